@@ -609,7 +609,7 @@ def sub_attention(dev, out):
                                            "algorithmic_gflop": round(fl8 / 1e9, 2)}
     ms = ev_time(lambda: pshattn.buck_swin_bwd(q, k, v, o, d_o, lse, dlt, dq, dk, dv, sc8, BS), 10)
     out["attention_scope8_4096_tokens_backward"] = {
-        "kernel": "bwd_delta_kernel<32> + bwd_dkdv_stream_kernel<32> + bwd_dq_stream_kernel<32>", "ms": round(ms, 4),
+        "kernel": "bwd_dq_kernel<32> + bwd_dkdv_kernel<32, 2>", "ms": round(ms, 4),
         "tflops": round(2.5 * fl8 / ms / 1e9, 2),
         "frac_of_bf16_mfma_peak": round(2.5 * fl8 / ms / 1e9 / MFMA_BF16_PEAK_TFLOPS, 4),
         "algorithmic_gflop": round(2.5 * fl8 / 1e9, 2)}

@@ -412,6 +412,31 @@ def test_backward_with_valid_lengths(oracle):
                 assert not t[:, b * bs + n:(b + 1) * bs].any(), f"bucket {b}: gradient on a masked row"
 
 
+@pytest.mark.parametrize("H,D,bs,scope_size,n_scope,lens", [
+    (8, 32, 128, 2, 32, None),                  # 64 keys a wave: one workgroup per (scope, head), 256 workgroups
+    (4, 16, 256, 2, 32, (1, 63, 64, 65, 0)),    # ... 16-wide heads, valid lengths around a 64-row tile
+    (5, 32, 384, 2, 18, (384, 32, 33, 127)),    # ... three workgroups per item, no multiple of eight units
+    (8, 32, 128, 1, 40, (128, 31, 0, 97)),      # scopes of 128 rows: 32 keys a wave
+    (1, 32, 512, 3, 2, (512, 1, 480)),          # few workgroups: 32 keys a wave
+    (2, 64, 256, 2, 3, (256, 40, 200)),
+    (2, 128, 128, 3, 2, (100, 128, 0)),         # 32-row tiles
+])
+def test_backward_key_split_and_tile_edges(oracle, H, D, bs, scope_size, n_scope, lens):
+    """both key counts per wave of the dK / dV kernel, bucket ends inside and at the edges of its tiles, permuted buckets"""
+    L = bs * scope_size * n_scope
+    Q, K, V = _qkv(17 + D + bs, 1, L, H, D)
+    dO = torch.randn(1, L, H, D, generator=torch.Generator().manual_seed(21)).to(torch.bfloat16)
+    scopes = np.random.default_rng(5).permuted(oracle.gen_scopes(L, bs, scope_size), axis=1)
+    kl = None if lens is None else np.resize(np.asarray(lens), L // bs)
+    dq, dk, dv, delta, O = _run_bwd(Q, K, V, dO, scopes, bs, kv_len=kl)
+    wq, wk, wv, wdelta = oracle.buck_swin_bwd(Q, K, V, dO, scopes, bs, kv_len=kl)
+    _check_grads((dq, dk, dv), (wq, wk, wv), f"H={H} D={D} bs={bs} scope={scope_size}")
+    # Delta of the library's own O: fp32 sums of D products, each below 64 here
+    assert (delta - (O * dO.float()).sum(-1)).abs().max().item() <= 2 * D * 2.0 ** -24 * 64
+    for b, n in enumerate(() if kl is None else kl):
+        assert not any(t[:, b * bs + n:(b + 1) * bs].any() for t in (dq, dk, dv)), f"bucket {b}: gradient on a masked row"
+
+
 def test_streaming_backward_more_than_65535_items(oracle):
     """8,192 one-bucket scopes of 128 tokens x 8 heads = 65,536 (batch, scope, head) items, one more than a launch's
     grid.y holds: the forward takes them in one launch, the backward in two.  Gradients of scopes at both ends of the
