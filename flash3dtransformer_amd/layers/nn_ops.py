@@ -381,8 +381,6 @@ class Linear(_CachedParamModule):
                                  tag=("ln", float(pre_norm.eps)))
             pshattn.ln_linear_bf16(x2, g, b, pre_norm.eps, w16, b16, r2, y, act)
         else:
-            if self.in_features > 512:     # long inner dimension: the output-panel kernel re-lays the weight
-                self._staged.arm(self.training, self.out_features, self.in_features, w16, b16, tag="ys")
             pshattn.linear_bf16(x2, w16, b16, r2, y, act)
         ln_w = None if pre_norm is None else pre_norm.weight
         ln_b = None if pre_norm is None else pre_norm.bias

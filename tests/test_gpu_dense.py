@@ -498,3 +498,32 @@ def test_staged_weights_are_reused_and_refreshed():
     with pytest.raises(RuntimeError, match="f3d_stage_weights"):
         pshattn.ln_linear_bf16(x[:64], g, g, 1e-5, w, None, None, y, None)
     pshattn.ln_linear_bf16(x[:64], g, g, 1e-5, w, None, None, y, None)     # the staging ended with the failed call
+
+
+@pytest.mark.parametrize("M,N,K,use_bias,use_res", [
+    (1, 128, 192, True, True),          # 128 x 128 panels: one row, the shortest inner dimension
+    (129, 384, 640, False, True),       # ... a second row panel of one row, three column panels, no bias
+    (9001, 512, 704, True, False),      # 256 x 128 panels, a ragged last row panel
+    (17001, 512, 576, True, True),      # 256 x 256 panels
+    (65537, 128, 1024, True, True),     # 256 x 128 panels, more than one round of the chip
+])
+def test_output_panel_linear_forms(M, N, K, use_bias, use_res):
+    """each panel form of the output-panel kernel at ragged row counts, with strided rows of x, residual and y"""
+    from flash3dtransformer_amd.lib import pshattn
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    rand = lambda *s: torch.randn(*s, device=DEV, generator=g).to(torch.bfloat16)
+    x, w = rand(M, K + 64)[:, :K], rand(N, K) * K ** -0.5
+    b, r = rand(N) if use_bias else None, rand(M, N + 8)[:, :N] if use_res else None
+    wide = torch.full((M + 3, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    y = wide[:M, :N]
+    pshattn.linear_bf16(x, w, b, r, y, None)
+    torch.cuda.synchronize()
+    z = x.double() @ w.double().t()
+    z = z if b is None else z + b.double()
+    want = z if r is None else z + r.double()
+    # the product and the sum are each rounded to bf16 (7 fraction bits: up to 2^-8 of their size, of the rounded product's
+    # too), after K fp32 additions of terms whose magnitudes sum to at most |x| |w|
+    acc = K * 2.0 ** -24 * (x.double().norm(dim=1, keepdim=True) * w.double().norm(dim=1))
+    bound = 2.0 ** -8 * (1 + 2.0 ** -8) * (z.abs() + (0 if r is None else want.abs())) + acc
+    assert ((y.double() - want).abs() <= bound).all()
+    assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()
