@@ -108,7 +108,7 @@ class _Bf16Cache:
         if training or torch.is_grad_enabled():
             self.clear()
             return p.detach().to(torch.bfloat16).contiguous()
-        key = (p.data_ptr(), p._version, p.dtype, p.device)
+        key = (p.data_ptr(), p._version, p.dtype, p.get_device())
         if key != self._key:
             self._val = p.detach().to(torch.bfloat16).contiguous()
             self._key = key
@@ -136,11 +136,10 @@ class _StagedWeights:
             self.clear()
             return
         live = [t for t in tensors if t is not None]
-        key = (tag, rows, cols) + tuple((t.data_ptr(), t._version, tuple(t.shape)) for t in live)
+        key = (tag, rows, cols) + tuple([(t.data_ptr(), t._version, t.shape) for t in live])
         need = 3 * rows * cols + 4 * rows + 2 * cols + 512
-        dev = live[0].device
-        if self._buf is None or self._buf.numel() < need or self._buf.device != dev:
-            self._buf = torch.empty(need, dtype=torch.uint8, device=dev)
+        if self._buf is None or self._buf.numel() < need or self._buf.get_device() != live[0].get_device():
+            self._buf = torch.empty(need, dtype=torch.uint8, device=live[0].device)
             self._key = None
         ready = key == self._key
         pshattn.stage_weights(self._buf, ready)

@@ -19,7 +19,55 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "libf3d_hip.so")
 _lib = None
 
-_u32, _i32, _f32, _vp = ctypes.c_uint32, ctypes.c_int, ctypes.c_float, ctypes.c_void_p
+_CTYPE = {"p": ctypes.c_void_p, "u": ctypes.c_uint32, "i": ctypes.c_int, "f": ctypes.c_float, "Q": ctypes.c_size_t}
+# argument kinds of every C entry point (include/f3d_hip.h): declared once, so that a call passes plain integers and ctypes
+# converts them in C instead of the call building an object for each of its 10 to 25 arguments
+_SIGNATURES = {
+    "f3d_last_error": "",
+    "f3d_init_dev_info": "i",
+    "f3d_set_sync_stream": "i",
+    "f3d_get_sync_stream": "",
+    "f3d_set_seed": "u",
+    "f3d_get_seed": "",
+    "f3d_batch_psh_scatter_pad_hash": "pppppuuuuuuupppppufuip",
+    "f3d_batch_psh_scatter_pad_hash_noalloc": "pppppuuuuuuupppppufuip",
+    "f3d_set_psh_rebalance": "i",
+    "f3d_get_psh_rebalance": "",
+    "f3d_set_quantiser": "i",
+    "f3d_get_quantiser": "",
+    "f3d_coord_bbox": "puppip",
+    "f3d_batch_subbuck_reduce": "pppuuuuuupppppppupuuuip",
+    "f3d_subbuck_build": "ppuuuuuppppupuip",
+    "f3d_reduce_feat": "puupuuupuip",
+    "f3d_reduce_feat_norm": "puupuuupuuppppfuip",
+    "f3d_additive_unpool_fwd": "ppppuuuuip",
+    "f3d_additive_unpool_norm_fwd": "ppppuuuuuppppfppppfuip",
+    "f3d_psh_scatter_feat_index": "pppppuuupuppuip",
+    "f3d_permute_rows": "pppuuuuip",
+    "f3d_additive_unpool_bwd": "ppppuuuuip",
+    "f3d_subbuck_reduce_bwd": "ppppuuuuuip",
+    "f3d_buck_swin_bwd": "pppuppppppppuuuuuuupip",
+    "f3d_buck_swin_bwd_strided": "pppupppppppupuuuuuuupip",
+    "f3d_buck_swin_fwd": "ppppppuuuuuuupip",
+    "f3d_buck_swin_fwd_strided": "pppupppuuuuuuupip",
+    "f3d_stage_weights": "pQi",
+    "f3d_gemm_sm_bf16": "pppuuuip",
+    "f3d_linear_bf16": "pupppupuuuuuip",
+    "f3d_ln_linear_bf16": "puppfpppupuuuuuip",
+    "f3d_ln_mlp_swiglu_bf16": "puppfpppppupuuuuip",
+    "f3d_proj_ln_mlp_swiglu_bf16": "pupppuppfpppppuuuuip",
+    "f3d_embed_proj_ln_mlp_swiglu_bf16": "puppppppfpppppuuuuip",
+    "f3d_embed_qkv_fold_bf16": "ppppfppuuuppip",
+    "f3d_embed_buck_swin_fwd": "ppppppuuuuuuuip",
+    "f3d_layernorm_bf16": "ppppuufip",
+    "f3d_coord_embed_bf16": "ppppuuip",
+    "f3d_embed_ln_linear_bf16": "ppppfpppuuuuip",
+    "f3d_affine_act_bf16": "ppppuuuip",
+    "f3d_linear_wgrad_bf16": "pupuppuuuuip",
+    "f3d_layernorm_bwd_bf16": "pupuppupuppuufuip",
+    "f3d_swiglu_bwd_bf16": "pupupupuuuip",
+    "f3d_mlp_gate_bwd_bf16": "pupuppppupuuuuip",
+}
 
 
 def _load():
@@ -29,9 +77,12 @@ def _load():
             raise RuntimeError(
                 f"{_LIB_PATH} is missing: build it with `python -m flash3dtransformer_amd.csrc.build` "
                 "(hipcc, gfx950). There is no CPU fallback for the Flash3D ops.")
-        _lib = ctypes.CDLL(_LIB_PATH)
-        _lib.f3d_last_error.restype = ctypes.c_char_p
-        _lib.f3d_get_seed.restype = ctypes.c_uint32
+        lib = ctypes.CDLL(_LIB_PATH)
+        for name, kinds in _SIGNATURES.items():
+            getattr(lib, name).argtypes = [_CTYPE[c] for c in kinds]
+        lib.f3d_last_error.restype = ctypes.c_char_p
+        lib.f3d_get_seed.restype = ctypes.c_uint32
+        _lib = lib
     return _lib
 
 
@@ -45,11 +96,11 @@ def _check(rc: int):
 
 
 def _ptr(t):
-    return _vp(t.data_ptr()) if t is not None else _vp(0)
+    return t.data_ptr() if t is not None else None
 
 
-def _stream(dev_index: int):
-    return _vp(torch.cuda.current_stream(dev_index).cuda_stream)
+# the current stream's handle without a torch.cuda.Stream object around it
+_stream = torch._C._cuda_getCurrentRawStream
 
 
 def assert_contiguous(tensors):
@@ -60,18 +111,22 @@ def assert_contiguous(tensors):
 
 
 def assert_same_device(tensors):
+    index = tensors[0].get_device()
+    for t in tensors:
+        if t.get_device() != index or not t.is_cuda:
+            break
+    else:
+        return index
     dev = tensors[0].device
     for i, t in enumerate(tensors):
         if t.device != dev:
             raise RuntimeError(f"Tensor #{i} is on {t.device}, expected {dev}.")
-    if dev.type != "cuda":
-        raise RuntimeError(f"Flash3D ops need tensors on a GPU device, got {dev}.")
-    return dev.index if dev.index is not None else torch.cuda.current_device()
+    raise RuntimeError(f"Flash3D ops need tensors on a GPU device, got {dev}.")
 
 
 def assert_dtype(tensors, dtype):
     for i, t in enumerate(tensors):
-        if t.dtype != dtype:
+        if t.dtype is not dtype:
             raise RuntimeError(f"Tensor #{i} has dtype {t.dtype}, expected {dtype}.")
 
 
@@ -95,26 +150,26 @@ class DeviceManagerSingleton:
         return DeviceManagerSingleton._inst
 
     def init_dev_info(self, dev_id: int):
-        _check(_load().f3d_init_dev_info(_i32(dev_id)))
+        _check(_load().f3d_init_dev_info(dev_id))
 
     def init_dispatchers(self):
         _load()  # kernels are selected at call time; loading the library is all there is to do
 
     def set_sync_stream(self, is_syncing: bool) -> bool:
-        return bool(_load().f3d_set_sync_stream(_i32(1 if is_syncing else 0)))
+        return bool(_load().f3d_set_sync_stream(1 if is_syncing else 0))
 
     def get_sync_stream(self) -> bool:
         return bool(_load().f3d_get_sync_stream())
 
     # extensions -----------------------------------------------------------------------------
     def set_seed(self, seed: int):
-        _check(_load().f3d_set_seed(_u32(seed)))
+        _check(_load().f3d_set_seed(seed))
 
     def get_seed(self) -> int:
         return int(_load().f3d_get_seed())
 
     def set_psh_rebalance(self, mode: int):
-        _check(_load().f3d_set_psh_rebalance(_i32(mode)))
+        _check(_load().f3d_set_psh_rebalance(mode))
 
     def get_psh_rebalance(self) -> int:
         return int(_load().f3d_get_psh_rebalance())
@@ -122,7 +177,7 @@ class DeviceManagerSingleton:
     def set_quantiser(self, mode: int):
         """0: quotient of the voxel quantiser as a multiply by the rounded reciprocal (a fast-math build of the
         reference, default); 1: IEEE division (src/psh/hash_fns.cuh:23-33 as written)"""
-        _check(_load().f3d_set_quantiser(_i32(mode)))
+        _check(_load().f3d_set_quantiser(mode))
 
     def get_quantiser(self) -> int:
         return int(_load().f3d_get_quantiser())
@@ -150,10 +205,10 @@ def batch_psh_scatter_pad_hash(coord, bucket_id, bucket_counter, bucket_offset, 
     fn = _load().f3d_batch_psh_scatter_pad_hash_noalloc if no_alloc else _load().f3d_batch_psh_scatter_pad_hash
     _check(fn(
         _ptr(coord), _ptr(bucket_id), _ptr(bucket_counter), _ptr(bucket_offset), _ptr(batch_sep),
-        _u32(batch_sep.shape[0]), _u32(coord.shape[0]), _u32(instance_max_N), _u32(num_bucket),
-        _u32(bucket_divisor), _u32(bucket_size), _u32(num_vox), _ptr(bbox_min), _ptr(bbox_max),
-        _ptr(probe_offsets), _ptr(cumsum_counter), _ptr(scatter_coord), _u32(scatter_coord.shape[0]),
-        _f32(pad_num), _u32(hash_type), _i32(dev), _stream(dev)))
+        batch_sep.shape[0], coord.shape[0], instance_max_N, num_bucket,
+        bucket_divisor, bucket_size, num_vox, _ptr(bbox_min), _ptr(bbox_max),
+        _ptr(probe_offsets), _ptr(cumsum_counter), _ptr(scatter_coord), scatter_coord.shape[0],
+        pad_num, hash_type, dev, _stream(dev)))
 
 
 def batch_psh_scatter_pad(coord, bucket_id, bucket_counter, bucket_offset, batch_sep, instance_max_N,
@@ -209,9 +264,9 @@ def psh_scatter_feat_index(bucket_id, bucket_counter, bucket_offset, batch_sep, 
     row_bytes = 0 if feat is None else _row_bytes(feat)
     _check(_load().f3d_psh_scatter_feat_index(
         _ptr(bucket_id), _ptr(bucket_offset), _ptr(bucket_counter), _ptr(cumsum_counter), _ptr(batch_sep),
-        _u32(batch_sep.shape[0]), _u32(bucket_id.shape[0]), _u32(bucket_counter.shape[1]),
-        _ptr(feat), _u32(row_bytes), _ptr(scatter_idx_out2in), _ptr(scattered_feat),
-        _u32(scatter_idx_out2in.shape[0]), _i32(dev), _stream(dev)))
+        batch_sep.shape[0], bucket_id.shape[0], bucket_counter.shape[1],
+        _ptr(feat), row_bytes, _ptr(scatter_idx_out2in), _ptr(scattered_feat),
+        scatter_idx_out2in.shape[0], dev, _stream(dev)))
 
 
 def permute_rows(index, src, dst, gather: bool):
@@ -233,8 +288,8 @@ def permute_rows(index, src, dst, gather: bool):
         if gather:
             dst.zero_()
         return
-    _check(_load().f3d_permute_rows(_ptr(index), _ptr(src), _ptr(dst), _u32(n_index), _u32(n_other),
-                                    _u32(_row_bytes(src)), _u32(1 if gather else 0), _i32(dev),
+    _check(_load().f3d_permute_rows(_ptr(index), _ptr(src), _ptr(dst), n_index, n_other,
+                                    _row_bytes(src), 1 if gather else 0, dev,
                                     _stream(dev)))
 
 
@@ -243,7 +298,7 @@ def coord_bbox(coord, bbox_min, bbox_max):
     assert_contiguous([coord, bbox_min, bbox_max])
     dev = assert_same_device([coord, bbox_min, bbox_max])
     assert_dtype([coord, bbox_min, bbox_max], torch.float16)
-    _check(_load().f3d_coord_bbox(_ptr(coord), _u32(coord.shape[0]), _ptr(bbox_min), _ptr(bbox_max), _i32(dev),
+    _check(_load().f3d_coord_bbox(_ptr(coord), coord.shape[0], _ptr(bbox_min), _ptr(bbox_max), dev,
                                   _stream(dev)))
 
 
@@ -311,11 +366,11 @@ def batch_subbuck_reduce(scattered_coord, scattered_feat, batch_sep, instance_ma
     # Rows of the feature tensor beyond the coordinate count are ignored, as in the reference
     # (total_N is taken from the coordinates, dispatcher :43).
     _check(_load().f3d_batch_subbuck_reduce(
-        _ptr(scattered_coord), _ptr(scattered_feat), _ptr(batch_sep), _u32(batch_sep.shape[0]),
-        _u32(scattered_coord.shape[0]), _u32(instance_max_N), _u32(scattered_feat.shape[1]), _u32(subbuck_size),
-        _u32(num_vox), _ptr(bbox_min.contiguous()), _ptr(bbox_max.contiguous()), _ptr(subbuck_id), _ptr(subbuck_off),
-        _ptr(reduced_batch_sep), _ptr(reduced_coord), _ptr(reduced_feat), _u32(reduced_feat.shape[0]),
-        _ptr(unpool_ind), _u32(unpool_ind.shape[0]), _u32(hash_type), _u32(red_op), _i32(dev), _stream(dev)))
+        _ptr(scattered_coord), _ptr(scattered_feat), _ptr(batch_sep), batch_sep.shape[0],
+        scattered_coord.shape[0], instance_max_N, scattered_feat.shape[1], subbuck_size,
+        num_vox, _ptr(bbox_min.contiguous()), _ptr(bbox_max.contiguous()), _ptr(subbuck_id), _ptr(subbuck_off),
+        _ptr(reduced_batch_sep), _ptr(reduced_coord), _ptr(reduced_feat), reduced_feat.shape[0],
+        _ptr(unpool_ind), unpool_ind.shape[0], hash_type, red_op, dev, _stream(dev)))
 
 
 def batch_subbuck_reduce_backward(grad_red_feat, input_feat, unpool_ind, grad_input_feat, subbuck_size, red_op):
@@ -334,8 +389,8 @@ def batch_subbuck_reduce_backward(grad_red_feat, input_feat, unpool_ind, grad_in
     if unpool_ind.shape[1] != subbuck_size:
         raise RuntimeError(f"unpool_ind width {unpool_ind.shape[1]} != subbuck_size {subbuck_size}")
     _check(_load().f3d_subbuck_reduce_bwd(
-        _ptr(grad_red_feat), _ptr(input_feat), _ptr(unpool_ind), _ptr(grad_input_feat), _u32(input_feat.shape[0]),
-        _u32(unpool_ind.shape[0]), _u32(input_feat.shape[1]), _u32(subbuck_size), _u32(red_op), _i32(dev), _stream(dev)))
+        _ptr(grad_red_feat), _ptr(input_feat), _ptr(unpool_ind), _ptr(grad_input_feat), input_feat.shape[0],
+        unpool_ind.shape[0], input_feat.shape[1], subbuck_size, red_op, dev, _stream(dev)))
 
 
 def additive_unpool_fwd(res_feat, down_feat, up_add_feat, unpool_ind, subbuck_size):
@@ -354,8 +409,8 @@ def additive_unpool_fwd(res_feat, down_feat, up_add_feat, unpool_ind, subbuck_si
     if down_feat.shape[0] < unpool_ind.shape[0]:
         raise RuntimeError(f"down_feat has {down_feat.shape[0]} rows, unpool_ind needs {unpool_ind.shape[0]}")
     _check(_load().f3d_additive_unpool_fwd(
-        _ptr(res_feat), _ptr(down_feat), _ptr(up_add_feat), _ptr(unpool_ind), _u32(res_feat.shape[0]),
-        _u32(unpool_ind.shape[0]), _u32(res_feat.shape[1]), _u32(subbuck_size), _i32(dev), _stream(dev)))
+        _ptr(res_feat), _ptr(down_feat), _ptr(up_add_feat), _ptr(unpool_ind), res_feat.shape[0],
+        unpool_ind.shape[0], res_feat.shape[1], subbuck_size, dev, _stream(dev)))
 
 
 ROW_NORM_LAYER, ROW_NORM_AFFINE = 1, 2
@@ -369,12 +424,12 @@ def _row_norm_args(norm, c):
         assert_dtype([g] + ([b] if b is not None else []), torch.bfloat16)
         if g.numel() != c or (b is not None and b.numel() != c):
             raise RuntimeError(f"LayerNorm parameters must hold {c} values")
-        return ROW_NORM_LAYER, [_ptr(g), _ptr(b), _vp(0), _vp(0), _f32(eps)]
+        return ROW_NORM_LAYER, [_ptr(g), _ptr(b), None, None, eps]
     _, sc, sh = norm
     assert_dtype([sc, sh], torch.float32)
     if sc.numel() != c or sh.numel() != c:
         raise RuntimeError(f"scale / shift must hold {c} values")
-    return ROW_NORM_AFFINE, [_vp(0), _vp(0), _ptr(sc), _ptr(sh), _f32(0.0)]
+    return ROW_NORM_AFFINE, [None, None, _ptr(sc), _ptr(sh), 0.0]
 
 
 def subbuck_build(scattered_coord, batch_sep, instance_max_N, subbuck_size, num_vox, subbuck_id, subbuck_off,
@@ -393,10 +448,10 @@ def subbuck_build(scattered_coord, batch_sep, instance_max_N, subbuck_size, num_
     if unpool_ind.shape[1] != subbuck_size:
         raise RuntimeError(f"Unpool_ind last dimension({unpool_ind.shape[1]}) != subbucket_size({subbuck_size})")
     _check(_load().f3d_subbuck_build(
-        _ptr(scattered_coord), _ptr(batch_sep), _u32(batch_sep.shape[0]), _u32(scattered_coord.shape[0]),
-        _u32(instance_max_N), _u32(subbuck_size), _u32(num_vox), _ptr(subbuck_id), _ptr(subbuck_off),
-        _ptr(reduced_batch_sep), _ptr(reduced_coord), _u32(reduced_coord.shape[0]), _ptr(unpool_ind),
-        _u32(unpool_ind.shape[0]), _i32(dev), _stream(dev)))
+        _ptr(scattered_coord), _ptr(batch_sep), batch_sep.shape[0], scattered_coord.shape[0],
+        instance_max_N, subbuck_size, num_vox, _ptr(subbuck_id), _ptr(subbuck_off),
+        _ptr(reduced_batch_sep), _ptr(reduced_coord), reduced_coord.shape[0], _ptr(unpool_ind),
+        unpool_ind.shape[0], dev, _stream(dev)))
 
 
 def reduce_feat_norm(feat, total_n, unpool_ind, reduced_feat, subbuck_size, red_op, norm, act=None):
@@ -417,8 +472,8 @@ def reduce_feat_norm(feat, total_n, unpool_ind, reduced_feat, subbuck_size, red_
     mode, nargs = _row_norm_args(norm, feat.shape[1])
     a = ACT[act] if not isinstance(act, int) else act
     _check(_load().f3d_reduce_feat_norm(
-        _ptr(feat), _u32(total_n), _u32(feat.shape[1]), _ptr(unpool_ind), _u32(unpool_ind.shape[0]), _u32(subbuck_size),
-        _u32(red_op), _ptr(reduced_feat), _u32(reduced_feat.shape[0]), _u32(mode), *nargs, _u32(a), _i32(dev),
+        _ptr(feat), total_n, feat.shape[1], _ptr(unpool_ind), unpool_ind.shape[0], subbuck_size,
+        red_op, _ptr(reduced_feat), reduced_feat.shape[0], mode, *nargs, a, dev,
         _stream(dev)))
 
 
@@ -445,8 +500,8 @@ def additive_unpool_norm_fwd(res_feat, down_feat, up_add_feat, unpool_ind, subbu
     _, da = _row_norm_args(norm_down, res_feat.shape[1])
     a = ACT[act] if not isinstance(act, int) else act
     _check(_load().f3d_additive_unpool_norm_fwd(
-        _ptr(res_feat), _ptr(down_feat), _ptr(up_add_feat), _ptr(unpool_ind), _u32(res_feat.shape[0]),
-        _u32(unpool_ind.shape[0]), _u32(res_feat.shape[1]), _u32(subbuck_size), _u32(mode), *ra, *da, _u32(a), _i32(dev),
+        _ptr(res_feat), _ptr(down_feat), _ptr(up_add_feat), _ptr(unpool_ind), res_feat.shape[0],
+        unpool_ind.shape[0], res_feat.shape[1], subbuck_size, mode, *ra, *da, a, dev,
         _stream(dev)))
 
 
@@ -466,8 +521,8 @@ def additive_unpool_bwd(grad_res, grad_down, grad_up_added, unpool_ind, subbuck_
     if unpool_ind.shape[1] != subbuck_size:
         raise RuntimeError(f"unpool_ind width {unpool_ind.shape[1]} != subbuck_size {subbuck_size}")
     _check(_load().f3d_additive_unpool_bwd(
-        _ptr(grad_res), _ptr(grad_down), _ptr(grad_up_added), _ptr(unpool_ind), _u32(grad_res.shape[0]),
-        _u32(unpool_ind.shape[0]), _u32(grad_res.shape[1]), _u32(subbuck_size), _i32(dev), _stream(dev)))
+        _ptr(grad_res), _ptr(grad_down), _ptr(grad_up_added), _ptr(unpool_ind), grad_res.shape[0],
+        unpool_ind.shape[0], grad_res.shape[1], subbuck_size, dev, _stream(dev)))
 
 
 # ---------------------------------------------------------------------------------------------
@@ -499,9 +554,9 @@ def buck_swin_fwd(Q, K, V, O, L, Scope_buckets, bucket_size, kv_len=None):
         assert_dtype([kv_len], torch.int32)
         assert_contiguous([kv_len])
     _check(_load().f3d_buck_swin_fwd_strided(
-        _ptr(Q), _ptr(K), _ptr(V), _u32(Q.stride(1)), _ptr(O), _ptr(L), _ptr(Scope_buckets),
-        _u32(Scope_buckets.shape[0]), _u32(Scope_buckets.shape[1]), _u32(bucket_size), _u32(B), _u32(Ls), _u32(H),
-        _u32(D), _ptr(kv_len), _i32(dev), _stream(dev)))
+        _ptr(Q), _ptr(K), _ptr(V), Q.stride(1), _ptr(O), _ptr(L), _ptr(Scope_buckets),
+        Scope_buckets.shape[0], Scope_buckets.shape[1], bucket_size, B, Ls, H,
+        D, _ptr(kv_len), dev, _stream(dev)))
 
 
 def buck_swin_bwd(Q, K, V, O, dO, LSE, Delta, dQ, dK, dV, Scope_buckets, bucket_size, kv_len=None):
@@ -536,9 +591,9 @@ def buck_swin_bwd(Q, K, V, O, dO, LSE, Delta, dQ, dK, dV, Scope_buckets, bucket_
         if t.stride(3) != 1 or t.stride(2) != D or t.stride(0) != t.stride(1) * Ls or t.stride() != dQ.stride():
             raise RuntimeError("dQ/dK/dV must be dense over (H, D) with identical strides")
     rc = _load().f3d_buck_swin_bwd_strided(
-        _ptr(Q), _ptr(K), _ptr(V), _u32(Q.stride(1)), _ptr(O), _ptr(dO), _ptr(LSE), _ptr(Delta), _ptr(dQ), _ptr(dK),
-        _ptr(dV), _u32(dQ.stride(1)), _ptr(Scope_buckets), _u32(Scope_buckets.shape[0]), _u32(Scope_buckets.shape[1]), _u32(bucket_size),
-        _u32(B), _u32(Ls), _u32(H), _u32(D), _ptr(kv_len), _i32(dev), _stream(dev))
+        _ptr(Q), _ptr(K), _ptr(V), Q.stride(1), _ptr(O), _ptr(dO), _ptr(LSE), _ptr(Delta), _ptr(dQ), _ptr(dK),
+        _ptr(dV), dQ.stride(1), _ptr(Scope_buckets), Scope_buckets.shape[0], Scope_buckets.shape[1], bucket_size,
+        B, Ls, H, D, _ptr(kv_len), dev, _stream(dev))
     if rc == 2:   # F3D_ERR_UNSUPPORTED: a shape outside the backward kernels
         raise NotImplementedError(_load().f3d_last_error().decode("utf-8", "replace"))
     _check(rc)
@@ -557,7 +612,7 @@ def gemm_sm_bf16(A, B, O):
     K2, N = B.shape
     if K != K2 or tuple(O.shape) != (M, N):
         raise RuntimeError(f"gemm shape mismatch: A{tuple(A.shape)} B{tuple(B.shape)} O{tuple(O.shape)}")
-    _check(_load().f3d_gemm_sm_bf16(_ptr(A), _ptr(B), _ptr(O), _u32(M), _u32(N), _u32(K), _i32(dev), _stream(dev)))
+    _check(_load().f3d_gemm_sm_bf16(_ptr(A), _ptr(B), _ptr(O), M, N, K, dev, _stream(dev)))
     torch.cuda.current_stream(dev).synchronize()  # the reference op always synchronises (gemm_dispatcher.cu:77)
 
 
@@ -585,8 +640,8 @@ def linear_bf16(x, w, bias, residual, y, act=None):
         if tuple(residual.shape) != (m, n_out) or residual.stride(1) != 1:
             raise RuntimeError("residual must be [m, n_out] row-major")
         ldr = residual.stride(0)
-    _check(_load().f3d_linear_bf16(_ptr(x), _u32(x.stride(0)), _ptr(w), _ptr(bias), _ptr(residual), _u32(ldr),
-                                   _ptr(y), _u32(y.stride(0)), _u32(m), _u32(n), _u32(k), _u32(a), _i32(dev),
+    _check(_load().f3d_linear_bf16(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), _ptr(residual), ldr,
+                                   _ptr(y), y.stride(0), m, n, k, a, dev,
                                    _stream(dev)))
 
 
@@ -611,9 +666,9 @@ def ln_linear_bf16(x, gamma, beta, eps, w, bias, residual, y, act=None):
         if tuple(residual.shape) != (m, n_out) or residual.stride(1) != 1:
             raise RuntimeError("residual must be [m, n_out] row-major")
         ldr = residual.stride(0)
-    _check(_load().f3d_ln_linear_bf16(_ptr(x), _u32(x.stride(0)), _ptr(gamma), _ptr(beta), _f32(eps), _ptr(w),
-                                      _ptr(bias), _ptr(residual), _u32(ldr), _ptr(y), _u32(y.stride(0)), _u32(m),
-                                      _u32(n), _u32(k), _u32(a), _i32(dev), _stream(dev)))
+    _check(_load().f3d_ln_linear_bf16(_ptr(x), x.stride(0), _ptr(gamma), _ptr(beta), eps, _ptr(w),
+                                      _ptr(bias), _ptr(residual), ldr, _ptr(y), y.stride(0), m,
+                                      n, k, a, dev, _stream(dev)))
 
 
 def ln_mlp_swiglu_bf16(x, gamma, beta, eps, w1, b1, w2, b2, residual, y) -> bool:
@@ -637,9 +692,9 @@ def ln_mlp_swiglu_bf16(x, gamma, beta, eps, w1, b1, w2, b2, residual, y) -> bool
         if tuple(residual.shape) != (m, c) or residual.stride(1) != 1:
             raise RuntimeError("residual must be [m, c] row-major")
         ldr = residual.stride(0)
-    rc = _load().f3d_ln_mlp_swiglu_bf16(_ptr(x), _u32(x.stride(0)), _ptr(gamma), _ptr(beta), _f32(eps), _ptr(w1),
-                                        _ptr(b1), _ptr(w2), _ptr(b2), _ptr(residual), _u32(ldr), _ptr(y),
-                                        _u32(y.stride(0)), _u32(m), _u32(c), _u32(hidden), _i32(dev), _stream(dev))
+    rc = _load().f3d_ln_mlp_swiglu_bf16(_ptr(x), x.stride(0), _ptr(gamma), _ptr(beta), eps, _ptr(w1),
+                                        _ptr(b1), _ptr(w2), _ptr(b2), _ptr(residual), ldr, _ptr(y),
+                                        y.stride(0), m, c, hidden, dev, _stream(dev))
     if rc == 2:
         return False
     _check(rc)
@@ -672,8 +727,8 @@ def embed_ln_linear_bf16(coord, table, gamma, beta, eps, w, bias, y) -> bool:
             or tuple(y.shape) != (m, n) or y.stride(1) != 1):
         raise RuntimeError(f"embed_ln_linear shape mismatch: coord{tuple(coord.shape)} table{tuple(table.shape)} "
                            f"w{tuple(w.shape)} y{tuple(y.shape)}")
-    rc = _load().f3d_embed_ln_linear_bf16(_ptr(coord), _ptr(table), _ptr(gamma), _ptr(beta), _f32(eps), _ptr(w), _ptr(bias),
-                                          _ptr(y), _u32(y.stride(0)), _u32(m), _u32(n), _u32(k), _i32(dev), _stream(dev))
+    rc = _load().f3d_embed_ln_linear_bf16(_ptr(coord), _ptr(table), _ptr(gamma), _ptr(beta), eps, _ptr(w), _ptr(bias),
+                                          _ptr(y), y.stride(0), m, n, k, dev, _stream(dev))
     if rc == 2:
         return False
     _check(rc)
@@ -699,9 +754,9 @@ def embed_qkv_fold(embed_w, embed_b, gamma, beta, eps, w_qkv, b_qkv, num_heads: 
                 raise RuntimeError("embed_qkv_fold: bias / beta length mismatch")
     table = torch.empty(num_heads, 4, 32, 16, dtype=torch.bfloat16, device=embed_w.device)
     chol = torch.empty(16, dtype=torch.float32, device=embed_w.device)
-    rc = _load().f3d_embed_qkv_fold_bf16(_ptr(embed_w), _ptr(embed_b), _ptr(gamma), _ptr(beta), _f32(eps), _ptr(w_qkv),
-                                         _ptr(b_qkv), _u32(c), _u32(num_heads), _u32(c // num_heads), _ptr(table),
-                                         _ptr(chol), _i32(dev), _stream(dev))
+    rc = _load().f3d_embed_qkv_fold_bf16(_ptr(embed_w), _ptr(embed_b), _ptr(gamma), _ptr(beta), eps, _ptr(w_qkv),
+                                         _ptr(b_qkv), c, num_heads, c // num_heads, _ptr(table),
+                                         _ptr(chol), dev, _stream(dev))
     if rc == 2:
         return None
     _check(rc)
@@ -727,8 +782,8 @@ def embed_buck_swin_fwd(coord, table, chol, O, L, Scope_buckets, bucket_size) ->
         raise RuntimeError(f"embed_buck_swin_fwd shape mismatch: coord{tuple(coord.shape)} table{tuple(table.shape)} "
                            f"O{tuple(O.shape)} L{tuple(L.shape)}")
     rc = _load().f3d_embed_buck_swin_fwd(_ptr(coord), _ptr(table), _ptr(chol), _ptr(O), _ptr(L), _ptr(Scope_buckets),
-                                         _u32(Scope_buckets.shape[0]), _u32(Scope_buckets.shape[1]), _u32(bucket_size),
-                                         _u32(B), _u32(Ls), _u32(H), _u32(D), _i32(dev), _stream(dev))
+                                         Scope_buckets.shape[0], Scope_buckets.shape[1], bucket_size,
+                                         B, Ls, H, D, dev, _stream(dev))
     if rc == 2:
         return False
     _check(rc)
@@ -751,10 +806,10 @@ def proj_ln_mlp_swiglu_bf16(a, w_proj, b_proj, x, gamma, beta, eps, w1, b1, w2, 
             or tuple(y.shape) != (m, c) or gamma.shape[0] != c):
         raise RuntimeError(f"proj_ln_mlp shape mismatch: a{tuple(a.shape)} x{tuple(x.shape)} w_proj{tuple(w_proj.shape)} "
                            f"w1{tuple(w1.shape)} w2{tuple(w2.shape)} y{tuple(y.shape)}")
-    rc = _load().f3d_proj_ln_mlp_swiglu_bf16(_ptr(a), _u32(a.stride(0)), _ptr(w_proj), _ptr(b_proj), _ptr(x),
-                                             _u32(x.stride(0)), _ptr(gamma), _ptr(beta), _f32(eps), _ptr(w1), _ptr(b1),
-                                             _ptr(w2), _ptr(b2), _ptr(y), _u32(y.stride(0)), _u32(m), _u32(c),
-                                             _u32(hidden), _i32(dev), _stream(dev))
+    rc = _load().f3d_proj_ln_mlp_swiglu_bf16(_ptr(a), a.stride(0), _ptr(w_proj), _ptr(b_proj), _ptr(x),
+                                             x.stride(0), _ptr(gamma), _ptr(beta), eps, _ptr(w1), _ptr(b1),
+                                             _ptr(w2), _ptr(b2), _ptr(y), y.stride(0), m, c,
+                                             hidden, dev, _stream(dev))
     if rc == 2:
         return False
     _check(rc)
@@ -779,10 +834,10 @@ def embed_proj_ln_mlp_swiglu_bf16(a, w_proj, b_proj, coord, table, gamma, beta, 
         raise RuntimeError(f"embed_proj_ln_mlp shape mismatch: a{tuple(a.shape)} coord{tuple(coord.shape)} "
                            f"table{tuple(table.shape)} w_proj{tuple(w_proj.shape)} w1{tuple(w1.shape)} w2{tuple(w2.shape)} "
                            f"y{tuple(y.shape)}")
-    rc = _load().f3d_embed_proj_ln_mlp_swiglu_bf16(_ptr(a), _u32(a.stride(0)), _ptr(w_proj), _ptr(b_proj), _ptr(coord),
-                                                   _ptr(table), _ptr(gamma), _ptr(beta), _f32(eps), _ptr(w1), _ptr(b1),
-                                                   _ptr(w2), _ptr(b2), _ptr(y), _u32(y.stride(0)), _u32(m), _u32(c),
-                                                   _u32(hidden), _i32(dev), _stream(dev))
+    rc = _load().f3d_embed_proj_ln_mlp_swiglu_bf16(_ptr(a), a.stride(0), _ptr(w_proj), _ptr(b_proj), _ptr(coord),
+                                                   _ptr(table), _ptr(gamma), _ptr(beta), eps, _ptr(w1), _ptr(b1),
+                                                   _ptr(w2), _ptr(b2), _ptr(y), y.stride(0), m, c,
+                                                   hidden, dev, _stream(dev))
     if rc == 2:
         return False
     _check(rc)
@@ -794,7 +849,7 @@ def stage_weights(buf: torch.Tensor, ready: bool):
     copies) in `buf` (uint8 device tensor, 256-byte aligned), or with `ready` reuses what an earlier call with the same
     weights left there and skips the preparation launch"""
     assert_dtype([buf], torch.uint8)
-    _check(_load().f3d_stage_weights(_ptr(buf), ctypes.c_size_t(buf.numel()), _i32(1 if ready else 0)))
+    _check(_load().f3d_stage_weights(_ptr(buf), buf.numel(), 1 if ready else 0))
 
 
 def layernorm_bf16(x, gamma, beta, y, eps=1e-5):
@@ -804,8 +859,8 @@ def layernorm_bf16(x, gamma, beta, y, eps=1e-5):
     assert_dtype([x, gamma, y], torch.bfloat16)
     _check_vectors(x, [beta])
     m, c = x.shape
-    _check(_load().f3d_layernorm_bf16(_ptr(x), _ptr(gamma), _ptr(beta), _ptr(y), _u32(m), _u32(c), _f32(eps),
-                                      _i32(dev), _stream(dev)))
+    _check(_load().f3d_layernorm_bf16(_ptr(x), _ptr(gamma), _ptr(beta), _ptr(y), m, c, eps,
+                                      dev, _stream(dev)))
 
 
 def _rows2d(ts, dtype=torch.bfloat16):
@@ -829,8 +884,8 @@ def linear_wgrad_bf16(dy, x, dw, db=None, accumulate=False):
         _check_vectors(dy, [db], torch.float32)
         if tuple(db.shape) != (n,):
             raise RuntimeError("db must be [n]")
-    _check(_load().f3d_linear_wgrad_bf16(_ptr(dy), _u32(dy.stride(0)), _ptr(x), _u32(x.stride(0)), _ptr(dw), _ptr(db),
-                                         _u32(m), _u32(n), _u32(k), _u32(1 if accumulate else 0), _i32(dev),
+    _check(_load().f3d_linear_wgrad_bf16(_ptr(dy), dy.stride(0), _ptr(x), x.stride(0), _ptr(dw), _ptr(db),
+                                         m, n, k, 1 if accumulate else 0, dev,
                                          _stream(dev)))
 
 
@@ -849,10 +904,10 @@ def layernorm_bwd_bf16(x, dh, gamma, dres, dx, dgamma, dbeta, eps=1e-5, accumula
             raise RuntimeError("layernorm_bwd: x, dh, dx, dres must share one shape")
     if tuple(gamma.shape) != (c,) or tuple(dgamma.shape) != (c,) or tuple(dbeta.shape) != (c,):
         raise RuntimeError("layernorm_bwd: gamma, dgamma, dbeta must be [c]")
-    rc = _load().f3d_layernorm_bwd_bf16(_ptr(x), _u32(x.stride(0)), _ptr(dh), _u32(dh.stride(0)), _ptr(gamma),
-                                        _ptr(dres), _u32(dres.stride(0) if dres is not None else 0), _ptr(dx),
-                                        _u32(dx.stride(0)), _ptr(dgamma), _ptr(dbeta), _u32(m), _u32(c), _f32(eps),
-                                        _u32(1 if accumulate else 0), _i32(dev), _stream(dev))
+    rc = _load().f3d_layernorm_bwd_bf16(_ptr(x), x.stride(0), _ptr(dh), dh.stride(0), _ptr(gamma),
+                                        _ptr(dres), dres.stride(0) if dres is not None else 0, _ptr(dx),
+                                        dx.stride(0), _ptr(dgamma), _ptr(dbeta), m, c, eps,
+                                        1 if accumulate else 0, dev, _stream(dev))
     if rc == 2:
         raise NotImplementedError(_load().f3d_last_error().decode("utf-8", "replace"))
     _check(rc)
@@ -865,9 +920,9 @@ def swiglu_bwd_bf16(z, da, dz, a=None):
     m, h = da.shape
     if tuple(z.shape) != (m, 2 * h) or tuple(dz.shape) != (m, 2 * h) or (a is not None and tuple(a.shape) != (m, h)):
         raise RuntimeError("swiglu_bwd shape mismatch")
-    _check(_load().f3d_swiglu_bwd_bf16(_ptr(z), _u32(z.stride(0)), _ptr(da), _u32(da.stride(0)), _ptr(dz),
-                                       _u32(dz.stride(0)), _ptr(a), _u32(a.stride(0) if a is not None else 0),
-                                       _u32(m), _u32(h), _i32(dev), _stream(dev)))
+    _check(_load().f3d_swiglu_bwd_bf16(_ptr(z), z.stride(0), _ptr(da), da.stride(0), _ptr(dz),
+                                       dz.stride(0), _ptr(a), a.stride(0) if a is not None else 0,
+                                       m, h, dev, _stream(dev)))
 
 
 def mlp_gate_bwd_bf16(h, dy, w1, b1, w2t, dz, a):
@@ -884,9 +939,9 @@ def mlp_gate_bwd_bf16(h, dy, w1, b1, w2t, dz, a):
     if tuple(dy.shape) != (m, c) or tuple(w1.shape) != (2 * hid, c) or tuple(w2t.shape) != (hid, c) \
             or tuple(dz.shape) != (m, 2 * hid) or tuple(a.shape) != (m, hid) or (b1 is not None and tuple(b1.shape) != (2 * hid,)):
         raise RuntimeError("mlp_gate_bwd shape mismatch")
-    rc = _load().f3d_mlp_gate_bwd_bf16(_ptr(h), _u32(h.stride(0)), _ptr(dy), _u32(dy.stride(0)), _ptr(w1), _ptr(b1),
-                                       _ptr(w2t), _ptr(dz), _u32(dz.stride(0)), _ptr(a), _u32(a.stride(0)), _u32(m),
-                                       _u32(c), _u32(hid), _i32(dev), _stream(dev))
+    rc = _load().f3d_mlp_gate_bwd_bf16(_ptr(h), h.stride(0), _ptr(dy), dy.stride(0), _ptr(w1), _ptr(b1),
+                                       _ptr(w2t), _ptr(dz), dz.stride(0), _ptr(a), a.stride(0), m,
+                                       c, hid, dev, _stream(dev))
     if rc == 2:
         return False
     _check(rc)
@@ -900,8 +955,8 @@ def coord_embed_bf16(coord, w, bias, y):
     assert_dtype([coord], torch.float16)
     assert_dtype([w, y], torch.bfloat16)
     _check_vectors(coord, [bias])
-    _check(_load().f3d_coord_embed_bf16(_ptr(coord), _ptr(w), _ptr(bias), _ptr(y), _u32(coord.shape[0]),
-                                        _u32(w.shape[0]), _i32(dev), _stream(dev)))
+    _check(_load().f3d_coord_embed_bf16(_ptr(coord), _ptr(w), _ptr(bias), _ptr(y), coord.shape[0],
+                                        w.shape[0], dev, _stream(dev)))
 
 
 def affine_act_bf16(x, scale, shift, y, act=None):
@@ -911,5 +966,5 @@ def affine_act_bf16(x, scale, shift, y, act=None):
     assert_dtype([x, y], torch.bfloat16)
     assert_dtype([scale, shift], torch.float32)
     a = ACT[act] if not isinstance(act, int) else act
-    _check(_load().f3d_affine_act_bf16(_ptr(x), _ptr(scale), _ptr(shift), _ptr(y), _u32(x.shape[0]),
-                                       _u32(x.shape[1]), _u32(a), _i32(dev), _stream(dev)))
+    _check(_load().f3d_affine_act_bf16(_ptr(x), _ptr(scale), _ptr(shift), _ptr(y), x.shape[0],
+                                       x.shape[1], a, dev, _stream(dev)))
