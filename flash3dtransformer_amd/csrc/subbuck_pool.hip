@@ -8,8 +8,12 @@
 // its own bounding box, keyed by the 13-bit z-order cell, and sorted by (cell, position) with an LDS
 // counting sort over the 8192 cells, as the reference does (shmem_cumsum_counter.cuh:25-167), made
 // deterministic: the atomic claim only yields a point's place inside its cell's run in arbitration
-// order; a second look at the run (almost always one or two points long) replaces it by the number of
-// run members that come earlier in the input.  Consecutive runs of S sorted points form a
+// order; a second look at the run replaces it by the number of run members that come earlier in the input.
+// In evenly spread points a run is one or two points long and its members are compared one by one.  In
+// LiDAR tiles hundreds of points share a cell (a few far points span the box); comparing them took up to
+// 60 us a tile, so runs of more than 32 points count through a bitmap of the tile's points: bucketed sweeps,
+// S = 2: 3 x 83k points 184 -> 32 us over three levels, 4 x 250k
+// 184 -> 61 us over four, 262,144 points at S = 8 41 -> 10 us.  Consecutive runs of S sorted points form a
 // sub-bucket.  Tile t owns output rows [t * tile_pts / S, ...) of its cloud, so no global counter
 // is needed.  Every output is a pure function of (coords, seps, S, seed).
 #include "f3d_device.h"
@@ -114,6 +118,12 @@ __global__ __launch_bounds__(kSubThreads) void subbuck_build_kernel(
   __shared__ uint16_t s_claim[kSubThreads];   // run position (arbitration order) -> point
   __shared__ uint16_t s_key[kSubThreads];     // rank (input order inside a run) -> point
   __shared__ uint32_t s_red[kWaves][3];       // per wave: packed keys of the minima and (complemented) maxima
+  // runs of more than kLongRun points: bit j of a run's bitmap = point j of the tile is a member; and the members before
+  // each 32-bit word.  Such runs start more than kLongRun ranks apart, so run start / (kLongRun + 1) numbers them.
+  constexpr uint32_t kLongRun = 32u, kMapWords = kSubThreads / 32u;
+  static_assert((kSubThreads / (kLongRun + 1u) + 1u) * kMapWords <= kSubThreads, "one bitmap word per thread");
+  __shared__ uint32_t s_map[kSubThreads];
+  __shared__ uint16_t s_map_pre[kSubThreads];
   __shared__ uint32_t s_wsum[kWaves];
   __shared__ float s_mat[9];                  // the tile's rotation
   __shared__ float s_bb[9];                   // min, max, 1 / (max - min) per axis
@@ -151,6 +161,7 @@ __global__ __launch_bounds__(kSubThreads) void subbuck_build_kernel(
   // thread t owns the counters of cells 8 t .. 8 t + 7 (four words) in the zero-fill and in the scan
   uint4* const my_cells = reinterpret_cast<uint4*>(s_cell) + tid;
   *my_cells = make_uint4(0u, 0u, 0u, 0u);
+  s_map[tid] = 0u;
   if (w == 0) {
     // the tile's rotation, once per workgroup
     float q[4], mat[9];
@@ -260,12 +271,27 @@ __global__ __launch_bounds__(kSubThreads) void subbuck_build_kernel(
   }
   __syncthreads();
   uint32_t run0 = 0, run1 = 0;
+  bool long_run = false;
+  uint32_t map0 = 0;
   if (valid) {
     run0 = (s_cell[cell >> 1] >> (16u * (cell & 1u))) & 0xFFFFu;
     run1 = (s_cell[(cell + 1u) >> 1] >> (16u * ((cell + 1u) & 1u))) & 0xFFFFu;
-    s_claim[run0 + claim] = (uint16_t)tid;
+    long_run = run1 - run0 > kLongRun;
+    map0 = run0 / (kLongRun + 1u) * kMapWords;
+    if (long_run) atomicOr(&s_map[map0 + tid / 32u], 1u << (tid % 32u));
+    else s_claim[run0 + claim] = (uint16_t)tid;
   }
-  __syncthreads();
+  if (__syncthreads_or(long_run)) {
+    const uint32_t mine = (uint32_t)__popc(s_map[tid]);
+    uint32_t incl = mine;
+#pragma unroll
+    for (int off = 1; off < (int)kMapWords; off <<= 1) {
+      const uint32_t up = __shfl_up(incl, off, kMapWords);
+      if (tid % kMapWords >= (uint32_t)off) incl += up;
+    }
+    s_map_pre[tid] = (uint16_t)(incl - mine);
+    __syncthreads();
+  }
   const uint32_t S = subbuck_size;
   const uint32_t rows_per_tile = tile_pts / S;
   const uint32_t row_base = rstart + tile * rows_per_tile;
@@ -274,7 +300,9 @@ __global__ __launch_bounds__(kSubThreads) void subbuck_build_kernel(
   if (valid) {
     // place inside the run = number of its members that come earlier in the input
     uint32_t before = 0;
-    if (run1 - run0 > 1u)
+    if (long_run)
+      before = s_map_pre[map0 + tid / 32u] + (uint32_t)__popc(s_map[map0 + tid / 32u] & ((1u << (tid % 32u)) - 1u));
+    else if (run1 - run0 > 1u)
       for (uint32_t j = run0; j < run1; ++j) before += (uint32_t)s_claim[j] < tid ? 1u : 0u;
     const uint32_t rank = run0 + before;
     s_key[rank] = (uint16_t)tid;

@@ -97,6 +97,26 @@ def test_c3_pool_unpool_full_size(oracle):
     assert np.array_equal(n_bf16_bits(up), want_up)
 
 
+@pytest.mark.parametrize("S,members", [(2, 1024), (8, 700), (2, 33), (3, 32), (4, 300)])
+def test_builder_many_points_in_one_cell(oracle, S, members):
+    """tiles whose points share cells: clusters of `members` equal or nearly equal points (runs at and around the length
+    from which a bitmap ranks them, several of them in a tile, one filling it) between points that span the tile's box"""
+    rng = np.random.default_rng(members)
+    n = 2 * 1024 + 517
+    coords = rng.uniform(-60, 60, (n, 3)).astype(np.float16)
+    at = rng.permutation(n)
+    for c in range(0, n - members + 1, members + 40):
+        coords[np.sort(at[c:c + members])] = (rng.uniform(-50, 50, 3) + rng.normal(0, 1e-3, (members, 3))).astype(np.float16)
+    coords[1024:2048] = coords[1024]                      # a tile that is one point: one cell, one run of all ranks
+    seps = np.array([1024 + 300, n], dtype=np.uint32)
+    feat = bf16_bits(rng.normal(0, 1, (n, 8)))
+    sb = _pool(coords, seps, feat, S, 0, 16, oracle)
+    sub_id, sub_off, unpool, red_coord, _ = oracle.subbuck_build(coords, seps, S, out_align=16)
+    assert np.array_equal(n_u32(sb.unpool_ind), unpool)
+    assert np.array_equal(n_u32(sb.subbuck_id), sub_id) and np.array_equal(n_u16(sb.subbuck_off), sub_off)
+    assert np.array_equal(n_f16(sb.reduced_coord).view(np.uint16)[:len(unpool)], red_coord.view(np.uint16)[:len(unpool)])
+
+
 @pytest.mark.parametrize("S,C", [(2, 64), (3, 24), (2, 12)])
 def test_unpool_bit_exact_with_empty_slots(oracle, S, C):
     """expected[r] = down[i] + res[r] (reference tests/test_unpooling.py:127-134); rows that no slot
