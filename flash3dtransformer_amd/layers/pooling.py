@@ -24,7 +24,7 @@ class SubbuckReduceFunction(Function):
                                      sb.subbuck_id, sb.subbuck_off, sb.reduced_sep, sb.reduced_coord, sb.reduced_feat,
                                      sb.unpool_ind, 1, reduction_op)
         ctx.save_for_backward(input_feat, sb.unpool_ind)
-        ctx.subbuck_size, ctx.reduction_op = subbuck_size, reduction_op
+        ctx.subbuck_size, ctx.reduction_op, ctx.covered = subbuck_size, reduction_op, sb.covers(input_feat.shape[0])
         sb.remove_unused_buffers()
         ctx.mark_non_differentiable(sb.reduced_coord)
         return sb.reduced_feat, sb
@@ -34,7 +34,8 @@ class SubbuckReduceFunction(Function):
         """only input_feat is differentiable (reference: layers/pooling.py:87-116)"""
         input_feat, unpool_ind = ctx.saved_tensors
         g = grad_reduced_feat if grad_reduced_feat.dtype == torch.bfloat16 else grad_reduced_feat.to(torch.bfloat16)
-        grad_input_feat = torch.zeros_like(input_feat)
+        # every row that has a slot is written
+        grad_input_feat = torch.empty_like(input_feat) if ctx.covered else torch.zeros_like(input_feat)
         pshattn.batch_subbuck_reduce_backward(g.contiguous(), input_feat, unpool_ind, grad_input_feat, ctx.subbuck_size,
                                               ctx.reduction_op)
         return None, grad_input_feat, None, None, None, None

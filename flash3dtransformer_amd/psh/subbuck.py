@@ -41,6 +41,13 @@ class SubbuckBuffers:
     reduced_coord: torch.Tensor
     reduced_feat: torch.Tensor
     unpool_ind: torch.Tensor
+    # (number of point rows, inverse map, its version) when the clouds cover all rows, so that every row has a slot
+    covered: tuple = None
+
+    def covers(self, rows: int) -> bool:
+        """whether each of `rows` point rows has a slot in `unpool_ind`, as the builder left it"""
+        c = self.covered
+        return c is not None and c[0] == rows and c[1] is self.unpool_ind and c[2] == self.unpool_ind._version
 
     @staticmethod
     def create_subbuck_buff(coords: torch.Tensor, input_feat: torch.Tensor, seps: torch.Tensor,
@@ -57,15 +64,21 @@ class SubbuckBuffers:
         bbox_max = torch.full((d,), 65504.0, dtype=torch.float16, device=dev)
         red_len, _, red_sep = calc_red_sep_sizes(seps, subbuck_size)
         aligned = cdiv(red_len, out_alignment) * out_alignment
-        return SubbuckBuffers(
+        sb = SubbuckBuffers(
             bbox_min, bbox_max, red_sep,
-            torch.zeros(total_n, dtype=torch.uint32, device=dev),
+            None,
             torch.empty(total_n, dtype=torch.uint16, device=dev),
             red_sep,
             torch.empty(aligned, d, dtype=torch.float16, device=dev),
             torch.empty(aligned, input_feat.shape[1], dtype=input_feat.dtype, device=dev),
             torch.full((red_len, subbuck_size), total_n + 3, dtype=torch.int32, device=dev).view(torch.uint32),
         )
+        if sum(f3dbatch.host_sizes(seps)) == total_n:      # every point's id is written, nothing to clear
+            sb.covered = (total_n, sb.unpool_ind, sb.unpool_ind._version)
+            sb.subbuck_id = torch.empty(total_n, dtype=torch.uint32, device=dev)
+        else:
+            sb.subbuck_id = torch.zeros(total_n, dtype=torch.uint32, device=dev)
+        return sb
 
     def remove_unused_buffers(self):
         del self.subbuck_id
@@ -84,8 +97,9 @@ class UnpoolBuffers:
 @dcls.dataclass(slots=True)
 class UnpoolGradients:
     """gradient buffers of additive unpooling (reference: psh/subbuck.py:119-132): grad_res like the output
-    gradient, grad_down with the aligned row count of the pooled features; both start from zero because the
-    kernel leaves rows that no slot refers to untouched"""
+    gradient, grad_down with the aligned row count of the pooled features.  The kernel leaves rows that no slot refers to
+    (grad_res) and rows past the inverse map (grad_down) untouched: only those are cleared (clearing both tensors took 20 of
+    the 176 us of pooling and unpooling 262,144 rows of 128 channels, forward and backward)"""
     grad_res: torch.Tensor
     grad_down: torch.Tensor
 
@@ -94,6 +108,8 @@ class UnpoolGradients:
         feat_dim = grad_up_added.shape[-1]
         if down_len is None:
             down_len = sb.reduced_feat.shape[0]
-        grad_res = torch.zeros_like(grad_up_added)
-        grad_down = torch.zeros(down_len, feat_dim, dtype=grad_up_added.dtype, device=grad_up_added.device)
+        grad_res = torch.empty_like(grad_up_added) if sb.covers(grad_up_added.shape[0]) else torch.zeros_like(grad_up_added)
+        grad_down = torch.empty(down_len, feat_dim, dtype=grad_up_added.dtype, device=grad_up_added.device)
+        if down_len > sb.unpool_ind.shape[0]:
+            grad_down[sb.unpool_ind.shape[0]:].zero_()
         return UnpoolGradients(grad_res, grad_down)

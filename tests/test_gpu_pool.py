@@ -117,6 +117,25 @@ def test_builder_many_points_in_one_cell(oracle, S, members):
     assert np.array_equal(n_f16(sb.reduced_coord).view(np.uint16)[:len(unpool)], red_coord.view(np.uint16)[:len(unpool)])
 
 
+@pytest.mark.parametrize("tail", [0, 5])
+def test_pool_unpool_gradients_of_rows_without_a_slot(tail):
+    """rows past the last cloud have no slot: their gradients are zero; rows of the pooled tensor past the map too"""
+    from flash3dtransformer_amd.layers.pooling import InbucketPoolingLayer
+    from flash3dtransformer_amd.layers.unpool import AdditiveUnpoolLayer
+    n, C = 1501, 16
+    g = torch.Generator(device=DEV).manual_seed(tail)
+    coords = torch.rand(n + tail, 3, device=DEV, generator=g).to(torch.float16)
+    for _ in range(3):      # memory that is handed out again holds the earlier gradients
+        feat, skip = [torch.randn(n + tail, C, device=DEV, generator=g).to(torch.bfloat16).requires_grad_() for _ in range(2)]
+        red, sb = InbucketPoolingLayer("mean", out_alignment=256)(coords, feat, t_u32(np.array([n], dtype=np.uint32)))
+        grad = torch.randn(n + tail, C, device=DEV, generator=g).to(torch.bfloat16)
+        red.retain_grad()
+        AdditiveUnpoolLayer(2)(skip, red, sb).backward(grad)
+        assert sb.covers(n + tail) == (tail == 0)
+        assert torch.equal(skip.grad[:n], grad[:n]) and not skip.grad[n:].any() and not feat.grad[n:].any()
+        assert not red.grad[sb.unpool_ind.shape[0]:].any() and torch.isfinite(feat.grad.float()).all()
+
+
 @pytest.mark.parametrize("S,C", [(2, 64), (3, 24), (2, 12)])
 def test_unpool_bit_exact_with_empty_slots(oracle, S, C):
     """expected[r] = down[i] + res[r] (reference tests/test_unpooling.py:127-134); rows that no slot
