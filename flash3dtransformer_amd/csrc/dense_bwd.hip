@@ -223,33 +223,47 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
 }
 
 // out[i] = (accumulate ? out[i] : 0) + sum over p of part[p][i], for two arrays in one launch (the weight gradient and,
-// in the workgroups past blocks_a, the bias gradient; len_b may be 0).  A workgroup owns 256 consecutive elements (64
-// lanes x 4 floats, lengths are multiples of 4); its 16 partial groups each sum every 16th partial (independent 16-byte
-// loads), then the first group adds the 16 group sums in ascending order: a fixed summation tree.
+// in the workgroups past blocks_a, the bias gradient; len_b may be 0).  A workgroup owns 4 LANES consecutive elements
+// (lengths are multiples of 4); its 1024 / LANES partial groups each sum every (1024 / LANES)-th partial, eight 16-byte
+// loads at a time (one at a time every partial waited for memory: 9.5 us a launch whatever the size), then the first
+// group adds the group sums in ascending order: a fixed summation tree.  Many partials (small gradients, 128 to 256
+// slabs) take 16 lanes and 64 groups, so that 32 x 32 elements still occupy 16 workgroups: 9.5 -> 4.7 us.
+template <int LANES>
 __global__ __launch_bounds__(1024) void sum_partials_kernel(const float* __restrict__ part_a, size_t len_a,
                                                             float* __restrict__ out_a, uint32_t blocks_a,
                                                             const float* __restrict__ part_b, size_t len_b,
                                                             float* __restrict__ out_b, uint32_t n_part,
                                                             uint32_t accumulate) {
-  __shared__ float4 s_sum[16][64];
+  constexpr uint32_t GROUPS = 1024u / LANES;
+  __shared__ float4 s_sum[GROUPS][LANES];
   const bool second = blockIdx.x >= blocks_a;
   const float* part = second ? part_b : part_a;
   float* out = second ? out_b : out_a;
   const size_t len = second ? len_b : len_a;
-  const uint32_t tid = threadIdx.x, l = tid & 63u, g = tid >> 6;
-  const size_t i = ((size_t)(blockIdx.x - (second ? blocks_a : 0u)) * 64u + l) * 4u;
+  const uint32_t tid = threadIdx.x, l = tid % LANES, g = tid / LANES;
+  const size_t i = ((size_t)(blockIdx.x - (second ? blocks_a : 0u)) * LANES + l) * 4u;
   float4 s = {0.f, 0.f, 0.f, 0.f};
-  if (i < len)
-    for (uint32_t p = g; p < n_part; p += 16u) {
-      const float4 v = *reinterpret_cast<const float4*>(part + (size_t)p * len + i);
-      s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+  if (n_part <= GROUPS) {      // uniform
+    if (i < len && g < n_part) s = *reinterpret_cast<const float4*>(part + (size_t)g * len + i);
+  } else if (i < len) {
+    for (uint32_t p = g; p < n_part; p += 8u * GROUPS) {
+      float4 v[8];
+#pragma unroll
+      for (uint32_t u = 0; u < 8u; ++u) {
+        v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (p + u * GROUPS < n_part) v[u] = *reinterpret_cast<const float4*>(part + (size_t)(p + u * GROUPS) * len + i);
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < 8u; ++u) { s.x += v[u].x; s.y += v[u].y; s.z += v[u].z; s.w += v[u].w; }
     }
+  }
   s_sum[g][l] = s;
   __syncthreads();
   if (g == 0 && i < len) {
     float4 t = {0.f, 0.f, 0.f, 0.f};
     if (accumulate) t = *reinterpret_cast<const float4*>(out + i);
-    for (int r = 0; r < 16; ++r) {
+#pragma unroll 16
+    for (uint32_t r = 0; r < GROUPS; ++r) {
       const float4 v = s_sum[r][l];
       t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
     }
@@ -382,8 +396,8 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(const uint16_t* z, uint
 }
 
 // dgamma / dbeta from the per-workgroup partial rows [dgamma | dbeta].  A workgroup owns 16 columns; its 64 row
-// groups each sum every 64th partial row (independent loads, so many are in flight), then one thread per column adds
-// the 64 group sums in ascending order: a fixed summation tree.
+// groups each sum every 64th partial row, eight loads at a time (2048 rows: 5 to 7 us a launch; one at a time 11.7), then
+// one thread per column adds the 64 group sums in ascending order: a fixed summation tree.
 __global__ __launch_bounds__(1024) void ln_bwd_reduce_kernel(const float* __restrict__ part, uint32_t n_part, uint32_t C,
                                                              float* __restrict__ dgamma, float* __restrict__ dbeta,
                                                              uint32_t accumulate) {
@@ -391,12 +405,19 @@ __global__ __launch_bounds__(1024) void ln_bwd_reduce_kernel(const float* __rest
   const uint32_t tid = threadIdx.x, col = blockIdx.x * 16u + (tid & 15u), rg = tid >> 4;
   float s = 0.f;
   if (col < 2u * C)
-    for (uint32_t p = rg; p < n_part; p += 64u) s += part[(size_t)p * 2u * C + col];
+    for (uint32_t p = rg; p < n_part; p += 512u) {
+      float v[8];
+#pragma unroll
+      for (uint32_t u = 0; u < 8u; ++u) v[u] = p + 64u * u < n_part ? part[(size_t)(p + 64u * u) * 2u * C + col] : 0.f;
+#pragma unroll
+      for (uint32_t u = 0; u < 8u; ++u) s += v[u];
+    }
   s_red[rg][tid & 15u] = s;
   __syncthreads();
   if (tid < 16u && col < 2u * C) {
     float* out = col < C ? dgamma + col : dbeta + (col - C);
     float t = accumulate ? *out : 0.f;
+#pragma unroll 16
     for (uint32_t r = 0; r < 64u; ++r) t += s_red[r][tid];
     *out = t;
   }
@@ -450,9 +471,13 @@ int f3d_linear_wgrad_bf16(const f3d_bf16_t* dy, uint32_t lddy, const f3d_bf16_t*
   const uint32_t n_items = tiles * slabs, items_per_xcd = cdiv_u32(n_items, kXcd);
   hipLaunchKernelGGL(linear_wgrad_kernel, dim3(items_per_xcd * kXcd), dim3(kWgThreads), kWgLds, s, dy, lddy, x, ldx,
                      part_w, part_b, m, n, k, n_tiles, k_tiles, slabs, slab_rows, items_per_xcd);
-  const uint32_t blocks_w = (uint32_t)((nk + 255) / 256), blocks_b = db ? cdiv_u32(n, 256) : 0u;
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(blocks_w + blocks_b), dim3(1024), 0, s, part_w, nk, dw, blocks_w, part_b,
-                     db ? (size_t)n : (size_t)0, db, slabs, accumulate);
+  auto sum = [&](auto kern, uint32_t per_block) {
+    const uint32_t blocks_w = (uint32_t)((nk + per_block - 1) / per_block), blocks_b = db ? cdiv_u32(n, per_block) : 0u;
+    hipLaunchKernelGGL(kern, dim3(blocks_w + blocks_b), dim3(1024), 0, s, part_w, nk, dw, blocks_w, part_b,
+                       db ? (size_t)n : (size_t)0, db, slabs, accumulate);
+  };
+  if (slabs > 64) sum(sum_partials_kernel<16>, 64u);
+  else sum(sum_partials_kernel<64>, 256u);
   F3D_CHECK_HIP(hipGetLastError());
   return F3D_OK;
 }

@@ -12,9 +12,8 @@
 // In evenly spread points a run is one or two points long and its members are compared one by one.  In
 // LiDAR tiles hundreds of points share a cell (a few far points span the box); comparing them took up to
 // 60 us a tile, so runs of more than 32 points count through a bitmap of the tile's points: bucketed sweeps,
-// S = 2: 3 x 83k points 184 -> 32 us over three levels, 4 x 250k
-// 184 -> 61 us over four, 262,144 points at S = 8 41 -> 10 us.  Consecutive runs of S sorted points form a
-// sub-bucket.  Tile t owns output rows [t * tile_pts / S, ...) of its cloud, so no global counter
+// S = 2: 3 x 83k points 184 -> 32 us over three levels, 4 x 250k 184 -> 61 us over four, 262,144 points at
+// S = 8 41 -> 10 us.  Consecutive runs of S sorted points form a sub-bucket.  Tile t owns output rows [t * tile_pts / S, ...) of its cloud, so no global counter
 // is needed.  Every output is a pure function of (coords, seps, S, seed).
 #include "f3d_device.h"
 #include "f3d_internal.h"

@@ -46,6 +46,37 @@ def test_linear_wgrad_matches_fp64(M, N, K):
     assert (db.double() - 2 * ref_b).abs().max().item() <= 2e-5 * ref_b.abs().max().item() + 1e-6
 
 
+@pytest.mark.parametrize("slabs", [1, 16, 17, 64, 65, 129, 200])
+def test_wgrad_partial_sums_by_slab_count(slabs):
+    """slab counts around the sizes at which the summation kernel changes its form; 32-row slabs of small integers, whose
+    products and sums are exact in fp32"""
+    from flash3dtransformer_amd.lib import pshattn
+    M, N, K = 32 * slabs - 5, 40, 24
+    g = torch.Generator().manual_seed(slabs)
+    dy, x = [torch.randint(-3, 4, (M, c), generator=g).to(torch.bfloat16).to(DEV) for c in (N, K)]
+    dw, db = torch.full((N, K), 7.0, device=DEV), torch.full((N,), 7.0, device=DEV)
+    pshattn.linear_wgrad_bf16(dy, x, dw, db)
+    assert torch.equal(dw, dy.float().t() @ x.float()) and torch.equal(db, dy.float().sum(0))
+
+
+@pytest.mark.parametrize("blocks", [1, 64, 65, 512, 513, 1100])
+def test_layernorm_backward_partial_rows(blocks):
+    """numbers of partial rows around the reduction's batch of 8 x 64"""
+    from flash3dtransformer_amd.lib import pshattn
+    C = 256
+    M = blocks * (256 // (C // 8)) - 1
+    g = torch.Generator().manual_seed(blocks)
+    x, dh = [torch.randn(M, C, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2)]
+    dx, dg, db = torch.empty_like(x), torch.empty(C, device=DEV), torch.empty(C, device=DEV)
+    pshattn.layernorm_bwd_bf16(x, dh, torch.ones(C, dtype=torch.bfloat16, device=DEV), None, dx, dg, db, 1e-5)
+    xd = x.double()
+    xhat = (xd - xd.mean(1, keepdim=True)) * torch.rsqrt(xd.var(1, unbiased=False, keepdim=True) + 1e-5)
+    # fp32 sums of M terms in three levels, each level at most M additions: M 2^-24 of the sum of magnitudes, and the
+    # statistics' own error of a few 2^-24 per term
+    for got, terms in ((dg, dh.double() * xhat), (db, dh.double())):
+        assert ((got.double() - terms.sum(0)).abs() <= (M + 16) * 2.0 ** -24 * terms.abs().sum(0)).all()
+
+
 def test_linear_wgrad_random_shapes():
     """shapes drawn at random (multiples of 8 in n and k, any row count), one of the operands a column slice"""
     from flash3dtransformer_amd.lib import pshattn
