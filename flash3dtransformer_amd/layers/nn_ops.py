@@ -203,6 +203,18 @@ def as_bf16_2d(x: torch.Tensor) -> torch.Tensor:
     return x
 
 
+def _fresh_copies(caches, params, transposed=()):
+    """bf16 copies of a layer's parameters for a forward that records gradients (they are made anew on every such forward,
+    as _Bf16Cache does), in one launch, with the transposed copies that the backward multiplies with.  None where a
+    parameter is not a contiguous fp32 tensor on the GPU: the caller then asks the caches one by one."""
+    for p in params:
+        if p is not None and not (p.dtype is torch.float32 and p.is_cuda and p.is_contiguous()):
+            return None
+    for c in caches:
+        c.clear()
+    return pshattn.cast_bf16(params, transposed)
+
+
 def _grad_out(g, like):
     """a gradient tensor in the dtype and shape autograd expects for `like`"""
     return g.to(like.dtype).reshape(like.shape)
@@ -245,14 +257,15 @@ class _LinearGrad(torch.autograd.Function):
     dw, db = f3d_linear_wgrad_bf16(dy, h), dh = f3d_linear_bf16(dy, w.T), then LayerNorm backward if there is one"""
 
     @staticmethod
-    def forward(ctx, y, x, weight, bias, residual, ln_w, ln_b, eps, w16, g16, b16):
-        ctx.save_for_backward(x, weight, bias, residual, ln_w, ln_b, w16, g16, b16)
+    def forward(ctx, y, x, weight, bias, residual, ln_w, ln_b, eps, w16, g16, b16, w16t):
+        """w16t: the transposed copy of the weight if there is one already, else None"""
+        ctx.save_for_backward(x, weight, bias, residual, ln_w, ln_b, w16 if w16t is None else None, g16, b16, w16t)
         ctx.eps = eps
         return y.view_as(y)
 
     @staticmethod
     def backward(ctx, dy):
-        x, weight, bias, residual, ln_w, ln_b, w16, g16, b16 = ctx.saved_tensors
+        x, weight, bias, residual, ln_w, ln_b, w16, g16, b16, w16t = ctx.saved_tensors
         need = ctx.needs_input_grad
         dy2 = as_bf16_2d(dy)
         x2 = as_bf16_2d(x)
@@ -271,7 +284,7 @@ class _LinearGrad(torch.autograd.Function):
             pshattn.linear_wgrad_bf16(dy2, h, dw, db)
         if need[1] or (ln_w is not None and (need[5] or need[6])):
             dh = torch.empty(m, k, dtype=torch.bfloat16, device=dev)
-            pshattn.linear_bf16(dy2, _transposed_bf16(w16), None, None, dh, None)
+            pshattn.linear_bf16(dy2, _transposed_bf16(w16) if w16t is None else w16t, None, None, dh, None)
             if ln_w is not None:
                 dx, dg, dbeta = _ln_backward(x2, dh, g16, None, ctx.eps)
             else:
@@ -280,7 +293,7 @@ class _LinearGrad(torch.autograd.Function):
                 _grad_out(db, bias) if bias is not None and need[3] else None,
                 _grad_out(dy2, residual) if residual is not None and need[4] else None,
                 _grad_out(dg, ln_w) if ln_w is not None and need[5] else None,
-                _grad_out(dbeta, ln_b) if ln_b is not None and need[6] else None, None, None, None, None)
+                _grad_out(dbeta, ln_b) if ln_b is not None and need[6] else None, None, None, None, None, None)
 
 
 class _GatedMLPGrad(torch.autograd.Function):
@@ -291,26 +304,29 @@ class _GatedMLPGrad(torch.autograd.Function):
     When the residual is the layer's own input, its gradient dy is added to dx inside the LayerNorm backward."""
 
     @staticmethod
-    def forward(ctx, y, x, residual, ln_w, ln_b, w1, b1, w2, b2, eps, g16, be16, w1_16, b1_16, w2_16):
-        ctx.save_for_backward(x, residual, ln_w, ln_b, w1, b1, w2, b2, g16, be16, w1_16, b1_16, w2_16)
+    def forward(ctx, y, x, residual, ln_w, ln_b, w1, b1, w2, b2, eps, g16, be16, w1_16, b1_16, w2_16, w1t, w2t):
+        """w1t, w2t: the transposed copies of the weights if there are some already, else None"""
+        ctx.save_for_backward(x, residual, ln_w, ln_b, w1, b1, w2, b2, g16, be16, w1_16, b1_16,
+                              w2_16 if w2t is None else None, w1t, w2t)
         ctx.eps = eps
         return y.view_as(y)
 
     @staticmethod
     def backward(ctx, dy):
-        x, residual, ln_w, ln_b, w1, b1, w2, b2, g16, be16, w1_16, b1_16, w2_16 = ctx.saved_tensors
+        x, residual, ln_w, ln_b, w1, b1, w2, b2, g16, be16, w1_16, b1_16, w2_16, w1t, w2t = ctx.saved_tensors
         need = ctx.needs_input_grad
         dy2 = as_bf16_2d(dy)
         x2 = as_bf16_2d(x).contiguous()
         m, c = x2.shape
-        hid = w2_16.shape[1]
+        hid = w2.shape[1]
         dev = x2.device
         bf = dict(dtype=torch.bfloat16, device=dev)
         f32 = dict(dtype=torch.float32, device=dev)
         h = torch.empty(m, c, **bf)
         pshattn.layernorm_bf16(x2, g16, be16, h, ctx.eps)
         dz, a = torch.empty(m, 2 * hid, **bf), torch.empty(m, hid, **bf)
-        w2t = _transposed_bf16(w2_16)
+        if w2t is None:
+            w1t, w2t = _transposed_bf16(w1_16), _transposed_bf16(w2_16)
         # one kernel where it exists (fc1 recomputed, da = dy @ w2 and the gate backward; neither z nor da is stored) ...
         if not pshattn.mlp_gate_bwd_bf16(h, dy2, w1_16, b1_16, w2t, dz, a):
             # ... otherwise fc1, da, then the gate backward in place (dz over z, a over da)
@@ -321,7 +337,7 @@ class _GatedMLPGrad(torch.autograd.Function):
         pshattn.linear_wgrad_bf16(dy2, a, dw2, db2)
         dw1, db1 = torch.empty(2 * hid, c, **f32), torch.empty(2 * hid, **f32)
         pshattn.linear_wgrad_bf16(dz, h, dw1, db1)
-        pshattn.linear_bf16(dz, _transposed_bf16(w1_16), None, None, h, None)     # h <- dh
+        pshattn.linear_bf16(dz, w1t, None, None, h, None)     # h <- dh
         # a residual that is the input itself: one gradient tensor for both routes
         shared = (residual is not None and need[1] and need[2] and residual.data_ptr() == x.data_ptr()
                   and residual.shape == x.shape and residual.dtype == x.dtype and residual.stride() == x.stride())
@@ -333,7 +349,7 @@ class _GatedMLPGrad(torch.autograd.Function):
                 _grad_out(dg, ln_w) if need[3] else None, _grad_out(dbeta, ln_b) if ln_b is not None and need[4] else None,
                 _grad_out(dw1, w1) if need[5] else None, _grad_out(db1, b1) if b1 is not None and need[6] else None,
                 _grad_out(dw2, w2) if need[7] else None, _grad_out(db2, b2) if b2 is not None and need[8] else None,
-                None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None)
 
 
 def _grad_wanted(*tensors) -> bool:
@@ -371,10 +387,21 @@ class Linear(_CachedParamModule):
         n_out = self.out_features // 2 if act == "swiglu" else self.out_features
         y = out if out is not None else torch.empty(x2.shape[0], n_out, dtype=torch.bfloat16, device=x.device)
         r2 = None if residual is None else as_bf16_2d(residual.reshape(-1, n_out))
-        w16, b16 = self._w.get(self.weight, self.training), self._b.get(self.bias, self.training)
-        g = b = None
+        g = b = w16t = fresh = None
+        if torch.is_grad_enabled():
+            own_norm = isinstance(pre_norm, LayerNorm)
+            caches, params = [self._w, self._b], [self.weight, self.bias]
+            if own_norm:
+                caches, params = caches + [pre_norm._w, pre_norm._b], params + [pre_norm.weight, pre_norm.bias]
+            wants_dx = act is None and _grad_wanted(x, *params[2:])
+            fresh = _fresh_copies(caches, params, (0,) if wants_dx else ())
+        if fresh is not None:
+            w16, b16 = fresh[0][:2]
+            w16t = fresh[1][0] if fresh[1] else None
+        else:
+            w16, b16 = self._w.get(self.weight, self.training), self._b.get(self.bias, self.training)
         if pre_norm is not None:
-            g, b = norm_params_bf16(pre_norm)
+            g, b = fresh[0][2:] if fresh is not None and own_norm else norm_params_bf16(pre_norm)
             if isinstance(pre_norm, LayerNorm):     # its bf16 copies are kept between calls, a torch norm's are not
                 self._staged.arm(self.training or pre_norm.training, self.out_features, self.in_features, w16, b16, g, b,
                                  tag=("ln", float(pre_norm.eps)))
@@ -390,7 +417,7 @@ class Linear(_CachedParamModule):
             return y.view(*lead, n_out)
         if act is None and _hip_backward_covers(x_in, self.in_features, self.out_features) and (
                 pre_norm is None or (self.in_features in pshattn.LN_BWD_WIDTHS and g is not None)):
-            out = _LinearGrad.apply(y, x_in, self.weight, self.bias, res_in, ln_w, ln_b, eps, w16, g, b)
+            out = _LinearGrad.apply(y, x_in, self.weight, self.bias, res_in, ln_w, ln_b, eps, w16, g, b, w16t)
         else:
             out = torch_backward(y, _linear_ref(act, eps), x_in, self.weight, self.bias, res_in, ln_w, ln_b)
         return out.view(*lead, n_out)
@@ -463,8 +490,10 @@ class LayerNorm(_CachedParamModule):
     def forward(self, x: torch.Tensor):
         x2 = as_bf16_2d(x.reshape(-1, x.shape[-1])).contiguous()
         y = torch.empty_like(x2)
-        g16 = self._w.get(self.weight, self.training)
-        pshattn.layernorm_bf16(x2, g16, self._b.get(self.bias, self.training), y, self.eps)
+        fresh = _fresh_copies((self._w, self._b), (self.weight, self.bias)) if torch.is_grad_enabled() else None
+        g16, b16 = fresh[0] if fresh is not None else (self._w.get(self.weight, self.training),
+                                                       self._b.get(self.bias, self.training))
+        pshattn.layernorm_bf16(x2, g16, b16, y, self.eps)
         x_in = x.reshape(-1, x.shape[-1])
         if _grad_wanted(x_in, self.weight, self.bias) and _hip_backward_covers(x_in) \
                 and self.normalized_shape in pshattn.LN_BWD_WIDTHS:
@@ -654,7 +683,15 @@ class LayerNormMLP(_CachedParamModule):
     def forward(self, x: torch.Tensor, residual: torch.Tensor = None):
         x2 = as_bf16_2d(x.reshape(-1, self.hidden_size)).contiguous()
         params = (self.layer_norm_weight, self.layer_norm_bias, self.fc1_weight, self.fc1_bias, self.fc2_weight, self.fc2_bias)
-        g16, be16, w1_16, b1_16, w2_16, b2_16 = (c.get(p, self.training) for c, p in zip(self._c, params))
+        fresh, w1t, w2t = None, None, None
+        if torch.is_grad_enabled():
+            fresh = _fresh_copies(self._c, params, (2, 4) if _grad_wanted(x, residual, *params) else ())
+        if fresh is not None:
+            g16, be16, w1_16, b1_16, w2_16, b2_16 = fresh[0]
+            if fresh[1]:
+                w1t, w2t = fresh[1]
+        else:
+            g16, be16, w1_16, b1_16, w2_16, b2_16 = (c.get(p, self.training) for c, p in zip(self._c, params))
         r2 = None if residual is None else as_bf16_2d(residual.reshape(-1, self.hidden_size))
         y = torch.empty_like(x2)
         # on request, the whole gated MLP in one kernel where one exists (hidden activations stay in registers) ...
@@ -685,7 +722,7 @@ class LayerNormMLP(_CachedParamModule):
             return y.view(x.shape)
         if self.activation == "swiglu" and self.hidden_size in pshattn.LN_BWD_WIDTHS \
                 and _hip_backward_covers(x_in, self.ffn_hidden_size) and (res_in is None or res_in.dtype == torch.bfloat16):
-            out = _GatedMLPGrad.apply(y, x_in, res_in, *params, self.eps, g16, be16, w1_16, b1_16, w2_16)
+            out = _GatedMLPGrad.apply(y, x_in, res_in, *params, self.eps, g16, be16, w1_16, b1_16, w2_16, w1t, w2t)
             return out.view(x.shape)
         act, eps = self.activation, self.eps
 

@@ -46,6 +46,7 @@ _SIGNATURES = {
     "f3d_permute_rows": "pppuuuuip",
     "f3d_additive_unpool_bwd": "ppppuuuuip",
     "f3d_subbuck_reduce_bwd": "ppppuuuuuip",
+    "f3d_cast_bf16": "puip",
     "f3d_buck_swin_bwd": "pppuppppppppuuuuuuupip",
     "f3d_buck_swin_bwd_strided": "pppupppppppupuuuuuuupip",
     "f3d_buck_swin_fwd": "ppppppuuuuuuupip",
@@ -617,6 +618,36 @@ def gemm_sm_bf16(A, B, O):
 
 
 ACT = {None: 0, "none": 0, "gelu": 1, "swiglu": 2, "silu": 3, "relu": 4}
+
+
+def cast_bf16(tensors, transposed=()):
+    """extension: bf16 copies of contiguous fp32 tensors of one or two axes (None entries are passed through), all made in
+    one launch and laid out in one buffer; `transposed`: positions whose transposed copies are wanted too.  Returns
+    (copies, transposed copies in the order of `transposed`)."""
+    live = [t for t in tensors if t is not None]
+    dev = assert_same_device(live)
+    assert_dtype(live, torch.float32)
+    assert_contiguous(live)
+    if len(live) > 16 or any(t.dim() not in (1, 2) for t in live):
+        raise RuntimeError("cast_bf16 takes up to 16 tensors of one or two axes")
+    places, total = [], 0      # every copy starts at a multiple of 16 bytes
+    for i, t in enumerate(tensors):
+        n = 0 if t is None else t.numel()
+        room = (n + 7) // 8 * 8
+        places.append((total, total + room))
+        total += 2 * room if i in transposed else room
+    flat = torch.empty(total, dtype=torch.bfloat16, device=live[0].device)
+    base = flat.data_ptr()
+    table, copies = [], []
+    for i, (t, (at, at_t)) in enumerate(zip(tensors, places)):
+        if t is None:
+            copies.append(None)
+            continue
+        rows, cols = t.shape if t.dim() == 2 else (1, t.shape[0])
+        table += (t.data_ptr(), base + 2 * at, base + 2 * at_t if i in transposed else 0, rows, cols)
+        copies.append(flat.as_strided(t.shape, (cols, 1) if t.dim() == 2 else (1,), at))
+    _check(_load().f3d_cast_bf16((ctypes.c_uint64 * len(table))(*table), len(live), dev, _stream(dev)))
+    return copies, [flat.as_strided(tensors[i].shape[::-1], (tensors[i].shape[0], 1), places[i][1]) for i in transposed]
 
 
 def linear_bf16(x, w, bias, residual, y, act=None):

@@ -223,6 +223,12 @@ int f3d_subbuck_reduce_bwd(const f3d_bf16_t* grad_red_feat, const f3d_bf16_t* in
                            f3d_bf16_t* grad_input_feat, uint32_t total_n, uint32_t reduced_n, uint32_t feat_dim,
                            uint32_t subbuck_size, uint32_t red_op, int device, void* stream);
 
+/* ---- bf16 copies of fp32 parameters, up to 16 tensors in one launch (no counterpart in the reference, whose autocast
+ *      casts tensor by tensor) ----
+ * table: host array of `count` rows of five words: src (fp32 [rows][cols]), dst (bf16 [rows][cols]), dst_t (bf16
+ * [cols][rows], may be 0), rows, cols.  Rounding to nearest even. */
+int f3d_cast_bf16(const uint64_t* table, uint32_t count, int device, void* stream);
+
 /* ---- bucketed attention backward: buck_swin_bwd, declared src/f3d_frontend.cu:94-97, called from
  *      flash3dxfmr/layers/buck_swin.py:69-95 (kernel source absent from the reference) ------------
  * q,k,v [batch,seq_len,num_head,head_dim] bf16 with row stride qkv_row_stride (elements); o, d_o, dq, dk, dv dense

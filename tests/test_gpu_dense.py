@@ -527,3 +527,27 @@ def test_output_panel_linear_forms(M, N, K, use_bias, use_res):
     bound = 2.0 ** -8 * (1 + 2.0 ** -8) * (z.abs() + (0 if r is None else want.abs())) + acc
     assert ((y.double() - want).abs() <= bound).all()
     assert (wide[M:] == 7).all() and (wide[:, N:] == 7).all()
+
+
+@pytest.mark.parametrize("shapes,transposed", [
+    ([(1, 1), (3,), (64, 64)], (0, 2)),                             # a single element, a short vector, one whole tile
+    ([(65, 63), (130, 4), (4, 130), None, (257,)], (0, 1, 2)),      # ragged tiles, rows not in pieces of four, a missing bias
+    ([(32, 3), (32,), (96, 32), (96,)], ()),                        # no transposed copies
+    ([(8 + i, 16) for i in range(16)], (0, 15)),                    # as many as one launch takes
+])
+def test_cast_bf16_many_tensors_at_once(shapes, transposed):
+    from flash3dtransformer_amd.lib import pshattn
+    g = torch.Generator().manual_seed(len(shapes))
+    src = [None if s is None else (torch.randn(*s, generator=g) * 10.0 ** torch.randint(-30, 30, s, generator=g)).to(DEV)
+           for s in shapes]
+    src[0].view(-1)[0] = float("-inf")
+    copies, flipped = pshattn.cast_bf16(src, transposed)
+    for t, c in zip(src, copies):
+        assert (c is None) if t is None else (torch.equal(c, t.to(torch.bfloat16)) and c.is_contiguous()
+                                              and c.data_ptr() % 16 == 0)
+    for i, t in zip(transposed, flipped):
+        assert torch.equal(t, src[i].to(torch.bfloat16).t()) and t.is_contiguous() and t.data_ptr() % 16 == 0
+    with pytest.raises(RuntimeError):
+        pshattn.cast_bf16([torch.zeros(4, 4, dtype=torch.bfloat16, device=DEV)])
+    with pytest.raises(RuntimeError):
+        pshattn.cast_bf16([torch.zeros(4, device=DEV)] * 17)
