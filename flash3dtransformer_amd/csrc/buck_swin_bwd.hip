@@ -25,14 +25,15 @@
 // multiply-type instructions over the two kernels next to 14 matrix products, about 900 clocks of issue; it takes 1400.
 // Hence: Delta enters as the start value of the dP product instead of 16 subtractions, masking costs nothing in the loops
 // (an infinite LSE for masked queries, 8 ANDs in a bucket's last key tile; a masked key or query of the wave itself
-// spoils only its own column and is zeroed by the store), the walk over buckets has no division, two 32-row sub-tiles
-// share a barrier, and all streamed data including LSE and Delta arrives by direct loads (passing LSE and Delta through
-// registers made one wave wait for memory in every tile).
+// spoils only its own column and is zeroed by the store), the walk over buckets has no division, up to four
+// 32-row sub-tiles share a barrier, and all streamed data including LSE and Delta arrives by direct loads (passing LSE and
+// Delta through registers made one wave wait for memory in every tile).
 // The sub-tile loop stays rolled: unrolled, the accumulators cost up to 128 registers more and half the occupancy.
 // Keeping a whole scope in LDS (one 16-wave workgroup per scope) is slower at 256 / 512 tokens too.  Measured, both
-// kernels, before -> now: 8 heads x 131,072 rows, 512-row scopes 432 -> 391 us, with valid lengths of 3/4 to full
-// buckets 590 -> 388; scopes of 8 x 512, 122,880 rows 562 -> 322, 24,576 rows 264 -> 133; 20,480 rows of 512-row
-// scopes 39 -> 26; 4 heads of 64: 234 -> 167, of 128: 257 -> 203.
+// kernels, before -> now: 8 heads x 131,072 rows, 512-row scopes 432 -> 381 us, with valid lengths of 3/4 to full
+// buckets 590 -> 390; scopes of 8 x 512, 122,880 rows 562 -> 322, 24,576 rows 264 -> 126; 20,480 rows of 512-row
+// scopes 39 -> 25; 4 heads of 64: 234 -> 167, of 128: 257 -> 203.  128 rows a tile against 64 (32-wide heads): 381 against
+// 397 us, 126 against 134.
 #include <algorithm>
 #include "f3d_device.h"
 #include "f3d_internal.h"
@@ -55,7 +56,7 @@ struct SGeom {
   static constexpr int CPK = D / 8;                // 16-byte pieces per row
   static constexpr int ROWB = D * 2;               // bytes per row
   static constexpr int RPB = 1024 / ROWB;          // rows one direct-load instruction fills
-  static constexpr int NSUB = D <= 64 ? 2 : 1;     // 32-row sub-tiles streamed per barrier
+  static constexpr int NSUB = D <= 32 ? 4 : D <= 64 ? 2 : 1;   // 32-row sub-tiles streamed per barrier
   static constexpr int SWZ_DIV = 16 / CPK;         // rows sharing one swizzle value
   static constexpr int TILEB = 32 * ROWB;          // bytes of a 32-row tile
 };
@@ -493,12 +494,14 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
     stream_fill_pair<D, ROWS>(reinterpret_cast<const char*>(q + base_qkv + grow * ld), ld * 2u,
                               reinterpret_cast<const char*>(d_o + base_o + grow * ldo), ldo * 2u, lds0 + b * 2u * TILEB, wave, lane);
     // LSE and Delta of the tile's rows by direct loads too: through registers one wave would wait for memory in every tile
-    if (wave < 2 && lane < (uint32_t)ROWS) {
-      const uint64_t g = (uint64_t)(uintptr_t)((wave ? delta : lse) + base_l + grow * num_head);
+    constexpr uint32_t LROWS = ROWS < 64 ? ROWS : 64;      // rows of one direct load
+    const uint32_t arr = wave & 1u, part = wave >> 1;
+    if (part * LROWS < (uint32_t)ROWS && lane < LROWS) {
+      const uint64_t g = (uint64_t)(uintptr_t)((arr ? delta : lse) + base_l + (grow + part * LROWS) * num_head);
       const uint64_t gu = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)g) |
                           ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(g >> 32)) << 32);
       stream_dma4(reinterpret_cast<const void*>((uintptr_t)gu), lane * num_head * 4u,
-                  __builtin_amdgcn_readfirstlane(lds0 + 4u * TILEB + (wave * 2u + b) * ROWS * 4u));
+                  __builtin_amdgcn_readfirstlane(lds0 + 4u * TILEB + ((arr * 2u + b) * ROWS + part * LROWS) * 4u));
     }
   };
   uint32_t b = 0;
@@ -506,8 +509,12 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
   while (!w.done()) {
     const int32_t q_valid = (int32_t)(w.len - w.r);
     __builtin_amdgcn_s_waitcnt(0);   // this wave's loads of the tile have landed
-    // queries past the bucket's valid length: an infinite LSE makes their P and dS zero (wave 0 has loaded the LSE)
-    if (wave == 0 && q_valid < ROWS && (int32_t)lane >= q_valid && lane < (uint32_t)ROWS) s_lse[b * ROWS + lane] = __builtin_inff();
+    // queries past the bucket's valid length: an infinite LSE makes their P and dS zero, put there by the wave that loaded
+    // the LSE (waves 0 and 2)
+    if ((wave & 1u) == 0u && q_valid < ROWS) {
+      const uint32_t i = (wave >> 1) * 64u + lane;
+      if (i < (uint32_t)ROWS && (int32_t)i >= q_valid) s_lse[b * ROWS + i] = __builtin_inff();
+    }
     __syncthreads();                 // ... everybody's; and everybody has left the other buffer
     w.next();
     if (!w.done()) fill(b ^ 1u);

@@ -4,8 +4,8 @@
 // backward multiplies with the transposed weights.  Tensor by tensor these are launches of 2 to 5 us for a few KB each: 172
 // casts and 53 transpositions, 0.72 ms of a 12.8 ms training step of the five-level model.  One launch per layer takes all
 // of a layer's tensors: a workgroup owns one 64 x 64 tile of one of them, writes it as it is and, through LDS,
-// transposed (55 launches, 0.27 ms; the step 12.75 -> 12.3 ms).  Bound by launch latency: 6 us for the six tensors of a 128-wide MLP, 10 for those of a 512-wide one
-// (25 MB moved).
+// transposed (55 launches, 0.27 ms; the step 12.75 -> 12.3 ms).  Bound by launch latency: 6 us for the six tensors of a
+// 128-wide MLP, 10 for those of a 512-wide one (25 MB moved).
 #include "f3d_device.h"
 #include "f3d_internal.h"
 

@@ -414,7 +414,8 @@ def test_backward_with_valid_lengths(oracle):
 
 @pytest.mark.parametrize("H,D,bs,scope_size,n_scope,lens", [
     (8, 32, 128, 2, 32, None),                  # 64 keys a wave: one workgroup per (scope, head), 256 workgroups
-    (4, 16, 256, 2, 32, (1, 63, 64, 65, 0)),    # ... 16-wide heads, valid lengths around a 64-row tile
+    (4, 16, 256, 2, 32, (1, 63, 64, 65, 0)),    # ... 16-wide heads, valid lengths around a direct load's 64 rows
+    (2, 32, 256, 1, 7, (127, 128, 129, 191, 256, 95, 96)),      # ... around a 128-row tile
     (5, 32, 384, 2, 18, (384, 32, 33, 127)),    # ... three workgroups per item, no multiple of eight units
     (8, 32, 128, 1, 40, (128, 31, 0, 97)),      # scopes of 128 rows: 32 keys a wave
     (1, 32, 512, 3, 2, (512, 1, 480)),          # few workgroups: 32 keys a wave
