@@ -13,7 +13,8 @@
 // LiDAR tiles hundreds of points share a cell (a few far points span the box); comparing them took up to
 // 60 us a tile, so runs of more than 32 points count through a bitmap of the tile's points: bucketed sweeps,
 // S = 2: 3 x 83k points 184 -> 32 us over three levels, 4 x 250k 184 -> 61 us over four, 262,144 points at
-// S = 8 41 -> 10 us.  Consecutive runs of S sorted points form a sub-bucket.  Tile t owns output rows [t * tile_pts / S, ...) of its cloud, so no global counter
+// S = 8 41 -> 10 us (4 M evenly spread points, no such run: 67 -> 68).  Consecutive runs of S sorted points form a
+// sub-bucket.  Tile t owns output rows [t * tile_pts / S, ...) of its cloud, so no global counter
 // is needed.  Every output is a pure function of (coords, seps, S, seed).
 #include "f3d_device.h"
 #include "f3d_internal.h"
@@ -123,6 +124,7 @@ __global__ __launch_bounds__(kSubThreads) void subbuck_build_kernel(
   static_assert((kSubThreads / (kLongRun + 1u) + 1u) * kMapWords <= kSubThreads, "one bitmap word per thread");
   __shared__ uint32_t s_map[kSubThreads];
   __shared__ uint16_t s_map_pre[kSubThreads];
+  __shared__ uint32_t s_any_long;
   __shared__ uint32_t s_wsum[kWaves];
   __shared__ float s_mat[9];                  // the tile's rotation
   __shared__ float s_bb[9];                   // min, max, 1 / (max - min) per axis
@@ -161,6 +163,7 @@ __global__ __launch_bounds__(kSubThreads) void subbuck_build_kernel(
   uint4* const my_cells = reinterpret_cast<uint4*>(s_cell) + tid;
   *my_cells = make_uint4(0u, 0u, 0u, 0u);
   s_map[tid] = 0u;
+  if (tid == 0) s_any_long = 0u;
   if (w == 0) {
     // the tile's rotation, once per workgroup
     float q[4], mat[9];
@@ -271,16 +274,19 @@ __global__ __launch_bounds__(kSubThreads) void subbuck_build_kernel(
   __syncthreads();
   uint32_t run0 = 0, run1 = 0;
   bool long_run = false;
-  uint32_t map0 = 0;
   if (valid) {
     run0 = (s_cell[cell >> 1] >> (16u * (cell & 1u))) & 0xFFFFu;
     run1 = (s_cell[(cell + 1u) >> 1] >> (16u * ((cell + 1u) & 1u))) & 0xFFFFu;
     long_run = run1 - run0 > kLongRun;
-    map0 = run0 / (kLongRun + 1u) * kMapWords;
-    if (long_run) atomicOr(&s_map[map0 + tid / 32u], 1u << (tid % 32u));
-    else s_claim[run0 + claim] = (uint16_t)tid;
+    if (long_run) {
+      atomicOr(&s_map[run0 / (kLongRun + 1u) * kMapWords + tid / 32u], 1u << (tid % 32u));
+      s_any_long = 1u;
+    } else {
+      s_claim[run0 + claim] = (uint16_t)tid;
+    }
   }
-  if (__syncthreads_or(long_run)) {
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(s_any_long)) {
     const uint32_t mine = (uint32_t)__popc(s_map[tid]);
     uint32_t incl = mine;
 #pragma unroll
@@ -299,9 +305,10 @@ __global__ __launch_bounds__(kSubThreads) void subbuck_build_kernel(
   if (valid) {
     // place inside the run = number of its members that come earlier in the input
     uint32_t before = 0;
-    if (long_run)
-      before = s_map_pre[map0 + tid / 32u] + (uint32_t)__popc(s_map[map0 + tid / 32u] & ((1u << (tid % 32u)) - 1u));
-    else if (run1 - run0 > 1u)
+    if (long_run) {
+      const uint32_t word = run0 / (kLongRun + 1u) * kMapWords + tid / 32u;
+      before = s_map_pre[word] + (uint32_t)__popc(s_map[word] & ((1u << (tid % 32u)) - 1u));
+    } else if (run1 - run0 > 1u)
       for (uint32_t j = run0; j < run1; ++j) before += (uint32_t)s_claim[j] < tid ? 1u : 0u;
     const uint32_t rank = run0 + before;
     s_key[rank] = (uint16_t)tid;
