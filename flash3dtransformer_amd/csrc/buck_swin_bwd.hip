@@ -21,19 +21,21 @@
 // Valid lengths (kv_len, may be null): keys at in-bucket position >= kv_len[bucket] have P = 0, and so have query rows
 // there (the forward gave them O = 0, LSE = 0): their gradients are zero and they add nothing to dK / dV.
 //
-// What bounds it: the vector issue port.  A 32 x 32 block at D = 32 takes 16 exponentials, 8 + 16 conversions and 80
-// multiply-type instructions over the two kernels next to 14 matrix products, about 900 clocks of issue; it takes 1400.
-// Hence: Delta enters as the start value of the dP product instead of 16 subtractions, masking costs nothing in the loops
-// (an infinite LSE for masked queries, 8 ANDs in a bucket's last key tile; a masked key or query of the wave itself
-// spoils only its own column and is zeroed by the store), the walk over buckets has no division, up to four
-// 32-row sub-tiles share a barrier, and all streamed data including LSE and Delta arrives by direct loads (passing LSE and
-// Delta through registers made one wave wait for memory in every tile).
+// What bounds it: mostly the vector issue port.  A 32 x 32 block at D = 32 takes 32 exponentials (16 clocks each), 16
+// conversions and 112 multiply-type instructions over the two kernels next to 14 matrix products, about 1,030 clocks of
+// issue; it takes 1,450.  Hence: masking costs nothing in the loops (an infinite LSE for masked queries, 8 ANDs in a bucket's
+// last key tile; a masked key or query of the wave itself spoils only its own column and is zeroed by the store), the walk
+// over buckets has no division, the LSE is brought to the exponent's units once per tile by the wave that loaded it, up to
+// four 32-row sub-tiles share a barrier, and all streamed data including LSE and Delta arrives by direct loads (passing LSE
+// and Delta through registers made one wave wait for memory in every tile).
+// Delta is subtracted behind the dP product.  As the product's start value it would save 32 subtractions a block (122,880
+// rows in scopes of 4,096: 274 us instead of 290), but dP - Delta then rounds differently, and the backward of batch
+// statistics enlarges the flipped last bits of dS to 1e-3 of a model's gradients.
 // The sub-tile loop stays rolled: unrolled, the accumulators cost up to 128 registers more and half the occupancy.
-// Keeping a whole scope in LDS (one 16-wave workgroup per scope) is slower at 256 / 512 tokens too.  Measured, both
-// kernels, before -> now: 8 heads x 131,072 rows, 512-row scopes 432 -> 381 us, with valid lengths of 3/4 to full
-// buckets 590 -> 390; scopes of 8 x 512, 122,880 rows 562 -> 322, 24,576 rows 264 -> 126; 20,480 rows of 512-row
-// scopes 39 -> 25; 4 heads of 64: 234 -> 167, of 128: 257 -> 203.  128 rows a tile against 64 (32-wide heads): 381 against
-// 397 us, 126 against 134.
+// Keeping a whole scope in LDS (one 16-wave workgroup per scope) is slower at 256 / 512 tokens too, and so were separate
+// Delta, dK / dV and dQ kernels.  Measured, both kernels, against those: 8 heads x 131,072 rows, 512-row scopes 435 -> 382 us,
+// with valid lengths of 3/4 to full buckets 550 -> 348; scopes of 8 x 512, 122,880 rows 528 -> 290, 24,576 rows 263 -> 120;
+// 20,480 rows of 512-row scopes 39 -> 24; 4 heads of 64, 65,536 rows: 233 -> 150, of 128, 32,768 rows: 256 -> 203.
 #include <algorithm>
 #include "f3d_device.h"
 #include "f3d_internal.h"
@@ -230,30 +232,32 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 ? 2 : 4) voi
   const uint32_t qrow = q_bucket * bs + q_in_b0 + lq;
   const int32_t q_len = __builtin_amdgcn_readfirstlane(s_len[qj]) - (int32_t)q_in_b0;   // valid ones of the wave's queries
   bf16x8_t qf[KSTEPS], dof[KSTEPS];
-  float lse2;
-  f32x16_t neg_delta;
+  float lse2, dlt;
   if (q_bucket < n_bucket) {
     const uint16_t* qr = q + base_qkv + (size_t)qrow * ld + half * 8;
     const uint16_t* dr = d_o + base_o + (size_t)qrow * ldo + half * 8;
     const uint16_t* orow = o + base_o + (size_t)qrow * ldo + half * 8;
-    float sum = 0.f;
+    dlt = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       qf[ks] = *reinterpret_cast<const bf16x8_t*>(qr + ks * 16);
       dof[ks] = *reinterpret_cast<const bf16x8_t*>(dr + ks * 16);
       const u32x4_t ov = *reinterpret_cast<const u32x4_t*>(orow + ks * 16);
       const u32x4_t dv = __builtin_bit_cast(u32x4_t, dof[ks]);
+      // one sum over the row's features in ascending order: 8 of them in the lane with half 0, the next 8 in the other
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        sum = __builtin_fmaf(bf16_lo(ov[e]), bf16_lo(dv[e]), sum);
-        sum = __builtin_fmaf(bf16_hi(ov[e]), bf16_hi(dv[e]), sum);
+      for (uint32_t h = 0; h < 2; ++h) {
+        float sum = dlt;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sum = __builtin_fmaf(bf16_lo(ov[e]), bf16_lo(dv[e]), sum);
+          sum = __builtin_fmaf(bf16_hi(ov[e]), bf16_hi(dv[e]), sum);
+        }
+        dlt = __shfl(sum, lq + 32u * h);
       }
     }
-    sum += __shfl_xor(sum, 32);
     lse2 = lse[base_l + (size_t)qrow * num_head] * 1.4426950408889634f;
-    if (half == 0) delta[base_l + (size_t)qrow * num_head] = sum;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) neg_delta[i] = -sum;
+    if (half == 0) delta[base_l + (size_t)qrow * num_head] = dlt;
   }
   if (!good) return;
 
@@ -285,20 +289,18 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 ? 2 : 4) voi
     uint32_t sb[8];
     f32x16_t s_acc, p_acc;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s_acc[i] = 0.f;
-    s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[0], qf[0], s_acc, 0, 0, 0);           // St[key][query]
-    p_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[0], dof[0], neg_delta, 0, 0, 0);      // dPt - Delta
+    for (int i = 0; i < 16; ++i) { s_acc[i] = 0.f; p_acc[i] = 0.f; }
 #pragma unroll
-    for (int ks = 1; ks < KSTEPS; ++ks) {
-      s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[ks], qf[ks], s_acc, 0, 0, 0);
-      p_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[ks], dof[ks], p_acc, 0, 0, 0);
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[ks], qf[ks], s_acc, 0, 0, 0);    // St[key][query]
+      p_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[ks], dof[ks], p_acc, 0, 0, 0);   // dPt[key][query]
     }
 #pragma unroll
     for (int i = 0; i < 16; i += 2) {
       float ds[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e)
-        ds[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[i + e], scale_log2, -lse2)) * p_acc[i + e];
+        ds[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[i + e], scale_log2, -lse2)) * (p_acc[i + e] - dlt);
       sb[i / 2] = pack_bf16x2(ds[0], ds[1]);
     }
     if (k_valid < 32) {      // uniform, a bucket's last tile
@@ -362,7 +364,7 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 ? 2 : 4) voi
 
 // ---- dK, dV -------------------------------------------------------------------------------------------------
 template <int D, int KT>
-__global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 2 : 4) void bwd_dkdv_kernel(
+__global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 2 : D > 16 ? 4 : 3) void bwd_dkdv_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, uint32_t ld,
     const uint16_t* __restrict__ d_o, const float* __restrict__ lse, const float* __restrict__ delta,
     uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, const uint32_t* __restrict__ scope_buckets,
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
   const uint32_t kj = kloc0 / bs, k_in_b0 = kloc0 - kj * bs;
   const uint32_t krow = __builtin_amdgcn_readfirstlane(s_bucket[kj]) * bs + k_in_b0 + lq;   // row inside the sequence
   const int32_t k_len = __builtin_amdgcn_readfirstlane(s_len[kj]) - (int32_t)k_in_b0;       // valid ones of the wave's keys
-  bf16x8_t kf[KT][KSTEPS], vf[KT][KSTEPS];   // vf holds -V: the product then starts from Delta and gives Delta - dP
+  bf16x8_t kf[KT][KSTEPS], vf[KT][KSTEPS];
 #pragma unroll
   for (int a = 0; a < KT; ++a) {
     const uint16_t* kr = k + base_qkv + (size_t)(krow + 32u * a) * ld + half * 8;
@@ -403,10 +405,7 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       kf[a][ks] = *reinterpret_cast<const bf16x8_t*>(kr + ks * 16);
-      u32x4_t raw = *reinterpret_cast<const u32x4_t*>(vr + ks * 16);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) raw[e] ^= 0x80008000u;
-      vf[a][ks] = __builtin_bit_cast(bf16x8_t, raw);
+      vf[a][ks] = *reinterpret_cast<const bf16x8_t*>(vr + ks * 16);
     }
   }
 
@@ -436,28 +435,25 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
       da[ks] = *reinterpret_cast<const bf16x8_t*>(sD + (dir_off ^ (ks * 32u)));
     }
     // register i of a lane is query (i/4)*8 + 4 half + i%4 of the tile, for the lane's key
-    f32x16_t dl;
-    float lse2[16];
+    float lse2[16], dl[16];
 #pragma unroll
     for (int g4 = 0; g4 < 4; ++g4) {
       const float4 l4 = *reinterpret_cast<const float4*>(lse_t + g4 * 8 + half * 4);
       const float4 d4 = *reinterpret_cast<const float4*>(dlt_t + g4 * 8 + half * 4);
       const float lv[4] = {l4.x, l4.y, l4.z, l4.w}, dv4[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) { lse2[g4 * 4 + r] = lv[r] * 1.4426950408889634f; dl[g4 * 4 + r] = dv4[r]; }
+      for (int r = 0; r < 4; ++r) { lse2[g4 * 4 + r] = lv[r]; dl[g4 * 4 + r] = dv4[r]; }
     }
     uint32_t pb[KT][8], sb[KT][8];
 #pragma unroll
     for (int a = 0; a < KT; ++a) {
       f32x16_t s_acc, p_acc;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s_acc[i] = 0.f;
-      s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[0], kf[a][0], s_acc, 0, 0, 0);   // S[query][key]
-      p_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(da[0], vf[a][0], dl, 0, 0, 0);      // Delta - dP[query][key]
+      for (int i = 0; i < 16; ++i) { s_acc[i] = 0.f; p_acc[i] = 0.f; }
 #pragma unroll
-      for (int ks = 1; ks < KSTEPS; ++ks) {
-        s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[ks], kf[a][ks], s_acc, 0, 0, 0);
-        p_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(da[ks], vf[a][ks], p_acc, 0, 0, 0);
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[ks], kf[a][ks], s_acc, 0, 0, 0);   // S[query][key]
+        p_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(da[ks], vf[a][ks], p_acc, 0, 0, 0);   // dP[query][key]
       }
 #pragma unroll
       for (int i = 0; i < 16; i += 2) {
@@ -465,7 +461,7 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[i + e], scale_log2, -lse2[i + e]));
-          ds[e] = -p_acc[i + e] * p[e];
+          ds[e] = p[e] * (p_acc[i + e] - dl[i + e]);
         }
         pb[a][i / 2] = pack_bf16x2(p[0], p[1]);
         sb[a][i / 2] = pack_bf16x2(ds[0], ds[1]);
@@ -511,9 +507,12 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
     __builtin_amdgcn_s_waitcnt(0);   // this wave's loads of the tile have landed
     // queries past the bucket's valid length: an infinite LSE makes their P and dS zero, put there by the wave that loaded
     // the LSE (waves 0 and 2)
-    if ((wave & 1u) == 0u && q_valid < ROWS) {
+    if ((wave & 1u) == 0u) {
       const uint32_t i = (wave >> 1) * 64u + lane;
-      if (i < (uint32_t)ROWS && (int32_t)i >= q_valid) s_lse[b * ROWS + i] = __builtin_inff();
+      if (i < (uint32_t)ROWS) {
+        const float l = s_lse[b * ROWS + i] * 1.4426950408889634f;
+        s_lse[b * ROWS + i] = (int32_t)i < q_valid ? l : __builtin_inff();
+      }
     }
     __syncthreads();                 // ... everybody's; and everybody has left the other buffer
     w.next();

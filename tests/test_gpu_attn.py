@@ -438,6 +438,24 @@ def test_backward_key_split_and_tile_edges(oracle, H, D, bs, scope_size, n_scope
         assert not any(t[:, b * bs + n:(b + 1) * bs].any() for t in (dq, dk, dv)), f"bucket {b}: gradient on a masked row"
 
 
+@pytest.mark.parametrize("H,D,bs,scope_size,masked", [(3, 16, 256, 4, False), (2, 32, 512, 8, False), (8, 32, 256, 1, True),
+                                                      (2, 64, 256, 2, True), (1, 128, 128, 2, False)])
+def test_backward_delta_is_one_sum_in_feature_order(H, D, bs, scope_size, masked):
+    """Delta = rowsum(dO * O) as one fp32 sum over the features in ascending order, bit for bit: dS, a difference of nearly
+    equal numbers, follows its last bit, and so do a model's gradients behind batch statistics.  Products of two bf16 are
+    exact in fp32, so adding them one by one rounds as the kernel's fused multiply-adds do."""
+    L = 2 * bs * scope_size
+    Q, K, V = _qkv(3 + D, 1, L, H, D)
+    dO = torch.randn(1, L, H, D, generator=torch.Generator().manual_seed(D)).to(torch.bfloat16)
+    scopes = np.arange(L // bs, dtype=np.uint32).reshape(-1, scope_size)
+    kl = np.resize(np.array([bs, bs - 37]), L // bs) if masked else None
+    delta, O = _run_bwd(Q, K, V, dO, scopes, bs, kv_len=kl)[3:]
+    want = torch.zeros(1, L, H)
+    for d in range(D):
+        want = want + dO[..., d].float() * O[..., d]
+    assert torch.equal(delta, want)
+
+
 def test_streaming_backward_more_than_65535_items(oracle):
     """8,192 one-bucket scopes of 128 tokens x 8 heads = 65,536 (batch, scope, head) items, one more than a launch's
     grid.y holds: the forward takes them in one launch, the backward in two.  Gradients of scopes at both ends of the
