@@ -224,17 +224,18 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
 
 // out[i] = (accumulate ? out[i] : 0) + sum over p of part[p][i], for two arrays in one launch (the weight gradient and,
 // in the workgroups past blocks_a, the bias gradient; len_b may be 0).  A workgroup owns 4 LANES consecutive elements
-// (lengths are multiples of 4); its 1024 / LANES partial groups each sum every (1024 / LANES)-th partial, eight 16-byte
-// loads at a time (one at a time every partial waited for memory: 9.5 us a launch whatever the size), then the first
-// group adds the group sums in ascending order: a fixed summation tree.  Many partials (small gradients, 128 to 256
-// slabs) take 16 lanes and 64 groups, so that 32 x 32 elements still occupy 16 workgroups: 9.5 -> 4.7 us.
-template <int LANES>
-__global__ __launch_bounds__(1024) void sum_partials_kernel(const float* __restrict__ part_a, size_t len_a,
-                                                            float* __restrict__ out_a, uint32_t blocks_a,
-                                                            const float* __restrict__ part_b, size_t len_b,
-                                                            float* __restrict__ out_b, uint32_t n_part,
-                                                            uint32_t accumulate) {
-  constexpr uint32_t GROUPS = 1024u / LANES;
+// (lengths are multiples of 4); its 16 partial groups each sum every 16th partial, BATCH 16-byte loads at a time (one at a
+// time every partial waited for memory), then the first group adds the group sums in
+// ascending order: one fixed summation tree for every LANES.  Many partials (small gradients, 128 to 256 slabs) take 16
+// lanes, so that 32 x 32 elements still occupy 16 workgroups: 6.1 -> 4.8 us.  (64 groups of 16 lanes took as long, and their
+// longer last sum raised the error of a bias gradient from 1.0e-7 to 1.9e-7 at 482,304 rows.)
+template <int LANES, uint32_t BATCH>
+__global__ __launch_bounds__(16 * LANES) void sum_partials_kernel(const float* __restrict__ part_a, size_t len_a,
+                                                                  float* __restrict__ out_a, uint32_t blocks_a,
+                                                                  const float* __restrict__ part_b, size_t len_b,
+                                                                  float* __restrict__ out_b, uint32_t n_part,
+                                                                  uint32_t accumulate) {
+  constexpr uint32_t GROUPS = 16u;
   __shared__ float4 s_sum[GROUPS][LANES];
   const bool second = blockIdx.x >= blocks_a;
   const float* part = second ? part_b : part_a;
@@ -246,15 +247,15 @@ __global__ __launch_bounds__(1024) void sum_partials_kernel(const float* __restr
   if (n_part <= GROUPS) {      // uniform
     if (i < len && g < n_part) s = *reinterpret_cast<const float4*>(part + (size_t)g * len + i);
   } else if (i < len) {
-    for (uint32_t p = g; p < n_part; p += 8u * GROUPS) {
-      float4 v[8];
+    for (uint32_t p = g; p < n_part; p += BATCH * GROUPS) {
+      float4 v[BATCH];
 #pragma unroll
-      for (uint32_t u = 0; u < 8u; ++u) {
+      for (uint32_t u = 0; u < BATCH; ++u) {
         v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (p + u * GROUPS < n_part) v[u] = *reinterpret_cast<const float4*>(part + (size_t)(p + u * GROUPS) * len + i);
       }
 #pragma unroll
-      for (uint32_t u = 0; u < 8u; ++u) { s.x += v[u].x; s.y += v[u].y; s.z += v[u].z; s.w += v[u].w; }
+      for (uint32_t u = 0; u < BATCH; ++u) { s.x += v[u].x; s.y += v[u].y; s.z += v[u].z; s.w += v[u].w; }
     }
   }
   s_sum[g][l] = s;
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(1024) void sum_partials_kernel(const float* __restr
   if (g == 0 && i < len) {
     float4 t = {0.f, 0.f, 0.f, 0.f};
     if (accumulate) t = *reinterpret_cast<const float4*>(out + i);
-#pragma unroll 16
+#pragma unroll
     for (uint32_t r = 0; r < GROUPS; ++r) {
       const float4 v = s_sum[r][l];
       t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
@@ -471,13 +472,14 @@ int f3d_linear_wgrad_bf16(const f3d_bf16_t* dy, uint32_t lddy, const f3d_bf16_t*
   const uint32_t n_items = tiles * slabs, items_per_xcd = cdiv_u32(n_items, kXcd);
   hipLaunchKernelGGL(linear_wgrad_kernel, dim3(items_per_xcd * kXcd), dim3(kWgThreads), kWgLds, s, dy, lddy, x, ldx,
                      part_w, part_b, m, n, k, n_tiles, k_tiles, slabs, slab_rows, items_per_xcd);
-  auto sum = [&](auto kern, uint32_t per_block) {
+  auto sum = [&](auto kern, uint32_t lanes) {
+    const uint32_t per_block = 4 * lanes;
     const uint32_t blocks_w = (uint32_t)((nk + per_block - 1) / per_block), blocks_b = db ? cdiv_u32(n, per_block) : 0u;
-    hipLaunchKernelGGL(kern, dim3(blocks_w + blocks_b), dim3(1024), 0, s, part_w, nk, dw, blocks_w, part_b,
+    hipLaunchKernelGGL(kern, dim3(blocks_w + blocks_b), dim3(16 * lanes), 0, s, part_w, nk, dw, blocks_w, part_b,
                        db ? (size_t)n : (size_t)0, db, slabs, accumulate);
   };
-  if (slabs > 64) sum(sum_partials_kernel<16>, 64u);
-  else sum(sum_partials_kernel<64>, 256u);
+  if (slabs > 64) sum(sum_partials_kernel<16, 16>, 16u);
+  else sum(sum_partials_kernel<64, 8>, 64u);
   F3D_CHECK_HIP(hipGetLastError());
   return F3D_OK;
 }

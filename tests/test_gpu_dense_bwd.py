@@ -59,6 +59,21 @@ def test_wgrad_partial_sums_by_slab_count(slabs):
     assert torch.equal(dw, dy.float().t() @ x.float()) and torch.equal(db, dy.float().sum(0))
 
 
+@pytest.mark.parametrize("slabs", [40, 80, 128, 200])
+def test_wgrad_partial_sums_keep_small_terms_beside_a_large_one(slabs):
+    """one partial of 2^25 and one of 127/128 from every other slab: a summation tree of 16 groups rounds at most
+    slabs / 16 + 15 times next to the large one, by half a unit of its last place (2) each"""
+    from flash3dtransformer_amd.lib import pshattn
+    dy = torch.zeros(32 * slabs, 32, dtype=torch.bfloat16)
+    dy[::32] = 127 / 128
+    dy[0] = 2.0 ** 25
+    dw, db = torch.empty(32, 32, device=DEV), torch.empty(32, device=DEV)
+    pshattn.linear_wgrad_bf16(dy.to(DEV), torch.ones(32 * slabs, 32, dtype=torch.bfloat16, device=DEV), dw, db)
+    want = 2.0 ** 25 + (slabs - 1) * 127 / 128
+    for got in (dw, db):
+        assert (got.double() - want).abs().max().item() <= 2 * (slabs / 16 + 15)
+
+
 @pytest.mark.parametrize("blocks", [1, 64, 65, 512, 513, 1100])
 def test_layernorm_backward_partial_rows(blocks):
     """numbers of partial rows around the reduction's batch of 8 x 64"""
