@@ -92,4 +92,16 @@ struct DeviceGuard {
 
 static inline uint32_t cdiv_u32(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
+// Whether y [rows][cols_y] may share an element with x [rows][cols_x] (row strides in elements).  Matrices whose address
+// ranges meet are told apart only when their rows have one pitch: y may then be other columns of the same buffer.
+static inline bool rows_overlap(const void* x, uint32_t ldx, uint32_t cols_x, const void* y, uint32_t ldy, uint32_t cols_y,
+                                uint32_t rows) {
+  if (rows == 0 || cols_x == 0 || cols_y == 0) return false;
+  const uint64_t x0 = (uintptr_t)x / 2, y0 = (uintptr_t)y / 2;      // in elements of two bytes
+  if (x0 + (uint64_t)(rows - 1) * ldx + cols_x <= y0 || y0 + (uint64_t)(rows - 1) * ldy + cols_y <= x0) return false;
+  if (ldx != ldy) return true;
+  const uint64_t at = y0 >= x0 ? (y0 - x0) % ldx : (ldx - (x0 - y0) % ldx) % ldx;   // y's first column in a row of x
+  return at < cols_x || at + cols_y > ldx;
+}
+
 }  // namespace f3d

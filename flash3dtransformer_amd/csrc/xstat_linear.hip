@@ -446,10 +446,12 @@ static int launch_k(bool ln, bool swiglu, hipStream_t s, const uint16_t* x, uint
   // Few rows leave most of the chip idle while each workgroup walks all output columns: the columns are then divided
   // over as many workgroups per row panel as the chip takes at once (each reads its rows again, from the L2).  Measured
   // at 512 -> 4096 with LayerNorm and gate: 30,208 rows 187 -> 121 us (two groups), 1,536 rows 178 -> 21 us; a panel
-  // count beyond half of the places gets no split (62,976 rows: two groups 257 against 250 us).
+  // count beyond half of the places gets no split (62,976 rows: two groups 257 against 250 us).  A y that lies on x gets none
+  // either: a workgroup holds its rows before it stores, but would store on rows that another one still has to read.
   const uint32_t panels = cdiv_u32(M, 32 * MT * WAVES), chunks = cdiv_u32(swiglu ? N / 2 : N, swiglu ? 32u : (uint32_t)kXsChunk);
   const uint32_t places = 256u * (WAVES == 8 ? 1u : 2u);          // workgroups the 256 CUs hold (LDS, registers)
-  const dim3 grid(panels, std::max(1u, std::min(chunks, places / panels))), block(64 * WAVES);
+  const bool in_place = x && rows_overlap(x, ldx, K, y, ldy, swiglu ? N / 2 : N, M);
+  const dim3 grid(panels, in_place ? 1u : std::max(1u, std::min(chunks, places / panels))), block(64 * WAVES);
 #define F3D_XS(L, S, E, ...)                                                                                       \
   do {                                                                                                             \
     static bool attr_set[64] = {};                                                                                 \

@@ -221,11 +221,14 @@ int launch_ystat_linear(const uint16_t* x, uint32_t ldx, const uint16_t* w, cons
   // 128 x 128 (K = 2048: 49.5, 37, 27.5 us up to 256 panels); the launch takes the form with the least panel time times rounds
   // of the chip.  N = 512, K = 2048: 30,208 rows 64 / 82 / 98 us, 8,192 rows 50 / 37 / 28; N = 128, K = 1024: 120,832 rows
   // (256 x 128, 128 x 128) 57 / 67 us, 32,768 rows 24 / 19.
+  // A y that lies on x is taken only where one workgroup holds all columns of its rows, and so reads them before it stores.
   const uint32_t rows2 = cdiv_u32(M, 256), rows1 = cdiv_u32(M, 128);
+  const bool in_place = rows_overlap(x, ldx, K, y, ldy, N, M);
+  if (in_place && N > 256) return F3D_ERR_UNSUPPORTED;
   auto cost = [](uint64_t panels, uint32_t weight) { return (panels + 255) / 256 * weight; };
   const uint64_t wide = N % 256 == 0 ? cost((uint64_t)rows2 * (N / 256), 20) : ~0ull;
   const uint64_t tall = cost((uint64_t)rows2 * (N / 128), 15), small = cost((uint64_t)rows1 * (N / 128), 11);
-  if (wide <= tall && wide <= small) return launch_ys<256, 2>(x, ldx, w, bias, residual, ldr, y, ldy, M, N, K, device, s);
+  if ((in_place && N == 256) || (wide <= tall && wide <= small)) return launch_ys<256, 2>(x, ldx, w, bias, residual, ldr, y, ldy, M, N, K, device, s);
   if (tall <= small) return launch_ys<128, 2>(x, ldx, w, bias, residual, ldr, y, ldy, M, N, K, device, s);
   return launch_ys<128, 1>(x, ldx, w, bias, residual, ldr, y, ldy, M, N, K, device, s);
 }

@@ -295,7 +295,9 @@ int f3d_gemm_sm_bf16(const f3d_bf16_t* a, const f3d_bf16_t* b, f3d_bf16_t* o, ui
  * (flash3dxfmr/layers/buck_swin.py:159,163; hourglass.py:65,148,150; flash3d.py:32).
  * x [m,k] bf16 (row stride ldx), w [n,k] bf16, bias [n] bf16 or NULL, residual [m,n_out] bf16 or
  * NULL (row stride ldr), y [m,n_out] bf16 (row stride ldy); n_out = n/2 for F3D_ACT_SWIGLU else n.
- * fp32 accumulate; k % 8 == 0. */
+ * fp32 accumulate; k % 8 == 0.  y may lie on x (rows on their own rows, any columns of them) where one workgroup holds all
+ * columns of its rows: k = 32, 64, 128, 256 or 512 with n % 32 == 0 (% 64 for F3D_ACT_SWIGLU), also with LayerNorm in front,
+ * and without activation k % 64 == 0 from 192 up with n = 128 or 256.  Elsewhere such a call's results are undefined. */
 int f3d_linear_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* w, const f3d_bf16_t* bias,
                     const f3d_bf16_t* residual, uint32_t ldr, f3d_bf16_t* y, uint32_t ldy, uint32_t m,
                     uint32_t n, uint32_t k, uint32_t act, int device, void* stream);

@@ -551,3 +551,32 @@ def test_cast_bf16_many_tensors_at_once(shapes, transposed):
         pshattn.cast_bf16([torch.zeros(4, 4, dtype=torch.bfloat16, device=DEV)])
     with pytest.raises(RuntimeError):
         pshattn.cast_bf16([torch.zeros(4, device=DEV)] * 17)
+
+
+@pytest.mark.parametrize("M,N,K,act,ln", [
+    (1536, 512, 512, None, False),      # few rows: the columns would be divided over eight workgroups a panel
+    (1537, 512, 512, None, True),       # ... with LayerNorm in front
+    (3001, 256, 256, "gelu", False),
+    (999, 128, 64, "swiglu", False),    # 64 outputs from 128 weight rows
+    (700, 128, 640, None, False),       # output-panel kernel, one panel of columns
+    (700, 256, 640, None, False),       # ... a y that lies on the first columns of x
+])
+def test_linear_in_place(M, N, K, act, ln):
+    """y on the rows of x gives what a separate y gives, and so does a y beside x in one buffer"""
+    from flash3dtransformer_amd.lib import pshattn
+    x0, w, b = _rand((M, K), 1).to(DEV), _rand((N, K), 2, scale=K ** -0.5).to(DEV), _rand((N,), 3).to(DEV)
+    g = (_rand((K,), 4) + 1.0).to(DEV)
+    n_out = N // 2 if act == "swiglu" else N
+
+    def run(x, y):
+        if ln:
+            pshattn.ln_linear_bf16(x, g, b[:K].contiguous() if N >= K else g, 1e-5, w, b, None, y, act)
+        else:
+            pshattn.linear_bf16(x, w, b, None, y, act)
+        return y
+    want = run(x0, torch.empty(M, n_out, dtype=torch.bfloat16, device=DEV))
+    for _ in range(5):
+        x = x0.clone()
+        assert torch.equal(run(x, x[:, :n_out]), want) and torch.equal(x[:, n_out:], x0[:, n_out:])
+    both = torch.cat([x0, torch.zeros_like(want)], dim=1)
+    assert torch.equal(run(both[:, :K], both[:, K:]), want) and torch.equal(both[:, :K], x0)
