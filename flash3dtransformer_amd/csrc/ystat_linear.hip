@@ -208,12 +208,13 @@ static int launch_ys(const uint16_t* x, uint32_t ldx, const uint16_t* w, const u
 }
 
 // Returns F3D_OK when launched, F3D_ERR_UNSUPPORTED when the shape is not covered (the caller then uses the tiled
-// GEMM), another code on failure.  Covered: no activation, N a multiple of 128, K a multiple of 64 from 192 up, row
-// offsets inside a workgroup's panel that fit 32 bits.
+// GEMM), another code on failure.  Covered: no activation, N a multiple of 128, K a multiple of 64 from 192 up, a bias
+// that can be read in 8-byte pieces (the entry point asks that of no bias), row offsets inside a workgroup's panel that fit
+// 32 bits.
 int launch_ystat_linear(const uint16_t* x, uint32_t ldx, const uint16_t* w, const uint16_t* bias,
                         const uint16_t* residual, uint32_t ldr, uint16_t* y, uint32_t ldy, uint32_t M, uint32_t N,
                         uint32_t K, uint32_t act, int device, hipStream_t s) {
-  if (act != F3D_ACT_NONE || N % 128 != 0 || K < 192 || K % 64 != 0) return F3D_ERR_UNSUPPORTED;
+  if (act != F3D_ACT_NONE || N % 128 != 0 || K < 192 || K % 64 != 0 || ((uintptr_t)bias & 7u) != 0) return F3D_ERR_UNSUPPORTED;
   if ((uint64_t)K * 2 * 8 >= (1ull << 32) || (uint64_t)256 * ldx * 2 >= (1ull << 31) ||
       (uint64_t)256 * std::max(ldy, ldr) >= (1ull << 32) || (uint64_t)cdiv_u32(M, 128) * (N / 128) > 0x7FFFF0ull)
     return F3D_ERR_UNSUPPORTED;

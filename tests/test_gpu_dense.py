@@ -580,3 +580,17 @@ def test_linear_in_place(M, N, K, act, ln):
         assert torch.equal(run(x, x[:, :n_out]), want) and torch.equal(x[:, n_out:], x0[:, n_out:])
     both = torch.cat([x0, torch.zeros_like(want)], dim=1)
     assert torch.equal(run(both[:, :K], both[:, K:]), want) and torch.equal(both[:, :K], x0)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 256, 640), (300, 128, 192), (300, 256, 256), (300, 40, 72)])
+@pytest.mark.parametrize("at", [1, 2, 3, 4])
+def test_linear_bias_at_any_element(M, N, K, at):
+    """a bias may be a slice that starts at any element: the kernels that read it in pieces leave such a call to others"""
+    from flash3dtransformer_amd.lib import pshattn
+    x, w, b = _rand((M, K), 1).to(DEV), _rand((N, K), 2, scale=K ** -0.5).to(DEV), _rand((N + 8,), 3).to(DEV)
+    y, y0 = torch.empty(M, N, dtype=torch.bfloat16, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    pshattn.linear_bf16(x, w, b[at:at + N], None, y, None)
+    pshattn.linear_bf16(x, w, b[at:at + N].clone(), None, y0, None)
+    # the same sums in another order: at most one bf16 rounding apart, by K fp32 additions of terms below |x| |w|
+    acc = K * 2.0 ** -23 * (x.double().norm(dim=1, keepdim=True) * w.double().norm(dim=1))
+    assert ((y.double() - y0.double()).abs() <= 2.0 ** -7 * y0.double().abs() + acc).all()
