@@ -63,11 +63,14 @@ __global__ __launch_bounds__(64 * kYsWaves, 2) void ystat_linear_kernel(
   const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
   const uint32_t lq = lane & 31u, half = lane >> 5;
   const uint32_t rb = wave & 3u, cg = wave >> 2;          // row block of 32 MT rows, half of the panel's columns
-  // the column panels of one row panel run on one XCD, whose L2 serves their reads of x after the first
-  const uint32_t n_pan = NT / N, slot = blockIdx.x / kYsXcd;
-  const uint32_t wg_row0 = (slot / n_pan * kYsXcd + blockIdx.x % kYsXcd) * ROWS_WG;
-  if (wg_row0 >= M) return;
-  const uint32_t pan = slot % n_pan, col0 = pan * N;
+  // Workgroups go round the XCDs in launch order.  The column panels of one row panel run on one XCD, whose L2 serves their
+  // reads of x after the first, as long as there are eight row panels to share out; the column panels of the last up to
+  // seven go to all XCDs (with those on one XCD each, 128 rows x 8,192 outputs, K = 1024, kept 32 CUs busy for two rounds:
+  // 27 us, the tiled GEMM 19, now 12.6)
+  const uint32_t n_pan = NT / N, whole = gridDim.x / n_pan / kYsXcd * kYsXcd * n_pan, slot = blockIdx.x / kYsXcd;
+  const bool grouped = blockIdx.x < whole;
+  const uint32_t row_pan = grouped ? slot / n_pan * kYsXcd + blockIdx.x % kYsXcd : blockIdx.x / n_pan;
+  const uint32_t wg_row0 = row_pan * ROWS_WG, col0 = (grouped ? slot : blockIdx.x) % n_pan * N;
   const uint32_t row0 = wg_row0 + rb * (32 * MT);
 
   // accumulators start from the bias: acc[o][mt][g*4+r] <-> output column (cg*OTW + o)*32 + g*8 + half*4 + r, row lq
@@ -201,8 +204,7 @@ static int launch_ys(const uint16_t* x, uint32_t ldx, const uint16_t* w, const u
     F3D_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if (device >= 0 && device < 64) attr_set[device] = true;
   }
-  const uint32_t groups = cdiv_u32(cdiv_u32(M, 128 * MT), kYsXcd);      // of eight row panels
-  hipLaunchKernelGGL(kern, dim3(groups * kYsXcd * (NT / N)), dim3(64 * kYsWaves), lds, s, x, ldx, w, bias, residual, ldr,
+  hipLaunchKernelGGL(kern, dim3(cdiv_u32(M, 128 * MT) * (NT / N)), dim3(64 * kYsWaves), lds, s, x, ldx, w, bias, residual, ldr,
                      y, ldy, M, K, NT);
   return F3D_OK;
 }

@@ -506,6 +506,8 @@ def test_staged_weights_are_reused_and_refreshed():
     (9001, 512, 704, True, False),      # 256 x 128 panels, a ragged last row panel
     (17001, 512, 576, True, True),      # 256 x 256 panels
     (65537, 128, 1024, True, True),     # 256 x 128 panels, more than one round of the chip
+    (130, 2048, 192, True, True),       # two row panels: their column panels go to all XCDs
+    (2300, 384, 640, True, False),      # eighteen: sixteen shared out, two to all XCDs
 ])
 def test_output_panel_linear_forms(M, N, K, use_bias, use_res):
     """each panel form of the output-panel kernel at ragged row counts, with strided rows of x, residual and y"""
