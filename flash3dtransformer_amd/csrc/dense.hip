@@ -396,7 +396,7 @@ int f3d_linear_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* w, cons
                 "row strides must be multiples of 8 and cover a row (ldx=%u ldy=%u ldr=%u)", ldx, ldy, ldr);
   F3D_CHECK_ARG((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)residual) & 15u) == 0,
                 "x/w/y/residual must be 16-byte aligned");
-  if (m == 0) return F3D_OK;
+  if (m == 0 || n_out == 0) return F3D_OK;
   DeviceGuard guard(device);
   F3D_CHECK_ARG(guard.ok, "cannot select device %d", device);
   hipStream_t s = (hipStream_t)stream;
@@ -427,7 +427,7 @@ int f3d_ln_linear_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* gamm
                 "row strides must be aligned and cover a row (ldx=%u ldy=%u ldr=%u)", ldx, ldy, ldr);
   F3D_CHECK_ARG((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)residual | (uintptr_t)gamma | (uintptr_t)beta) & 15u) == 0,
                 "x/w/y/residual/gamma/beta must be 16-byte aligned");
-  if (m == 0) return F3D_OK;
+  if (m == 0 || n_out == 0) return F3D_OK;
   DeviceGuard guard(device);
   F3D_CHECK_ARG(guard.ok, "cannot select device %d", device);
   hipStream_t s = (hipStream_t)stream;

@@ -88,3 +88,14 @@ def test_no_alloc_psh_rejects_batches_beyond_its_scratch_array(lib):
         dummy, dummy, dummy, dummy, dummy, u32(1), u32(512), u32(512), u32(64), u32(512), u32(512), u32(0xFFFF), dummy,
         dummy, dummy, dummy, dummy, u32(512), ctypes.c_float(0.0), u32(1), ctypes.c_int(0), vp(0)) == 1
     assert b"bucket divisor too small" in lib.f3d_last_error()
+
+
+@pytest.mark.parametrize("m,n,k,act", [(0, 64, 64, 0), (16, 0, 640, 0), (16, 0, 64, 2)])
+def test_linear_without_outputs_launches_nothing(lib, m, n, k, act):
+    """no rows or no columns: done, whatever the kernel that the other sizes would choose, and before a device is selected"""
+    p, none, u = ctypes.c_void_p(4096), ctypes.c_void_p(0), ctypes.c_uint32
+    end = ctypes.c_int(0), none
+    assert lib.f3d_linear_bf16(p, u(k), p, none, none, u(0), p, u(64), u(m), u(n), u(k), u(act), *end) == 0
+    if k == 64:
+        assert lib.f3d_ln_linear_bf16(p, u(k), p, none, ctypes.c_float(1e-5), p, none, none, u(0), p, u(64), u(m), u(n), u(k),
+                                      u(act), *end) == 0
