@@ -19,7 +19,8 @@
 // LDS rows are unpadded with their 16-byte pieces XOR-swizzled (conflict-free 128-bit operand reads); the transposing
 // reads address 8-byte pieces per lane and apply the same swizzle to their addresses.
 // Valid lengths (kv_len, may be null): keys at in-bucket position >= kv_len[bucket] have P = 0, and so have query rows
-// there (the forward gave them O = 0, LSE = 0): their gradients are zero and they add nothing to dK / dV.
+// there (the forward gave them O = 0, LSE = 0): their gradients are zero and they add nothing to dK / dV.  Masked rows of
+// q, k, v, o, dO and LSE may hold anything: the tiles repeat the last valid row instead of reading them.
 //
 // What bounds it: mostly the vector issue port.  A 32 x 32 block at D = 32 takes 32 exponentials (16 clocks each), 16
 // conversions and 112 multiply-type instructions over the two kernels next to 14 matrix products, about 1,030 clocks of
@@ -29,13 +30,13 @@
 // four 32-row sub-tiles share a barrier, and all streamed data including LSE and Delta arrives by direct loads (passing LSE
 // and Delta through registers made one wave wait for memory in every tile).
 // Delta is subtracted behind the dP product.  As the product's start value it would save 32 subtractions a block (122,880
-// rows in scopes of 4,096: 274 us instead of 290), but dP - Delta then rounds differently, and the backward of batch
+// rows in scopes of 4,096: 275 us instead of 292), but dP - Delta then rounds differently, and the backward of batch
 // statistics enlarges the flipped last bits of dS to 1e-3 of a model's gradients.
 // The sub-tile loop stays rolled: unrolled, the accumulators cost up to 128 registers more and half the occupancy.
 // Keeping a whole scope in LDS (one 16-wave workgroup per scope) is slower at 256 / 512 tokens too, and so were separate
-// Delta, dK / dV and dQ kernels.  Measured, both kernels, against those: 8 heads x 131,072 rows, 512-row scopes 435 -> 382 us,
-// with valid lengths of 3/4 to full buckets 550 -> 348; scopes of 8 x 512, 122,880 rows 528 -> 290, 24,576 rows 263 -> 120;
-// 20,480 rows of 512-row scopes 39 -> 24; 4 heads of 64, 65,536 rows: 233 -> 150, of 128, 32,768 rows: 256 -> 203.
+// Delta, dK / dV and dQ kernels.  Measured, both kernels, against those: 8 heads x 131,072 rows, 512-row scopes 430 -> 382 us,
+// with valid lengths of 3/4 to full buckets 538 -> 342; scopes of 8 x 512, 122,880 rows 524 -> 292, 24,576 rows 263 -> 126;
+// 20,480 rows of 512-row scopes 39 -> 24; 4 heads of 64, 65,536 rows: 236 -> 154, of 128, 32,768 rows: 257 -> 208.
 #include <algorithm>
 #include "f3d_device.h"
 #include "f3d_internal.h"
@@ -78,10 +79,11 @@ __device__ __forceinline__ void stream_dma4(const void* gbase, uint32_t voff, ui
 }
 
 // Two runs of ROWS consecutive rows (g0, ld0 bytes a row; g1, ld1) -> two swizzled LDS tiles, one behind the other; the
-// direct loads are shared by the workgroup's waves
+// direct loads are shared by the workgroup's waves.  Rows past `last` are copies of row `last`: what lies there in memory
+// (masked rows, which may hold anything) is not read.
 template <int D, int ROWS>
 __device__ __forceinline__ void stream_fill_pair(const char* g0, uint32_t ld0, const char* g1, uint32_t ld1,
-                                                 uint32_t lds_tile, uint32_t wave, uint32_t lane) {
+                                                 uint32_t last, uint32_t lds_tile, uint32_t wave, uint32_t lane) {
   using G = SGeom<D>;
   constexpr int BLK = ROWS / G::RPB;
   const uint32_t r = lane / G::CPK, pos = lane % G::CPK;
@@ -92,10 +94,11 @@ __device__ __forceinline__ void stream_fill_pair(const char* g0, uint32_t ld0, c
       const bool second = n >= (uint32_t)BLK;
       const uint32_t blk = second ? n - BLK : n, ld = second ? ld1 : ld0;
       const uint32_t ck = pos ^ (((blk * G::RPB + r) / G::SWZ_DIV) & (G::CPK - 1));
-      const uint64_t g = (uint64_t)(uintptr_t)(second ? g1 : g0) + (uint64_t)blk * G::RPB * ld;
+      const uint32_t row0 = min(blk * G::RPB, last);
+      const uint64_t g = (uint64_t)(uintptr_t)(second ? g1 : g0) + (uint64_t)row0 * ld;
       const uint64_t gu = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)g) |
                           ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(g >> 32)) << 32);
-      stream_dma16(reinterpret_cast<const void*>((uintptr_t)gu), r * ld + ck * 16u,
+      stream_dma16(reinterpret_cast<const void*>((uintptr_t)gu), min(r, last - row0) * ld + ck * 16u,
                    __builtin_amdgcn_readfirstlane(lds_tile + n * 1024u));
     }
   }
@@ -326,8 +329,9 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 ? 2 : 4) voi
   StreamWalk<ROWS> w(s_bucket, s_len, scope_size, bs);
   auto fill = [&](uint32_t b) {   // the walk's tile -> buffer b
     const size_t grow = w.row0 + w.r;
+    const uint32_t last = min(w.len - w.r, (uint32_t)ROWS) - 1u;
     stream_fill_pair<D, ROWS>(reinterpret_cast<const char*>(k + base_qkv + grow * ld), ld * 2u,
-                              reinterpret_cast<const char*>(v + base_qkv + grow * ld), ld * 2u, lds0 + b * 2u * TILEB, wave, lane);
+                              reinterpret_cast<const char*>(v + base_qkv + grow * ld), ld * 2u, last, lds0 + b * 2u * TILEB, wave, lane);
   };
   uint32_t b = 0;
   if (!w.done()) fill(b);
@@ -487,16 +491,18 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
   StreamWalk<ROWS> w(s_bucket, s_len, scope_size, bs);
   auto fill = [&](uint32_t b) {   // the walk's tile -> buffer b
     const size_t grow = w.row0 + w.r;
+    const uint32_t last = min(w.len - w.r, (uint32_t)ROWS) - 1u;
     stream_fill_pair<D, ROWS>(reinterpret_cast<const char*>(q + base_qkv + grow * ld), ld * 2u,
-                              reinterpret_cast<const char*>(d_o + base_o + grow * ldo), ldo * 2u, lds0 + b * 2u * TILEB, wave, lane);
+                              reinterpret_cast<const char*>(d_o + base_o + grow * ldo), ldo * 2u, last, lds0 + b * 2u * TILEB, wave, lane);
     // LSE and Delta of the tile's rows by direct loads too: through registers one wave would wait for memory in every tile
     constexpr uint32_t LROWS = ROWS < 64 ? ROWS : 64;      // rows of one direct load
     const uint32_t arr = wave & 1u, part = wave >> 1;
     if (part * LROWS < (uint32_t)ROWS && lane < LROWS) {
-      const uint64_t g = (uint64_t)(uintptr_t)((arr ? delta : lse) + base_l + (grow + part * LROWS) * num_head);
+      const uint32_t part0 = min(part * LROWS, last);
+      const uint64_t g = (uint64_t)(uintptr_t)((arr ? delta : lse) + base_l + (grow + part0) * num_head);
       const uint64_t gu = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)g) |
                           ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(g >> 32)) << 32);
-      stream_dma4(reinterpret_cast<const void*>((uintptr_t)gu), lane * num_head * 4u,
+      stream_dma4(reinterpret_cast<const void*>((uintptr_t)gu), min(lane, last - part0) * num_head * 4u,
                   __builtin_amdgcn_readfirstlane(lds0 + 4u * TILEB + ((arr * 2u + b) * ROWS + part * LROWS) * 4u));
     }
   };
@@ -505,8 +511,8 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
   while (!w.done()) {
     const int32_t q_valid = (int32_t)(w.len - w.r);
     __builtin_amdgcn_s_waitcnt(0);   // this wave's loads of the tile have landed
-    // queries past the bucket's valid length: an infinite LSE makes their P and dS zero, put there by the wave that loaded
-    // the LSE (waves 0 and 2)
+    // the LSE in the exponent's units, by the wave that loaded it (waves 0 and 2); queries past the bucket's valid length get
+    // an infinite one, which makes their P and dS zero
     if ((wave & 1u) == 0u) {
       const uint32_t i = (wave >> 1) * 64u + lane;
       if (i < (uint32_t)ROWS) {

@@ -235,8 +235,8 @@ int f3d_cast_bf16(const uint64_t* table, uint32_t count, int device, void* strea
  * [batch,seq_len,num_head,head_dim] bf16; lse (from the forward), delta (output: rowsum(d_o * o))
  * [batch,seq_len,num_head] fp32.  Rows that no scope covers are not written.  kv_len (may be NULL)
  * [seq_len/bucket_size] i32 is the forward's extension: rows of a bucket at or past its valid length get zero
- * gradients and add nothing to the others (they must still hold finite numbers).  Supported: head_dim 16, 32, 64 or
- * 128, scopes of any number of buckets up to 4096 (the reference's test shapes, tests/test_attn_bwd.py: head_dim 64 and
+ * gradients and add nothing to the others, whatever they hold (delta there follows o and d_o).  Supported: head_dim 16,
+ * 32, 64 or 128, scopes of any number of buckets up to 4096 (the reference's test shapes, tests/test_attn_bwd.py: head_dim 64 and
  * 128, 32 buckets of 256 in one scope); other head sizes return F3D_ERR_UNSUPPORTED. */
 int f3d_buck_swin_bwd(const f3d_bf16_t* q, const f3d_bf16_t* k, const f3d_bf16_t* v, uint32_t qkv_row_stride,
                       const f3d_bf16_t* o, const f3d_bf16_t* d_o, const float* lse, float* delta, f3d_bf16_t* dq,

@@ -438,6 +438,44 @@ def test_backward_key_split_and_tile_edges(oracle, H, D, bs, scope_size, n_scope
         assert not any(t[:, b * bs + n:(b + 1) * bs].any() for t in (dq, dk, dv)), f"bucket {b}: gradient on a masked row"
 
 
+@pytest.mark.parametrize("H,D,bs,scope_size,lens", [
+    (8, 32, 256, 1, (256, 127, 128, 1)),        # 128-row tiles
+    (8, 32, 512, 8, (512, 300, 0, 511)),
+    (4, 16, 256, 2, (256, 40, 200)),
+    (2, 64, 256, 2, (255, 63, 64)),             # 64-row tiles
+    (2, 128, 128, 3, (100, 128, 0, 31)),        # 32-row tiles
+])
+def test_backward_masked_rows_may_hold_anything(H, D, bs, scope_size, lens):
+    """NaN and infinities in the rows past a bucket's valid length change no gradient"""
+    from flash3dtransformer_amd.lib import pshattn
+    L = bs * scope_size * (2 if scope_size > 2 else 40)
+    kl = np.resize(np.asarray(lens), L // bs)
+    masked = torch.from_numpy((np.arange(bs) >= kl[:, None]).reshape(-1)).to(DEV)
+    Q, K, V = [t.to(DEV) for t in _qkv(5 + D, 1, L, H, D)]
+    dO = torch.randn(1, L, H, D, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(DEV)
+    O, LSE = torch.zeros_like(Q), torch.zeros(1, L, H, device=DEV)
+    sc = torch.arange(L // bs, dtype=torch.int32, device=DEV).view(-1, scope_size).view(torch.uint32)
+    kv = torch.from_numpy(kl.astype(np.int32)).to(DEV)
+    pshattn.buck_swin_fwd(Q, K, V, O, LSE, sc, bs, kv_len=kv)
+
+    def grads(q, k, v, o, do, lse):
+        out = [torch.zeros_like(Q) for _ in range(3)]
+        pshattn.buck_swin_bwd(q, k, v, o, do, lse, torch.zeros_like(LSE), *out, sc, bs, kv_len=kv)
+        return out
+    want = grads(Q, K, V, O, dO, LSE)
+    assert all(torch.isfinite(t.float()).all() for t in want)
+    junk = torch.tensor([float("nan"), float("inf"), float("-inf"), 3e38], device=DEV)
+    for only in (range(6), (0,), (1,), (2,), (3,), (4,), (5,)):
+        poisoned = []
+        for i, t in enumerate((Q, K, V, O, dO, LSE)):
+            t = t.clone()
+            if i in only:
+                t[:, masked] = junk[torch.arange(t[:, masked].numel(), device=DEV) % 4].view_as(t[:, masked]).to(t.dtype)
+            poisoned.append(t)
+        for g, w, n in zip(grads(*poisoned), want, ("dQ", "dK", "dV")):
+            assert torch.equal(g, w), f"{n} changed with junk in {only}"
+
+
 @pytest.mark.parametrize("H,D,bs,scope_size,masked", [(3, 16, 256, 4, False), (2, 32, 512, 8, False), (8, 32, 256, 1, True),
                                                       (2, 64, 256, 2, True), (1, 128, 128, 2, False)])
 def test_backward_delta_is_one_sum_in_feature_order(H, D, bs, scope_size, masked):
