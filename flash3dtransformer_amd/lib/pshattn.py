@@ -100,8 +100,9 @@ def _ptr(t):
     return t.data_ptr() if t is not None else None
 
 
-# the current stream's handle without a torch.cuda.Stream object around it
-_stream = torch._C._cuda_getCurrentRawStream
+# the current stream's handle, without a torch.cuda.Stream object around it where torch has such a call (a build without
+# GPU support has not, and still has to import the host-side modules)
+_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda dev: torch.cuda.current_stream(dev).cuda_stream)
 
 
 def assert_contiguous(tensors):

@@ -1,6 +1,8 @@
 """The argument kinds the Python binding declares for the C entry points, against the header they are compiled from."""
 import os
 import re
+import subprocess
+import sys
 
 from flash3dtransformer_amd.lib import pshattn
 
@@ -16,3 +18,14 @@ def test_declared_signatures_match_the_header():
     found = {name: "".join(kind(a.strip()) for a in args.split(",") if a.strip() not in ("", "void"))
              for name, args in re.findall(r"\b(f3d_\w+)\s*\(([^()]*)\)\s*;", text)}
     assert len(found) > 40 and found == pshattn._SIGNATURES
+
+
+def test_host_side_modules_import_on_a_torch_without_gpu_support():
+    """such a torch has no raw stream call; sizes, planning and the layers' construction need none"""
+    code = ("import torch; hasattr(torch._C, '_cuda_getCurrentRawStream') and delattr(torch._C, '_cuda_getCurrentRawStream')\n"
+            "from flash3dtransformer_amd.psh import batching\n"
+            "from flash3dtransformer_amd import layers\n"
+            "print(batching.host_sizes(torch.tensor([3, 7])), layers.Linear(8, 4).weight.shape[0])")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert got.returncode == 0 and got.stdout.split() == ["[3,", "4]", "4"], got.stderr[-2000:]
