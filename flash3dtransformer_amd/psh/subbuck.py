@@ -74,7 +74,8 @@ class SubbuckBuffers:
             torch.full((red_len, subbuck_size), total_n + 3, dtype=torch.int32, device=dev).view(torch.uint32),
         )
         if sum(f3dbatch.host_sizes(seps)) == total_n:      # every point's id is written, nothing to clear
-            sb.covered = (total_n, sb.unpool_ind, sb.unpool_ind._version)
+            if not sb.unpool_ind.is_inference():      # a tensor made in inference mode keeps no version to check later
+                sb.covered = (total_n, sb.unpool_ind, sb.unpool_ind._version)
             sb.subbuck_id = torch.empty(total_n, dtype=torch.uint32, device=dev)
         else:
             sb.subbuck_id = torch.zeros(total_n, dtype=torch.uint32, device=dev)

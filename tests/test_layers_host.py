@@ -94,3 +94,19 @@ def test_layernorm_qkv_of_a_rank4_embedding_folds_to_four_numbers_per_feature():
     # a dropped mean, a missing gamma or the uncentred Gram matrix are not the same function
     assert ((rstd * (c @ ((w * gamma[None, :]) @ E).T) + bp) - want).abs().max().item() > 1e-3
     assert ((rstd * (c @ (w @ Ep).T) + bp) - want).abs().max().item() > 1e-3
+
+
+def _pool_buffers(n, tail=0):
+    from flash3dtransformer_amd.psh import subbuck
+    seps = torch.tensor([3, n], dtype=torch.int32)
+    coords, feat = torch.zeros(n + tail, 3, dtype=torch.float16), torch.zeros(n + tail, 8, dtype=torch.bfloat16)
+    return seps, lambda **kw: subbuck.SubbuckBuffers.create_subbuck_buff(coords, feat, seps, 2, out_alignment=16, **kw)
+
+
+def test_pooling_buffers_in_inference_mode():
+    """tensors made there keep no version counter; separators seen before stay usable"""
+    seps, make = _pool_buffers(40)
+    make()
+    with torch.inference_mode():
+        sb = make()
+        assert not sb.covers(40) and sb.unpool_ind.shape == (21, 2)
