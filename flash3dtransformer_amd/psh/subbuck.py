@@ -49,13 +49,20 @@ class SubbuckBuffers:
         c = self.covered
         return c is not None and c[0] == rows and c[1] is self.unpool_ind and c[2] == self.unpool_ind._version
 
+    def mark_built(self, seps: torch.Tensor, rows: int):
+        """called once the builder has filled the map for these clouds: notes whether they cover all `rows` point rows.  A
+        map made in inference mode keeps no version to check later and counts as not covering."""
+        if not self.unpool_ind.is_inference() and sum(f3dbatch.host_sizes(seps)) == rows:
+            self.covered = (rows, self.unpool_ind, self.unpool_ind._version)
+
     @staticmethod
     def create_subbuck_buff(coords: torch.Tensor, input_feat: torch.Tensor, seps: torch.Tensor,
-                            subbuck_size=2, out_alignment=1):
+                            subbuck_size=2, out_alignment=1, build_follows=False):
         """Allocation contract of batch_subbuck_reduce (subbuck.py:68-102).  `unpool_ind` MUST be
         prefilled with an index >= N: that marks a slot no point was mapped to.  The reduced length is
         rounded up to `out_alignment` so the next level's attention buckets divide it; the op
-        zero-fills the extra rows (the reference leaves them uninitialised)."""
+        zero-fills the extra rows (the reference leaves them uninitialised).  build_follows: the caller runs the builder on
+        these clouds next, which writes the id of every point of them; only rows behind them then need clearing."""
         total_n, d = coords.shape
         dev = coords.device
         # The op quantises inside each tile's own box; the whole-batch box is part of the reference
@@ -64,22 +71,16 @@ class SubbuckBuffers:
         bbox_max = torch.full((d,), 65504.0, dtype=torch.float16, device=dev)
         red_len, _, red_sep = calc_red_sep_sizes(seps, subbuck_size)
         aligned = cdiv(red_len, out_alignment) * out_alignment
-        sb = SubbuckBuffers(
+        all_written = build_follows and sum(f3dbatch.host_sizes(seps)) == total_n
+        return SubbuckBuffers(
             bbox_min, bbox_max, red_sep,
-            None,
+            (torch.empty if all_written else torch.zeros)(total_n, dtype=torch.uint32, device=dev),
             torch.empty(total_n, dtype=torch.uint16, device=dev),
             red_sep,
             torch.empty(aligned, d, dtype=torch.float16, device=dev),
             torch.empty(aligned, input_feat.shape[1], dtype=input_feat.dtype, device=dev),
             torch.full((red_len, subbuck_size), total_n + 3, dtype=torch.int32, device=dev).view(torch.uint32),
         )
-        if sum(f3dbatch.host_sizes(seps)) == total_n:      # every point's id is written, nothing to clear
-            if not sb.unpool_ind.is_inference():      # a tensor made in inference mode keeps no version to check later
-                sb.covered = (total_n, sb.unpool_ind, sb.unpool_ind._version)
-            sb.subbuck_id = torch.empty(total_n, dtype=torch.uint32, device=dev)
-        else:
-            sb.subbuck_id = torch.zeros(total_n, dtype=torch.uint32, device=dev)
-        return sb
 
     def remove_unused_buffers(self):
         del self.subbuck_id

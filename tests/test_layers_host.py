@@ -103,10 +103,35 @@ def _pool_buffers(n, tail=0):
     return seps, lambda **kw: subbuck.SubbuckBuffers.create_subbuck_buff(coords, feat, seps, 2, out_alignment=16, **kw)
 
 
+def test_pooling_buffers_cover_rows_only_once_built():
+    """a map nobody has filled has no slot for any row: gradients start from zero, and so do the point ids"""
+    from flash3dtransformer_amd.psh import subbuck
+    for _ in range(3):      # memory that is handed out again holds something
+        seps, make = _pool_buffers(4001)
+        junk = [torch.full((4001, 8), 7.0).to(torch.bfloat16), torch.full((4001,), 7, dtype=torch.int32)]
+        del junk
+        sb = make()
+        assert not sb.covers(4001) and not sb.subbuck_id.view(torch.int32).any()
+        grads = subbuck.UnpoolGradients.create_unpool_grad(torch.ones(4001, 8, dtype=torch.bfloat16), sb, 2016)
+        assert not grads.grad_res.any() and not grads.grad_down[sb.unpool_ind.shape[0]:].any()
+    sb.mark_built(seps, 4001)
+    assert sb.covers(4001) and not sb.covers(4000)
+    sb.unpool_ind.view(torch.int32).add_(1)             # changed since
+    assert not sb.covers(4001)
+    seps, make = _pool_buffers(4001, tail=5)            # rows behind the last cloud
+    sb = make(build_follows=True)
+    sb.mark_built(seps, 4006)
+    assert not sb.covers(4006) and not sb.subbuck_id.view(torch.int32).any()
+
+
 def test_pooling_buffers_in_inference_mode():
     """tensors made there keep no version counter; separators seen before stay usable"""
+    from flash3dtransformer_amd.psh import batching
     seps, make = _pool_buffers(40)
     make()
+    batching.host_sizes(seps)
     with torch.inference_mode():
-        sb = make()
-        assert not sb.covers(40) and sb.unpool_ind.shape == (21, 2)
+        for how in ({}, dict(build_follows=True)):
+            sb = make(**how)
+            sb.mark_built(seps, 40)
+            assert not sb.covers(40) and sb.unpool_ind.shape == (21, 2)
