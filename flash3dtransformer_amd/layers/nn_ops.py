@@ -203,16 +203,18 @@ def as_bf16_2d(x: torch.Tensor) -> torch.Tensor:
     return x
 
 
-def _fresh_copies(caches, params, transposed=()):
+def _fresh_copies(caches, params, transposed=(), apart=()):
     """bf16 copies of a layer's parameters for a forward that records gradients (they are made anew on every such forward,
-    as _Bf16Cache does), in one launch, with the transposed copies that the backward multiplies with.  None where a
-    parameter is not a contiguous fp32 tensor on the GPU: the caller then asks the caches one by one."""
+    as _Bf16Cache does), in one launch, with the transposed copies that the backward multiplies with; a forward whose backward
+    never runs pays for those too.  `apart`: copies that the backward does not read, in memory of their own that is free
+    again after the forward.  None where a parameter is not a contiguous fp32 tensor on the GPU: the caller then asks the
+    caches one by one."""
     for p in params:
         if p is not None and not (p.dtype is torch.float32 and p.is_cuda and p.is_contiguous()):
             return None
     for c in caches:
         c.clear()
-    return pshattn.cast_bf16(params, transposed)
+    return pshattn.cast_bf16(params, transposed, apart)
 
 
 def _grad_out(g, like):
@@ -388,13 +390,15 @@ class Linear(_CachedParamModule):
         y = out if out is not None else torch.empty(x2.shape[0], n_out, dtype=torch.bfloat16, device=x.device)
         r2 = None if residual is None else as_bf16_2d(residual.reshape(-1, n_out))
         g = b = w16t = fresh = None
+        hip_backward = act is None and _hip_backward_covers(x, self.in_features, self.out_features) and (
+            pre_norm is None or (self.in_features in pshattn.LN_BWD_WIDTHS and pre_norm.weight is not None))
         if torch.is_grad_enabled():
             own_norm = isinstance(pre_norm, LayerNorm)
             caches, params = [self._w, self._b], [self.weight, self.bias]
             if own_norm:
                 caches, params = caches + [pre_norm._w, pre_norm._b], params + [pre_norm.weight, pre_norm.bias]
-            wants_dx = act is None and _grad_wanted(x, *params[2:])
-            fresh = _fresh_copies(caches, params, (0,) if wants_dx else ())
+            flipped = (0,) if hip_backward and _grad_wanted(x, *params[2:]) else ()      # the weight, for dx
+            fresh = _fresh_copies(caches, params, flipped, flipped)
         if fresh is not None:
             w16, b16 = fresh[0][:2]
             w16t = fresh[1][0] if fresh[1] else None
@@ -415,8 +419,7 @@ class Linear(_CachedParamModule):
         res_in = None if residual is None else residual.reshape(-1, n_out)
         if not _grad_wanted(x_in, self.weight, self.bias, res_in, ln_w, ln_b):
             return y.view(*lead, n_out)
-        if act is None and _hip_backward_covers(x_in, self.in_features, self.out_features) and (
-                pre_norm is None or (self.in_features in pshattn.LN_BWD_WIDTHS and g is not None)):
+        if hip_backward:
             out = _LinearGrad.apply(y, x_in, self.weight, self.bias, res_in, ln_w, ln_b, eps, w16, g, b, w16t)
         else:
             out = torch_backward(y, _linear_ref(act, eps), x_in, self.weight, self.bias, res_in, ln_w, ln_b)
@@ -684,8 +687,12 @@ class LayerNormMLP(_CachedParamModule):
         x2 = as_bf16_2d(x.reshape(-1, self.hidden_size)).contiguous()
         params = (self.layer_norm_weight, self.layer_norm_bias, self.fc1_weight, self.fc1_bias, self.fc2_weight, self.fc2_bias)
         fresh, w1t, w2t = None, None, None
+        hip_backward = self.activation == "swiglu" and self.hidden_size in pshattn.LN_BWD_WIDTHS \
+            and _hip_backward_covers(x, self.ffn_hidden_size) and (residual is None or residual.dtype == torch.bfloat16)
         if torch.is_grad_enabled():
-            fresh = _fresh_copies(self._c, params, (2, 4) if _grad_wanted(x, residual, *params) else ())
+            # the backward takes fc1 as it is (to form the gate again) and both weights transposed
+            flipped = (2, 4) if hip_backward and _grad_wanted(x, residual, *params) else ()
+            fresh = _fresh_copies(self._c, params, flipped, flipped[1:])
         if fresh is not None:
             g16, be16, w1_16, b1_16, w2_16, b2_16 = fresh[0]
             if fresh[1]:
@@ -720,8 +727,7 @@ class LayerNormMLP(_CachedParamModule):
         res_in = None if residual is None else residual.reshape(-1, self.hidden_size)
         if not _grad_wanted(x_in, res_in, *params):
             return y.view(x.shape)
-        if self.activation == "swiglu" and self.hidden_size in pshattn.LN_BWD_WIDTHS \
-                and _hip_backward_covers(x_in, self.ffn_hidden_size) and (res_in is None or res_in.dtype == torch.bfloat16):
+        if hip_backward:
             out = _GatedMLPGrad.apply(y, x_in, res_in, *params, self.eps, g16, be16, w1_16, b1_16, w2_16, w1t, w2t)
             return out.view(x.shape)
         act, eps = self.activation, self.eps

@@ -621,9 +621,10 @@ def gemm_sm_bf16(A, B, O):
 ACT = {None: 0, "none": 0, "gelu": 1, "swiglu": 2, "silu": 3, "relu": 4}
 
 
-def cast_bf16(tensors, transposed=()):
+def cast_bf16(tensors, transposed=(), apart=()):
     """extension: bf16 copies of contiguous fp32 tensors of one or two axes (None entries are passed through), all made in
-    one launch and laid out in one buffer; `transposed`: positions whose transposed copies are wanted too.  Returns
+    one launch and laid out in one buffer; `transposed`: positions whose transposed copies are wanted too; `apart`: positions
+    whose copies lie in a second buffer, so that their memory does not live as long as that of the others.  Returns
     (copies, transposed copies in the order of `transposed`)."""
     live = [t for t in tensors if t is not None]
     dev = assert_same_device(live)
@@ -631,13 +632,18 @@ def cast_bf16(tensors, transposed=()):
     assert_contiguous(live)
     if len(live) > 16 or any(t.dim() not in (1, 2) for t in live):
         raise RuntimeError("cast_bf16 takes up to 16 tensors of one or two axes")
-    places, total = [], 0      # every copy starts at a multiple of 16 bytes
+    places, total, total_apart = [], 0, 0      # every copy starts at a multiple of 16 bytes
     for i, t in enumerate(tensors):
-        n = 0 if t is None else t.numel()
-        room = (n + 7) // 8 * 8
-        places.append((total, total + room))
-        total += 2 * room if i in transposed else room
+        room = 0 if t is None else (t.numel() + 7) // 8 * 8
+        if i in apart:
+            at, total_apart = total_apart, total_apart + room
+        else:
+            at, total = total, total + room
+        places.append((at, total))
+        if i in transposed:
+            total += room
     flat = torch.empty(total, dtype=torch.bfloat16, device=live[0].device)
+    second = torch.empty(total_apart, dtype=torch.bfloat16, device=live[0].device) if total_apart else flat
     base = flat.data_ptr()
     table, copies = [], []
     for i, (t, (at, at_t)) in enumerate(zip(tensors, places)):
@@ -645,8 +651,9 @@ def cast_bf16(tensors, transposed=()):
             copies.append(None)
             continue
         rows, cols = t.shape if t.dim() == 2 else (1, t.shape[0])
-        table += (t.data_ptr(), base + 2 * at, base + 2 * at_t if i in transposed else 0, rows, cols)
-        copies.append(flat.as_strided(t.shape, (cols, 1) if t.dim() == 2 else (1,), at))
+        buf = second if i in apart else flat
+        table += (t.data_ptr(), buf.data_ptr() + 2 * at, base + 2 * at_t if i in transposed else 0, rows, cols)
+        copies.append(buf.as_strided(t.shape, (cols, 1) if t.dim() == 2 else (1,), at))
     _check(_load().f3d_cast_bf16((ctypes.c_uint64 * len(table))(*table), len(live), dev, _stream(dev)))
     return copies, [flat.as_strided(tensors[i].shape[::-1], (tensors[i].shape[0], 1), places[i][1]) for i in transposed]
 

@@ -549,6 +549,13 @@ def test_cast_bf16_many_tensors_at_once(shapes, transposed):
                                               and c.data_ptr() % 16 == 0)
     for i, t in zip(transposed, flipped):
         assert torch.equal(t, src[i].to(torch.bfloat16).t()) and t.is_contiguous() and t.data_ptr() % 16 == 0
+    apart = transposed[:1]      # the same copies with one of them in a buffer of its own
+    copies2, flipped2 = pshattn.cast_bf16(src, transposed, apart)
+    for a, b in zip(copies + flipped, copies2 + flipped2):
+        assert (a is None and b is None) or torch.equal(a, b)
+    storage = lambda t: t.untyped_storage().data_ptr()
+    for i in apart:
+        assert all(storage(copies2[i]) != storage(t) for j, t in enumerate(copies2 + flipped2) if t is not None and j != i)
     with pytest.raises(RuntimeError):
         pshattn.cast_bf16([torch.zeros(4, 4, dtype=torch.bfloat16, device=DEV)])
     with pytest.raises(RuntimeError):

@@ -237,3 +237,51 @@ def test_gated_mlp_layer_gradients_vs_autograd(M, C, hid):
     assert rel(x.grad, xr.grad) <= 1e-2
     for k, p in mlp.named_parameters():
         assert rel(p.grad, ps[k].grad) <= 1e-2, (k, rel(p.grad, ps[k].grad))
+
+
+@pytest.mark.parametrize("layer", ["linear", "norm_linear", "mlp"])
+def test_bf16_weight_copies_kept_for_the_backward(layer):
+    """what a forward keeps beside parameters and activations: one layout of a weight, both only where the backward reads both"""
+    from flash3dtransformer_amd import layers as L
+    C, H, M = 256, 1024, 64
+    x = torch.randn(M, C, device=DEV).to(torch.bfloat16).requires_grad_()
+    if layer == "mlp":
+        mods, weights = [L.LayerNormMLP(C, H).to(DEV)], 2 * 2 * H * C + C * H      # fc1 twice, fc2 once
+        call = lambda: mods[0](x)
+    else:
+        mods, weights = [L.Linear(C, H).to(DEV), L.LayerNorm(C).to(DEV)], H * C
+        call = lambda: mods[0](x, pre_norm=mods[1] if layer == "norm_linear" else None)
+    known = {p.untyped_storage().data_ptr() for m in mods for p in m.parameters()} | {x.untyped_storage().data_ptr()}
+    kept = {}
+
+    def pack(t):
+        if t.untyped_storage().data_ptr() not in known:
+            kept[t.untyped_storage().data_ptr()] = t.untyped_storage().nbytes()
+        return t
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        y = call()
+    vectors = 4 * (C + 8) + 2 * (2 * H + 8)
+    assert sum(kept.values()) <= 2 * (weights + vectors), kept
+    y.float().sum().backward()
+    assert x.grad is not None
+
+
+@pytest.mark.parametrize("what", ["gelu mlp", "fp32 input", "width", "gelu linear", "no dx"])
+def test_no_transposed_copies_without_the_kernels_that_read_them(what, monkeypatch):
+    from flash3dtransformer_amd import layers as L
+    from flash3dtransformer_amd.lib import pshattn
+    asked, cast = [], pshattn.cast_bf16
+    monkeypatch.setattr(pshattn, "cast_bf16", lambda ts, transposed=(), *rest: (asked.append(tuple(transposed)), cast(ts, transposed, *rest))[1])
+    x = torch.randn(40, 256, device=DEV).to(torch.bfloat16).requires_grad_(what != "no dx")
+    if what == "gelu mlp":
+        y = L.LayerNormMLP(256, 512, activation="gelu").to(DEV)(x)
+    elif what == "fp32 input":
+        y = L.LayerNormMLP(256, 512).to(DEV)(x.detach().float().requires_grad_())
+    elif what == "width":      # no LayerNorm backward kernel: torch differentiates
+        y = L.LayerNormMLP(96, 192).to(DEV)(torch.randn(40, 96, device=DEV).to(torch.bfloat16).requires_grad_())
+    elif what == "gelu linear":
+        y = L.Linear(256, 64).to(DEV)(x, act="gelu")
+    else:
+        y = L.Linear(256, 64).to(DEV)(x)
+    y.float().sum().backward()
+    assert asked and not any(asked), asked
