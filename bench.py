@@ -252,7 +252,7 @@ def main():
                "embed_proj_ln_mlp_residual": "ln_mlp_swiglu_kernel<256, true, true> + mlp_prep_kernel",
                "ln_fc1_act": "xstat_linear_kernel<256,2,8,3,LN,swiglu> + ln_fold_kernel",
                "proj_residual": "xstat_linear_kernel<256,2,8,3,residual>",
-               "fc2_residual": "ystat_linear_kernel<256> + ys_w_prep_kernel",
+               "fc2_residual": "ystat_linear_kernel<256, 2>",
                "ln_mlp_residual": "ln_mlp_swiglu_kernel<256, false> + mlp_prep_kernel",
                "proj_ln_mlp_residual": "ln_mlp_swiglu_kernel<256, true> + mlp_prep_kernel"}
     all_flops = dict(flops)

@@ -648,7 +648,7 @@ class LayerNormMLP(_CachedParamModule):
         nn.init.normal_(self.fc1_weight, std=0.023)
         nn.init.normal_(self.fc2_weight, std=0.023)
         self._c = [_Bf16Cache() for _ in range(6)]
-        self._staged = [_StagedWeights(), _StagedWeights()]      # fused kernel / fc1 of the two-kernel path; fc2
+        self._staged = _StagedWeights()      # fused kernel / fc1 of the two-kernel path
 
     def after_projection(self, a: torch.Tensor, proj: "Linear", x: torch.Tensor):
         """x1 = proj(a) + x;  x1 + MLP(x1) in one kernel (x1 is never stored): the second half of a transformer block
@@ -669,7 +669,7 @@ class LayerNormMLP(_CachedParamModule):
         g16, be16, w1_16, b1_16, w2_16, b2_16 = (c.get(p, self.training) for c, p in zip(self._c, params))
         wp16, bp16 = proj._w.get(proj.weight, proj.training), proj._b.get(proj.bias, proj.training)
         y = torch.empty(a2.shape[0], self.hidden_size, dtype=torch.bfloat16, device=a.device)
-        self._staged[0].arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16, w2_16, b2_16,
+        self._staged.arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16, w2_16, b2_16,
                             tag=("mlp", float(self.eps)))
         if lazy is not None:
             ok = pshattn.embed_proj_ln_mlp_swiglu_bf16(a2, wp16, bp16, lazy.coord, lazy.table(), g16, be16, self.eps, w1_16,
@@ -706,22 +706,20 @@ class LayerNormMLP(_CachedParamModule):
         fused = (want_fused and self.activation == "swiglu" and self.hidden_size in FUSED_MLP_WIDTHS
                  and self.ffn_hidden_size % 32 == 0)
         if fused:
-            self._staged[0].arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16, w2_16, b2_16,
+            self._staged.arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16, w2_16, b2_16,
                                 tag=("mlp", float(self.eps)))
             fused = pshattn.ln_mlp_swiglu_bf16(x2, g16, be16, self.eps, w1_16, b1_16, w2_16, b2_16, r2, y)
         if not fused:
             # ... otherwise LayerNorm + fc1 + activation, then fc2 + residual
             h = torch.empty(x2.shape[0], self.ffn_hidden_size, dtype=torch.bfloat16, device=x.device)
             if self.hidden_size in FUSABLE_LN_WIDTHS:
-                self._staged[0].arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16,
+                self._staged.arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16,
                                     tag=("fc1", float(self.eps)))
                 pshattn.ln_linear_bf16(x2, g16, be16, self.eps, w1_16, b1_16, None, h, self.activation)
             else:
                 ln = torch.empty_like(x2)
                 pshattn.layernorm_bf16(x2, g16, be16, ln, self.eps)
                 pshattn.linear_bf16(ln, w1_16, b1_16, None, h, self.activation)
-            if self.ffn_hidden_size > 512:
-                self._staged[1].arm(self.training, self.hidden_size, self.ffn_hidden_size, w2_16, b2_16, tag="ys")
             pshattn.linear_bf16(h, w2_16, b2_16, r2, y, None)
         x_in = x.reshape(-1, self.hidden_size)
         res_in = None if residual is None else residual.reshape(-1, self.hidden_size)

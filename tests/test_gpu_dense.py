@@ -457,13 +457,13 @@ def test_staged_weights_are_reused_and_refreshed():
     ln = L.LayerNorm(256).to(DEV).eval()
     lin = L.Linear(256, 768).to(DEV).eval()
     mlp = L.LayerNormMLP(256, 1024).to(DEV).eval()
-    wide = L.LayerNormMLP(512, 2048).to(DEV).eval()          # two-kernel path: fc1 fold and the re-laid fc2 weight
+    wide = L.LayerNormMLP(512, 2048).to(DEV).eval()          # two-kernel path: fc1 fold (fc2 reads its weight as it is)
     x = torch.randn(40000, 256, device=DEV).to(torch.bfloat16)
     xw = torch.randn(40000, 512, device=DEV).to(torch.bfloat16)
     with torch.no_grad():
         ln.weight.add_(torch.randn_like(ln.weight) * 0.1)
         first = [lin(x, pre_norm=ln), mlp(x, residual=x), wide(xw)]
-        assert lin._staged._key is not None and mlp._staged[0]._key is not None and wide._staged[1]._key is not None
+        assert all(m._staged._key is not None for m in (lin, mlp, wide))
         second = [lin(x, pre_norm=ln), mlp(x, residual=x), wide(xw)]
         for a, b in zip(first, second):
             assert torch.equal(a, b)

@@ -96,6 +96,12 @@ def test_layernorm_qkv_of_a_rank4_embedding_folds_to_four_numbers_per_feature():
     assert ((rstd * (c @ (w @ Ep).T) + bp) - want).abs().max().item() > 1e-3
 
 
+def test_layers_keep_one_buffer_of_prepared_weights():
+    """only the kernel with the LayerNorm inside prepares weights: one buffer a layer, the second linear of an MLP has none"""
+    for layer in (L.Linear(512, 512), L.LayerNormMLP(512, 2048), L.LayerNormMLP(128, 512, activation="gelu")):
+        assert sum(isinstance(c, nn_ops._StagedWeights) for c in layer._bf16_caches()) == 1
+
+
 def _pool_buffers(n, tail=0):
     from flash3dtransformer_amd.psh import subbuck
     seps = torch.tensor([3, n], dtype=torch.int32)
