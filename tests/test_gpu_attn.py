@@ -357,10 +357,10 @@ def test_backward_vs_oracle(oracle, B, L, H, D, bs, scope_size, fused):
     (2, 2048, 3, 64, 256, 2, True),      # 64-wide heads
     (1, 2048, 2, 128, 256, 4, False),    # 128-wide heads
     (1, 1536, 1, 16, 128, 6, False),     # 16-wide heads, a scope of six buckets
-    (1, 1024, 5, 64, 512, 1, False),     # wide heads on a scope the resident kernels would hold
+    (1, 1024, 5, 64, 512, 1, False),     # wide heads, scopes of one bucket
 ])
 def test_streaming_backward_vs_oracle(oracle, B, L, H, D, bs, scope_size, fused):
-    """head sizes and scopes beyond the scope-resident kernels: the streaming kernels"""
+    """the other head sizes, and scopes of more buckets"""
     Q, K, V = _qkv(70 + D + bs, B, L, H, D)
     dO = torch.randn(B, L, H, D, generator=torch.Generator().manual_seed(13)).to(torch.bfloat16)
     nb = L // bs
@@ -391,8 +391,7 @@ def test_backward_reference_test_shape_one_global_scope(oracle, D):
 
 
 def test_backward_with_valid_lengths(oracle):
-    """kv_len in the backward: full lengths (through the streaming kernels' mask path) agree with no lengths (the
-    resident kernels) within tolerance; ragged, one-key and empty buckets follow the oracle and give exact zeros on
+    """kv_len in the backward: full lengths agree with no lengths within tolerance; ragged, one-key and empty buckets follow the oracle and give exact zeros on
     the masked rows"""
     B, L, H, D, bs = 1, 4096, 2, 32, 512
     Q, K, V = _qkv(90, B, L, H, D)
@@ -401,7 +400,7 @@ def test_backward_with_valid_lengths(oracle):
         scopes = oracle.gen_scopes(L, bs, scope_size)
         plain = _run_bwd(Q, K, V, dO, scopes, bs)
         full = _run_bwd(Q, K, V, dO, scopes, bs, kv_len=np.full(L // bs, bs))
-        _check_grads(full[:3], plain[:3], "full lengths vs resident kernels")
+        _check_grads(full[:3], plain[:3], "full lengths vs none")
         kl = np.random.default_rng(1003).integers(300, 513, L // bs)
         kl[0], kl[1], kl[5] = 1, 0, 33
         dq, dk, dv, delta, O = _run_bwd(Q, K, V, dO, scopes, bs, kv_len=kl)
@@ -495,9 +494,8 @@ def test_backward_delta_is_one_sum_in_feature_order(H, D, bs, scope_size, masked
 
 
 def test_streaming_backward_more_than_65535_items(oracle):
-    """8,192 one-bucket scopes of 128 tokens x 8 heads = 65,536 (batch, scope, head) items, one more than a launch's
-    grid.y holds: the forward takes them in one launch, the backward in two.  Gradients of scopes at both ends of the
-    list (the last item is the one the second launch covers) against the oracle."""
+    """8,192 one-bucket scopes of 128 tokens x 8 heads = 65,536 (batch, scope, head) items, more than 16 bits number: forward
+    and backward take them in one launch.  Gradients of scopes at both ends of the list against the oracle."""
     B, H, D, bs = 1, 8, 16, 128
     n_scope = 8192
     L = n_scope * bs
