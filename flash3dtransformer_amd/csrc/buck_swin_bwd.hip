@@ -22,9 +22,11 @@
 // there (the forward gave them O = 0, LSE = 0): their gradients are zero and they add nothing to dK / dV.  Masked rows of
 // q, k, v, o, dO and LSE may hold anything: the tiles repeat the last valid row instead of reading them.
 //
-// What bounds it: mostly the vector issue port.  A 32 x 32 block at D = 32 takes 32 exponentials (16 clocks each), 16
-// conversions and 112 multiply-type instructions over the two kernels next to 14 matrix products, about 1,030 clocks of
-// issue; it takes 1,450.  Hence: masking costs nothing in the loops (an infinite LSE for masked queries, 8 ANDs in a bucket's
+// What bounds it: mostly vector issue.  A 32 x 32 block at D = 32 (32 exponentials, 16 conversions, 112 multiply-type
+// instructions and 14 matrix products over the two kernels) keeps a SIMD's vector ALU active for 880 clocks and takes 1,120
+// in scopes of 4,096 rows (counters: dK / dV 73 % of 615 clocks, dQ 86 % of 503); in scopes of 512 it is 970 of 1,560, where
+// loading the wave's own rows and storing its gradients weigh against 16 blocks instead of 128.
+// Hence: masking costs nothing in the loops (an infinite LSE for masked queries, 8 ANDs in a bucket's
 // last key tile; a masked key or query of the wave itself spoils only its own column and is zeroed by the store), the walk
 // over buckets has no division, the LSE is brought to the exponent's units once per tile by the wave that loaded it, up to
 // four 32-row sub-tiles share a barrier, and all streamed data including LSE and Delta arrives by direct loads (passing LSE
