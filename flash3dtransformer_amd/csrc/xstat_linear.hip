@@ -6,10 +6,11 @@
 //
 // Why not an output-tiled GEMM: with K this small a 128x128 tile re-reads 128 KB of operands per
 // 8 MFLOP, which saturates L2 long before the matrix cores.  Here a workgroup owns a panel of
-// 32 * MT * WAVES rows of x for ALL output columns (for a share of them where the rows alone leave CUs idle): every wave keeps its 32 * MT rows, already in the
-// MFMA B-operand layout, in registers for the whole kernel (x is read from HBM exactly once), while w
-// streams through LDS in chunks of 64 output features.  Each 16-byte LDS fragment read feeds MT MFMAs;
-// with MT = 1 the LDS read port is as busy as the matrix cores, so the large configuration uses MT = 2.
+// 32 * MT * WAVES rows of x for ALL output columns (for a share of them where the rows alone leave CUs
+// idle): every wave keeps its 32 * MT rows, already in the MFMA B-operand layout, in registers for the
+// whole kernel (x is read from HBM exactly once), while w streams through LDS in chunks of 64 output
+// features.  Each 16-byte LDS fragment read feeds MT MFMAs; with MT = 1 the LDS read port is as busy as
+// the matrix cores, so the large configuration uses MT = 2.
 // The product is formed transposed (A = w rows, B = x rows) so a lane owns 4 consecutive output columns
 // of one row for the epilogue (bias, GELU / SiLU / ReLU / swiglu, residual, bf16 store).
 //
