@@ -13,6 +13,8 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "lib", "libf3d_hip.so")
+HOST_SRC = os.path.join(HERE, "host", "f3d_host.cpp")
+HOST_LIB = os.path.join(PKG, "lib", "_f3d_host.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 COMMON = [
@@ -56,6 +58,32 @@ def _compile(src, incremental=False):
     return obj
 
 
+def _build_host(incremental=False):
+    """the layers' native driver: a Python module over torch's C++ API that calls the library beside it"""
+    import sysconfig
+
+    import torch
+    newest = max(os.path.getmtime(HOST_SRC), os.path.getmtime(os.path.join(os.path.dirname(PKG), "include", "f3d_hip.h")),
+                 os.path.getmtime(__file__))
+    if incremental and os.path.exists(HOST_LIB) and os.path.getmtime(HOST_LIB) > newest:
+        return HOST_LIB
+    root = os.path.dirname(torch.__file__)
+    inc, libs = os.path.join(root, "include"), os.path.join(root, "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-DTORCH_EXTENSION_NAME=_f3d_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+           "-isystem", sysconfig.get_paths()["include"], HOST_SRC, "-o", HOST_LIB,
+           "-L" + os.path.dirname(LIB), "-lf3d_hip", "-L" + libs, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch",
+           "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    p = subprocess.run(cmd, capture_output=True, text=True)
+    if p.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SRC}:\n{p.stderr}")
+    if p.stderr.strip():
+        sys.stderr.write(p.stderr + "\n")
+    return HOST_LIB
+
+
 def build(verbose=True, jobs=None, incremental=False):
     """incremental=True keeps objects that are newer than their source, every header and this file (a developer's
     shortcut: `python -m flash3dtransformer_amd.csrc.build -i`); the default compiles everything."""
@@ -69,6 +97,7 @@ def build(verbose=True, jobs=None, incremental=False):
     p = subprocess.run(cmd, capture_output=True, text=True)
     if p.returncode != 0:
         raise RuntimeError(f"link failed:\n{p.stderr}")
+    _build_host(incremental)
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources")
     return LIB

@@ -141,7 +141,12 @@ class BucketSwinAttentionModule(nn.Module):
         if attn_out is None:
             # pre_norm: LayerNorm applied inside the projection kernel; a CoordEmbedding is formed there too
             qkv = self.qkv.embedded(x, pre_norm).view(B, L, -1) if isinstance(x, CoordEmbedding) else self.qkv(x, pre_norm=pre_norm)
-            if qkv.dtype == torch.bfloat16 and qkv.is_contiguous():
+            if qkv.is_cuda:
+                attn_out = pshattn.host().attention_qkv(qkv, scope_buckets, self.attn.buck_size, self.num_heads,
+                                                        _covers(scope_buckets, self.attn.buck_size, L))
+            if attn_out is not None:
+                pass
+            elif qkv.dtype == torch.bfloat16 and qkv.is_contiguous():
                 attn_out = BuckSwinQKVFunction.apply(qkv, scope_buckets, self.attn.buck_size, self.num_heads)
             else:
                 q, k, v = (t.view(B, L, self.num_heads, self.head_dim) for t in torch.chunk(qkv, 3, dim=-1))

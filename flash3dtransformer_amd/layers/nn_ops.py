@@ -158,12 +158,40 @@ class _DerivedCache(_Bf16Cache):
         return self._val
 
 
+class _HostCache:
+    """The native driver's copies of a block's parameters (`WeightCache` of csrc/host/f3d_host.cpp, same rules as
+    `_Bf16Cache` and `_StagedWeights`).  A copied or unpickled module starts with an empty one."""
+
+    def __init__(self):
+        self._native = None
+        self._generation = None
+
+    def __reduce__(self):
+        return _HostCache, ()
+
+    def clear(self):
+        if self._native is not None:
+            self._native.clear()
+
+    def get(self, modules):
+        """current for the parameters' addresses and versions by itself; dropped here when one of the modules that own them
+        was refreshed since"""
+        generation = [m._generation for m in modules]
+        if self._native is None:
+            self._native = pshattn.host().WeightCache()
+        elif generation != self._generation:
+            self._native.clear()
+        self._generation = generation
+        return self._native
+
+
 class _CachedParamModule(nn.Module):
     """nn.Module whose kernels read bf16 copies of its parameters (`_Bf16Cache` attributes or lists of them)"""
+    _generation = 0      # counts refresh_weights(): a cache outside the module notices that its copies are to be dropped
 
     def _bf16_caches(self):
         for v in self.__dict__.values():
-            if isinstance(v, (_Bf16Cache, _StagedWeights)):
+            if isinstance(v, (_Bf16Cache, _StagedWeights, _HostCache)):
                 yield v
             elif isinstance(v, (list, tuple)):
                 for c in v:
@@ -171,6 +199,7 @@ class _CachedParamModule(nn.Module):
                         yield c
 
     def refresh_weights(self):
+        self._generation += 1
         for c in self._bf16_caches():
             c.clear()
 
@@ -384,6 +413,20 @@ class Linear(_CachedParamModule):
     def forward(self, x: torch.Tensor, residual: torch.Tensor = None, act=None, out: torch.Tensor = None,
                 pre_norm=None):
         """`pre_norm`: a LayerNorm-like module (weight, bias, eps) applied to x inside the same kernel"""
+        if act is None and out is None and x.requires_grad and torch.is_grad_enabled() and x.is_cuda and (
+                pre_norm is None or (isinstance(pre_norm, LayerNorm) and self.in_features in pshattn.LN_BWD_WIDTHS)):
+            if pre_norm is None:
+                y = pshattn.host().linear_train(x, self.weight, self.bias, residual, None, None, 0.0)
+            else:
+                y = pshattn.host().linear_train(x, self.weight, self.bias, residual, pre_norm.weight, pre_norm.bias, pre_norm.eps)
+            if y is not None:
+                for c in (self._w, self._b) if pre_norm is None else (self._w, self._b, pre_norm._w, pre_norm._b):
+                    c.clear()
+                return y
+        elif act is None and out is None and pre_norm is None and x.is_cuda and not torch.is_grad_enabled():
+            y = pshattn.host().linear_infer(x, self._w.get(self.weight, self.training), self._b.get(self.bias, self.training), residual)
+            if y is not None:
+                return y
         lead = x.shape[:-1]
         x2 = as_bf16_2d(x.reshape(-1, x.shape[-1]))
         n_out = self.out_features // 2 if act == "swiglu" else self.out_features
@@ -683,7 +726,21 @@ class LayerNormMLP(_CachedParamModule):
         return not (torch.is_grad_enabled() or self.activation != "swiglu" or self.hidden_size not in PROJ_MLP_WIDTHS
                     or self.ffn_hidden_size % 32 != 0 or self.fused is False or (self.hidden_size == 256 and rows < 30000))
 
+    def one_kernel(self, rows: int) -> bool:
+        """whether the whole MLP runs as one kernel (hidden activations stay in registers) at `rows` rows"""
+        want = self.fused if self.fused is not None else (self.hidden_size <= 128 or rows >= 30000)
+        return (want and self.activation == "swiglu" and self.hidden_size in FUSED_MLP_WIDTHS
+                and self.ffn_hidden_size % 32 == 0)
+
     def forward(self, x: torch.Tensor, residual: torch.Tensor = None):
+        if self.activation == "swiglu" and x.requires_grad and torch.is_grad_enabled() and x.is_cuda \
+                and self.hidden_size in pshattn.LN_BWD_WIDTHS:
+            y = pshattn.host().mlp_train(x, residual, self.layer_norm_weight, self.layer_norm_bias, self.fc1_weight, self.fc1_bias,
+                                         self.fc2_weight, self.fc2_bias, self.eps, self.one_kernel(x.numel() // self.hidden_size))
+            if y is not None:
+                for c in self._c:
+                    c.clear()
+                return y
         x2 = as_bf16_2d(x.reshape(-1, self.hidden_size)).contiguous()
         params = (self.layer_norm_weight, self.layer_norm_bias, self.fc1_weight, self.fc1_bias, self.fc2_weight, self.fc2_bias)
         fresh, w1t, w2t = None, None, None
@@ -701,10 +758,8 @@ class LayerNormMLP(_CachedParamModule):
             g16, be16, w1_16, b1_16, w2_16, b2_16 = (c.get(p, self.training) for c, p in zip(self._c, params))
         r2 = None if residual is None else as_bf16_2d(residual.reshape(-1, self.hidden_size))
         y = torch.empty_like(x2)
-        # on request, the whole gated MLP in one kernel where one exists (hidden activations stay in registers) ...
-        want_fused = self.fused if self.fused is not None else (self.hidden_size <= 128 or x2.shape[0] >= 30000)
-        fused = (want_fused and self.activation == "swiglu" and self.hidden_size in FUSED_MLP_WIDTHS
-                 and self.ffn_hidden_size % 32 == 0)
+        # on request, the whole gated MLP in one kernel where one exists ...
+        fused = self.one_kernel(x2.shape[0])
         if fused:
             self._staged.arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16, w2_16, b2_16,
                                 tag=("mlp", float(self.eps)))

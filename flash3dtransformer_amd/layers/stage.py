@@ -6,10 +6,12 @@ import torch
 import torch.cuda.nvtx as nvtx
 from torch import nn
 
+from ..lib import pshattn
 from ..psh import bucket_scope
 from ..psh import dev_context as f3ddev
 from . import buck_swin, elem_wise
-from .nn_ops import CoordEmbedding, apply_norm, is_fusable_layernorm, materialize
+from .nn_ops import (CoordEmbedding, LayerNorm, LayerNormMLP, Linear, _CachedParamModule, _HostCache, apply_norm,
+                     is_fusable_layernorm, materialize)
 
 
 @dataclass(slots=True)
@@ -22,7 +24,19 @@ class XFMRSpecs:
     norm_layer: callable
 
 
-class XFMR(nn.Module):
+def _as_built(module: nn.Module, kind: type) -> bool:
+    """the package's own class with no hooks and no forward of its own: skipping its __call__ changes nothing"""
+    return type(module) is kind and "forward" not in module.__dict__ and not (
+        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+def _global_hooks() -> bool:
+    m = torch.nn.modules.module
+    return bool(m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
+                or m._global_backward_pre_hooks)
+
+
+class XFMR(_CachedParamModule):
     """mid = proj(attention(qkv(norm(x)))) + x;  out = MLP(mid) + mid   (stage.py:71-102 of the reference).
     Takes the (coord, feat, sep) triplet of the submodule interface and uses only `feat`."""
     NVTX_SCOPE = "XFMR"
@@ -35,12 +49,34 @@ class XFMR(nn.Module):
         self.norm = norm_layer(channels)
         self.bwa = buck_swin.BucketSwinAttentionModule(channels, num_heads, buck_size, qkv_bias)
         self.mlp = elem_wise.MLP(channels, hid_chann, mlp_activation)
+        self._host = _HostCache()
+
+    def _whole_block(self, x: torch.Tensor, scope_bucks: torch.Tensor):
+        """The block at inference through one call of the native driver, which runs the kernels the code in forward() runs;
+        None where it does not apply (training mode, hooks, modules of other classes, other dtypes or widths)."""
+        norm, bwa, mlp = self.norm, self.bwa, self.mlp
+        if not (_as_built(norm, LayerNorm) and _as_built(bwa, buck_swin.BucketSwinAttentionModule) and _as_built(mlp, elem_wise.MLP)):
+            return None
+        qkv, proj, ff = bwa.qkv, bwa.proj, mlp.mlp
+        if not (_as_built(qkv, Linear) and _as_built(proj, Linear) and _as_built(ff, LayerNormMLP)) or _global_hooks() \
+                or norm.training or qkv.training or proj.training or ff.training or ff.activation != "swiglu" or f3ddev.get_nvtx():
+            return None
+        rows = x.shape[0]
+        params = [norm.weight, norm.bias, qkv.weight, qkv.bias, proj.weight, proj.bias, ff.layer_norm_weight, ff.layer_norm_bias,
+                  ff.fc1_weight, ff.fc1_bias, ff.fc2_weight, ff.fc2_bias]
+        return pshattn.host().block_infer(
+            self._host.get((norm, qkv, proj, ff)), x, params, norm.eps, ff.eps, scope_bucks, bwa.attn.buck_size, bwa.num_heads,
+            buck_swin._covers(scope_bucks, bwa.attn.buck_size, rows), ff.takes_projection(rows), ff.one_kernel(rows))
 
     def forward(self, reduced_coord, reduced_feat: torch.Tensor, reduced_sep) -> torch.Tensor:
         assert reduced_feat.dim() == 2, f"Expect input features have two axes [N, C], but got shape={reduced_feat.shape}"
         N, C = reduced_feat.shape
         assert C == self.set_chnn, f"Expect input feat_dim={self.set_chnn}, but got {C}"
         scope_bucks = self.swin_plan.gen_scopes_from_plan(N, reduced_feat.device)
+        if type(reduced_feat) is torch.Tensor and reduced_feat.is_cuda and not torch.is_grad_enabled():
+            out = self._whole_block(reduced_feat, scope_bucks)
+            if out is not None:
+                return out
         if f3ddev.get_nvtx():
             nvtx.range_push(self.NVTX_SCOPE)
         fused_ln = is_fusable_layernorm(self.norm, C)   # norm -> qkv in one kernel

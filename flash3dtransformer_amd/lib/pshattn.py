@@ -91,6 +91,23 @@ def library_path() -> str:
     return _LIB_PATH
 
 
+_host = None
+
+
+def host():
+    """the native driver of the layers' hot calls (csrc/host/f3d_host.cpp), beside the library it calls"""
+    global _host
+    if _host is None:
+        _load()
+        try:
+            from . import _f3d_host
+        except ImportError as e:
+            raise RuntimeError(f"the native driver beside {_LIB_PATH} is missing or does not load ({e}): build it with "
+                               "`python -m flash3dtransformer_amd.csrc.build`") from e
+        _host = _f3d_host
+    return _host
+
+
 def _check(rc: int):
     if rc != 0:
         raise RuntimeError(_load().f3d_last_error().decode("utf-8", "replace"))

@@ -1,0 +1,190 @@
+"""The native driver of the layers against the layers' own Python code: the same kernels in the same order on the same
+operands, so every output and gradient is compared bit for bit."""
+import copy
+
+import pytest
+import torch
+from torch import nn
+
+from tests.gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+class _Declines:
+    """a driver that takes no call: the layers run their Python code"""
+    class WeightCache:
+        def clear(self):
+            pass
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+@pytest.fixture
+def python_path(monkeypatch):
+    from flash3dtransformer_amd.lib import pshattn
+
+    def run(f):
+        with monkeypatch.context() as m:
+            m.setattr(pshattn, "_host", _Declines())
+            return f()
+    return run
+
+
+def _same(a, b):
+    assert type(a) is type(b)
+    if isinstance(a, torch.Tensor):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+    elif isinstance(a, (list, tuple)):
+        assert len(a) == len(b)
+        for x, y in zip(a, b):
+            _same(x, y)
+    else:
+        assert a == b
+
+
+def _step(module, call, x, grad_seed=3):
+    """output, dx and every parameter's gradient of one step"""
+    x = x.detach().clone().requires_grad_()
+    module.zero_grad(set_to_none=True)
+    y = call(x)
+    g = torch.randn(y.shape, generator=torch.Generator(device=DEV).manual_seed(grad_seed), device=DEV).to(y.dtype)
+    y.backward(g)
+    return [y.detach(), x.grad] + [p.grad for p in module.parameters() if p.requires_grad]
+
+
+@pytest.mark.parametrize("rows,k,n,bias,norm,residual,form", [
+    (1, 32, 8, True, True, False, "2d"), (33, 64, 192, True, True, False, "3d"), (1000, 256, 256, True, False, True, "3d"),
+    (257, 512, 1536, False, True, False, "2d"), (515, 40, 24, True, False, False, "2d"), (300, 128, 64, True, False, True, "columns"),
+    (96, 96, 32, False, False, False, "frozen weight"),
+])
+def test_linear_training_step(rows, k, n, bias, norm, residual, form, python_path):
+    from flash3dtransformer_amd import layers as L
+    torch.manual_seed(rows + k)
+    lin = L.Linear(k, n, bias=bias)
+    both = nn.ModuleList([lin] + ([L.LayerNorm(k)] if norm else [])).to(DEV)
+    if form == "frozen weight":
+        lin.weight.requires_grad_(False)
+    x = torch.randn(rows, 2 * k if form == "columns" else k, device=DEV).to(torch.bfloat16)
+    res = torch.randn(rows, n, device=DEV).to(torch.bfloat16).requires_grad_() if residual else None
+
+    def call(t):
+        if form == "3d":
+            return lin(t.view(1, rows, k), residual=None if res is None else res.view(1, rows, n), pre_norm=both[1] if norm else None)
+        return lin(t[:, k:] if form == "columns" else t, residual=res, pre_norm=both[1] if norm else None)
+
+    def run():
+        if res is not None:
+            res.grad = None
+        return _step(both, call, x) + ([res.grad] if res is not None else [])
+    _same(run(), python_path(run))
+
+
+@pytest.mark.parametrize("rows,c,hid,own_residual", [(1, 32, 128, True), (333, 64, 256, True), (130, 128, 96, False), (700, 256, 1024, True),
+                                                     (65, 512, 2048, None)])
+def test_mlp_training_step(rows, c, hid, own_residual, python_path):
+    from flash3dtransformer_amd import layers as L
+    torch.manual_seed(c)
+    mlp = L.LayerNormMLP(c, hid).to(DEV)
+    x = torch.randn(rows, c, device=DEV).to(torch.bfloat16)
+    other = torch.randn(rows, c, device=DEV).to(torch.bfloat16).requires_grad_()
+
+    def run():
+        other.grad = None
+        got = _step(mlp, lambda t: mlp(t, None if own_residual is None else t if own_residual else other), x)
+        return got + ([other.grad] if own_residual is False else [])
+    _same(run(), python_path(run))
+
+
+@pytest.mark.parametrize("c,heads,scope,rows,whole", [(64, 2, 1, 1536, True), (32, 2, 2, 2048, True), (128, 2, 1, 1024, False)])
+def test_block_training_step(c, heads, scope, rows, whole, python_path):
+    """whole: a table that covers all rows, as a plan makes it; otherwise a table of the first bucket alone"""
+    from flash3dtransformer_amd import layers as L
+    from flash3dtransformer_amd.psh.bucket_scope import SwinPlan
+    torch.manual_seed(c + scope)
+    blk = L.XFMR(c, 4 * c, heads, 512, True, SwinPlan("swin", 512, scope, 0), lambda ch: L.LayerNorm(ch)).to(DEV)
+    x = torch.randn(rows, c, device=DEV).to(torch.bfloat16)
+    if whole:
+        run = lambda: _step(blk, lambda t: blk(None, t, None), x)
+    else:
+        table = torch.zeros(1, 1, dtype=torch.int32, device=DEV).view(torch.uint32)
+        run = lambda: _step(blk, lambda t: blk.bwa(t.view(1, rows, c), table, skip_proj=True)[:, :512], x)
+    _same(run(), python_path(run))
+
+
+@pytest.mark.parametrize("c,heads,rows,scope", [(32, 1, 512, 1), (64, 2, 4096, 8), (128, 4, 1024, 1), (256, 8, 1536, 1), (256, 8, 30208, 1),
+                                                (512, 16, 1024, 2)])
+def test_block_inference(c, heads, rows, scope, python_path):
+    """equal bits; a changed, replaced or refreshed parameter shows; hooks and other classes take the Python code"""
+    from flash3dtransformer_amd import layers as L
+    from flash3dtransformer_amd.psh.bucket_scope import SwinPlan
+    torch.manual_seed(c)
+    blk = L.XFMR(c, 4 * c, heads, 512, True, SwinPlan("swin", 512, scope, 0), lambda ch: L.LayerNorm(ch)).to(DEV).eval()
+    x = torch.randn(rows, c, device=DEV).to(torch.bfloat16)
+    wide = torch.randn(rows, c + 8, device=DEV).to(torch.bfloat16)
+    run = lambda t=x: blk(None, t, None)
+    with torch.no_grad():
+        first = run()
+        _same(first, python_path(run))
+        _same(run(), first)
+        _same(run(wide[:, :c]), python_path(lambda: run(wide[:, :c])))
+        blk.mlp.mlp.fc1_weight.mul_(1.5)
+        blk.norm.bias.add_(0.25)
+        changed = run()
+        assert not torch.equal(changed, first)
+        _same(changed, python_path(run))
+        blk.bwa.proj.bias.data.add_(1.0)      # leaves address and version alone
+        L.refresh_weights(blk.bwa)
+        refreshed = run()
+        assert not torch.equal(refreshed, changed)
+        _same(refreshed, python_path(run))
+        twin = copy.deepcopy(blk)
+        _same(twin(None, x, None), refreshed)
+        seen = []
+        handle = blk.bwa.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+        _same(run(), refreshed)
+        assert seen
+        handle.remove()
+        blk.to(torch.bfloat16)
+        _same(run(), python_path(run))
+        blk.train()
+        _same(run(), python_path(run))
+
+
+def test_attention_outside_the_kernels_is_told_apart():
+    from flash3dtransformer_amd.layers.buck_swin import BucketSwinAttentionModule
+    m = BucketSwinAttentionModule(48, 2, 512).to(DEV)      # 24-wide heads
+    table = torch.zeros(1, 1, dtype=torch.int32, device=DEV).view(torch.uint32)
+    with pytest.raises(RuntimeError, match="head_dim"):
+        m(torch.zeros(1, 512, 48, dtype=torch.bfloat16, device=DEV), table)
+
+
+@pytest.mark.parametrize("rows,k,n,residual", [(1, 64, 8, False), (2049, 32, 64, True), (300, 136, 72, False)])
+def test_linear_inference(rows, k, n, residual, python_path):
+    from flash3dtransformer_amd import layers as L
+    torch.manual_seed(rows)
+    lin = L.Linear(k, n).to(DEV).eval()
+    x = torch.randn(rows, k, device=DEV).to(torch.bfloat16)
+    res = torch.randn(rows, n, device=DEV).to(torch.bfloat16) if residual else None
+    with torch.no_grad():
+        run = lambda: [lin(x, residual=res), lin(x.view(1, rows, k)), lin(x.float())]
+        _same(run(), python_path(run))
+
+
+def test_saved_tensor_hooks_and_in_place_changes_are_seen():
+    """the native nodes save through autograd: pack hooks run, and a weight changed between forward and backward is refused"""
+    from flash3dtransformer_amd import layers as L
+    lin = L.Linear(64, 64).to(DEV)
+    mlp = L.LayerNormMLP(64, 128).to(DEV)
+    x = torch.randn(40, 64, device=DEV).to(torch.bfloat16).requires_grad_()
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t)[1], lambda t: t):
+        y = mlp(lin(x))
+    assert len(packed) >= 10
+    y.float().sum().backward()
+    y = mlp(lin(x))
+    with torch.no_grad():
+        mlp.fc2_weight.add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.float().sum().backward()
