@@ -8,13 +8,20 @@
 // Weight gradient  dw[n][k] = sum_m dy[m][n] x[m][k]  (fp32 out, bf16 in):
 //   the reduction runs over the rows, which is the slow axis of both operands in memory, so both MFMA operands are
 //   read TRANSPOSED from LDS (ds_read_b64_tr_b16: a lane receives four consecutive rows of one column).  A workgroup of
-//   eight waves (4 x 2, two per SIMD) owns a 256 x 256 tile of dw and one slab of rows; a wave holds 64 x 128 of it in
-//   128 accumulator registers and skips the 32 x 32 blocks that lie outside dw.  32-row stages stream HBM -> LDS
-//   directly (global_load ... lds, no registers) through four stage buffers, so three stages are in flight behind the
-//   one being multiplied; one barrier per stage.  Slabs are sized so that the launch is one round of the chip; every
-//   slab writes its partial tile to the workspace and a second kernel sums the slabs in a fixed order (no atomics: the
-//   result does not depend on scheduling).  The bias gradient rides along in the waves of the first k-tile as one more
-//   product with a matrix of ones.
+//   eight waves (two per SIMD) owns a tile of dw, as wide in either direction as its columns (32, 64, 128 or 256), and one
+//   slab of rows; a wave holds up to 64 x 128 of it in accumulator registers and skips the 32 x 32 blocks that lie outside dw.
+//   Stages of 32 (256 x 256) to 256 rows (32 x 32), 24 to 40 KB each, stream HBM -> LDS directly (global_load ... lds,
+//   no registers) through four stage buffers, so three stages are in flight behind the one being multiplied; one barrier per
+//   stage.  Where a tile has fewer blocks than waves, the waves share the rows of a stage and add their sums at the end.
+//   Slabs are sized so that the launch is one round of the chip; every slab writes its partial tile to the workspace and a second
+//   kernel sums the slabs in a fixed order (no atomics: the result does not depend on scheduling).  The bias gradient rides
+//   along in the waves of the first k-tile as one more product with a matrix of ones.
+//   What bounds it: the rows' way in.  In tiles of 256 x 256 alone, a 32 x 32 gradient moved 4 KB a stage (12 KB a CU in flight) and
+//   fetched seven of eight pieces twice; slabs of consecutive rows made the chip read 256 runs of rows megabytes apart.
+//   Both kernels of a call, operands not in any cache, before -> now: 482,304 rows 32 x 32 47.6 -> 29.9 us, 96 x 32 61 -> 51,
+//   32 x 128 70 -> 61, 256 x 32 117 -> 101; 241,152 rows 64 x 64 37 -> 30, 512 x 64 118 -> 110; 120,832 rows 1024 x 128 121 -> 115;
+//   5,000 rows 64 x 256 19 -> 14; 30,208 rows 4096 x 512 177 (0.71 PFLOP/s) either way.  Errors against fp64 equal or smaller
+//   (2.8e-7 -> 1.4e-7 of a 32 x 32 gradient).
 #include "f3d_device.h"
 #include "f3d_internal.h"
 
@@ -28,16 +35,24 @@ typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 
 constexpr int kXcd = 8;
 constexpr int kWgThreads = 512, kWgWaves = kWgThreads / kWave;
-constexpr int kWgNT = 256, kWgKT = 256;      // tile of dw per workgroup
-constexpr int kWgMT = 32;                    // rows per stage
 constexpr int kWgNBuf = 4;                   // stage buffers: three stages in flight behind the one being multiplied
-constexpr int kRowB = 512;                   // bytes per LDS row of either operand tile (256 bf16, no padding)
-constexpr int kTileB = kWgMT * kRowB;        // one operand tile of a stage
-constexpr int kWgBuf = 2 * kTileB;
-constexpr int kWgLds = kWgNBuf * kWgBuf;
-constexpr int kDmaPerTile = kTileB / 1024 / kWgWaves;   // direct loads (1 KB each) per wave, operand and stage
-static_assert(kWgNT == 256 && kWgKT == 256 && kRowB == 512, "one direct load fills two LDS rows of 32 pieces");
-static_assert(kDmaPerTile * kWgWaves * 1024 == kTileB && kWgLds <= 160 * 1024, "stage geometry");
+
+// A workgroup's tile of dw: WN x WK columns of dy and x (32, 64, 128 or 256 each), MT rows a stage
+template <int WN, int WK>
+struct WgGeom {
+  static constexpr int ROW = 2 * (WN + WK);                       // bytes of a row of both operands
+  static constexpr int MT = ROW * 256 <= 40960 ? 256 : ROW * 128 <= 40960 ? 128 : ROW * 64 <= 40960 ? 64 : 32;
+  static constexpr int RA = 2 * WN, RB = 2 * WK;                  // bytes of an LDS row, no padding
+  static constexpr int TILE_A = MT * RA, STAGE = MT * ROW, LDS = kWgNBuf * STAGE;
+  static constexpr int DMA_A = TILE_A / 1024, DMA = STAGE / 1024;             // direct loads (1 KB each) of a stage
+  static constexpr int DMA_WAVE = (DMA + kWgWaves - 1) / kWgWaves;            // ... of a wave (a last one may repeat)
+  // the eight waves: over the 32-column blocks of dy, then those of x, what is left of them over the rows of a stage
+  static constexpr int NB = WN / 32, KB = WK / 32;
+  static constexpr int GN = NB < 4 ? NB : 4, GK = KB < 8 / GN ? KB : 8 / GN, GR = 8 / (GN * GK);
+  static constexpr int NI = NB / GN, NJ = KB / GK;                // blocks of a wave
+  static constexpr int KS = MT / 16 / GR;                         // k-steps of a wave and stage
+};
+static_assert(WgGeom<256, 256>::LDS == 128 * 1024 && WgGeom<128, 32>::LDS == 160 * 1024, "stage geometry");
 
 // 16 bytes per lane from global memory straight into LDS: lane l of the wave lands at lds + 16 l
 __device__ __forceinline__ void wg_dma16(const void* gbase, uint32_t voff, const char* lds) {
@@ -51,21 +66,32 @@ __device__ __forceinline__ void wg_dma16(const void* gbase, uint32_t voff, const
 
 // two transposing reads -> one 8-value MFMA operand: slots 0..3 = rows r .. r+3, slots 4..7 = rows r+4 .. r+7 of the
 // lane's column (the same row order for both operands, so the products pair up)
+template <int ROWB>
 __device__ __forceinline__ bf16x8_t read_tr8(const char* p) {
   const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)p);
-  const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(p + 4 * kRowB));
+  const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(p + 4 * ROWB));
   return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// LDS layout of an operand tile: row r at r * 512 bytes, its 16-byte piece c stored at position c ^ 4 (r % 4).  The
+// LDS layout of an operand tile: row r at r ROWB, its 16-byte piece c stored at position c ^ wg_swizzle(r).  The
 // direct loads write positions linearly (a lane picks the global piece that belongs at its position).  A transposing
 // read has 32 lanes touch 64 bytes of each of four consecutive rows; the swizzle sends the four rows to the four
-// 64-byte quarters of the 256 bytes the 64 banks serve per clock (without it the rows, a multiple of 256 bytes apart,
-// would all meet in the same banks).
+// 64-byte quarters of the 256 bytes the 64 banks serve per clock (without it rows a multiple of 256 bytes apart would all
+// meet in the same banks; rows of 128 bytes two by two; rows of 64 bytes need none).
+template <int ROWB>
+__device__ __forceinline__ uint32_t wg_swizzle(uint32_t r) {
+  return ROWB >= 256 ? (r & 3u) << 2 : ROWB == 128 ? ((r >> 1) & 1u) << 2 : 0u;
+}
+
+// A slab's rows are every slabs-th stage of the whole: at any time the chip reads one run of rows, not 256 runs that start
+// megabytes apart.
+template <int WN, int WK>
 __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
     const uint16_t* __restrict__ dy, uint32_t lddy, const uint16_t* __restrict__ x, uint32_t ldx,
     float* __restrict__ part_w, float* __restrict__ part_b, uint32_t M, uint32_t N, uint32_t K, uint32_t n_tiles,
-    uint32_t k_tiles, uint32_t slabs, uint32_t slab_rows, uint32_t items_per_xcd) {
+    uint32_t k_tiles, uint32_t slabs, uint32_t items_per_xcd) {
+  using G = WgGeom<WN, WK>;
+  constexpr int MT = G::MT, RA = G::RA, RB = G::RB, NI = G::NI, NJ = G::NJ, KS = G::KS;
   extern __shared__ __attribute__((aligned(16))) char lds_wg[];
   // workgroups of one XCD take consecutive items, so the tiles of one slab (which re-read the same rows of x and
   // dy) meet in one L2
@@ -73,62 +99,64 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
   const uint32_t item = (blockIdx.x % kXcd) * items_per_xcd + blockIdx.x / kXcd;
   if (blockIdx.x / kXcd >= items_per_xcd || item >= n_items) return;
   const uint32_t slab = item / tiles, tile = item % tiles;
-  const uint32_t n0 = (tile / k_tiles) * kWgNT, k0 = (tile % k_tiles) * kWgKT;
-  const uint32_t m_begin = slab * slab_rows, m_end = min(M, m_begin + slab_rows);
+  const uint32_t n0 = (tile / k_tiles) * WN, k0 = (tile % k_tiles) * WK;
   const uint32_t tid = threadIdx.x, lane = tid % kWave;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  // 4 x 2 waves; the two waves of a SIMD (wave, wave + 4) sit in different k halves
-  const uint32_t nw = wave & 3u, kw = wave >> 2;
+  const uint32_t nw = wave % G::GN, kw = wave / G::GN % G::GK, rw = wave / (G::GN * G::GK);
   const bool with_bias = part_b != nullptr && k0 == 0 && kw == 0;
-  // 32 x 32 blocks of this wave's 64 x 128 that lie inside dw
-  const uint32_t n_w = n0 + nw * 64u, k_w = k0 + kw * 128u;
-  const uint32_t ni = n_w >= N ? 0u : min(2u, (N - n_w + 31u) / 32u), nj = k_w >= K ? 0u : min(4u, (K - k_w + 31u) / 32u);
+  // 32 x 32 blocks of this wave that lie inside dw
+  const uint32_t n_w = n0 + nw * 32u * NI, k_w = k0 + kw * 32u * NJ;
+  const uint32_t ni = n_w >= N ? 0u : min((uint32_t)NI, (N - n_w + 31u) / 32u), nj = k_w >= K ? 0u : min((uint32_t)NJ, (K - k_w + 31u) / 32u);
 
-  // ---- direct loads: instruction q of a tile fills rows 2q, 2q + 1; this wave issues q = kDmaPerTile wave + i.
+  // ---- direct loads: load q of a stage fills 1 KB of LDS, the tile of dy first; this wave issues q = wave + 8 i.
   //      Pieces beyond the last column are clamped to the last valid piece (they only reach blocks of dw that are
-  //      never stored), rows beyond the slab to its last row (and zeroed in LDS once they have landed). ----
-  const uint32_t pieces_a = min(32u, (N - n0) / 8u), pieces_b = min(32u, (K - k0) / 8u);
-  uint32_t d_row[kDmaPerTile], d_ca[kDmaPerTile], d_cb[kDmaPerTile];
+  //      never stored), rows beyond the last to it (and zeroed in LDS once they have landed). ----
+  const uint32_t pieces_a = min((uint32_t)RA / 16u, (N - n0) / 8u), pieces_b = min((uint32_t)RB / 16u, (K - k0) / 8u);
+  // (wave < 8: which operand load i belongs to is known at compile time but for one i at most)
+  auto dma = [&](int i) { return G::DMA % kWgWaves == 0 ? wave + 8u * i : min(wave + 8u * i, (uint32_t)G::DMA - 1u); };
+  auto of_dy = [&](int i) { return 8 * i + 7 < G::DMA_A || (8 * i < G::DMA_A && wave + 8u * i < (uint32_t)G::DMA_A); };
+  uint32_t d_row[G::DMA_WAVE], d_col[G::DMA_WAVE];
 #pragma unroll
-  for (int i = 0; i < kDmaPerTile; ++i) {
-    const uint32_t q = kDmaPerTile * wave + i;
-    d_row[i] = 2u * q + lane / 32u;
-    const uint32_t c = (lane & 31u) ^ ((d_row[i] & 3u) << 2);
-    d_ca[i] = min(c, pieces_a - 1u) * 16u;
-    d_cb[i] = min(c, pieces_b - 1u) * 16u;
+  for (int i = 0; i < G::DMA_WAVE; ++i) {
+    const uint32_t q = dma(i);
+    const bool a = of_dy(i);
+    const uint32_t at = (a ? q : q - G::DMA_A) * 1024u + lane * 16u;
+    const uint32_t row = at / (a ? (uint32_t)RA : (uint32_t)RB), pos = at % (a ? (uint32_t)RA : (uint32_t)RB) / 16u;
+    const uint32_t c = pos ^ (a ? wg_swizzle<RA>(row) : wg_swizzle<RB>(row));
+    d_row[i] = row;
+    d_col[i] = min(c, (a ? pieces_a : pieces_b) - 1u) * 16u;
   }
+  auto first_row = [&](uint32_t st) { return (st * slabs + slab) * MT; };
   auto issue = [&](uint32_t st) {
-    const uint32_t m0 = m_begin + st * kWgMT, last = m_end - 1u - m0;   // m0 < m_end
+    const uint32_t m0 = first_row(st), last = M - 1u - m0;   // m0 < M
     const char* ga = reinterpret_cast<const char*>(dy + (size_t)m0 * lddy + n0);
     const char* gb = reinterpret_cast<const char*>(x + (size_t)m0 * ldx + k0);
-    char* buf = lds_wg + (st % kWgNBuf) * kWgBuf;
+    char* buf = lds_wg + (st % kWgNBuf) * G::STAGE;
 #pragma unroll
-    for (int i = 0; i < kDmaPerTile; ++i) {
-      const uint32_t r = min(d_row[i], last), q = kDmaPerTile * wave + i;
-      wg_dma16(ga, r * lddy * 2u + d_ca[i], buf + q * 1024);
-      wg_dma16(gb, r * ldx * 2u + d_cb[i], buf + kTileB + q * 1024);
+    for (int i = 0; i < G::DMA_WAVE; ++i) {
+      const bool a = of_dy(i);      // uniform
+      wg_dma16(a ? ga : gb, min(d_row[i], last) * (a ? lddy : ldx) * 2u + d_col[i], buf + dma(i) * 1024);
     }
   };
 
   // ---- the lane's place in a transposing read: lane p of a 16-lane block points at row p / 4, columns 4 (p % 4)..;
-  //      the swizzle value 4 (row % 4) = 4 (p / 4) is the same for every row the lane ever reads ----
-  const uint32_t half = lane >> 5, p16 = lane & 15u, cgrp = (lane >> 4) & 1u;
-  const uint32_t row_off = (8u * half + p16 / 4u) * kRowB, sw = (p16 / 4u) << 2, in_piece = 8u * (p16 & 1u);
-  uint32_t a_off[2], b_off[4];
+  //      the swizzle value of row p / 4 is that of every row the lane ever reads (they differ by multiples of 4) ----
+  const uint32_t half = lane >> 5, p16 = lane & 15u, cgrp = (lane >> 4) & 1u, r0 = 8u * half + p16 / 4u, in_piece = 8u * (p16 & 1u);
+  uint32_t a_off[NI], b_off[NJ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-    a_off[i] = row_off + (((nw * 8u + 4u * i + 2u * cgrp + ((p16 & 3u) >> 1)) ^ sw) << 4) + in_piece;
+  for (int i = 0; i < NI; ++i)
+    a_off[i] = r0 * RA + ((((nw * NI + i) * 4u + 2u * cgrp + ((p16 & 3u) >> 1)) ^ wg_swizzle<RA>(r0)) << 4) + in_piece;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    b_off[j] = kTileB + row_off + (((kw * 16u + 4u * j + 2u * cgrp + ((p16 & 3u) >> 1)) ^ sw) << 4) + in_piece;
+  for (int j = 0; j < NJ; ++j)
+    b_off[j] = G::TILE_A + r0 * RB + ((((kw * NJ + j) * 4u + 2u * cgrp + ((p16 & 3u) >> 1)) ^ wg_swizzle<RB>(r0)) << 4) + in_piece;
 
-  f32x16_t acc[2][4], accb[2];
+  f32x16_t acc[NI][NJ], accb[NI];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < NI; ++i) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) accb[i][e] = 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   }
@@ -136,54 +164,53 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
 
-  const uint32_t n_stage = m_end > m_begin ? (m_end - m_begin + kWgMT - 1) / kWgMT : 0u;
-  static_assert(kWgMT == 32, "two k-steps per stage");
-  // waits until this wave's loads of stage st have landed (at most the loads of the later stages, two of them at
+  const uint32_t all_stages = (M + MT - 1) / MT;
+  const uint32_t n_stage = all_stages > slab ? (all_stages - slab + slabs - 1) / slabs : 0u;
+// waits until this wave's loads of stage st have landed (at most the loads of the later stages, two of them at
   // that point, stay outstanding), zeroes the rows past the slab, and meets the other waves: after the barrier the
   // whole stage is in LDS and every wave has its operands of the stages before it in registers
   auto stage_ready = [&](uint32_t st) {
     const uint32_t later = min(n_stage - 1u - st, 2u);
-    if (later == 2u) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * kDmaPerTile) : "memory");
-    else if (later == 1u) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kDmaPerTile) : "memory");
+    if (later == 2u) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * G::DMA_WAVE) : "memory");
+    else if (later == 1u) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::DMA_WAVE) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const uint32_t rows_left = m_end - (m_begin + st * kWgMT);
-    if (rows_left < (uint32_t)kWgMT) {
-      char* buf = lds_wg + (st % kWgNBuf) * kWgBuf;
+    const uint32_t rows_left = M - first_row(st);
+    if (rows_left < (uint32_t)MT) {
+      char* buf = lds_wg + (st % kWgNBuf) * G::STAGE;
 #pragma unroll
-      for (int i = 0; i < kDmaPerTile; ++i)
-        if (d_row[i] >= rows_left) {
-          const uint32_t pos = (kDmaPerTile * wave + i) * 1024u + lane * 16u;
-          *reinterpret_cast<u32x4_t*>(buf + pos) = u32x4_t{0u, 0u, 0u, 0u};
-          *reinterpret_cast<u32x4_t*>(buf + kTileB + pos) = u32x4_t{0u, 0u, 0u, 0u};
-        }
+      for (int i = 0; i < G::DMA_WAVE; ++i)
+        if (d_row[i] >= rows_left)
+          *reinterpret_cast<u32x4_t*>(buf + dma(i) * 1024u + lane * 16u) = u32x4_t{0u, 0u, 0u, 0u};
     }
     wg_barrier_lds();
   };
-  bf16x8_t fa[2][2], fb[2][4];
-  auto frags = [&](uint32_t st, int ks, bf16x8_t (&a)[2], bf16x8_t (&b)[4]) {
-    const char* buf = lds_wg + (st % kWgNBuf) * kWgBuf;
+  bf16x8_t fa[2][NI], fb[2][NJ];
+  // k-step ks of this wave: rows 16 (GR ks + rw) .. of the stage
+  auto frags = [&](uint32_t st, int ks, bf16x8_t (&a)[NI], bf16x8_t (&b)[NJ]) {
+    const char* buf = lds_wg + (st % kWgNBuf) * G::STAGE;
+    const uint32_t row = 16u * (G::GR * ks + rw);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      if ((uint32_t)i < ni) a[i] = read_tr8(buf + a_off[i] + ks * 16 * kRowB);
+    for (int i = 0; i < NI; ++i)
+      if ((uint32_t)i < ni) a[i] = read_tr8<RA>(buf + a_off[i] + row * RA);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if ((uint32_t)j < nj) b[j] = read_tr8(buf + b_off[j] + ks * 16 * kRowB);
+    for (int j = 0; j < NJ; ++j)
+      if ((uint32_t)j < nj) b[j] = read_tr8<RB>(buf + b_off[j] + row * RB);
   };
-  auto products = [&](const bf16x8_t (&a)[2], const bf16x8_t (&b)[4]) {
+  auto products = [&](const bf16x8_t (&a)[NI], const bf16x8_t (&b)[NJ]) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < NJ; ++j)
         if ((uint32_t)i < ni && (uint32_t)j < nj)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
     if (with_bias) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < NI; ++i)
         if ((uint32_t)i < ni) accb[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], ones, accb[i], 0, 0, 0);
     }
   };
   // Three stages are requested ahead.  The hand-over to the next stage (wait, barrier, first operand reads) sits
-  // between the two k-steps of a stage, so the products of the second k-step run over it.
+  // in front of the last k-step's products of a stage, which run over it.
 #pragma unroll
   for (int st = 0; st < kWgNBuf - 1; ++st)
     if ((uint32_t)st < n_stage) issue(st);
@@ -191,28 +218,64 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
     stage_ready(0);
     frags(0, 0, fa[0], fb[0]);
   }
+  static_assert(KS % 2 == 0, "operands of k-step 0 are in the first buffer");
   for (uint32_t st = 0; st < n_stage; ++st) {
     // the buffer of stage st - 1 is free: every wave read the last of it before the barrier that made stage st ready
     if (st + kWgNBuf - 1 < n_stage) issue(st + kWgNBuf - 1);
-    frags(st, 1, fa[1], fb[1]);
-    products(fa[0], fb[0]);
-    if (st + 1 < n_stage) {
-      stage_ready(st + 1);   // stages st + 2 and st + 3 are the ones still in flight
-      frags(st + 1, 0, fa[0], fb[0]);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      if (ks + 1 < KS) {
+        frags(st, ks + 1, fa[(ks + 1) & 1], fb[(ks + 1) & 1]);
+      } else if (st + 1 < n_stage) {
+        stage_ready(st + 1);   // stages st + 2 and st + 3 are the ones still in flight
+        frags(st + 1, 0, fa[0], fb[0]);
+      }
+      products(fa[ks & 1], fb[ks & 1]);
     }
-    products(fa[1], fb[1]);
+  }
+
+  // ---- waves that shared the rows of a stage: their sums are added in ascending order of the row group ----
+  if constexpr (G::GR > 1) {
+    __syncthreads();      // the stage buffers are free
+    constexpr uint32_t WAVE_B = (NI * NJ + NI) * 4096;
+    static_assert((G::GR - 1) * G::GN * G::GK * WAVE_B <= G::LDS, "the waves' sums fit the stage buffers");
+    float* const mine = reinterpret_cast<float*>(lds_wg + (wave - G::GN * G::GK) * WAVE_B);
+    if (rw > 0) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j <= NJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) mine[((i * (NJ + 1) + j) * 16 + e) * 64 + lane] = j < NJ ? acc[i][j < NJ ? j : 0][e] : accb[i][e];
+    }
+    __syncthreads();
+    if (rw > 0) return;
+#pragma unroll 1
+    for (uint32_t r = 1; r < (uint32_t)G::GR; ++r) {
+      const float* theirs = reinterpret_cast<const float*>(lds_wg + ((r - 1) * G::GN * G::GK + wave) * WAVE_B);
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j <= NJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float v = theirs[((i * (NJ + 1) + j) * 16 + e) * 64 + lane];
+            if (j < NJ) acc[i][j < NJ ? j : 0][e] += v;
+            else accb[i][e] += v;
+          }
+    }
   }
 
   // ---- this slab's partial tile: accumulator slot e of a lane is row 8 (e / 4) + 4 half + e % 4, column lane % 32 ----
   float* pw = part_w + (size_t)slab * N * K;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < NI; ++i) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const uint32_t n = n_w + 32u * i + 8u * (e / 4) + 4u * half + (e % 4);
       if (n >= N) continue;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < NJ; ++j) {
         const uint32_t k = k_w + 32u * j + (lane & 31u);
         if (k < K) pw[(size_t)n * K + k] = acc[i][j][e];
       }
@@ -431,6 +494,39 @@ int n_cu_of(int device, uint32_t* n_cu) {
   return F3D_OK;
 }
 
+struct WgLaunch {
+  const uint16_t *dy, *x;
+  uint32_t lddy, ldx, m, n, k, n_tiles, k_tiles, n_cu;
+  int device;
+  bool bias;
+  hipStream_t stream;
+  uint32_t slabs;               // out: row slabs, and where their partial tiles lie
+  float *part_w, *part_b;
+};
+
+template <int WN, int WK>
+int launch_wgrad(WgLaunch& l) {
+  using G = WgGeom<WN, WK>;
+  // one round of the chip: as many row slabs as there are compute units per tile
+  const uint32_t tiles = l.n_tiles * l.k_tiles, stages = cdiv_u32(l.m, G::MT);
+  l.slabs = tiles >= l.n_cu ? 1u : l.n_cu / tiles;
+  if (l.slabs > stages) l.slabs = stages ? stages : 1u;
+  const size_t part_w_bytes = (size_t)l.slabs * l.n * l.k * 4, part_b_bytes = l.bias ? (size_t)l.slabs * l.n * 4 : 0;
+  char* ws = (char*)workspace(l.device, part_w_bytes + part_b_bytes, l.stream);
+  if (!ws) return F3D_ERR_RUNTIME;
+  l.part_w = (float*)ws;
+  l.part_b = l.bias ? (float*)(ws + part_w_bytes) : nullptr;
+  static bool attr_set[64] = {};
+  if (l.device >= 0 && l.device < 64 && !attr_set[l.device]) {
+    F3D_CHECK_HIP(hipFuncSetAttribute((const void*)linear_wgrad_kernel<WN, WK>, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
+    attr_set[l.device] = true;
+  }
+  const uint32_t items_per_xcd = cdiv_u32(tiles * l.slabs, kXcd);
+  hipLaunchKernelGGL((linear_wgrad_kernel<WN, WK>), dim3(items_per_xcd * kXcd), dim3(kWgThreads), G::LDS, l.stream, l.dy, l.lddy, l.x,
+                     l.ldx, l.part_w, l.part_b, l.m, l.n, l.k, l.n_tiles, l.k_tiles, l.slabs, items_per_xcd);
+  return F3D_OK;
+}
+
 }  // namespace
 }  // namespace f3d
 
@@ -451,34 +547,27 @@ int f3d_linear_wgrad_bf16(const f3d_bf16_t* dy, uint32_t lddy, const f3d_bf16_t*
   SyncBracket sync(s);
   uint32_t n_cu = 0;
   if (int rc = n_cu_of(device, &n_cu)) return rc;
-  const uint32_t n_tiles = cdiv_u32(n, kWgNT), k_tiles = cdiv_u32(k, kWgKT), tiles = n_tiles * k_tiles;
-  // one round of the chip: as many row slabs as there are compute units per tile
-  uint32_t slabs = tiles >= n_cu ? 1u : n_cu / tiles;
-  const uint32_t stages = cdiv_u32(m, kWgMT);
-  if (slabs > stages) slabs = stages ? stages : 1u;
-  const uint32_t slab_rows = cdiv_u32(cdiv_u32(m, slabs), kWgMT) * kWgMT;
-  if (m) slabs = cdiv_u32(m, slab_rows);
+  // tile of dw per workgroup: the narrowest width that holds all columns, 256 where none does
+  auto width = [](uint32_t c) { return c <= 32u ? 32u : c <= 64u ? 64u : c <= 128u ? 128u : 256u; };
+  const uint32_t wn = width(n), wk = width(k);
+  const uint32_t n_tiles = cdiv_u32(n, wn), k_tiles = cdiv_u32(k, wk);
   const size_t nk = (size_t)n * k;
-  const size_t part_w_bytes = (size_t)slabs * nk * 4, part_b_bytes = db ? (size_t)slabs * n * 4 : 0;
-  char* ws = (char*)workspace(device, part_w_bytes + part_b_bytes, s);
-  if (!ws) return F3D_ERR_RUNTIME;
-  float* part_w = (float*)ws;
-  float* part_b = db ? (float*)(ws + part_w_bytes) : nullptr;
-  static bool attr_set[64] = {};
-  if (device >= 0 && device < 64 && !attr_set[device]) {
-    F3D_CHECK_HIP(hipFuncSetAttribute((const void*)linear_wgrad_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kWgLds));
-    attr_set[device] = true;
-  }
-  const uint32_t n_items = tiles * slabs, items_per_xcd = cdiv_u32(n_items, kXcd);
-  hipLaunchKernelGGL(linear_wgrad_kernel, dim3(items_per_xcd * kXcd), dim3(kWgThreads), kWgLds, s, dy, lddy, x, ldx,
-                     part_w, part_b, m, n, k, n_tiles, k_tiles, slabs, slab_rows, items_per_xcd);
+  WgLaunch l = {dy, x, lddy, ldx, m, n, k, n_tiles, k_tiles, n_cu, device, db != nullptr, s};
+  int rc = F3D_OK;
+#define F3D_WG(WN, WK) \
+  if (wn == WN && wk == WK) rc = launch_wgrad<WN, WK>(l)
+#define F3D_WGS(WN) F3D_WG(WN, 32); F3D_WG(WN, 64); F3D_WG(WN, 128); F3D_WG(WN, 256)
+  F3D_WGS(32); F3D_WGS(64); F3D_WGS(128); F3D_WGS(256);
+#undef F3D_WGS
+#undef F3D_WG
+  if (rc != F3D_OK) return rc;
   auto sum = [&](auto kern, uint32_t lanes) {
     const uint32_t per_block = 4 * lanes;
     const uint32_t blocks_w = (uint32_t)((nk + per_block - 1) / per_block), blocks_b = db ? cdiv_u32(n, per_block) : 0u;
-    hipLaunchKernelGGL(kern, dim3(blocks_w + blocks_b), dim3(16 * lanes), 0, s, part_w, nk, dw, blocks_w, part_b,
-                       db ? (size_t)n : (size_t)0, db, slabs, accumulate);
+    hipLaunchKernelGGL(kern, dim3(blocks_w + blocks_b), dim3(16 * lanes), 0, s, l.part_w, nk, dw, blocks_w,
+                       l.part_b, db ? (size_t)n : (size_t)0, db, l.slabs, accumulate);
   };
-  if (slabs > 64) sum(sum_partials_kernel<16, 16>, 16u);
+  if (l.slabs > 64) sum(sum_partials_kernel<16, 16>, 16u);
   else sum(sum_partials_kernel<64, 8>, 64u);
   F3D_CHECK_HIP(hipGetLastError());
   return F3D_OK;

@@ -92,6 +92,23 @@ def test_layernorm_backward_partial_rows(blocks):
         assert ((got.double() - terms.sum(0)).abs() <= (M + 16) * 2.0 ** -24 * terms.abs().sum(0)).all()
 
 
+@pytest.mark.parametrize("N", [8, 32, 40, 72, 264])
+@pytest.mark.parametrize("K", [16, 64, 128, 136])
+def test_linear_wgrad_tile_widths(N, K):
+    """every width of tile in both operands (32, 64, 128, 256; exact, ragged, several tiles) around its stages of 32 to 256 rows: one
+    row, one row short of a stage, two stages and a row, more stages than slabs.  Sums of M products of at most `top`: M 2^-24
+    of the sum of magnitudes, in a tree that is at most as deep as a plain sum."""
+    from flash3dtransformer_amd.lib import pshattn
+    for M in (1, 255, 513, 256 * 260 + 7 if N * K <= 64 * 64 else 9001):
+        g = torch.Generator(device=DEV).manual_seed(M + N + K)
+        dy, x = (torch.randn(M, c, device=DEV, generator=g).to(torch.bfloat16) for c in (N, K))
+        dw, db = torch.full((N, K), 3.0, device=DEV), torch.full((N,), 3.0, device=DEV)
+        pshattn.linear_wgrad_bf16(dy, x, dw, db)
+        for got, ref, size in ((dw.double(), dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()),
+                               (db.double(), dy.double().sum(0), dy.double().abs().sum(0))):
+            assert ((got - ref).abs() <= M * 2.0 ** -24 * size).all(), (M, N, K)
+
+
 def test_linear_wgrad_random_shapes():
     """shapes drawn at random (multiples of 8 in n and k, any row count), one of the operands a column slice"""
     from flash3dtransformer_amd.lib import pshattn
