@@ -1039,15 +1039,19 @@ __global__ __launch_bounds__(64 * WAVES) void buck_swin_fwd_scope_kernel(
       const bool row_ok = (int32_t)lq < q_len[b] && l_tot > 0.f;
       const float inv = row_ok ? 1.0f / l_tot : 0.f;
       const uint32_t orow_b = q_row[b] * num_head * D * 2u;
+      // a lane holds features 8 g + 4 half .. + 3 of its row: the lower half-wave's odd groups against the upper one's even ones
+      // make 8 consecutive features a lane, one 16-byte store instead of two of 8 bytes (8 heads x 131,072 rows in 512-row scopes
+      // 105 -> 101 us, in 256-row scopes 68 -> 63.5)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const uint32_t d0 = g * 8 + half * 4;
-        if (D >= 32 || d0 < (uint32_t)D) {
-          uint2 w;
-          w.x = pack_bf16x2(acc[b][g * 4 + 0] * inv, acc[b][g * 4 + 1] * inv);
-          w.y = pack_bf16x2(acc[b][g * 4 + 2] * inv, acc[b][g * 4 + 3] * inv);
-          *reinterpret_cast<uint2*>(op + (orow_b + d0 * 2u)) = w;
-        }
+      for (int g = 0; g < (D < 32 ? D : 32) / 8; g += 2) {
+        uint32_t w[2][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) w[h][e] = pack_bf16x2(acc[b][(g + h) * 4 + 2 * e] * inv, acc[b][(g + h) * 4 + 2 * e + 1] * inv);
+        const auto lo = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
+        *reinterpret_cast<u32x4_t*>(op + (orow_b + (g + half) * 16u)) = u32x4_t{lo[0], hi[0], lo[1], hi[1]};
       }
       if (half == 0) {
         const float ln2 = 0.69314718055994530942f;

@@ -39,6 +39,12 @@
 // Delta, dK / dV and dQ kernels.  Measured, both kernels, against those: 8 heads x 131,072 rows, 512-row scopes 430 -> 382 us,
 // with valid lengths of 3/4 to full buckets 538 -> 342; scopes of 8 x 512, 122,880 rows 524 -> 292, 24,576 rows 263 -> 126;
 // 20,480 rows of 512-row scopes 39 -> 24; 4 heads of 64, 65,536 rows: 236 -> 154, of 128, 32,768 rows: 257 -> 208.
+// The score products of both key tiles of a wave are issued before the first exponential, and gradients leave in 16-byte
+// pieces (the halves of a wave exchange registers; 8-byte pieces touched twice the lines per store): 482,304 rows of 512-row scopes
+// 182 -> 175 us, 30,208 rows x 16 heads 181 -> 171, 8 heads x 131,072 rows 405 -> 390, in 256-row scopes 269 -> 253, 64-wide
+// heads 158 -> 148, same bits.  One kernel for dQ, dK and dV (five products a block instead of seven, dQ summed in LDS by eight waves
+// that pass its tiles on) reached 340 at 8 heads x 131,072 rows, but 35 instead of 25 at 20,480 rows: with both P and dS turned
+// round through LDS, two waves a SIMD and a hand-over per tile, a step took 3,400 clocks for 2,000 of vector issue.
 #include <algorithm>
 #include "f3d_device.h"
 #include "f3d_internal.h"
@@ -201,6 +207,23 @@ constexpr size_t stream_lds_bytes(uint32_t scope_size) {
   return (size_t)4 * SGeom<D>::TILEB * SGeom<D>::NSUB + (size_t)4 * 32 * SGeom<D>::NSUB * 4 + (size_t)scope_size * 8;
 }
 
+// a 32 x 32 accumulator tile (transposed output: the lane's row, features 8 g + 4 half .. + 3 per group g) as bf16 in 16-byte pieces:
+// the lower half-wave's second group is exchanged with the upper half-wave's first, so that a lane holds 8 consecutive features
+template <int N>
+__device__ __forceinline__ void store_features(uint16_t* row, uint32_t half, const f32x16_t& x, float f, bool ok) {
+#pragma unroll
+  for (int g = 0; g < N / 8; g += 2) {
+    uint32_t w[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) w[h][e] = ok ? pack_bf16x2(x[(g + h) * 4 + 2 * e] * f, x[(g + h) * 4 + 2 * e + 1] * f) : 0u;
+    const auto lo = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
+    *reinterpret_cast<u32x4_t*>(row + (g + half) * 8) = u32x4_t{lo[0], hi[0], lo[1], hi[1]};
+  }
+}
+
 // ---- Delta, dQ ------------------------------------------------------------------------------------------------
 // Runs first: Delta of the wave's queries is formed from its O and dO rows (dO is in registers anyway).
 template <int D>
@@ -355,17 +378,7 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 ? 2 : 4) voi
   uint16_t* dqrow = dq + base_g + (size_t)qrow * ldg;
   const bool q_ok = (int32_t)lq < q_len;
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const uint32_t d0 = dt * 32 + g4 * 8 + half * 4;
-      if (d0 < (uint32_t)D) {
-        uint2 x;
-        x.x = pack_bf16x2(acc[dt][g4 * 4 + 0] * scale, acc[dt][g4 * 4 + 1] * scale);
-        x.y = pack_bf16x2(acc[dt][g4 * 4 + 2] * scale, acc[dt][g4 * 4 + 3] * scale);
-        *reinterpret_cast<uint2*>(dqrow + d0) = q_ok ? x : make_uint2(0u, 0u);
-      }
-    }
+  for (int dt = 0; dt < DT; ++dt) store_features<D < 32 ? D : 32>(dqrow + dt * 32, half, acc[dt], scale, q_ok);
 }
 
 // ---- dK, dV -------------------------------------------------------------------------------------------------
@@ -451,16 +464,21 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
       for (int r = 0; r < 4; ++r) { lse2[g4 * 4 + r] = lv[r]; dl[g4 * 4 + r] = dv4[r]; }
     }
     uint32_t pb[KT][8], sb[KT][8];
+    f32x16_t s_all[KT], p_all[KT];
 #pragma unroll
     for (int a = 0; a < KT; ++a) {
-      f32x16_t s_acc, p_acc;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) { s_acc[i] = 0.f; p_acc[i] = 0.f; }
+      for (int i = 0; i < 16; ++i) { s_all[a][i] = 0.f; p_all[a][i] = 0.f; }
 #pragma unroll
       for (int ks = 0; ks < KSTEPS; ++ks) {
-        s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[ks], kf[a][ks], s_acc, 0, 0, 0);   // S[query][key]
-        p_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(da[ks], vf[a][ks], p_acc, 0, 0, 0);   // dP[query][key]
+        s_all[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[ks], kf[a][ks], s_all[a], 0, 0, 0);   // S[query][key]
+        p_all[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(da[ks], vf[a][ks], p_all[a], 0, 0, 0);   // dP[query][key]
       }
+    }
+    if constexpr (KT > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int a = 0; a < KT; ++a) {
+      const f32x16_t &s_acc = s_all[a], &p_acc = p_all[a];
 #pragma unroll
       for (int i = 0; i < 16; i += 2) {
         float p[2], ds[2];
@@ -544,20 +562,10 @@ __global__ __launch_bounds__(64 * kStreamWaves, D > 64 ? 1 : D > 32 || KT > 1 ? 
     uint16_t* dvrow = dv + base_g + (size_t)(krow + 32u * a) * ldg;
     const bool key_ok = (int32_t)(32u * a + lq) < k_len;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const uint32_t d0 = dt * 32 + g4 * 8 + half * 4;
-        if (d0 < (uint32_t)D) {
-          uint2 x, y;
-          x.x = pack_bf16x2(acc_dk[a][dt][g4 * 4 + 0] * scale, acc_dk[a][dt][g4 * 4 + 1] * scale);
-          x.y = pack_bf16x2(acc_dk[a][dt][g4 * 4 + 2] * scale, acc_dk[a][dt][g4 * 4 + 3] * scale);
-          y.x = pack_bf16x2(acc_dv[a][dt][g4 * 4 + 0], acc_dv[a][dt][g4 * 4 + 1]);
-          y.y = pack_bf16x2(acc_dv[a][dt][g4 * 4 + 2], acc_dv[a][dt][g4 * 4 + 3]);
-          *reinterpret_cast<uint2*>(dkrow + d0) = key_ok ? x : make_uint2(0u, 0u);
-          *reinterpret_cast<uint2*>(dvrow + d0) = key_ok ? y : make_uint2(0u, 0u);
-        }
-      }
+    for (int dt = 0; dt < DT; ++dt) {
+      store_features<D < 32 ? D : 32>(dkrow + dt * 32, half, acc_dk[a][dt], scale, key_ok);
+      store_features<D < 32 ? D : 32>(dvrow + dt * 32, half, acc_dv[a][dt], 1.0f, key_ok);
+    }
   }
 }
 
