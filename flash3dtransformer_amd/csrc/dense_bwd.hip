@@ -338,8 +338,10 @@ __global__ __launch_bounds__(16 * LANES) void sum_partials_kernel(const float* _
 // ---- LayerNorm backward: LPR lanes per row, 8 channels per lane.
 //   xhat = (x - mean) rstd, g = dh gamma, dx = rstd (g - mean(g) - xhat mean(g xhat)) (+ dres),
 //   dgamma = sum_rows dh xhat, dbeta = sum_rows dh.  A thread walks rows with a grid stride and keeps its 8 + 8 column
-//   sums in registers; the workgroup combines them through LDS and writes one partial per workgroup. ----
-template <int LPR>
+//   sums in registers; the workgroup combines them through LDS and writes one partial per workgroup.
+//   APART: dx is rounded to bf16 before dres is added, as two tensors added afterwards would be (the bits of that sum, without
+//   writing dx and reading both again: 14 additions of 19 us in a training step of 482,304 rows). ----
+template <int LPR, bool APART>
 __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const uint16_t* __restrict__ x, uint32_t ldx,
                                                             const uint16_t* dh, uint32_t lddh,
                                                             const uint16_t* __restrict__ gamma,
@@ -403,9 +405,15 @@ __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const uint16_t* __re
       u32x4_t t;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float f0 = rstd * (dv[2 * e] * g8[2 * e] - s1 - xv[2 * e] * s2) + bf16_lo(vr[e]);
-        float f1 = rstd * (dv[2 * e + 1] * g8[2 * e + 1] - s1 - xv[2 * e + 1] * s2) + bf16_hi(vr[e]);
-        t[e] = pack_bf16x2(f0, f1);
+        if constexpr (APART) {
+          const uint32_t own = pack_bf16x2(rstd * (dv[2 * e] * g8[2 * e] - s1 - xv[2 * e] * s2),
+                                           rstd * (dv[2 * e + 1] * g8[2 * e + 1] - s1 - xv[2 * e + 1] * s2));
+          t[e] = pack_bf16x2(bf16_lo(own) + bf16_lo(vr[e]), bf16_hi(own) + bf16_hi(vr[e]));
+        } else {
+          float f0 = rstd * (dv[2 * e] * g8[2 * e] - s1 - xv[2 * e] * s2) + bf16_lo(vr[e]);
+          float f1 = rstd * (dv[2 * e + 1] * g8[2 * e + 1] - s1 - xv[2 * e + 1] * s2) + bf16_hi(vr[e]);
+          t[e] = pack_bf16x2(f0, f1);
+        }
       }
       *reinterpret_cast<u32x4_t*>(dx + (size_t)row * lddx + sub * 8) = t;
     }
@@ -573,10 +581,9 @@ int f3d_linear_wgrad_bf16(const f3d_bf16_t* dy, uint32_t lddy, const f3d_bf16_t*
   return F3D_OK;
 }
 
-int f3d_layernorm_bwd_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* dh, uint32_t lddh,
-                           const f3d_bf16_t* gamma, const f3d_bf16_t* dres, uint32_t lddr, f3d_bf16_t* dx, uint32_t lddx,
-                           float* dgamma, float* dbeta, uint32_t m, uint32_t c, float eps, uint32_t accumulate,
-                           int device, void* stream) {
+static int layernorm_bwd(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* dh, uint32_t lddh, const f3d_bf16_t* gamma,
+                         const f3d_bf16_t* dres, uint32_t lddr, f3d_bf16_t* dx, uint32_t lddx, float* dgamma, float* dbeta,
+                         uint32_t m, uint32_t c, float eps, uint32_t accumulate, bool apart, int device, void* stream) {
   using namespace f3d;
   F3D_CHECK_ARG(((x && dh && dx) || m == 0) && gamma && dgamma && dbeta, "null tensor pointer");
   if (!(c == 32 || c == 64 || c == 128 || c == 256 || c == 512)) {
@@ -600,9 +607,13 @@ int f3d_layernorm_bwd_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* 
   if (wgs == 0) wgs = 1;
   float* part = (float*)workspace(device, (size_t)wgs * 2u * c * 4u, s);
   if (!part) return F3D_ERR_RUNTIME;
-#define F3D_LNB(LPR)                                                                                                \
-  hipLaunchKernelGGL((layernorm_bwd_kernel<LPR>), dim3(wgs), dim3(256), 0, s, x, ldx, dh, lddh, gamma, dres, lddr, \
-                     dx, lddx, part, m, eps)
+#define F3D_LNB(LPR)                                                                                                          \
+  if (apart)                                                                                                                 \
+    hipLaunchKernelGGL((layernorm_bwd_kernel<LPR, true>), dim3(wgs), dim3(256), 0, s, x, ldx, dh, lddh, gamma, dres, lddr, dx, \
+                       lddx, part, m, eps);                                                                                  \
+  else                                                                                                                       \
+    hipLaunchKernelGGL((layernorm_bwd_kernel<LPR, false>), dim3(wgs), dim3(256), 0, s, x, ldx, dh, lddh, gamma, dres, lddr, dx, \
+                       lddx, part, m, eps)
   switch (c) {
     case 32: F3D_LNB(4); break;
     case 64: F3D_LNB(8); break;
@@ -615,6 +626,21 @@ int f3d_layernorm_bwd_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* 
                      accumulate);
   F3D_CHECK_HIP(hipGetLastError());
   return F3D_OK;
+}
+
+int f3d_layernorm_bwd_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* dh, uint32_t lddh,
+                           const f3d_bf16_t* gamma, const f3d_bf16_t* dres, uint32_t lddr, f3d_bf16_t* dx, uint32_t lddx,
+                           float* dgamma, float* dbeta, uint32_t m, uint32_t c, float eps, uint32_t accumulate,
+                           int device, void* stream) {
+  return layernorm_bwd(x, ldx, dh, lddh, gamma, dres, lddr, dx, lddx, dgamma, dbeta, m, c, eps, accumulate, false, device, stream);
+}
+
+int f3d_layernorm_bwd_add_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* dh, uint32_t lddh,
+                               const f3d_bf16_t* gamma, const f3d_bf16_t* dres, uint32_t lddr, f3d_bf16_t* dx, uint32_t lddx,
+                               float* dgamma, float* dbeta, uint32_t m, uint32_t c, float eps, uint32_t accumulate,
+                               int device, void* stream) {
+  F3D_CHECK_ARG(dres || m == 0, "null tensor pointer");
+  return layernorm_bwd(x, ldx, dh, lddh, gamma, dres, lddr, dx, lddx, dgamma, dbeta, m, c, eps, accumulate, true, device, stream);
 }
 
 int f3d_swiglu_bwd_bf16(const f3d_bf16_t* z, uint32_t ldz, const f3d_bf16_t* da, uint32_t ldda, f3d_bf16_t* dz,

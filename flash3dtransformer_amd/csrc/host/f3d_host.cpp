@@ -56,6 +56,7 @@ bool plain(const Tensor& t) { return !t.is_inference() && t.layout() == at::kStr
 bool activations(const Tensor& t, int64_t cols) {
   return t.defined() && t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() >= 1 && t.size(-1) == cols && plain(t);
 }
+bool fold_width(int64_t c) { return c == 32 || c == 64 || c == 128 || c == 256 || c == 512; }      // LayerNorm kernels
 Tensor two_axes(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
 
 // bf16 copies of fp32 tensors in one launch and one buffer, transposed copies where asked, and a second buffer for copies
@@ -131,12 +132,14 @@ Tensor as_grad_of(const Tensor& g, const Tensor& like) {
 struct LnGrads {
   Tensor dx, dg, db;
 };
-LnGrads ln_backward(const Tensor& x, const Tensor& dh, const Tensor& g16, const Tensor& dres, double eps) {
+// dres: another gradient of x, added before the one rounding to bf16, or (`apart`) after it
+LnGrads ln_backward(const Tensor& x, const Tensor& dh, const Tensor& g16, const Tensor& dres, double eps, bool apart = false) {
   const int64_t m = x.size(0), c = x.size(1);
   LnGrads r{empty_like_device({m, c}, at::kBFloat16, x), empty_like_device({c}, at::kFloat, x), empty_like_device({c}, at::kFloat, x)};
   const Place p = place_of(x);
-  check_covered(f3d_layernorm_bwd_bf16(bf(x), ld(x), bf(dh), ld(dh), bf(g16), bf(dres), ld(dres), bf(r.dx), ld(r.dx), f32(r.dg), f32(r.db),
-                               (uint32_t)m, (uint32_t)c, (float)eps, 0, p.device, p.stream));
+  check_covered((apart ? f3d_layernorm_bwd_add_bf16 : f3d_layernorm_bwd_bf16)(
+      bf(x), ld(x), bf(dh), ld(dh), bf(g16), bf(dres), ld(dres), bf(r.dx), ld(r.dx), f32(r.dg), f32(r.db), (uint32_t)m, (uint32_t)c,
+      (float)eps, 0, p.device, p.stream));
   return r;
 }
 void wgrad(const Tensor& dy, const Tensor& x, const Tensor& dw, const Tensor& db) {
@@ -228,6 +231,46 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
   }
 };
 
+// y = LayerNorm(x) w^T + b and x itself once more, for a residual: the gradient that comes back by that way is added where
+// LayerNorm's own dx is written (with the bits of adding the two tensors), instead of by a pass over both
+struct ForkNode : torch::autograd::Function<ForkNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const OptTensor& bias_, const Tensor& ln_w,
+                               const OptTensor& ln_b_, double eps) {
+    const Tensor bias = or_undefined(bias_), ln_b = or_undefined(ln_b_);
+    const Copies c = cast({weight, bias, ln_w, ln_b}, {0}, {0});
+    const Tensor x2 = bf16_rows(x);
+    const Tensor y = empty_like_device({x2.size(0), weight.size(0)}, at::kBFloat16, x);
+    ln_linear(x2, c.copy[2], c.copy[3], eps, c.copy[0], c.copy[1], Tensor(), y, F3D_ACT_NONE);
+    ctx->save_for_backward({x, weight, bias, ln_w, ln_b, c.copy[2], c.copy[3], c.turned[0]});
+    ctx->saved_data["edges"] = edges({&x, &weight, &bias, &ln_w, &ln_b});
+    ctx->saved_data["eps"] = eps;
+    return {y, x};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const Tensor &x = s[0], &weight = s[1], &bias = s[2], &ln_w = s[3], &ln_b = s[4], &g16 = s[5], &b16 = s[6], &wt = s[7];
+    const Wanted want(ctx, "edges");
+    const double eps = ctx->saved_data["eps"].toDouble();
+    const Tensor dy = bf16_rows(grads[0]), dres = bf16_rows(grads[1]), x2 = bf16_rows(x);
+    const int64_t m = x2.size(0), k = x2.size(1), n = dy.size(1);
+    const Tensor h = empty_like_device({m, k}, at::kBFloat16, x2);
+    layernorm(x2.contiguous(), g16, b16, h, eps);
+    Tensor dw, db;
+    if (want(1) || want(2)) {
+      dw = empty_like_device({n, k}, at::kFloat, x2);
+      if (bias.defined()) db = empty_like_device({n}, at::kFloat, x2);
+      wgrad(dy, h, dw, db);
+    }
+    LnGrads r;
+    if (want(0) || want(3) || want(4)) {
+      linear(dy, wt, Tensor(), Tensor(), h);      // h <- dh
+      r = ln_backward(x2, h, g16, dres, eps, true);
+    }
+    return {want(0) ? as_grad_of(r.dx, x) : Tensor(), want(1) ? as_grad_of(dw, weight) : Tensor(), want(2) ? as_grad_of(db, bias) : Tensor(),
+            want(3) ? as_grad_of(r.dg, ln_w) : Tensor(), want(4) ? as_grad_of(r.db, ln_b) : Tensor(), Tensor()};
+  }
+};
+
 // None: not a case of this module (the caller's Python path takes it, and raises what there is to raise)
 py::object linear_train(const Tensor& x, const Tensor& weight, const OptTensor& bias, const OptTensor& residual, const OptTensor& ln_w,
                         const OptTensor& ln_b, double eps) {
@@ -247,6 +290,19 @@ py::object linear_train(const Tensor& x, const Tensor& weight, const OptTensor& 
   std::vector<int64_t> shape = x.sizes().vec();
   shape.back() = n;
   return py::cast(y.view(shape));
+}
+
+py::object linear_fork(const Tensor& x, const Tensor& weight, const OptTensor& bias, const Tensor& ln_w, const OptTensor& ln_b, double eps) {
+  if (weight.dim() != 2) return py::none();
+  const int64_t n = weight.size(0), k = weight.size(1);
+  if (!activations(x, k) || !x.requires_grad() || n % 8 || !fold_width(k) || !master(weight, x, {n, k}) || !master(or_undefined(bias), x, {n}) ||
+      !master(ln_w, x, {k}) || !master(or_undefined(ln_b), x, {k}))
+    return py::none();
+  const variable_list r = ForkNode::apply(two_axes(x), weight, bias, ln_w, ln_b, eps);
+  if (x.dim() == 2) return py::make_tuple(r[0], r[1]);
+  std::vector<int64_t> shape = x.sizes().vec();
+  shape.back() = n;
+  return py::make_tuple(r[0].view(shape), r[1].view(x.sizes()));
 }
 
 // the gated MLP with its LayerNorm (+ residual); the backward of layers/nn_ops.py: _GatedMLPGrad
@@ -299,8 +355,6 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
             want(6) ? as_grad_of(dw2, w2) : Tensor(), want(7) ? as_grad_of(db2, b2) : Tensor(), Tensor(), Tensor()};
   }
 };
-
-bool fold_width(int64_t c) { return c == 32 || c == 64 || c == 128 || c == 256 || c == 512; }
 
 py::object mlp_train(const Tensor& x, const OptTensor& residual, const Tensor& ln_w, const Tensor& ln_b, const Tensor& w1, const Tensor& b1,
                      const Tensor& w2, const Tensor& b2, double eps, bool one_kernel) {
@@ -531,6 +585,7 @@ py::object block_infer(WeightCache& cache, const Tensor& x, const std::vector<Op
 
 PYBIND11_MODULE(_f3d_host, m) {
   m.def("linear_train", &linear_train);
+  m.def("linear_fork", &linear_fork);
   m.def("mlp_train", &mlp_train);
   m.def("attention_qkv", &attention_qkv);
   m.def("linear_infer", &linear_infer);

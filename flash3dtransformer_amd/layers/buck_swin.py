@@ -9,7 +9,7 @@ from torch.autograd import Function
 from ..lib import pshattn
 from ..psh import dev_context as f3ddev
 from ..psh import swin_attn as sa
-from .nn_ops import CoordEmbedding, LayerNorm, Linear, _DerivedCache, norm_params_bf16
+from .nn_ops import CoordEmbedding, LayerNorm, Linear, _as_built, _DerivedCache, _global_hooks, norm_params_bf16
 
 
 class BuckSwinFwdFunction(Function):
@@ -140,7 +140,17 @@ class BucketSwinAttentionModule(nn.Module):
         attn_out = self._attention_of_embedding(x, pre_norm, scope_buckets) if isinstance(x, CoordEmbedding) else None
         if attn_out is None:
             # pre_norm: LayerNorm applied inside the projection kernel; a CoordEmbedding is formed there too
-            qkv = self.qkv.embedded(x, pre_norm).view(B, L, -1) if isinstance(x, CoordEmbedding) else self.qkv(x, pre_norm=pre_norm)
+            forked = None
+            if residual is x and not skip_proj and type(x) is torch.Tensor and x.requires_grad and torch.is_grad_enabled() and x.is_cuda \
+                    and isinstance(pre_norm, LayerNorm) and _as_built(self.qkv, Linear) and not _global_hooks():
+                # x also runs past the attention: its two gradients meet in the backward of this layer's LayerNorm
+                forked = self.qkv.forked(x, pre_norm)
+            if forked is not None:
+                qkv, residual = forked
+            elif isinstance(x, CoordEmbedding):
+                qkv = self.qkv.embedded(x, pre_norm).view(B, L, -1)
+            else:
+                qkv = self.qkv(x, pre_norm=pre_norm)
             if qkv.is_cuda:
                 attn_out = pshattn.host().attention_qkv(qkv, scope_buckets, self.attn.buck_size, self.num_heads,
                                                         _covers(scope_buckets, self.attn.buck_size, L))

@@ -224,6 +224,18 @@ def refresh_weights(module: nn.Module) -> None:
         _BN_AFFINE.pop(m, None)
 
 
+def _as_built(module: nn.Module, kind: type) -> bool:
+    """exactly this class, with no hooks and no forward of its own: skipping its __call__ changes nothing"""
+    return type(module) is kind and "forward" not in module.__dict__ and not (
+        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+def _global_hooks() -> bool:
+    m = torch.nn.modules.module
+    return bool(m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
+                or m._global_backward_pre_hooks)
+
+
 def as_bf16_2d(x: torch.Tensor) -> torch.Tensor:
     if x.dtype != torch.bfloat16:
         x = x.to(torch.bfloat16)
@@ -467,6 +479,15 @@ class Linear(_CachedParamModule):
         else:
             out = torch_backward(y, _linear_ref(act, eps), x_in, self.weight, self.bias, res_in, ln_w, ln_b)
         return out.view(*lead, n_out)
+
+    def forked(self, x: torch.Tensor, pre_norm: "LayerNorm"):
+        """(forward(x, pre_norm=pre_norm), x) in training, x to be used in place of the argument for a residual: the gradient
+        that reaches it is added inside the LayerNorm backward.  None where the kernels do not apply."""
+        got = pshattn.host().linear_fork(x, self.weight, self.bias, pre_norm.weight, pre_norm.bias, pre_norm.eps)
+        if got is not None:
+            for c in (self._w, self._b, pre_norm._w, pre_norm._b):
+                c.clear()
+        return got
 
     def embedded(self, emb: "CoordEmbedding", pre_norm):
         """forward(emb.materialize(), pre_norm=pre_norm) without storing the embedding: inference only"""

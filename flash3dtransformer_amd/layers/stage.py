@@ -10,8 +10,8 @@ from ..lib import pshattn
 from ..psh import bucket_scope
 from ..psh import dev_context as f3ddev
 from . import buck_swin, elem_wise
-from .nn_ops import (CoordEmbedding, LayerNorm, LayerNormMLP, Linear, _CachedParamModule, _HostCache, apply_norm,
-                     is_fusable_layernorm, materialize)
+from .nn_ops import (CoordEmbedding, LayerNorm, LayerNormMLP, Linear, _as_built, _CachedParamModule, _global_hooks, _HostCache,
+                     apply_norm, is_fusable_layernorm, materialize)
 
 
 @dataclass(slots=True)
@@ -22,18 +22,6 @@ class XFMRSpecs:
     qkv_bias: bool
     swin_plan: bucket_scope.SwinPlan
     norm_layer: callable
-
-
-def _as_built(module: nn.Module, kind: type) -> bool:
-    """the package's own class with no hooks and no forward of its own: skipping its __call__ changes nothing"""
-    return type(module) is kind and "forward" not in module.__dict__ and not (
-        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
-
-
-def _global_hooks() -> bool:
-    m = torch.nn.modules.module
-    return bool(m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
-                or m._global_backward_pre_hooks)
 
 
 class XFMR(_CachedParamModule):
@@ -94,7 +82,9 @@ class XFMR(_CachedParamModule):
                 mid = self.bwa.proj(attn, residual=materialize(reduced_feat))
                 out = self.mlp(mid, residual=mid)
         else:
-            mid = self.bwa(x.view(1, N, C), scope_bucks, residual=reduced_feat.view(1, N, C), pre_norm=pre).view(N, C)
+            x_in = x.view(1, N, C)
+            mid = self.bwa(x_in, scope_bucks, residual=x_in if x is reduced_feat else reduced_feat.view(1, N, C),
+                           pre_norm=pre).view(N, C)
             out = self.mlp(mid, residual=mid)
         if f3ddev.get_nvtx():
             nvtx.range_pop()

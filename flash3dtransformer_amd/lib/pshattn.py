@@ -66,6 +66,7 @@ _SIGNATURES = {
     "f3d_affine_act_bf16": "ppppuuuip",
     "f3d_linear_wgrad_bf16": "pupuppuuuuip",
     "f3d_layernorm_bwd_bf16": "pupuppupuppuufuip",
+    "f3d_layernorm_bwd_add_bf16": "pupuppupuppuufuip",
     "f3d_swiglu_bwd_bf16": "pupupupuuuip",
     "f3d_mlp_gate_bwd_bf16": "pupuppppupuuuuip",
 }

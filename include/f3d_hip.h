@@ -432,6 +432,12 @@ int f3d_layernorm_bwd_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* 
                            float* dgamma, float* dbeta, uint32_t m, uint32_t c, float eps, uint32_t accumulate,
                            int device, void* stream);
 
+/* The same with dres added as a second tensor would be: dx = bf16(bf16(LayerNorm's own dx) + dres).  dres is not NULL. */
+int f3d_layernorm_bwd_add_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* dh, uint32_t lddh,
+                               const f3d_bf16_t* gamma, const f3d_bf16_t* dres, uint32_t lddr, f3d_bf16_t* dx, uint32_t lddx,
+                               float* dgamma, float* dbeta, uint32_t m, uint32_t c, float eps, uint32_t accumulate,
+                               int device, void* stream);
+
 /* Backward of the gated activation a = silu(z[:, :h]) * z[:, h:] (F3D_ACT_SWIGLU):
  *   dz[:, :h] = da * z2 * s (1 + z1 (1 - s)),  dz[:, h:] = da * silu(z1),  s = sigmoid(z1).
  * z, dz [m,2h] bf16, da [m,h] bf16, a [m,h] bf16 or NULL (the recomputed activation, which the weight gradient of

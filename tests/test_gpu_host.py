@@ -81,6 +81,27 @@ def test_linear_training_step(rows, k, n, bias, norm, residual, form, python_pat
     _same(run(), python_path(run))
 
 
+@pytest.mark.parametrize("rows,k,n", [(1, 32, 96), (33, 64, 8), (257, 128, 384), (515, 256, 768), (70, 512, 64)])
+def test_input_that_is_used_twice(rows, k, n, python_path):
+    """Linear.forked against the layer and its input used by themselves, their two gradients added by autograd"""
+    from flash3dtransformer_amd import layers as L
+    torch.manual_seed(rows)
+    both = nn.ModuleList([L.Linear(k, n), L.LayerNorm(k)]).to(DEV)
+    x = torch.randn(rows, k, device=DEV).to(torch.bfloat16)
+    scale = torch.randn(rows, k, device=DEV).to(torch.bfloat16)
+
+    def run(forked):
+        def call(t):
+            y, again = both[0].forked(t, both[1]) if forked else (both[0](t, pre_norm=both[1]), t)
+            return torch.cat([y, again * scale], dim=1)
+        return _step(both, call, x)
+    _same(run(True), python_path(lambda: run(False)))
+    hooked = []
+    both[0].register_forward_hook(lambda *a: hooked.append(1))
+    run(False)
+    assert hooked
+
+
 @pytest.mark.parametrize("rows,c,hid,own_residual", [(1, 32, 128, True), (333, 64, 256, True), (130, 128, 96, False), (700, 256, 1024, True),
                                                      (65, 512, 2048, None)])
 def test_mlp_training_step(rows, c, hid, own_residual, python_path):
@@ -97,7 +118,8 @@ def test_mlp_training_step(rows, c, hid, own_residual, python_path):
     _same(run(), python_path(run))
 
 
-@pytest.mark.parametrize("c,heads,scope,rows,whole", [(64, 2, 1, 1536, True), (32, 2, 2, 2048, True), (128, 2, 1, 1024, False)])
+@pytest.mark.parametrize("c,heads,scope,rows,whole", [(64, 2, 1, 1536, True), (32, 2, 2, 2048, True), (128, 2, 1, 1024, False),
+                                                        (256, 8, 1, 512, True), (512, 16, 1, 512, True)])
 def test_block_training_step(c, heads, scope, rows, whole, python_path):
     """whole: a table that covers all rows, as a plan makes it; otherwise a table of the first bucket alone"""
     from flash3dtransformer_amd import layers as L
