@@ -22,7 +22,7 @@ class SubbuckReduceFunction(Function):
                                                            out_alignment=out_alignment, build_follows=True)
         pshattn.batch_subbuck_reduce(coords, input_feat, seps, max_n, subbuck_size, NUM_VOX, sb.bbox_min, sb.bbox_max,
                                      sb.subbuck_id, sb.subbuck_off, sb.reduced_sep, sb.reduced_coord, sb.reduced_feat,
-                                     sb.unpool_ind, 1, reduction_op)
+                                     sb.unpool_ind, 1, reduction_op, fill=True)
         sb.mark_built(seps, coords.shape[0])
         ctx.save_for_backward(input_feat, sb.unpool_ind)
         ctx.subbuck_size, ctx.reduction_op, ctx.covered = subbuck_size, reduction_op, sb.covers(input_feat.shape[0])
@@ -69,7 +69,7 @@ class InbucketPoolingLayer(nn.Module):
         sb = f3dsubbuck.SubbuckBuffers.create_subbuck_buff(coords, feat, seps, self.subbuck_size,
                                                            out_alignment=self.out_align, build_follows=True)
         pshattn.subbuck_build(coords, seps, max_n, self.subbuck_size, NUM_VOX, sb.subbuck_id, sb.subbuck_off,
-                              sb.reduced_sep, sb.reduced_coord, sb.unpool_ind)
+                              sb.reduced_sep, sb.reduced_coord, sb.unpool_ind, (sb.bbox_min, sb.bbox_max))
         pshattn.reduce_feat_norm(feat, coords.shape[0], sb.unpool_ind, sb.reduced_feat, self.subbuck_size,
                                  self.reduction_op, post[0], post[1])
         sb.remove_unused_buffers()

@@ -38,6 +38,7 @@ _SIGNATURES = {
     "f3d_coord_bbox": "puppip",
     "f3d_batch_subbuck_reduce": "pppuuuuuupppppppupuuuip",
     "f3d_subbuck_build": "ppuuuuuppppupuip",
+    "f3d_subbuck_build_filled": "ppuuuuuppppupuppip",
     "f3d_reduce_feat": "puupuuupuip",
     "f3d_reduce_feat_norm": "puupuuupuuppppfuip",
     "f3d_additive_unpool_fwd": "ppppuuuuip",
@@ -364,8 +365,9 @@ def batch_bucket_sanitizer_cpu(bucket_id, bucket_counter, bucket_offset, offset_
 
 def batch_subbuck_reduce(scattered_coord, scattered_feat, batch_sep, instance_max_N, subbuck_size, num_vox,
                          bbox_min, bbox_max, subbuck_id, subbuck_off, reduced_batch_sep, reduced_coord,
-                         reduced_feat, unpool_ind, hash_type, red_op):
-    """src/f3d_frontend.cu:60-66 -> src/psh/batch_subbuck_pooling_dispatcher.cu:35-144"""
+                         reduced_feat, unpool_ind, hash_type, red_op, fill=False):
+    """src/f3d_frontend.cu:60-66 -> src/psh/batch_subbuck_pooling_dispatcher.cu:35-144.  fill: unpool_ind and the box come as
+    they were allocated, see subbuck_build"""
     ts = [scattered_coord, scattered_feat, batch_sep, subbuck_id, subbuck_off, reduced_batch_sep, reduced_coord,
           reduced_feat]
     assert_contiguous(ts + [unpool_ind])
@@ -385,6 +387,15 @@ def batch_subbuck_reduce(scattered_coord, scattered_feat, batch_sep, instance_ma
         raise RuntimeError(f"Unpool_ind last dimension({unpool_ind.shape[1]}) != subbucket_size({subbuck_size})")
     # Rows of the feature tensor beyond the coordinate count are ignored, as in the reference
     # (total_N is taken from the coordinates, dispatcher :43).
+    if fill:
+        if red_op not in (0, 1, 2, 3):
+            raise RuntimeError(f"Unsupported reduction operation id-{red_op}")
+        subbuck_build(scattered_coord, batch_sep, instance_max_N, subbuck_size, num_vox, subbuck_id, subbuck_off,
+                      reduced_batch_sep, reduced_coord, unpool_ind, (bbox_min, bbox_max))
+        _check(_load().f3d_reduce_feat(
+            _ptr(scattered_feat), scattered_coord.shape[0], scattered_feat.shape[1], _ptr(unpool_ind), unpool_ind.shape[0],
+            subbuck_size, red_op, _ptr(reduced_feat), reduced_feat.shape[0], dev, _stream(dev)))
+        return
     _check(_load().f3d_batch_subbuck_reduce(
         _ptr(scattered_coord), _ptr(scattered_feat), _ptr(batch_sep), batch_sep.shape[0],
         scattered_coord.shape[0], instance_max_N, scattered_feat.shape[1], subbuck_size,
@@ -453,9 +464,11 @@ def _row_norm_args(norm, c):
 
 
 def subbuck_build(scattered_coord, batch_sep, instance_max_N, subbuck_size, num_vox, subbuck_id, subbuck_off,
-                  reduced_batch_sep, reduced_coord, unpool_ind):
+                  reduced_batch_sep, reduced_coord, unpool_ind, fill=None):
     """the first half of batch_subbuck_reduce alone (local_subbuck_ker, src/psh/batch_psh_subbuck_reduce.cuh:104-298):
-    sub-bucket ids / offsets, the inverse map and the reduced coordinates"""
+    sub-bucket ids / offsets, the inverse map and the reduced coordinates.  unpool_ind is prefilled with a value >= the number
+    of points, or comes as it was allocated with fill = (bbox_min, bbox_max): the builder then marks the empty slots of the
+    clouds' rows with the number of points + 3 and sets the box to the representable range"""
     ts = [scattered_coord, batch_sep, subbuck_id, subbuck_off, reduced_batch_sep, reduced_coord, unpool_ind]
     assert_contiguous(ts)
     dev = assert_same_device(ts)
@@ -467,11 +480,19 @@ def subbuck_build(scattered_coord, batch_sep, instance_max_N, subbuck_size, num_
                            f"dim({reduced_coord.shape[1]}) are NOT 3D.")
     if unpool_ind.shape[1] != subbuck_size:
         raise RuntimeError(f"Unpool_ind last dimension({unpool_ind.shape[1]}) != subbucket_size({subbuck_size})")
-    _check(_load().f3d_subbuck_build(
-        _ptr(scattered_coord), _ptr(batch_sep), batch_sep.shape[0], scattered_coord.shape[0],
-        instance_max_N, subbuck_size, num_vox, _ptr(subbuck_id), _ptr(subbuck_off),
-        _ptr(reduced_batch_sep), _ptr(reduced_coord), reduced_coord.shape[0], _ptr(unpool_ind),
-        unpool_ind.shape[0], dev, _stream(dev)))
+    args = [_ptr(scattered_coord), _ptr(batch_sep), batch_sep.shape[0], scattered_coord.shape[0],
+            instance_max_N, subbuck_size, num_vox, _ptr(subbuck_id), _ptr(subbuck_off),
+            _ptr(reduced_batch_sep), _ptr(reduced_coord), reduced_coord.shape[0], _ptr(unpool_ind),
+            unpool_ind.shape[0]]
+    if fill is None:
+        _check(_load().f3d_subbuck_build(*args, dev, _stream(dev)))
+        return
+    assert_contiguous(list(fill))
+    assert_same_device([scattered_coord, *fill])
+    assert_dtype(list(fill), torch.float16)
+    if any(b.numel() != 3 for b in fill):
+        raise RuntimeError("The box holds three coordinates a corner")
+    _check(_load().f3d_subbuck_build_filled(*args, _ptr(fill[0]), _ptr(fill[1]), dev, _stream(dev)))
 
 
 def reduce_feat_norm(feat, total_n, unpool_ind, reduced_feat, subbuck_size, red_op, norm, act=None):

@@ -62,14 +62,20 @@ class SubbuckBuffers:
         prefilled with an index >= N: that marks a slot no point was mapped to.  The reduced length is
         rounded up to `out_alignment` so the next level's attention buckets divide it; the op
         zero-fills the extra rows (the reference leaves them uninitialised).  build_follows: the caller runs the builder on
-        these clouds next, which writes the id of every point of them; only rows behind them then need clearing."""
+        these clouds next and has it fill the box and the map (`fill` of pshattn.subbuck_build); it writes the id of every
+        point of them, so only rows behind them then need clearing."""
         total_n, d = coords.shape
         dev = coords.device
+        red_len, _, red_sep = calc_red_sep_sizes(seps, subbuck_size)
+        filled = build_follows and red_len > 0
+
+        def full(shape, value, dtype):
+            return torch.empty(shape, dtype=dtype, device=dev) if filled else torch.full(shape, value, dtype=dtype, device=dev)
+
         # The op quantises inside each tile's own box; the whole-batch box is part of the reference
         # signature only.  It is kept cheap: no reduction pass, just the representable range.
-        bbox_min = torch.full((d,), -65504.0, dtype=torch.float16, device=dev)
-        bbox_max = torch.full((d,), 65504.0, dtype=torch.float16, device=dev)
-        red_len, _, red_sep = calc_red_sep_sizes(seps, subbuck_size)
+        bbox_min = full((d,), -65504.0, torch.float16)
+        bbox_max = full((d,), 65504.0, torch.float16)
         aligned = cdiv(red_len, out_alignment) * out_alignment
         all_written = build_follows and sum(f3dbatch.host_sizes(seps)) == total_n
         return SubbuckBuffers(
@@ -79,7 +85,7 @@ class SubbuckBuffers:
             red_sep,
             torch.empty(aligned, d, dtype=torch.float16, device=dev),
             torch.empty(aligned, input_feat.shape[1], dtype=input_feat.dtype, device=dev),
-            torch.full((red_len, subbuck_size), total_n + 3, dtype=torch.int32, device=dev).view(torch.uint32),
+            full((red_len, subbuck_size), total_n + 3, torch.int32).view(torch.uint32),
         )
 
     def remove_unused_buffers(self):

@@ -148,6 +148,14 @@ int f3d_subbuck_build(const f3d_half_t* coord, const uint32_t* batch_sep, uint32
                       uint32_t* subbuck_id, uint16_t* subbuck_off, const uint32_t* reduced_batch_sep,
                       f3d_half_t* reduced_coord, uint32_t reduced_aligned_n, uint32_t* unpool_ind,
                       uint32_t reduced_n, int device, void* stream);
+/* The same, for buffers that come as they were allocated: slots of the clouds' rows of unpool_ind that no point is mapped to
+ * are set to total_n + 3, and bbox_min / bbox_max [3] fp16 to the representable range (-65504, 65504).  A batch without
+ * points writes none of these. */
+int f3d_subbuck_build_filled(const f3d_half_t* coord, const uint32_t* batch_sep, uint32_t batch_size,
+                             uint32_t total_n, uint32_t instance_max_n, uint32_t subbuck_size, uint32_t num_vox,
+                             uint32_t* subbuck_id, uint16_t* subbuck_off, const uint32_t* reduced_batch_sep,
+                             f3d_half_t* reduced_coord, uint32_t reduced_aligned_n, uint32_t* unpool_ind,
+                             uint32_t reduced_n, f3d_half_t* bbox_min, f3d_half_t* bbox_max, int device, void* stream);
 int f3d_reduce_feat(const f3d_bf16_t* feat, uint32_t total_n, uint32_t feat_dim, const uint32_t* unpool_ind,
                     uint32_t reduced_n, uint32_t subbuck_size, uint32_t red_op, f3d_bf16_t* reduced_feat,
                     uint32_t reduced_aligned_n, int device, void* stream);

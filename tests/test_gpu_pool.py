@@ -48,6 +48,36 @@ def test_builder_and_reduce_bit_exact(oracle, S, op, sizes, C):
     assert np.array_equal(n_bf16_bits(sb.reduced_feat), want), "reduced features differ"
 
 
+@pytest.mark.parametrize("S,sizes,behind", [
+    (1, [1500, 1], 0), (2, [7, 1024, 1, 2051], 0), (3, [1023, 1024, 2], 5), (8, [4097, 0, 3], 0), (32, [2100, 33], 9),
+    (24, [1008, 1009, 23], 0), (1000, [999, 2001], 0), (1024, [1025, 1], 2),
+])
+@pytest.mark.parametrize("op", [0, 3])
+def test_builder_marks_empty_slots_itself(S, sizes, behind, op):
+    """buffers as they were allocated: the builder leaves the map, the box and all the rest as with a prefilled map, also
+    where clouds do not cover all rows, hold no point, or end on the first or last point of a tile"""
+    from flash3dtransformer_amd.lib import pshattn
+    from flash3dtransformer_amd.psh import subbuck
+    n = sum(sizes) + behind
+    rng = np.random.default_rng(S + n)
+    c = t_f16(rng.uniform(-30, 30, (n, 3)).astype(np.float16))
+    f, s = t_bf16_bits(bf16_bits(rng.normal(0, 1, (n, 16)))), t_u32(np.cumsum(sizes).astype(np.uint32))
+    out = []
+    for fill in (False, True):
+        sb = subbuck.SubbuckBuffers.create_subbuck_buff(c, f, s, S, out_alignment=16, build_follows=fill)
+        if fill:      # whatever the memory held
+            for t in (sb.unpool_ind.view(torch.int32), sb.bbox_min, sb.bbox_max, sb.reduced_coord, sb.reduced_feat):
+                t.fill_(3)
+        pshattn.batch_subbuck_reduce(c, f, s, max(sizes), S, 0xFFFF, sb.bbox_min, sb.bbox_max, sb.subbuck_id, sb.subbuck_off,
+                                     sb.reduced_sep, sb.reduced_coord, sb.reduced_feat, sb.unpool_ind, 1, op, fill=fill)
+        torch.cuda.synchronize()
+        out.append([sb.unpool_ind.view(torch.int32), sb.bbox_min, sb.bbox_max, sb.subbuck_id.view(torch.int32),
+                    sb.subbuck_off.view(torch.int16)[:sum(sizes)], sb.reduced_coord.view(torch.int16),
+                    sb.reduced_feat.view(torch.int16)])
+    for want, got in zip(*out):
+        assert torch.equal(want, got)
+
+
 def test_builder_long_runs_of_one_cell_bit_exact(oracle):
     """Clouds whose points share few distinct positions (one position only; three; a 2000-point cloud of 40 positions):
     whole tiles fall into one or a few cells of the counting sort, so the order inside a cell's run (input order) is
