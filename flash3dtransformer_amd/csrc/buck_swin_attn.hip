@@ -487,17 +487,22 @@ struct ScopeGen {
 // is consumed, exactly as the next item does otherwise) and the accumulators live across them.  Fixed-reference softmax
 // only: a wave whose row sums leave its range writes NaN into its rows' LSE instead of a result, and the launcher runs
 // the streaming kernel after this one for the workgroups that own such rows.
-template <int D, int T, int WAVES, bool GEN = false, bool STREAM = false>
+//
+// PARTS > 1: few items.  An item's queries are divided over PARTS workgroups of T / 32 / PARTS waves; each reads the whole
+// K and V.  A row's own sums do not change with it.
+template <int D, int T, int WAVES, bool GEN = false, bool STREAM = false, int PARTS = 1>
 __global__ __launch_bounds__(64 * WAVES) void buck_swin_fwd_scope_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, uint32_t ld,
     uint16_t* __restrict__ o, float* __restrict__ lse, const uint32_t* __restrict__ scope_buckets,
     uint32_t num_scope, uint32_t scope_size, uint32_t bs, uint32_t seq_len, uint32_t num_head,
     const int32_t* __restrict__ kv_len, float scale_log2, uint32_t n_items, uint32_t items_per_xcd,
     uint32_t n_slots, ScopeGen gen) {
-  constexpr int QB = T / (32 * WAVES);     // 32-query blocks per wave
+  constexpr int QB = T / (32 * WAVES * PARTS);     // 32-query blocks per wave
   static_assert(!GEN || (QB == 1 && D == 32), "rows formed in the kernel: one 32-row block per wave, 32-wide heads");
   static_assert(!(GEN && STREAM), "rows are formed in the kernel for resident scopes only");
+  static_assert(PARTS == 1 || !(GEN || STREAM), "queries are divided for resident scopes read from memory only");
   const uint32_t n_kb = STREAM ? scope_size : 1u;       // key buckets an item walks
+  const uint32_t n_qb = STREAM ? scope_size : (uint32_t)PARTS;    // items that share a (batch, scope, head): query buckets or parts
   constexpr int KSTEPS = D / 16;
   constexpr int CPK = D / 8;               // 16-byte chunks per row
   constexpr int ROWB = D * 2;              // bytes per K / V row in LDS
@@ -549,19 +554,19 @@ __global__ __launch_bounds__(64 * WAVES) void buck_swin_fwd_scope_kernel(
   // advances by a mixed-radix addition with carries, one division at the start and none per item (the scalar unit
   // is shared by all waves of a SIMD, and every wave does this bookkeeping).
   struct Pos {
-    uint32_t qb, head, scope, batch;      // qb: the item's query bucket inside its scope (STREAM; 0 otherwise)
+    uint32_t qb, head, scope, batch;      // qb: the item's query bucket (STREAM) or part (PARTS > 1) inside its scope, or 0
   };
-  // STREAM: the query bucket is the fastest index, so that the items that share a scope's K and V run at the same time
+  // the query bucket or part is the fastest index, so that the items that share a scope's K and V run at the same time
   // on one XCD
-  const uint32_t slots_h = n_slots / n_kb;
-  const uint32_t d_qb = n_slots % n_kb, d_head = slots_h % num_head, d_scope = (slots_h / num_head) % num_scope,
+  const uint32_t slots_h = n_slots / n_qb;
+  const uint32_t d_qb = n_slots % n_qb, d_head = slots_h % num_head, d_scope = (slots_h / num_head) % num_scope,
                  d_batch = slots_h / (num_head * num_scope);
   auto advance = [&](Pos p) {
     uint32_t carry = 0;
-    if constexpr (STREAM) {
+    if constexpr (STREAM || PARTS > 1) {
       p.qb += d_qb;
-      carry = p.qb >= n_kb ? 1u : 0u;
-      p.qb -= carry ? n_kb : 0u;
+      carry = p.qb >= n_qb ? 1u : 0u;
+      p.qb -= carry ? n_qb : 0u;
     }
     p.head += d_head + carry;
     carry = p.head >= num_head ? 1u : 0u;
@@ -610,9 +615,11 @@ __global__ __launch_bounds__(64 * WAVES) void buck_swin_fwd_scope_kernel(
     if (i < (uint32_t)BPW) lds_dma16_at(reinterpret_cast<const char*>(k) + g, dma_k, buf_addr + blk * 1024);
     else lds_dma16_at(reinterpret_cast<const char*>(v) + g, dma_v, buf_addr + OPB + blk * 1024);
   };
+  // first query of the wave's block b inside the scope (STREAM: inside the query bucket)
+  auto q_local_of = [&](const Pos& p, uint32_t b) { return (PARTS > 1 ? p.qb * (T / PARTS) : 0u) + (wave * QB + b) * 32u; };
   // row inside the sequence of query lq of block b (0 when the scope entry names no bucket of the sequence)
   auto q_row_of = [&](const Pos& p, const Scope& sc, uint32_t b) {
-    const uint32_t q_local = (wave * QB + b) * 32u, qj = STREAM ? 0u : q_local / bs;
+    const uint32_t q_local = q_local_of(p, b), qj = STREAM ? 0u : q_local / bs;
     const uint32_t id = bucket_of(sc, STREAM ? p.qb : qj);
     return (id < n_bucket ? id : 0u) * bs + (q_local - qj * bs) + lq;
   };
@@ -626,8 +633,8 @@ __global__ __launch_bounds__(64 * WAVES) void buck_swin_fwd_scope_kernel(
   };
 
   // ---- prologue: the first item's scope, K / V / Q; the second item's bucket ids ----
-  const uint32_t item_h = item_lo / n_kb;
-  Pos p_cur = {item_lo % n_kb, item_h % num_head, (item_h / num_head) % num_scope, item_h / (num_head * num_scope)};
+  const uint32_t item_h = item_lo / n_qb;
+  Pos p_cur = {item_lo % n_qb, item_h % num_head, (item_h / num_head) % num_scope, item_h / (num_head * num_scope)};
   Pos p_nxt = advance(p_cur);
   Scope cur, nxt;
   cur.ids = load_ids(p_cur);
@@ -787,7 +794,7 @@ __global__ __launch_bounds__(64 * WAVES) void buck_swin_fwd_scope_kernel(
       any_keys = false;
 #pragma unroll
       for (int b = 0; b < QB; ++b) {
-        const uint32_t q_local = (wave * QB + b) * 32u, qj = STREAM ? p_cur.qb : q_local / bs;
+        const uint32_t q_local = q_local_of(p_cur, b), qj = STREAM ? p_cur.qb : q_local / bs;
         const int32_t in_b = (int32_t)(STREAM ? q_local : q_local - qj * bs);
         q_exists[b] = bucket_of(cur, qj) < n_bucket;
         q_len[b] = len_of(cur, qj) - in_b;               // valid rows of the block, counted from its first row
@@ -1075,12 +1082,12 @@ __global__ __launch_bounds__(64 * WAVES) void buck_swin_fwd_scope_kernel(
   }
 }
 
-template <int D, int T, int WAVES, bool GEN = false, bool STREAM = false>
+template <int D, int T, int WAVES, bool GEN = false, bool STREAM = false, int PARTS = 1>
 static int launch_attn_scope(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint32_t ld, uint16_t* o, float* lse,
                              const uint32_t* scope_buckets, uint32_t num_scope, uint32_t scope_size, uint32_t bs,
                              uint32_t batch, uint32_t seq_len, uint32_t num_head, const int32_t* kv_len, int device,
                              hipStream_t s, ScopeGen gen = ScopeGen{nullptr, nullptr, nullptr}) {
-  const uint64_t n_items64 = (uint64_t)batch * num_scope * num_head * (STREAM ? scope_size : 1u);
+  const uint64_t n_items64 = (uint64_t)batch * num_scope * num_head * (STREAM ? scope_size : (uint32_t)PARTS);
   if (n_items64 == 0) return F3D_OK;
   if (n_items64 > 0x7FFFFFF0ull / (STREAM ? scope_size : 1u)) {
     set_error("attention problem too large for one launch (%llu items)", (unsigned long long)n_items64);
@@ -1092,9 +1099,9 @@ static int launch_attn_scope(const uint16_t* q, const uint16_t* k, const uint16_
   static int wg_per_cu[64] = {};
   int per_cu = (device >= 0 && device < 64) ? wg_per_cu[device] : 0;
   if (per_cu == 0) {
-    F3D_CHECK_HIP(hipFuncSetAttribute((const void*)buck_swin_fwd_scope_kernel<D, T, WAVES, GEN, STREAM>,
+    F3D_CHECK_HIP(hipFuncSetAttribute((const void*)buck_swin_fwd_scope_kernel<D, T, WAVES, GEN, STREAM, PARTS>,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    F3D_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, buck_swin_fwd_scope_kernel<D, T, WAVES, GEN, STREAM>,
+    F3D_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, buck_swin_fwd_scope_kernel<D, T, WAVES, GEN, STREAM, PARTS>,
                                                                64 * WAVES, lds));
     if (per_cu < 1) per_cu = 1;
     if (device >= 0 && device < 64) wg_per_cu[device] = per_cu;
@@ -1105,7 +1112,7 @@ static int launch_attn_scope(const uint16_t* q, const uint16_t* k, const uint16_
   const uint32_t items_per_xcd = cdiv_u32(n_items, kNumXcd);
   const uint32_t n_slots = std::max(1u, std::min((uint32_t)n_cu * (uint32_t)per_cu / kNumXcd, items_per_xcd));
   const float scale_log2 = 1.4426950408889634f / sqrtf((float)D);
-  hipLaunchKernelGGL((buck_swin_fwd_scope_kernel<D, T, WAVES, GEN, STREAM>), dim3(n_slots * kNumXcd), dim3(64 * WAVES), lds, s, q, k,
+  hipLaunchKernelGGL((buck_swin_fwd_scope_kernel<D, T, WAVES, GEN, STREAM, PARTS>), dim3(n_slots * kNumXcd), dim3(64 * WAVES), lds, s, q, k,
                      v, ld, o, lse, scope_buckets, num_scope, scope_size, bs, seq_len, num_head, kv_len, scale_log2,
                      n_items, items_per_xcd, n_slots, gen);
   return F3D_OK;
@@ -1258,13 +1265,30 @@ int f3d_buck_swin_fwd_strided(const f3d_bf16_t* q, const f3d_bf16_t* k, const f3
   const uint32_t scope_tokens = scope_size * bucket_size;
   if (head_dim <= 32 && scope_size <= (uint32_t)kResMaxScope && (scope_tokens == 256 || scope_tokens == 512) &&
       (uint64_t)seq_len * qkv_row_stride * 2 < (1ull << 32)) {
-#define F3D_RES(DD, TT)                                                                                         \
-  rc = launch_attn_scope<DD, TT, TT / 32>(q, k, v, qkv_row_stride, o, lse, scope_buckets, num_scope, scope_size, \
-                                          bucket_size, batch, seq_len, num_head, kv_len, device, s)
-    if (head_dim == 16) {
-      if (scope_tokens == 256) F3D_RES(16, 256); else F3D_RES(16, 512);
+    // Too few (batch, scope, head) items for one a CU: several workgroups take parts of an item's queries, each with all of
+    // the scope's K and V, as long as every part still finds a CU of its own (the buffers leave room for one 512-token
+    // workgroup a CU).  512 tokens, 8 heads of 32, 1 / 2 / 4 parts in us: 48 items 11.7 / 8.4 / 7.5, 64 items 11.9 / 8.5 /
+    // 7.9, 96 items 12.1 / 8.8 / 11.8, 128 items 12.4 / 9.5 / 12.1, 192 items 12.8 / 14.6 / 16.6.  256 tokens: 48 items
+    // 5.3 / 4.7 / 5.1, 128 items 5.8 / 5.4 / 6.6, 256 items 6.4 / 7.1 / 10.5: four parts never pay there.
+    int n_cu = 0;
+    F3D_CHECK_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, device));
+    const uint64_t n_items = (uint64_t)batch * num_scope * num_head;
+#define F3D_RES(DD, TT, PP)                                                                                                 \
+  rc = launch_attn_scope<DD, TT, TT / 32 / PP, false, false, PP>(q, k, v, qkv_row_stride, o, lse, scope_buckets, num_scope, \
+                                                                 scope_size, bucket_size, batch, seq_len, num_head, kv_len, \
+                                                                 device, s)
+    if (scope_tokens == 512 && 4u * n_items <= (uint64_t)n_cu) {
+      if (head_dim == 16) F3D_RES(16, 512, 4); else F3D_RES(32, 512, 4);
+    } else if (2u * n_items <= (uint64_t)n_cu) {
+      if (head_dim == 16) {
+        if (scope_tokens == 256) F3D_RES(16, 256, 2); else F3D_RES(16, 512, 2);
+      } else {
+        if (scope_tokens == 256) F3D_RES(32, 256, 2); else F3D_RES(32, 512, 2);
+      }
+    } else if (head_dim == 16) {
+      if (scope_tokens == 256) F3D_RES(16, 256, 1); else F3D_RES(16, 512, 1);
     } else {
-      if (scope_tokens == 256) F3D_RES(32, 256); else F3D_RES(32, 512);
+      if (scope_tokens == 256) F3D_RES(32, 256, 1); else F3D_RES(32, 512, 1);
     }
 #undef F3D_RES
     if (rc != F3D_OK) return rc;

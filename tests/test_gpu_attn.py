@@ -52,6 +52,33 @@ def test_single_global_scope_is_full_attention(oracle, B, L, H, D, bs):
     assert (LSE > 0).all()          # reference checks strict positivity at these sizes (:404-411)
 
 
+@pytest.mark.parametrize("D,bs,scope,buckets,H", [
+    (32, 512, 1, 16, 4), (32, 512, 1, 13, 5), (16, 512, 1, 8, 8), (32, 512, 1, 16, 8), (16, 512, 1, 43, 3),
+    (32, 256, 1, 16, 8), (16, 256, 1, 3, 1), (32, 256, 2, 8, 3), (16, 128, 4, 32, 9), (32, 128, 2, 32, 8), (32, 128, 2, 34, 8),
+])
+@pytest.mark.parametrize("scale,masked", [(1.0, False), (1.0, True), (12.0, True)])
+def test_few_items_divide_their_queries(D, bs, scope, buckets, H, scale, masked):
+    """Up to a quarter or half as many (scope, head) items as there are CUs, several workgroups take parts of an item's
+    queries: rows are what they are in a batch with enough items for one each, bit for bit (a row's own products, their
+    order and the choice of its wave's pass are the same), with masks, entries outside the sequence and sums out of the
+    fast pass's range."""
+    rng = np.random.default_rng(D + bs + buckets)
+    L = buckets * bs
+    Q, K, V = _qkv(D * buckets + H, 1, L, H, D, scale)
+    scopes = rng.permutation(buckets).astype(np.uint32).reshape(-1, scope)
+    kv_len = None
+    if masked:
+        kv_len = rng.integers(0, bs + 1, buckets)
+        kv_len[:2] = 0, 1
+        scopes[0, -1] = buckets + 7
+    many = -(-300 // (H * len(scopes)))          # 300 items and more: one workgroup each
+    few = _run(Q, K, V, scopes, bs, kv_len)
+    rep = _run(*(t.expand(many, -1, -1, -1).contiguous() for t in (Q, K, V)), scopes, bs, kv_len)
+    for a, b in zip(few, rep):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[0], b[-1])
+    assert few[0].abs().sum() > 0
+
+
 def test_permuted_bucket_order_inside_scope(oracle):
     """reference test_attn_fwd.py:418-452"""
     B, L, H, D, bs = 4, 1280, 2, 128, 256
