@@ -584,8 +584,11 @@ __global__ __launch_bounds__(64 * kMlpSmallWaves) void ln_mlp_swiglu_small_kerne
     for (int e = 0; e < 8; ++e) idf[j][e] = (lq == (uint32_t)(16 * j + e) + 8u * half) ? (__bf16)1.0f : (__bf16)0.0f;
   const uint32_t poff = lq * ROWB + (((half ^ G::swz(lq)) & (uint32_t)(G::CPR - 1)) << 4);
   const uint32_t tile_step = gridDim.x * WAVES;
-  if (blockIdx.x * WAVES + wave < ntiles) request_x(blockIdx.x * WAVES + wave);
-  for (uint32_t tile = blockIdx.x * WAVES + wave; tile < ntiles; tile += tile_step) {
+  // with fewer tiles than waves, the first wave of every workgroup gets one before the second of any; otherwise a workgroup's
+  // waves take neighbouring tiles (480,000 rows, C = 32: 38.3 us, spread 40.7)
+  const uint32_t tile0 = ntiles < tile_step ? wave * gridDim.x + blockIdx.x : blockIdx.x * WAVES + wave;
+  if (tile0 < ntiles) request_x(tile0);
+  for (uint32_t tile = tile0; tile < ntiles; tile += tile_step) {
     const uint32_t row0 = tile * 32;
     // ---- the tile's rows of x -> registers (B-operand layout) through the wave's patch ----
     bf16x8_t xf[KS];
@@ -795,7 +798,10 @@ static int launch_mlp(const uint16_t* x, uint32_t ldx, float eps, const uint16_t
     if (device >= 0 && device < 64) attr_set[device] = true;
   }
   // Whole turns of the chip run 256-row workgroups; what is left over is spread over all CUs in panels of fewer rows
-  // (fewer waves with work per workgroup), so that the last turn is shorter than a full one.
+  // (fewer waves with work per workgroup), so that the last turn is shorter than a full one.  That holds for a call of less
+  // than one turn too: four waves or fewer have a SIMD each.  C = 128, weights prepared with it, in us, 256-row panels and now:
+  // 5,632 rows 33.0 -> 24.4, 16,384 rows 33.8 -> 25.3, 32,000 rows 34.9 -> 28.4, 45,000 rows 35.7 -> 34.7; C = 256: 2,816
+  // rows 86.8 -> 60.6, 16,384 rows 88.6 -> 63.5.
   static int cus[64] = {};
   int n_cu = 256;
   if (device >= 0 && device < 64) {
@@ -805,7 +811,7 @@ static int launch_mlp(const uint16_t* x, uint32_t ldx, float eps, const uint16_t
   constexpr uint32_t kRows = 32 * kMlpWaves;
   const uint32_t panels = cdiv_u32(M, kRows);
   uint32_t main_wgs = panels, tail_rows = kRows, tail_wgs = 0;
-  if (panels > (uint32_t)n_cu && panels % (uint32_t)n_cu != 0) {
+  if (panels % (uint32_t)n_cu != 0) {
     main_wgs = panels / (uint32_t)n_cu * (uint32_t)n_cu;
     const uint32_t left = M - main_wgs * kRows;
     tail_rows = cdiv_u32(cdiv_u32(left, (uint32_t)n_cu), 32u) * 32u;
@@ -835,9 +841,14 @@ static int launch_mlp_small(const uint16_t* x, uint32_t ldx, float eps, const ui
     F3D_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if (device >= 0 && device < 64) attr_lds[device] = lds;
   }
-  // as many resident workgroups as the LDS allows; each wave then walks its share of the 32-row tiles
+  // As many resident workgroups as the LDS allows; each wave then walks its share of the 32-row tiles.  Up to a tile for
+  // every wave of one workgroup a CU there are no more than that: the tiles spread over the CUs before a second wave of a
+  // workgroup gets one, and no CU loads the weights twice.  In us, weights prepared with it, eight tiles a workgroup
+  // and now: C = 64: 3,000 rows 14.6 -> 11.1, 10,752 rows 14.9 -> 11.5, 60,000 rows 17.7 -> 16.7; C = 32: 3,000 rows 8.6 -> 7.0,
+  // 21,504 rows 8.8 -> 7.5, 40,000 rows 8.9 -> 8.7 (with a tile a workgroup 11.4), 80,000 rows 13.4 -> 12.1.
   const uint32_t per_cu = (uint32_t)std::max<size_t>(1, std::min<size_t>(4, (160 * 1024) / lds));
-  const uint32_t wgs = std::min<uint32_t>(cdiv_u32(cdiv_u32(M, 32), kMlpSmallWaves), (uint32_t)n_cu * per_cu);
+  const uint32_t tiles = cdiv_u32(M, 32);
+  const uint32_t wgs = std::min<uint32_t>(tiles, (uint32_t)n_cu * (tiles <= (uint32_t)(n_cu * kMlpSmallWaves) ? 1u : per_cu));
   hipLaunchKernelGGL(kern, dim3(wgs), dim3(64 * kMlpSmallWaves), lds, s, x, ldx, eps, w1p, b32, w2p, bias2, residual, ldr,
                      y, ldy, M, H, pj);
   return F3D_OK;

@@ -290,6 +290,22 @@ def test_proj_residual_mlp_in_one_kernel(oracle, M, C, H, use_bias):
     assert err_us.mean() <= 1.25 * err_ref.mean() + 1e-4, (err_us.mean(), err_ref.mean())
 
 
+@pytest.mark.parametrize("C,H,many", [(128, 512, 65536), (256, 64, 65536), (64, 256, 90000), (32, 128, 90000)])
+def test_mlp_rows_do_not_depend_on_the_panel_they_fall_into(C, H, many):
+    """Calls of less than one turn of the chip spread their rows over all CUs (panels of 32 to 256 rows, one tile a wave): each
+    row is what it is in a call of whole panels, bit for bit, at the edges of every panel height."""
+    from flash3dtransformer_amd.lib import pshattn
+    g = torch.Generator().manual_seed(C)
+    mk = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    a, x, wp, gam, w1, w2 = mk(many, C), mk(many, C), mk(C, C), mk(C), mk(2 * H, C), mk(C, H)
+    full = torch.empty_like(x)
+    assert pshattn.proj_ln_mlp_swiglu_bf16(a, wp, None, x, gam, None, 1e-5, w1, None, w2, None, full)
+    for m in (1, 32, 33, 257, 8192, 8193, 16385, 24577, 32769, 57345, 65503):
+        y = torch.full((m + 1, C), 3.0, dtype=torch.bfloat16, device=DEV)
+        assert pshattn.proj_ln_mlp_swiglu_bf16(a[:m], wp, None, x[:m], gam, None, 1e-5, w1, None, w2, None, y[:m])
+        assert torch.equal(y[:m], full[:m]) and (y[m] == 3.0).all(), m
+
+
 def test_proj_residual_mlp_unsupported_width_is_reported():
     from flash3dtransformer_amd.lib import pshattn
     mk = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=DEV)
