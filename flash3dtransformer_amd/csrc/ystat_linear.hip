@@ -3,7 +3,7 @@
 // where the reference runs te.LayerNormMLP's second GEMM) and the input gradients of QKV and fc1.
 //
 // The row-panel kernel keeps x in registers, which stops at 512 inner features.  Here the OUTPUT is what stays in
-// registers: a workgroup of eight waves owns 128 or 256 rows x 128 or 256 output columns; waves w and w + 4 (the two waves
+// registers: a workgroup of eight waves owns 128 or 256 rows x 64 to 256 output columns; waves w and w + 4 (the two waves
 // of a SIMD) share a block of rows and split the columns, so a wave holds at most 64 rows x 128 columns of fp32
 // accumulators (128 registers) and two waves per SIMD fit.  Rows of x and of w stream through LDS 64 inner features at a
 // time, straight from HBM / L2 (global_load ... lds).  The product is formed transposed (A operand = rows of w) so that a
@@ -13,13 +13,13 @@
 // loads: 64), measured on L2-resident data.  With x fetched in 32-byte pieces in operand order the loads took twice
 // the time of the products; in whole lines with the pieces swizzled they take half of it, w needs no re-laid copy, and
 // the matrix cores set the pace.  30,208 x 512, K = 4096: 155 -> 126 us (1.0 PFLOP/s; the tiled GEMM 207), 60,416 x 256,
-// K = 1024: 48 -> 40 us, 8,192 x 512, K = 4096: 46 us (tiled GEMM 70), 1,536 x 512, K = 2048: 24 us (37).
+// K = 1024: 48 -> 40 us, 8,192 x 512, K = 4096: 46 us (tiled GEMM 70), 1,536 x 512, K = 2048: 24 us (37), 20 in 64 columns.
 #include "xstat_common.h"
 #include <algorithm>
 
 namespace f3d {
 
-// A ring of 2 (256 x 256) to 5 (128 x 128) buffers, each w and x of one chunk.
+// A ring of 2 (256 x 256) to 6 (128 x 64) buffers, each w and x of one chunk.
 constexpr int kYsWaves = 8, kYsChunkK = 64;
 constexpr uint32_t kYsXcd = 8;
 
@@ -231,6 +231,11 @@ int launch_ystat_linear(const uint16_t* x, uint32_t ldx, const uint16_t* w, cons
   auto cost = [](uint64_t panels, uint32_t weight) { return (panels + 255) / 256 * weight; };
   const uint64_t wide = N % 256 == 0 ? cost((uint64_t)rows2 * (N / 256), 20) : ~0ull;
   const uint64_t tall = cost((uint64_t)rows2 * (N / 128), 15), small = cost((uint64_t)rows1 * (N / 128), 11);
+  // Fewer than half as many 128 x 128 panels as CUs: 128 x 64 ones, three quarters of the bytes a chunk and twice the CUs that
+  // ask for them.  K = 2048, N = 512, in us: 1,536 rows 22.0 -> 19.5, 4,096 rows 23.3 -> 20.6, but 8,192 rows 29 -> 39 (two
+  // rounds); K = 1024, N = 256: 5,632 rows 12.7 -> 11.4.
+  if (!in_place && 2u * (uint64_t)rows1 * (N / 128) <= 256)
+    return launch_ys<64, 1>(x, ldx, w, bias, residual, ldr, y, ldy, M, N, K, device, s);
   if ((in_place && N == 256) || (wide <= tall && wide <= small)) return launch_ys<256, 2>(x, ldx, w, bias, residual, ldr, y, ldy, M, N, K, device, s);
   if (tall <= small) return launch_ys<128, 2>(x, ldx, w, bias, residual, ldr, y, ldy, M, N, K, device, s);
   return launch_ys<128, 1>(x, ldx, w, bias, residual, ldr, y, ldy, M, N, K, device, s);

@@ -290,6 +290,21 @@ def test_proj_residual_mlp_in_one_kernel(oracle, M, C, H, use_bias):
     assert err_us.mean() <= 1.25 * err_ref.mean() + 1e-4, (err_us.mean(), err_ref.mean())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 128, 576), (127, 512, 1024), (4096, 512, 1088), (4097, 512, 1088), (130, 8192, 1024)])
+def test_few_output_panels_are_halved(M, N, K):
+    """up to half as many 128 x 128 panels as CUs run as 128 x 64 ones: rows are what they are in a larger call, bit for bit (a
+    value's products and their order are the same), and nothing is written past the last row"""
+    from flash3dtransformer_amd.lib import pshattn
+    g = torch.Generator().manual_seed(M + N)
+    mk = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    many = max(2 * M, 128 * (300 // (N // 128)))
+    x, w, b, r = mk(many, K), mk(N, K), mk(N), mk(many, N)
+    full, y = torch.empty_like(r), torch.full((M + 1, N), 3.0, dtype=torch.bfloat16, device=DEV)
+    pshattn.linear_bf16(x, w, b, r, full)
+    pshattn.linear_bf16(x[:M], w, b, r[:M], y[:M])
+    assert torch.equal(y[:M], full[:M]) and (y[M] == 3.0).all()
+
+
 @pytest.mark.parametrize("C,H,many", [(128, 512, 65536), (256, 64, 65536), (64, 256, 90000), (32, 128, 90000)])
 def test_mlp_rows_do_not_depend_on_the_panel_they_fall_into(C, H, many):
     """Calls of less than one turn of the chip spread their rows over all CUs (panels of 32 to 256 rows, one tile a wave): each
