@@ -443,7 +443,7 @@ int f3d_ln_linear_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* gamm
   }
   if (rc != F3D_OK) return rc;
   F3D_CHECK_HIP(hipGetLastError());
-  return F3D_OK;
+  return staged.succeeded();
 }
 
 int f3d_embed_ln_linear_bf16(const f3d_half_t* coord, const f3d_bf16_t* embed_table, const f3d_bf16_t* gamma,
@@ -470,7 +470,7 @@ int f3d_embed_ln_linear_bf16(const f3d_half_t* coord, const f3d_bf16_t* embed_ta
                                      s, coord, embed_table);
   if (rc != F3D_OK) return rc;
   F3D_CHECK_HIP(hipGetLastError());
-  return F3D_OK;
+  return staged.succeeded();
 }
 
 int f3d_gemm_sm_bf16(const f3d_bf16_t* a, const f3d_bf16_t* b, f3d_bf16_t* o, uint32_t m, uint32_t n, uint32_t k,

@@ -26,8 +26,10 @@ void* workspace(int device, size_t bytes, hipStream_t stream);
 // *ready: the staged buffer already holds this call's prepared weights, the preparation launch is skipped.
 // nullptr + error message when the staged buffer is too small or the workspace cannot grow.
 void* weight_area(int device, size_t bytes, bool* ready, hipStream_t stream);
-// Declared at the top of every dense entry point: whatever the call does, the staging ends with it.
+// Declared at the top of every dense entry point: whatever the call does, the staging ends with it.  An entry point that
+// asks for a weight_area returns succeeded() (F3D_OK) behind its last launch: f3d_staged_weights_kept then says so.
 struct StagedWeightsScope {
+  int succeeded();
   ~StagedWeightsScope();
 };
 

@@ -70,6 +70,7 @@ static thread_local struct {
   void* buf = nullptr;
   size_t bytes = 0;
   bool ready = false, armed = false;
+  bool taken = false, kept = false;      // the call asked for the buffer; it returned F3D_OK after that
 } g_staged;
 
 void* weight_area(int device, size_t bytes, bool* ready, hipStream_t stream) {
@@ -80,11 +81,16 @@ void* weight_area(int device, size_t bytes, bool* ready, hipStream_t stream) {
       return nullptr;
     }
     *ready = g_staged.ready;
+    g_staged.taken = true;
     return g_staged.buf;
   }
   return workspace(device, bytes, stream);
 }
 
+int StagedWeightsScope::succeeded() {
+  if (g_staged.armed && g_staged.taken) g_staged.kept = true;
+  return F3D_OK;
+}
 StagedWeightsScope::~StagedWeightsScope() { g_staged.armed = false; }
 
 bool sync_stream_enabled() { return g_sync; }
@@ -152,7 +158,14 @@ int f3d_stage_weights(void* buf, size_t bytes, int ready) {
   f3d::g_staged.bytes = bytes;
   f3d::g_staged.ready = ready != 0;
   f3d::g_staged.armed = true;
+  f3d::g_staged.taken = f3d::g_staged.kept = false;
   return F3D_OK;
+}
+
+int f3d_staged_weights_kept(void) {
+  const bool kept = f3d::g_staged.kept;
+  f3d::g_staged.armed = f3d::g_staged.taken = f3d::g_staged.kept = false;
+  return kept ? 1 : 0;
 }
 
 }  // extern "C"

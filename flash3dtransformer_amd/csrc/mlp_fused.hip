@@ -905,7 +905,7 @@ int f3d_ln_mlp_swiglu_bf16(const f3d_bf16_t* x, uint32_t ldx, const f3d_bf16_t* 
   else rc = launch_mlp<128>(x, ldx, eps, w1p, b32, w2p, b2, residual, ldr, y, ldy, m, hidden, device, s);
   if (rc != F3D_OK) return rc;
   F3D_CHECK_HIP(hipGetLastError());
-  return F3D_OK;
+  return staged.succeeded();
 }
 
 // x != NULL: the block input is read; else coord / embed_table say how it is formed
@@ -964,7 +964,7 @@ static int proj_ln_mlp_impl(const f3d_bf16_t* a, uint32_t lda, const f3d_bf16_t*
 #undef F3D_PM
   if (rc != F3D_OK) return rc;
   F3D_CHECK_HIP(hipGetLastError());
-  return F3D_OK;
+  return staged.succeeded();
 }
 
 int f3d_proj_ln_mlp_swiglu_bf16(const f3d_bf16_t* a, uint32_t lda, const f3d_bf16_t* w_proj, const f3d_bf16_t* b_proj,

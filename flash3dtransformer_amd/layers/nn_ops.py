@@ -130,11 +130,13 @@ class _StagedWeights:
     def clear(self):
         self._key = self._src = None
 
-    def arm(self, training: bool, rows: int, cols: int, *tensors, tag=None):
-        """call right before the dense op: stages the buffer for it (no-op while weights may change)"""
+    def call(self, training: bool, rows: int, cols: int, tensors, tag, op, *args):
+        """op(*args), a dense op on these weights, with the buffer staged for it (not while the weights may change).  The
+        buffer counts as current only once the op has left the prepared weights there, which one that raises or has no
+        rows does not"""
         if training or torch.is_grad_enabled():
             self.clear()
-            return
+            return op(*args)
         live = [t for t in tensors if t is not None]
         key = (tag, rows, cols) + tuple([(t.data_ptr(), t._version, t.shape) for t in live])
         need = 3 * rows * cols + 4 * rows + 2 * cols + 512
@@ -142,8 +144,16 @@ class _StagedWeights:
             self._buf = torch.empty(need, dtype=torch.uint8, device=live[0].device)
             self._key = None
         ready = key == self._key
+        if not ready:
+            self.clear()
         pshattn.stage_weights(self._buf, ready)
-        self._key, self._src = key, live
+        try:
+            return op(*args)
+        finally:
+            if not pshattn.staged_weights_kept():
+                self.clear()
+            elif not ready:
+                self._key, self._src = key, live
 
 
 class _DerivedCache(_Bf16Cache):
@@ -462,9 +472,10 @@ class Linear(_CachedParamModule):
         if pre_norm is not None:
             g, b = fresh[0][2:] if fresh is not None and own_norm else norm_params_bf16(pre_norm)
             if isinstance(pre_norm, LayerNorm):     # its bf16 copies are kept between calls, a torch norm's are not
-                self._staged.arm(self.training or pre_norm.training, self.out_features, self.in_features, w16, b16, g, b,
-                                 tag=("ln", float(pre_norm.eps)))
-            pshattn.ln_linear_bf16(x2, g, b, pre_norm.eps, w16, b16, r2, y, act)
+                self._staged.call(self.training or pre_norm.training, self.out_features, self.in_features, (w16, b16, g, b),
+                                  ("ln", float(pre_norm.eps)), pshattn.ln_linear_bf16, x2, g, b, pre_norm.eps, w16, b16, r2, y, act)
+            else:
+                pshattn.ln_linear_bf16(x2, g, b, pre_norm.eps, w16, b16, r2, y, act)
         else:
             pshattn.linear_bf16(x2, w16, b16, r2, y, act)
         ln_w = None if pre_norm is None else pre_norm.weight
@@ -495,9 +506,9 @@ class Linear(_CachedParamModule):
             w16, b16 = self._w.get(self.weight, self.training), self._b.get(self.bias, self.training)
             g, b = norm_params_bf16(pre_norm)
             y = torch.empty(emb.shape[0], self.out_features, dtype=torch.bfloat16, device=emb.device)
-            self._staged.arm(self.training or pre_norm.training, self.out_features, self.in_features, w16, b16, g, b,
-                             tag=("ln", float(pre_norm.eps)))
-            if pshattn.embed_ln_linear_bf16(emb.coord, emb.table(), g, b, pre_norm.eps, w16, b16, y):
+            if self._staged.call(self.training or pre_norm.training, self.out_features, self.in_features, (w16, b16, g, b),
+                                 ("ln", float(pre_norm.eps)), pshattn.embed_ln_linear_bf16, emb.coord, emb.table(), g, b,
+                                 pre_norm.eps, w16, b16, y):
                 return y
         return self.forward(emb.materialize(), pre_norm=pre_norm)
 
@@ -733,13 +744,13 @@ class LayerNormMLP(_CachedParamModule):
         g16, be16, w1_16, b1_16, w2_16, b2_16 = (c.get(p, self.training) for c, p in zip(self._c, params))
         wp16, bp16 = proj._w.get(proj.weight, proj.training), proj._b.get(proj.bias, proj.training)
         y = torch.empty(a2.shape[0], self.hidden_size, dtype=torch.bfloat16, device=a.device)
-        self._staged.arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16, w2_16, b2_16,
-                            tag=("mlp", float(self.eps)))
+        weights = (g16, be16, w1_16, b1_16, w2_16, b2_16)
         if lazy is not None:
-            ok = pshattn.embed_proj_ln_mlp_swiglu_bf16(a2, wp16, bp16, lazy.coord, lazy.table(), g16, be16, self.eps, w1_16,
-                                                       b1_16, w2_16, b2_16, y)
+            op, x_args = pshattn.embed_proj_ln_mlp_swiglu_bf16, (lazy.coord, lazy.table())
         else:
-            ok = pshattn.proj_ln_mlp_swiglu_bf16(a2, wp16, bp16, x2, g16, be16, self.eps, w1_16, b1_16, w2_16, b2_16, y)
+            op, x_args = pshattn.proj_ln_mlp_swiglu_bf16, (x2,)
+        ok = self._staged.call(self.training, w1_16.shape[0], self.hidden_size, weights, ("mlp", float(self.eps)), op, a2, wp16,
+                               bp16, *x_args, g16, be16, self.eps, w1_16, b1_16, w2_16, b2_16, y)
         return y.view(x.shape) if ok else None
 
     def takes_projection(self, rows: int) -> bool:
@@ -782,16 +793,16 @@ class LayerNormMLP(_CachedParamModule):
         # on request, the whole gated MLP in one kernel where one exists ...
         fused = self.one_kernel(x2.shape[0])
         if fused:
-            self._staged.arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16, w2_16, b2_16,
-                                tag=("mlp", float(self.eps)))
-            fused = pshattn.ln_mlp_swiglu_bf16(x2, g16, be16, self.eps, w1_16, b1_16, w2_16, b2_16, r2, y)
+            fused = self._staged.call(self.training, w1_16.shape[0], self.hidden_size, (g16, be16, w1_16, b1_16, w2_16, b2_16),
+                                      ("mlp", float(self.eps)), pshattn.ln_mlp_swiglu_bf16, x2, g16, be16, self.eps, w1_16, b1_16,
+                                      w2_16, b2_16, r2, y)
         if not fused:
             # ... otherwise LayerNorm + fc1 + activation, then fc2 + residual
             h = torch.empty(x2.shape[0], self.ffn_hidden_size, dtype=torch.bfloat16, device=x.device)
             if self.hidden_size in FUSABLE_LN_WIDTHS:
-                self._staged.arm(self.training, w1_16.shape[0], self.hidden_size, g16, be16, w1_16, b1_16,
-                                    tag=("fc1", float(self.eps)))
-                pshattn.ln_linear_bf16(x2, g16, be16, self.eps, w1_16, b1_16, None, h, self.activation)
+                self._staged.call(self.training, w1_16.shape[0], self.hidden_size, (g16, be16, w1_16, b1_16),
+                                  ("fc1", float(self.eps)), pshattn.ln_linear_bf16, x2, g16, be16, self.eps, w1_16, b1_16, None, h,
+                                  self.activation)
             else:
                 ln = torch.empty_like(x2)
                 pshattn.layernorm_bf16(x2, g16, be16, ln, self.eps)

@@ -53,6 +53,7 @@ _SIGNATURES = {
     "f3d_buck_swin_fwd": "ppppppuuuuuuupip",
     "f3d_buck_swin_fwd_strided": "pppupppuuuuuuupip",
     "f3d_stage_weights": "pQi",
+    "f3d_staged_weights_kept": "",
     "f3d_gemm_sm_bf16": "pppuuuip",
     "f3d_linear_bf16": "pupppupuuuuuip",
     "f3d_ln_linear_bf16": "puppfpppupuuuuuip",
@@ -928,6 +929,11 @@ def stage_weights(buf: torch.Tensor, ready: bool):
     weights left there and skips the preparation launch"""
     assert_dtype([buf], torch.uint8)
     _check(_load().f3d_stage_weights(_ptr(buf), buf.numel(), 1 if ready else 0))
+
+
+def staged_weights_kept() -> bool:
+    """whether the dense call after stage_weights left its prepared weights in the buffer; ends a staging that no call used"""
+    return _load().f3d_staged_weights_kept() != 0
 
 
 def layernorm_bf16(x, gamma, beta, y, eps=1e-5):

@@ -290,8 +290,13 @@ int f3d_buck_swin_fwd_strided(const f3d_bf16_t* q, const f3d_bf16_t* k, const f3
  * weight of n rows and k columns 3 n k + 4 n + 2 k + 512 bytes cover every case, with n = the fc1 rows for the
  * gated MLP), or, with ready != 0, takes what an earlier call with the same weights and shapes left there and skips
  * the preparation launch.  The staging ends with that call whatever its outcome.  A buffer that is too small makes
- * the call fail with a message. */
+ * the call fail with a message.
+ * f3d_staged_weights_kept, asked right after that call, returns 1 if the buffer now holds the prepared weights: the call
+ * used it and returned F3D_OK.  0 after a call that failed, that had no rows or columns (it returns before it prepares
+ * anything) or that prepares nothing: the buffer is then to be staged with ready = 0 again.  It also ends a staging that no
+ * dense call followed. */
 int f3d_stage_weights(void* buf, size_t bytes, int ready);
+int f3d_staged_weights_kept(void);
 
 /* ---- dense layers --------------------------------------------------------------------------
  * gemm_sm_bf16(A[M,K], B[K,N], O[M,N]) — src/f3d_frontend.cu:87-88, src/psh/gemm_dispatcher.cu;

@@ -99,3 +99,18 @@ def test_linear_without_outputs_launches_nothing(lib, m, n, k, act):
     if k == 64:
         assert lib.f3d_ln_linear_bf16(p, u(k), p, none, ctypes.c_float(1e-5), p, none, none, u(0), p, u(64), u(m), u(n), u(k),
                                       u(act), *end) == 0
+
+
+def test_staged_buffer_is_not_kept_by_a_call_that_prepares_nothing(lib):
+    """a refused call, an empty one and none at all: f3d_staged_weights_kept says no, and ends the staging"""
+    at = lambda a: ctypes.c_void_p(a)
+    u, f = ctypes.c_uint32, ctypes.c_float
+
+    def ln_linear(x, m):
+        return lib.f3d_ln_linear_bf16(at(x), u(256), at(4096), None, f(1e-5), at(8192), None, None, u(0), at(16384), u(64), u(m), u(64),
+                                      u(256), u(0), 0, None)
+    assert lib.f3d_staged_weights_kept() == 0
+    for call in (lambda: ln_linear(2, 8) != 0, lambda: ln_linear(32768, 0) == 0, lambda: True):
+        assert lib.f3d_stage_weights(at(65536), ctypes.c_size_t(1 << 20), 0) == 0
+        assert call()
+        assert lib.f3d_staged_weights_kept() == 0

@@ -532,6 +532,35 @@ def test_staged_weights_are_reused_and_refreshed():
     pshattn.ln_linear_bf16(x[:64], g, g, 1e-5, w, None, None, y, None)     # the staging ended with the failed call
 
 
+@pytest.mark.parametrize("bad", ["misaligned", "shapes"])
+@pytest.mark.parametrize("kind", ["linear", "narrow mlp", "mlp", "two-kernel mlp"])
+def test_staged_weights_are_current_only_once_prepared(kind, bad):
+    """a first call that raises, in the library or in the binding ahead of it, leaves the staged buffer as it was allocated: the next
+    call prepares it, and no other layer's call meets a staging that was left behind"""
+    from flash3dtransformer_amd import layers as L
+    C = {"linear": 256, "narrow mlp": 64, "mlp": 128, "two-kernel mlp": 512}[kind]
+
+    def make(seed):
+        torch.manual_seed(seed)
+        norm, layer = L.LayerNorm(C).to(DEV).eval(), (L.Linear(C, C) if kind == "linear" else L.LayerNormMLP(C, 4 * C)).to(DEV).eval()
+        return layer, (lambda x, r=None: layer(x, residual=r, pre_norm=norm)) if kind == "linear" else lambda x, r=None: layer(x, residual=r)
+    x, wide = [torch.randn(96, c, device=DEV).to(torch.bfloat16) for c in (C, C + 8)]
+    with torch.no_grad():
+        (layer, call), (other, other_call) = make(1), make(2)
+        rows = layer.weight.shape[0] if kind == "linear" else 8 * C
+        need = 3 * rows * C + 4 * rows + 2 * C + 512
+        junk = [torch.full((need,), 255, dtype=torch.uint8, device=DEV) for _ in range(4)]      # NaN, should it be read as weights
+        del junk
+        with pytest.raises(RuntimeError):
+            call(x, wide[:, 1:1 + C] if bad == "misaligned" else x[:95])
+        other.train()      # prepares per call, into the library's own memory
+        got_other = other_call(x)
+        got = call(x)
+        layer.train()
+        assert torch.isfinite(got).all() and torch.equal(got, call(x))
+        assert torch.equal(got_other, other_call(x))
+
+
 @pytest.mark.parametrize("M,N,K,use_bias,use_res", [
     (1, 128, 192, True, True),          # 128 x 128 panels: one row, the shortest inner dimension
     (129, 384, 640, False, True),       # ... a second row panel of one row, three column panels, no bias
