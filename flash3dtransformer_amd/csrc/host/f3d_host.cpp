@@ -152,11 +152,15 @@ void linear(const Tensor& x, const Tensor& w, const Tensor& b, const Tensor& res
   check(f3d_linear_bf16(bf(x), ld(x), bf(w), bf(b), bf(residual), ld(residual), bf(y), ld(y), (uint32_t)x.size(0),
                         (uint32_t)w.size(0), (uint32_t)w.size(1), F3D_ACT_NONE, p.device, p.stream));
 }
+int ln_linear_code(const Tensor& x, const Tensor& g, const Tensor& be, double eps, const Tensor& w, const Tensor& b,
+                   const Tensor& residual, const Tensor& y, uint32_t act) {
+  const Place p = place_of(x);
+  return f3d_ln_linear_bf16(bf(x), ld(x), bf(g), bf(be), (float)eps, bf(w), bf(b), bf(residual), ld(residual), bf(y), ld(y),
+                            (uint32_t)x.size(0), (uint32_t)w.size(0), (uint32_t)w.size(1), act, p.device, p.stream);
+}
 void ln_linear(const Tensor& x, const Tensor& g, const Tensor& be, double eps, const Tensor& w, const Tensor& b,
                const Tensor& residual, const Tensor& y, uint32_t act) {
-  const Place p = place_of(x);
-  check(f3d_ln_linear_bf16(bf(x), ld(x), bf(g), bf(be), (float)eps, bf(w), bf(b), bf(residual), ld(residual), bf(y), ld(y),
-                           (uint32_t)x.size(0), (uint32_t)w.size(0), (uint32_t)w.size(1), act, p.device, p.stream));
+  check(ln_linear_code(x, g, be, eps, w, b, residual, y, act));
 }
 void layernorm(const Tensor& x, const Tensor& g, const Tensor& be, const Tensor& y, double eps) {
   const Place p = place_of(x);
@@ -503,19 +507,26 @@ struct WeightCache {
     }
     return true;
   }
-  // right before the dense call that prepares w [rows, cols]
-  void stage(int b, const Tensor& w, double eps, int kind) {
+  // the code of call(), the dense call that prepares w [rows, cols], with the buffer staged for it.  The buffer is ready once
+  // the call has left the weights there, and the staging ends, however the call ends.
+  template <typename Call>
+  int staged_call(int b, const Tensor& w, double eps, int kind, Call call) {
     const int64_t rows = w.size(0), cols = w.size(1), need = 3 * rows * cols + 4 * rows + 2 * cols + 512;
     Staged& s = staged[b];
     if (!s.buf.defined() || s.buf.numel() < need || s.buf.device() != w.device()) {
-      s.buf = empty_like_device({need}, at::kByte, w);
       s.ready = false;
+      s.buf = empty_like_device({need}, at::kByte, w);
     }
-    if (s.eps != eps || s.kind != kind) s.ready = false;
-    check(f3d_stage_weights(s.buf.data_ptr(), (size_t)s.buf.numel(), s.ready ? 1 : 0));
-    s.ready = true;
+    const bool ready = s.ready && s.eps == eps && s.kind == kind;
+    s.ready = false;
     s.eps = eps;
     s.kind = kind;
+    check(f3d_stage_weights(s.buf.data_ptr(), (size_t)s.buf.numel(), ready ? 1 : 0));
+    struct End {
+      Staged& s;
+      ~End() { s.ready = f3d_staged_weights_kept() != 0; }
+    } end{s};
+    return call();
   }
 };
 
@@ -543,40 +554,38 @@ py::object block_infer(WeightCache& cache, const Tensor& x, const std::vector<Op
   if (!cache.update(ps, {0, 4, 6, 12})) return py::none();
   auto w = [&](int i) -> const Tensor& { return cache.slots[i].value; };
 
-  const Tensor qkv = empty_like_device({1, m, 3 * c}, at::kBFloat16, x);
-  cache.stage(0, w(2), eps, 0);
-  ln_linear(x, w(0), w(1), eps, w(2), w(3), Tensor(), qkv.view({m, 3 * c}), F3D_ACT_NONE);
+  const Tensor qkv = empty_like_device({1, m, 3 * c}, at::kBFloat16, x), qkv_rows = qkv.view({m, 3 * c});
+  check(cache.staged_call(0, w(2), eps, 0,
+                          [&] { return ln_linear_code(x, w(0), w(1), eps, w(2), w(3), Tensor(), qkv_rows, F3D_ACT_NONE); }));
   const Tensor o = attention(qkv, scopes, bucket, heads, covers).O.view({m, c});
   const Tensor y = empty_like_device({m, c}, at::kBFloat16, x);
   const Place p = place_of(x);
   if (one_half) {
-    cache.stage(1, w(8), mlp_eps, 1);
-    const int rc = f3d_proj_ln_mlp_swiglu_bf16(bf(o), ld(o), bf(w(4)), bf(w(5)), bf(x), ld(x), bf(w(6)), bf(w(7)), (float)mlp_eps, bf(w(8)),
-                                               bf(w(9)), bf(w(10)), bf(w(11)), bf(y), ld(y), (uint32_t)m, (uint32_t)c, (uint32_t)hid, p.device,
-                                               p.stream);
+    const int rc = cache.staged_call(1, w(8), mlp_eps, 1, [&] {
+      return f3d_proj_ln_mlp_swiglu_bf16(bf(o), ld(o), bf(w(4)), bf(w(5)), bf(x), ld(x), bf(w(6)), bf(w(7)), (float)mlp_eps, bf(w(8)),
+                                         bf(w(9)), bf(w(10)), bf(w(11)), bf(y), ld(y), (uint32_t)m, (uint32_t)c, (uint32_t)hid, p.device,
+                                         p.stream);
+    });
     if (rc != F3D_ERR_UNSUPPORTED) {
-      if (rc != F3D_OK) cache.staged[1].ready = false;
       check(rc);
       return py::cast(y);
     }
-    cache.staged[1].ready = false;
   }
   const Tensor mid = empty_like_device({m, c}, at::kBFloat16, x);
   linear(o, w(4), w(5), x, mid);
   if (one_mlp) {
-    cache.stage(1, w(8), mlp_eps, 1);
-    const int rc = f3d_ln_mlp_swiglu_bf16(bf(mid), ld(mid), bf(w(6)), bf(w(7)), (float)mlp_eps, bf(w(8)), bf(w(9)), bf(w(10)), bf(w(11)), bf(mid),
-                                          ld(mid), bf(y), ld(y), (uint32_t)m, (uint32_t)c, (uint32_t)hid, p.device, p.stream);
+    const int rc = cache.staged_call(1, w(8), mlp_eps, 1, [&] {
+      return f3d_ln_mlp_swiglu_bf16(bf(mid), ld(mid), bf(w(6)), bf(w(7)), (float)mlp_eps, bf(w(8)), bf(w(9)), bf(w(10)), bf(w(11)), bf(mid),
+                                    ld(mid), bf(y), ld(y), (uint32_t)m, (uint32_t)c, (uint32_t)hid, p.device, p.stream);
+    });
     if (rc != F3D_ERR_UNSUPPORTED) {
-      if (rc != F3D_OK) cache.staged[1].ready = false;
       check(rc);
       return py::cast(y);
     }
-    cache.staged[1].ready = false;
   }
-  cache.stage(1, w(8), mlp_eps, 2);
   const Tensor h = empty_like_device({m, hid}, at::kBFloat16, x);
-  ln_linear(mid, w(6), w(7), mlp_eps, w(8), w(9), Tensor(), h, F3D_ACT_SWIGLU);
+  check(cache.staged_call(1, w(8), mlp_eps, 2,
+                          [&] { return ln_linear_code(mid, w(6), w(7), mlp_eps, w(8), w(9), Tensor(), h, F3D_ACT_SWIGLU); }));
   linear(h, w(10), w(11), mid, y);
   return py::cast(y);
 }

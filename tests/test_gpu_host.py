@@ -174,6 +174,50 @@ def test_block_inference(c, heads, rows, scope, python_path):
         _same(run(), python_path(run))
 
 
+def _fresh_block(c, heads):
+    """an inference block whose driver has prepared nothing yet, behind freed memory that reads as NaN"""
+    from flash3dtransformer_amd import layers as L
+    from flash3dtransformer_amd.psh.bucket_scope import SwinPlan
+    torch.manual_seed(c)
+    blk = L.XFMR(c, 4 * c, heads, 512, True, SwinPlan("swin", 512, 1, 0), lambda ch: L.LayerNorm(ch)).to(DEV).eval()
+    junk = [torch.full((3 * n * c * c + 4 * n * c + 2 * c + 512,), 255, dtype=torch.uint8, device=DEV) for n in (3, 8) for _ in range(2)]
+    del junk
+    return blk
+
+
+@pytest.mark.parametrize("c,heads", [(64, 2), (256, 8), (512, 16)])
+def test_block_after_a_call_that_was_refused(c, heads, python_path):
+    """an input off 16 bytes raises before anything is prepared; the next call prepares"""
+    blk = _fresh_block(c, heads)
+    x, wide = [torch.randn(1024, w, device=DEV).to(torch.bfloat16) for w in (c, c + 8)]
+    with torch.no_grad():
+        with pytest.raises(RuntimeError, match="16-byte"):
+            blk(None, wide[:, 1:1 + c], None)
+        got = blk(None, x, None)
+        _same(got, python_path(lambda: blk(None, x, None)))
+
+
+def test_block_after_a_call_that_ran_out_of_memory(python_path):
+    """the hidden activations (268 MB at 65,536 rows), last and largest, do not fit; a smaller call prepares the MLP's weights"""
+    blk = _fresh_block(512, 16)
+    rows, x = 65536, torch.randn(1024, 512, device=DEV).to(torch.bfloat16)
+    with torch.no_grad():
+        big = torch.zeros(rows, 512, dtype=torch.bfloat16, device=DEV)
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        room = rows * (3 * 512 * 2 + 3 * 512 * 2 + 16 * 4) + (64 << 20)      # qkv; o, mid, y; lse; weight copies
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / total)
+        try:
+            with pytest.raises(torch.cuda.OutOfMemoryError):
+                blk(None, big, None)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert blk._host._native is not None
+        got = blk(None, x, None)
+        _same(got, python_path(lambda: blk(None, x, None)))
+
+
 def test_attention_outside_the_kernels_is_told_apart():
     from flash3dtransformer_amd.layers.buck_swin import BucketSwinAttentionModule
     m = BucketSwinAttentionModule(48, 2, 512).to(DEV)      # 24-wide heads
