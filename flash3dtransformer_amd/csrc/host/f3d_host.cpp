@@ -281,7 +281,7 @@ py::object linear_train(const Tensor& x, const Tensor& weight, const OptTensor& 
   if (weight.dim() != 2) return py::none();
   const int64_t n = weight.size(0), k = weight.size(1);
   const bool norm = ln_w.has_value();
-  if (!activations(x, k) || !x.requires_grad() || n % 8 || k % 8 || !master(weight, x, {n, k}) || !master(or_undefined(bias), x, {n}) ||
+  if (n == 0 || k == 0 || !activations(x, k) || !x.requires_grad() || n % 8 || k % 8 || !master(weight, x, {n, k}) || !master(or_undefined(bias), x, {n}) ||
       (norm && !master(*ln_w, x, {k})) || (ln_b.has_value() && (!norm || !master(*ln_b, x, {k}))))
     return py::none();
   Tensor r2;
@@ -438,12 +438,12 @@ py::object attention_qkv(const Tensor& qkv, const Tensor& scopes, int64_t bucket
 // y = x w^T + b (+ residual) on bf16 copies of the parameters
 py::object linear_infer(const Tensor& x, const Tensor& w, const OptTensor& b_, const OptTensor& residual_) {
   const Tensor b = or_undefined(b_), residual = or_undefined(residual_);
-  if (w.dim() != 2 || x.dim() < 1 || x.numel() == 0) return py::none();
+  if (w.dim() != 2 || w.numel() == 0 || x.dim() < 1 || x.numel() == 0) return py::none();
   const int64_t n = w.size(0), k = w.size(1);
   auto ours = [&](const Tensor& t) { return t.scalar_type() == at::kBFloat16 && t.layout() == at::kStrided && t.device() == x.device(); };
   if (!x.is_cuda() || !ours(x) || x.size(-1) != k || x.stride(-1) != 1 || !ours(w) || !w.is_contiguous() ||
       (b.defined() && (!ours(b) || !b.is_contiguous() || b.dim() != 1 || b.size(0) != n)) ||
-      (residual.defined() && (!ours(residual) || residual.size(-1) != n || residual.stride(-1) != 1 || residual.numel() / n != x.numel() / k)))
+      (residual.defined() && (!ours(residual) || residual.dim() < 1 || residual.size(-1) != n || residual.stride(-1) != 1 || residual.numel() / n != x.numel() / k)))
     return py::none();
   const Tensor x2 = two_axes(x), y = empty_like_device({x2.size(0), n}, at::kBFloat16, x);
   linear(x2, w, b, residual.defined() ? two_axes(residual) : residual, y);

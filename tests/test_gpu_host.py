@@ -238,6 +238,21 @@ def test_linear_inference(rows, k, n, residual, python_path):
         _same(run(), python_path(run))
 
 
+def test_layers_without_columns_raise():
+    """no output columns, or no input columns, beside a residual: an error, in training and in inference"""
+    from flash3dtransformer_amd import layers as L
+    from flash3dtransformer_amd.lib import pshattn
+    lin = L.Linear(64, 0).to(DEV)
+    x, res = torch.zeros(5, 64, dtype=torch.bfloat16, device=DEV), torch.zeros(5, 0, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(RuntimeError):
+        lin(x.requires_grad_(), residual=res)
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        lin(x, residual=res)
+    nothing = torch.zeros(5, 0, dtype=torch.bfloat16, device=DEV, requires_grad=True)
+    assert pshattn.host().linear_train(nothing, torch.zeros(8, 0, device=DEV), None, torch.zeros(5, 8, dtype=torch.bfloat16, device=DEV), None,
+                                       None, 0.0) is None
+
+
 def test_saved_tensor_hooks_and_in_place_changes_are_seen():
     """the native nodes save through autograd: pack hooks run, and a weight changed between forward and backward is refused"""
     from flash3dtransformer_amd import layers as L
