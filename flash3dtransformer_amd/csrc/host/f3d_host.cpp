@@ -52,9 +52,9 @@ Tensor bf16_rows(const Tensor& t) {      // bf16 with unit column stride
 bool master(const Tensor& p, const Tensor& x, at::IntArrayRef shape) {      // an fp32 parameter this module takes
   return !p.defined() || (p.scalar_type() == at::kFloat && p.device() == x.device() && p.is_contiguous() && p.sizes() == shape);
 }
-bool plain(const Tensor& t) { return !t.is_inference() && t.layout() == at::kStrided && !t.is_neg() && !t.is_conj(); }
-bool activations(const Tensor& t, int64_t cols) {
-  return t.defined() && t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() >= 1 && t.size(-1) == cols && plain(t);
+bool plain(const Tensor& t) { return t.layout() == at::kStrided && !t.is_neg() && !t.is_conj(); }
+bool activations(const Tensor& t, int64_t cols) {      // ... of a training node, which saves them: no inference tensors
+  return t.defined() && t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() >= 1 && t.size(-1) == cols && plain(t) && !t.is_inference();
 }
 bool fold_width(int64_t c) { return c == 32 || c == 64 || c == 128 || c == 256 || c == 512; }      // LayerNorm kernels
 Tensor two_axes(const Tensor& t) { return t.dim() == 2 ? t : t.reshape({-1, t.size(-1)}); }
@@ -454,7 +454,8 @@ py::object linear_infer(const Tensor& x, const Tensor& w, const OptTensor& b_, c
 }
 
 // bf16 copies of a block's parameters and the buffers in which the kernels keep what they prepare from them, between
-// eval-mode forwards under no_grad: current while every parameter keeps its address, version, dtype and device
+// eval-mode forwards without gradients: current while every parameter keeps its address, version, dtype and device (one without a
+// version is not taken; activations need none)
 struct WeightCache {
   struct Key {
     const void* at = nullptr;

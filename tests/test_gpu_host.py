@@ -218,6 +218,33 @@ def test_block_after_a_call_that_ran_out_of_memory(python_path):
         _same(got, python_path(lambda: blk(None, x, None)))
 
 
+@pytest.mark.parametrize("c,heads,rows", [(32, 1, 1024), (256, 8, 1536), (512, 16, 512)])
+def test_block_in_inference_mode(c, heads, rows, monkeypatch):
+    """the driver takes the block there as under no_grad, cold and warm, with equal bits; copies made there serve later calls"""
+    from flash3dtransformer_amd.lib import pshattn
+    taken = []
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(native, name)
+            return f if name == "WeightCache" else lambda *a: (lambda r: (taken.append((name, r is not None)), r)[1])(f(*a))
+    native = pshattn.host()
+    monkeypatch.setattr(pshattn, "_host", Spy())
+    blk, twin = _fresh_block(c, heads), _fresh_block(c, heads)
+    x = torch.randn(rows, c, device=DEV).to(torch.bfloat16)
+    with torch.no_grad():
+        want = twin(None, x, None)
+    with torch.inference_mode():
+        for t in (x, x.clone(), x.clone()):
+            _same(blk(None, t, None).clone(), want)
+    with torch.no_grad():
+        _same(blk(None, x, None), want)
+        blk.mlp.mlp.fc2_bias.add_(1.0)
+        twin.mlp.mlp.fc2_bias.add_(1.0)
+        _same(blk(None, x, None), twin(None, x, None))
+    assert taken and all(t == ("block_infer", True) for t in taken)
+
+
 def test_attention_outside_the_kernels_is_told_apart():
     from flash3dtransformer_amd.layers.buck_swin import BucketSwinAttentionModule
     m = BucketSwinAttentionModule(48, 2, 512).to(DEV)      # 24-wide heads
