@@ -110,7 +110,8 @@ class _Bf16Cache:
             return p.detach().to(torch.bfloat16).contiguous()
         key = (p.data_ptr(), p._version, p.dtype, p.get_device())
         if key != self._key:
-            self._val = p.detach().to(torch.bfloat16).contiguous()
+            with torch.inference_mode(False):      # a copy with a version of its own, whatever mode it is made in
+                self._val = p.detach().to(torch.bfloat16).contiguous()
             self._key = key
         return self._val
 

@@ -36,8 +36,9 @@ def with_last_separator(seps: torch.Tensor, total: int) -> torch.Tensor:
     facts = host_facts(seps)
     key = ("with_last", int(total))
     if key not in facts:
-        out = seps.clone()
-        out.view(torch.int32)[-1] = int(total)
+        with torch.inference_mode(False):      # kept between calls of any mode: a tensor with a version
+            out = seps.clone()
+            out.view(torch.int32)[-1] = int(total)
         if "sizes" in facts:
             sizes = list(facts["sizes"])
             sizes[-1] += int(total) - sum(sizes)
@@ -60,7 +61,10 @@ _HOST_FACTS = {}   # id(separator tensor) -> (weak reference, tensor version, fa
 def host_facts(seps: torch.Tensor) -> dict:
     """Per-tensor memo for values derived from a separator tensor that live on the host.  Keyed by the
     tensor OBJECT (a weak reference proves it is still the same one: a new tensor that happens to reuse
-    the address is a different object) and its version counter (in-place torch ops bump it)."""
+    the address is a different object) and its version counter (in-place torch ops bump it).  A tensor made in inference
+    mode has no version to tell a change by: nothing is remembered for it."""
+    if seps.is_inference():
+        return {}
     key = id(seps)
     hit = _HOST_FACTS.get(key)
     if hit is not None and hit[0]() is seps and hit[1] == seps._version:

@@ -312,6 +312,46 @@ def test_restore_input_order_without_point_features():
     assert torch.equal(out[:c.shape[0]], per_point[idx])
 
 
+@pytest.mark.parametrize("features", [False, True])
+@pytest.mark.parametrize("batch_made_in_inference_mode", [False, True])
+def test_first_forward_in_inference_mode(features, batch_made_in_inference_mode):
+    """a model whose first forward is one under torch.inference_mode gives the bits of no_grad, and serves no_grad and training after"""
+    import copy
+    from flash3dtransformer_amd import layers as L
+    import bench_workloads as synth
+    from flash3dtransformer_amd.psh.bucket_scope import SwinPlan
+    bs = 256
+    torch.manual_seed(5)
+    ln, bn = (lambda ch: L.LayerNorm(ch)), (lambda ch: torch.nn.BatchNorm1d(ch, eps=1e-3))
+    spec = lambda c, h: L.XFMRSpecs(c, 2 * c, h, True, SwinPlan("swin", bs, 1, 0), ln)
+    levels = [L.F3DLevelSpecs([spec(32, 1)], [spec(32, 1)], "mean", bs, ln, None, bn, torch.nn.GELU),
+              L.F3DLevelSpecs([spec(64, 2)], [spec(64, 2)], "max", bs, bn, torch.nn.GELU, ln, None),
+              L.F3DLevelSpecs([spec(128, 4)], [spec(128, 4)], "mean", bs, None, None, None, None)]
+    model = L.Flash3D(levels, bs, 1, 2, in_feat_dim=4 if features else None).to(DEV).eval()
+    twin = copy.deepcopy(model)
+    rng = np.random.default_rng(10)
+    coords, seps = synth.batch_of([rng.normal(0, 10, (n, 3)).astype(np.float32) for n in (9000, 8200)])
+
+    def batch():
+        c = torch.from_numpy(coords).to(DEV)
+        s = torch.from_numpy(seps.view(np.int32)).to(DEV).view(torch.uint32)
+        return c, torch.sin(torch.arange(4 * c.shape[0], device=DEV).view(-1, 4) * 0.37) if features else None, s
+    with torch.inference_mode(batch_made_in_inference_mode):
+        args = batch()
+    with torch.no_grad():
+        want = twin(*batch())
+    with torch.inference_mode():
+        first, second = model(*args), model(*args)
+        assert torch.equal(first, want) and torch.equal(second, want)
+    with torch.no_grad():
+        assert torch.equal(model(*batch()), want)
+        if not batch_made_in_inference_mode:
+            assert torch.equal(model(*args), want)
+    model.train()
+    model(*batch()).float().square().mean().backward()
+    assert all(q.grad is not None for q in model.module_tree.parameters())
+
+
 def test_state_dict_names_match_reference_module_tree():
     """parameter names a reference checkpoint would carry (flash3dxfmr/layers/*.py module attributes;
     TransformerEngine's LayerNormMLP / Linear parameter names)"""

@@ -1,5 +1,6 @@
 """Host-side logic of the layer modules that needs no GPU: when the bf16 weight copies the kernels read are made anew,
 and loading a checkpoint that carries TransformerEngine's per-module `_extra_state` entries."""
+import pytest
 import torch
 
 from flash3dtransformer_amd import layers as L
@@ -141,3 +142,34 @@ def test_pooling_buffers_in_inference_mode():
             sb = make(**how)
             sb.mark_built(seps, 40)
             assert not sb.covers(40) and sb.unpool_ind.shape == (21, 2)
+
+
+@pytest.mark.parametrize("made_in_inference_mode", [False, True])
+def test_separators_in_inference_mode(made_in_inference_mode):
+    """sizes, padded separators and pooled ones of a first call there; what is derived from them has a version and is remembered"""
+    from flash3dtransformer_amd.psh import batching, subbuck
+    with torch.inference_mode(made_in_inference_mode):
+        seps = torch.tensor([3, 40], dtype=torch.int32)
+    with torch.inference_mode():
+        assert batching.host_sizes(seps) == [3, 37] and batching.max_inslen_from_seps(seps) == 37
+        padded = batching.with_last_separator(seps, 48)
+        assert padded.tolist() == [3, 48] and batching.host_sizes(padded) == [3, 45]
+        rows, sizes, cum = subbuck.calc_red_sep_sizes(padded, 2)
+        assert rows == 25 and sizes.tolist() == [2, 23] and cum.tolist() == [2, 25]
+        assert subbuck.calc_red_sep_sizes(padded, 2)[2] is cum and batching.host_facts(cum)["sizes"] == [2, 23]
+        assert (batching.with_last_separator(seps, 48) is padded) == (not made_in_inference_mode)
+        if made_in_inference_mode:      # a change leaves no trace, so sizes are read again
+            seps[1] = 44
+            assert batching.host_sizes(seps) == [3, 41]
+    seps2 = torch.tensor([5], dtype=torch.int32)
+    assert batching.host_facts(seps2) is batching.host_facts(seps2)
+
+
+def test_weight_copies_made_in_inference_mode_have_a_version():
+    cache, p = nn_ops._Bf16Cache(), torch.nn.Parameter(torch.ones(4))
+    with torch.inference_mode():
+        copy = cache.get(p)
+    with torch.no_grad():
+        assert copy._version == 0 and cache.get(p) is copy
+        p.add_(1.0)
+        assert cache.get(p).tolist() == [2.0] * 4
