@@ -28,6 +28,7 @@ class XFMR(_CachedParamModule):
     """mid = proj(attention(qkv(norm(x)))) + x;  out = MLP(mid) + mid   (stage.py:71-102 of the reference).
     Takes the (coord, feat, sep) triplet of the submodule interface and uses only `feat`."""
     NVTX_SCOPE = "XFMR"
+    _host = None      # a block pickled without one makes it in its first inference call
 
     def __init__(self, channels: int, hid_chann: int, num_heads: int, buck_size: int, qkv_bias: bool,
                  swin_plan: bucket_scope.SwinPlan, norm_layer: callable, mlp_activation: str = "swiglu"):
@@ -49,6 +50,8 @@ class XFMR(_CachedParamModule):
         if not (_as_built(qkv, Linear) and _as_built(proj, Linear) and _as_built(ff, LayerNormMLP)) or _global_hooks() \
                 or norm.training or qkv.training or proj.training or ff.training or ff.activation != "swiglu" or f3ddev.get_nvtx():
             return None
+        if self._host is None:
+            self._host = _HostCache()
         rows = x.shape[0]
         params = [norm.weight, norm.bias, qkv.weight, qkv.bias, proj.weight, proj.bias, ff.layer_norm_weight, ff.layer_norm_bias,
                   ff.fc1_weight, ff.fc1_bias, ff.fc2_weight, ff.fc2_bias]

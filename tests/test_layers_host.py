@@ -173,3 +173,26 @@ def test_weight_copies_made_in_inference_mode_have_a_version():
         assert copy._version == 0 and cache.get(p) is copy
         p.add_(1.0)
         assert cache.get(p).tolist() == [2.0] * 4
+
+
+def test_block_pickled_without_the_drivers_cache(monkeypatch):
+    """the state of a block from before there was one; its first inference call makes it"""
+    import pickle
+    from flash3dtransformer_amd.lib import pshattn
+    from flash3dtransformer_amd.psh.bucket_scope import SwinPlan
+
+    class Driver:
+        class WeightCache:
+            pass
+
+        def block_infer(self, cache, x, *rest):
+            return (type(cache).__name__, x)
+    monkeypatch.setattr(pshattn, "_host", Driver())
+    plan = SwinPlan("swin", 512, 1, 0)
+    blk = L.XFMR(64, 256, 2, 512, True, plan, L.LayerNorm).eval()
+    del blk.__dict__["_host"]
+    old = pickle.loads(pickle.dumps(blk))
+    assert "_host" not in old.__dict__
+    x = torch.zeros(512, 64, dtype=torch.bfloat16)
+    for _ in range(2):
+        assert old._whole_block(x, plan.gen_scopes_from_plan(512, "cpu"))[0] == "WeightCache"
