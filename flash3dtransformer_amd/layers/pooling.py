@@ -19,7 +19,7 @@ class SubbuckReduceFunction(Function):
     def forward(ctx, coords, input_feat, seps, subbuck_size, reduction_op, out_alignment=1):
         max_n = f3dbatch.max_inslen_from_seps(seps)
         sb = f3dsubbuck.SubbuckBuffers.create_subbuck_buff(coords, input_feat, seps, subbuck_size,
-                                                           out_alignment=out_alignment, build_follows=True)
+                                                           out_alignment=out_alignment, build_follows=True, builder_fills=True)
         pshattn.batch_subbuck_reduce(coords, input_feat, seps, max_n, subbuck_size, NUM_VOX, sb.bbox_min, sb.bbox_max,
                                      sb.subbuck_id, sb.subbuck_off, sb.reduced_sep, sb.reduced_coord, sb.reduced_feat,
                                      sb.unpool_ind, 1, reduction_op, fill=True)
@@ -67,7 +67,7 @@ class InbucketPoolingLayer(nn.Module):
         feat = feat.contiguous()
         max_n = f3dbatch.max_inslen_from_seps(seps)
         sb = f3dsubbuck.SubbuckBuffers.create_subbuck_buff(coords, feat, seps, self.subbuck_size,
-                                                           out_alignment=self.out_align, build_follows=True)
+                                                           out_alignment=self.out_align, build_follows=True, builder_fills=True)
         pshattn.subbuck_build(coords, seps, max_n, self.subbuck_size, NUM_VOX, sb.subbuck_id, sb.subbuck_off,
                               sb.reduced_sep, sb.reduced_coord, sb.unpool_ind, (sb.bbox_min, sb.bbox_max))
         pshattn.reduce_feat_norm(feat, coords.shape[0], sb.unpool_ind, sb.reduced_feat, self.subbuck_size,

@@ -58,17 +58,18 @@ class SubbuckBuffers:
 
     @staticmethod
     def create_subbuck_buff(coords: torch.Tensor, input_feat: torch.Tensor, seps: torch.Tensor,
-                            subbuck_size=2, out_alignment=1, build_follows=False):
+                            subbuck_size=2, out_alignment=1, build_follows=False, builder_fills=False):
         """Allocation contract of batch_subbuck_reduce (subbuck.py:68-102).  `unpool_ind` MUST be
         prefilled with an index >= N: that marks a slot no point was mapped to.  The reduced length is
         rounded up to `out_alignment` so the next level's attention buckets divide it; the op
         zero-fills the extra rows (the reference leaves them uninitialised).  build_follows: the caller runs the builder on
-        these clouds next and has it fill the box and the map (`fill` of pshattn.subbuck_build); it writes the id of every
-        point of them, so only rows behind them then need clearing."""
+        these clouds next, which writes the id of every point of them; only rows behind them then need clearing.
+        builder_fills: and has it mark the empty slots and set the box (`fill` of pshattn.subbuck_build); neither is then
+        prefilled."""
         total_n, d = coords.shape
         dev = coords.device
         red_len, _, red_sep = calc_red_sep_sizes(seps, subbuck_size)
-        filled = build_follows and red_len > 0
+        filled = builder_fills and red_len > 0
 
         def full(shape, value, dtype):
             return torch.empty(shape, dtype=dtype, device=dev) if filled else torch.full(shape, value, dtype=dtype, device=dev)

@@ -131,6 +131,17 @@ def test_pooling_buffers_cover_rows_only_once_built():
     assert not sb.covers(4006) and not sb.subbuck_id.view(torch.int32).any()
 
 
+def test_pooling_buffers_are_prefilled_unless_the_builder_fills_them():
+    """a caller who runs the builder without `fill` finds the marker of an empty slot in the whole map, and the box set"""
+    for how in ({}, dict(build_follows=True)):
+        for _ in range(3):      # memory that is handed out again holds something
+            junk = [torch.full((2002, 2), 7, dtype=torch.int32), torch.zeros(3, dtype=torch.float16), torch.zeros(3, dtype=torch.float16)]
+            del junk
+            sb = _pool_buffers(4001)[1](**how)
+            assert (sb.unpool_ind.view(torch.int32) == 4004).all() and sb.unpool_ind.shape == (2001, 2)
+            assert sb.bbox_min.tolist() == [-65504.0] * 3 and sb.bbox_max.tolist() == [65504.0] * 3
+
+
 def test_pooling_buffers_in_inference_mode():
     """tensors made there keep no version counter; separators seen before stay usable"""
     from flash3dtransformer_amd.psh import batching
