@@ -391,8 +391,8 @@ def batch_subbuck_reduce(scattered_coord, scattered_feat, batch_sep, instance_ma
     if fill:
         if red_op not in (0, 1, 2, 3):
             raise RuntimeError(f"Unsupported reduction operation id-{red_op}")
-        subbuck_build(scattered_coord, batch_sep, instance_max_N, subbuck_size, num_vox, subbuck_id, subbuck_off,
-                      reduced_batch_sep, reduced_coord, unpool_ind, (bbox_min, bbox_max))
+        _run_builder(dev, scattered_coord, batch_sep, instance_max_N, subbuck_size, num_vox, subbuck_id, subbuck_off,
+                     reduced_batch_sep, reduced_coord, unpool_ind, (bbox_min, bbox_max))
         _check(_load().f3d_reduce_feat(
             _ptr(scattered_feat), scattered_coord.shape[0], scattered_feat.shape[1], _ptr(unpool_ind), unpool_ind.shape[0],
             subbuck_size, red_op, _ptr(reduced_feat), reduced_feat.shape[0], dev, _stream(dev)))
@@ -481,6 +481,15 @@ def subbuck_build(scattered_coord, batch_sep, instance_max_N, subbuck_size, num_
                            f"dim({reduced_coord.shape[1]}) are NOT 3D.")
     if unpool_ind.shape[1] != subbuck_size:
         raise RuntimeError(f"Unpool_ind last dimension({unpool_ind.shape[1]}) != subbucket_size({subbuck_size})")
+    if fill is not None:
+        assert_dtype(list(fill), torch.float16)
+    _run_builder(dev, scattered_coord, batch_sep, instance_max_N, subbuck_size, num_vox, subbuck_id, subbuck_off,
+                 reduced_batch_sep, reduced_coord, unpool_ind, fill)
+
+
+def _run_builder(dev, scattered_coord, batch_sep, instance_max_N, subbuck_size, num_vox, subbuck_id, subbuck_off,
+                 reduced_batch_sep, reduced_coord, unpool_ind, fill):
+    """the builder's call; all but the layout and the device of `fill` has been checked"""
     args = [_ptr(scattered_coord), _ptr(batch_sep), batch_sep.shape[0], scattered_coord.shape[0],
             instance_max_N, subbuck_size, num_vox, _ptr(subbuck_id), _ptr(subbuck_off),
             _ptr(reduced_batch_sep), _ptr(reduced_coord), reduced_coord.shape[0], _ptr(unpool_ind),
@@ -488,9 +497,8 @@ def subbuck_build(scattered_coord, batch_sep, instance_max_N, subbuck_size, num_
     if fill is None:
         _check(_load().f3d_subbuck_build(*args, dev, _stream(dev)))
         return
-    assert_contiguous(list(fill))
+    assert_contiguous(fill)
     assert_same_device([scattered_coord, *fill])
-    assert_dtype(list(fill), torch.float16)
     if any(b.numel() != 3 for b in fill):
         raise RuntimeError("The box holds three coordinates a corner")
     _check(_load().f3d_subbuck_build_filled(*args, _ptr(fill[0]), _ptr(fill[1]), dev, _stream(dev)))
