@@ -436,6 +436,7 @@ class Linear(_CachedParamModule):
     def forward(self, x: torch.Tensor, residual: torch.Tensor = None, act=None, out: torch.Tensor = None,
                 pre_norm=None):
         """`pre_norm`: a LayerNorm-like module (weight, bias, eps) applied to x inside the same kernel"""
+        copies = None
         if act is None and out is None and x.requires_grad and torch.is_grad_enabled() and x.is_cuda and (
                 pre_norm is None or (isinstance(pre_norm, LayerNorm) and self.in_features in pshattn.LN_BWD_WIDTHS)):
             if pre_norm is None:
@@ -447,7 +448,8 @@ class Linear(_CachedParamModule):
                     c.clear()
                 return y
         elif act is None and out is None and pre_norm is None and x.is_cuda and not torch.is_grad_enabled():
-            y = pshattn.host().linear_infer(x, self._w.get(self.weight, self.training), self._b.get(self.bias, self.training), residual)
+            copies = self._w.get(self.weight, self.training), self._b.get(self.bias, self.training)
+            y = pshattn.host().linear_infer(x, *copies, residual)
             if y is not None:
                 return y
         lead = x.shape[:-1]
@@ -469,7 +471,7 @@ class Linear(_CachedParamModule):
             w16, b16 = fresh[0][:2]
             w16t = fresh[1][0] if fresh[1] else None
         else:
-            w16, b16 = self._w.get(self.weight, self.training), self._b.get(self.bias, self.training)
+            w16, b16 = copies or (self._w.get(self.weight, self.training), self._b.get(self.bias, self.training))
         if pre_norm is not None:
             g, b = fresh[0][2:] if fresh is not None and own_norm else norm_params_bf16(pre_norm)
             if isinstance(pre_norm, LayerNorm):     # its bf16 copies are kept between calls, a torch norm's are not

@@ -265,6 +265,22 @@ def test_linear_inference(rows, k, n, residual, python_path):
         _same(run(), python_path(run))
 
 
+@pytest.mark.parametrize("training", [False, True])
+def test_linear_inference_copies_its_parameters_once(training, monkeypatch):
+    """also for an input that the driver declines"""
+    from flash3dtransformer_amd import layers as L
+    from flash3dtransformer_amd.layers import nn_ops
+    asked, get = [], nn_ops._Bf16Cache.get
+    monkeypatch.setattr(nn_ops._Bf16Cache, "get", lambda self, p, t=False: (asked.append(p), get(self, p, t))[1])
+    lin = L.Linear(64, 32).to(DEV).train(training)
+    x = torch.randn(40, 64, device=DEV)
+    with torch.no_grad():
+        want = lin(x.to(torch.bfloat16))
+        asked.clear()
+        assert torch.equal(lin(x), want)
+    assert len(asked) == 2
+
+
 def test_layers_without_columns_raise():
     """no output columns, or no input columns, beside a residual: an error, in training and in inference"""
     from flash3dtransformer_amd import layers as L
