@@ -22,6 +22,8 @@
 //   32 x 128 70 -> 61, 256 x 32 117 -> 101; 241,152 rows 64 x 64 37 -> 30, 512 x 64 118 -> 110; 120,832 rows 1024 x 128 121 -> 115;
 //   5,000 rows 64 x 256 19 -> 14; 30,208 rows 4096 x 512 177 (0.71 PFLOP/s) either way.  Errors against fp64 equal or smaller
 //   (2.8e-7 -> 1.4e-7 of a 32 x 32 gradient).
+#include <algorithm>
+
 #include "f3d_device.h"
 #include "f3d_internal.h"
 
@@ -37,11 +39,16 @@ constexpr int kXcd = 8;
 constexpr int kWgThreads = 512, kWgWaves = kWgThreads / kWave;
 constexpr int kWgNBuf = 4;                   // stage buffers: three stages in flight behind the one being multiplied
 
+// rows of a stage of wn + wk columns: 24 to 40 KB
+constexpr int wg_stage_rows(int wn, int wk) {
+  const int row = 2 * (wn + wk);
+  return row * 256 <= 40960 ? 256 : row * 128 <= 40960 ? 128 : row * 64 <= 40960 ? 64 : 32;
+}
 // A workgroup's tile of dw: WN x WK columns of dy and x (32, 64, 128 or 256 each), MT rows a stage
 template <int WN, int WK>
 struct WgGeom {
   static constexpr int ROW = 2 * (WN + WK);                       // bytes of a row of both operands
-  static constexpr int MT = ROW * 256 <= 40960 ? 256 : ROW * 128 <= 40960 ? 128 : ROW * 64 <= 40960 ? 64 : 32;
+  static constexpr int MT = wg_stage_rows(WN, WK);
   static constexpr int RA = 2 * WN, RB = 2 * WK;                  // bytes of an LDS row, no padding
   static constexpr int TILE_A = MT * RA, STAGE = MT * ROW, LDS = kWgNBuf * STAGE;
   static constexpr int DMA_A = TILE_A / 1024, DMA = STAGE / 1024;             // direct loads (1 KB each) of a stage
@@ -166,7 +173,7 @@ __global__ __launch_bounds__(kWgThreads) void linear_wgrad_kernel(
 
   const uint32_t all_stages = (M + MT - 1) / MT;
   const uint32_t n_stage = all_stages > slab ? (all_stages - slab + slabs - 1) / slabs : 0u;
-// waits until this wave's loads of stage st have landed (at most the loads of the later stages, two of them at
+  // waits until this wave's loads of stage st have landed (at most the loads of the later stages, two of them at
   // that point, stay outstanding), zeroes the rows past the slab, and meets the other waves: after the barrier the
   // whole stage is in LDS and every wave has its operands of the stages before it in registers
   auto stage_ready = [&](uint32_t st) {
@@ -557,7 +564,12 @@ int f3d_linear_wgrad_bf16(const f3d_bf16_t* dy, uint32_t lddy, const f3d_bf16_t*
   if (int rc = n_cu_of(device, &n_cu)) return rc;
   // tile of dw per workgroup: the narrowest width that holds all columns, 256 where none does
   auto width = [](uint32_t c) { return c <= 32u ? 32u : c <= 64u ? 64u : c <= 128u ? 128u : 256u; };
-  const uint32_t wn = width(n), wk = width(k);
+  uint32_t wn = width(n), wk = width(k);
+  // The direct loads take 32-bit byte offsets from a stage's first row.  Rows so far apart that a tall stage does not fit
+  // (8.4 million elements at 256 rows a stage) take the widest tile, whose stages have 32 rows.
+  auto reach = [&](uint32_t rows) { return (uint64_t)(std::min(rows, std::max(m, 1u)) - 1u) * std::max(lddy, ldx) * 2u + 512u; };
+  if (reach((uint32_t)wg_stage_rows((int)wn, (int)wk)) >> 32) wn = wk = 256u;
+  F3D_CHECK_ARG(reach((uint32_t)wg_stage_rows((int)wn, (int)wk)) >> 32 == 0, "rows of %u or %u elements lie too far apart", lddy, ldx);
   const uint32_t n_tiles = cdiv_u32(n, wn), k_tiles = cdiv_u32(k, wk);
   const size_t nk = (size_t)n * k;
   WgLaunch l = {dy, x, lddy, ldx, m, n, k, n_tiles, k_tiles, n_cu, device, db != nullptr, s};

@@ -109,6 +109,21 @@ def test_linear_wgrad_tile_widths(N, K):
             assert ((got - ref).abs() <= M * 2.0 ** -24 * size).all(), (M, N, K)
 
 
+def test_linear_wgrad_rows_far_apart():
+    """row strides at which the 256 rows of a narrow tile's stage span more than 32-bit offsets reach; small integers, exact sums"""
+    from flash3dtransformer_amd.lib import pshattn
+    M, N, K, ld = 300, 32, 24, 8500000
+    g = torch.Generator().manual_seed(1)
+    dy, x = [torch.randint(-3, 4, (M, c), generator=g).to(torch.bfloat16).to(DEV) for c in (N, K)]
+    far = torch.empty((M - 1) * ld + K, dtype=torch.bfloat16, device=DEV).as_strided((M, K), (ld, 1))
+    far.copy_(x)
+    dw, db = torch.full((N, K), 7.0, device=DEV), torch.full((N,), 7.0, device=DEV)
+    pshattn.linear_wgrad_bf16(dy, far, dw, db)
+    assert torch.equal(dw, dy.float().t() @ x.float()) and torch.equal(db, dy.float().sum(0))
+    with pytest.raises(RuntimeError, match="too far apart"):      # 32 rows, the fewest a stage has
+        pshattn.linear_wgrad_bf16(dy[:33], far.as_strided((33, K), (70000000, 1)), dw, db)
+
+
 def test_linear_wgrad_random_shapes():
     """shapes drawn at random (multiples of 8 in n and k, any row count), one of the operands a column slice"""
     from flash3dtransformer_amd.lib import pshattn
