@@ -48,10 +48,10 @@ def test_linear_wgrad_matches_fp64(M, N, K):
 
 @pytest.mark.parametrize("slabs", [1, 16, 17, 64, 65, 129, 200])
 def test_wgrad_partial_sums_by_slab_count(slabs):
-    """slab counts around the sizes at which the summation kernel changes its form; 32-row slabs of small integers, whose
-    products and sums are exact in fp32"""
+    """slab counts around the sizes at which the summation kernel changes its form: a slab of one 128-row stage each (64 x 32
+    tile); small integers, whose products and sums are exact in fp32"""
     from flash3dtransformer_amd.lib import pshattn
-    M, N, K = 32 * slabs - 5, 40, 24
+    M, N, K = 128 * slabs - 5, 40, 24
     g = torch.Generator().manual_seed(slabs)
     dy, x = [torch.randint(-3, 4, (M, c), generator=g).to(torch.bfloat16).to(DEV) for c in (N, K)]
     dw, db = torch.full((N, K), 7.0, device=DEV), torch.full((N,), 7.0, device=DEV)
@@ -61,14 +61,14 @@ def test_wgrad_partial_sums_by_slab_count(slabs):
 
 @pytest.mark.parametrize("slabs", [40, 80, 128, 200])
 def test_wgrad_partial_sums_keep_small_terms_beside_a_large_one(slabs):
-    """one partial of 2^25 and one of 127/128 from every other slab: a summation tree of 16 groups rounds at most
-    slabs / 16 + 15 times next to the large one, by half a unit of its last place (2) each"""
+    """one partial of 2^25 and one of 127/128 from every other slab (one 256-row stage each): a summation tree of 16 groups rounds
+    at most slabs / 16 + 15 times next to the large one, by half a unit of its last place (2) each"""
     from flash3dtransformer_amd.lib import pshattn
-    dy = torch.zeros(32 * slabs, 32, dtype=torch.bfloat16)
-    dy[::32] = 127 / 128
+    dy = torch.zeros(256 * slabs, 32, dtype=torch.bfloat16)
+    dy[::256] = 127 / 128
     dy[0] = 2.0 ** 25
     dw, db = torch.empty(32, 32, device=DEV), torch.empty(32, device=DEV)
-    pshattn.linear_wgrad_bf16(dy.to(DEV), torch.ones(32 * slabs, 32, dtype=torch.bfloat16, device=DEV), dw, db)
+    pshattn.linear_wgrad_bf16(dy.to(DEV), torch.ones(256 * slabs, 32, dtype=torch.bfloat16, device=DEV), dw, db)
     want = 2.0 ** 25 + (slabs - 1) * 127 / 128
     for got in (dw, db):
         assert (got.double() - want).abs().max().item() <= 2 * (slabs / 16 + 15)
@@ -96,17 +96,34 @@ def test_layernorm_backward_partial_rows(blocks):
 @pytest.mark.parametrize("K", [16, 64, 128, 136])
 def test_linear_wgrad_tile_widths(N, K):
     """every width of tile in both operands (32, 64, 128, 256; exact, ragged, several tiles) around its stages of 32 to 256 rows: one
-    row, one row short of a stage, two stages and a row, more stages than slabs.  Sums of M products of at most `top`: M 2^-24
-    of the sum of magnitudes, in a tree that is at most as deep as a plain sum."""
+    row, one row short of a stage, two stages and a row, more stages than slabs.  Integers of at most 3: sums of up to
+    66,567 products are below 2^24, exact in fp32 in any order, so that a row left out or taken twice shows.  And ordinary
+    values, to fp32 accumulation noise."""
     from flash3dtransformer_amd.lib import pshattn
     for M in (1, 255, 513, 256 * 260 + 7 if N * K <= 64 * 64 else 9001):
         g = torch.Generator(device=DEV).manual_seed(M + N + K)
-        dy, x = (torch.randn(M, c, device=DEV, generator=g).to(torch.bfloat16) for c in (N, K))
-        dw, db = torch.full((N, K), 3.0, device=DEV), torch.full((N,), 3.0, device=DEV)
-        pshattn.linear_wgrad_bf16(dy, x, dw, db)
-        for got, ref, size in ((dw.double(), dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()),
-                               (db.double(), dy.double().sum(0), dy.double().abs().sum(0))):
-            assert ((got - ref).abs() <= M * 2.0 ** -24 * size).all(), (M, N, K)
+        for whole in (True, False):
+            dy, x = ((torch.randint(-3, 4, (M, c), device=DEV, generator=g) if whole else torch.randn(M, c, device=DEV, generator=g))
+                     .to(torch.bfloat16) for c in (N, K))
+            dw, db = torch.full((N, K), 3.0, device=DEV), torch.full((N,), 3.0, device=DEV)
+            pshattn.linear_wgrad_bf16(dy, x, dw, db)
+            for got, ref in ((dw.double(), dy.double().t() @ x.double()), (db.double(), dy.double().sum(0))):
+                bound = 0.0 if whole else 1e-5 * ref.abs().max().item() + 1e-6
+                assert (got - ref).abs().max().item() <= bound, (M, N, K, whole)
+
+
+@pytest.mark.parametrize("N,K,stage", [(32, 32, 256), (32, 64, 128), (64, 32, 128), (64, 64, 128), (32, 128, 128), (128, 32, 128)])
+def test_linear_wgrad_many_stages_a_slab(N, K, stage):
+    """tiles whose waves share the rows of a stage, six stages a slab and more, the last one ragged: the four stage buffers come
+    round again.  Integers of at most 3, sums below 2^24: exact"""
+    from flash3dtransformer_amd.lib import pshattn
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    M = stage * (6 * cus + 3) - 5
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    dy, x = (torch.randint(-3, 4, (M, c), device=DEV, generator=g).to(torch.bfloat16) for c in (N, K))
+    dw, db = torch.full((N, K), 3.0, device=DEV), torch.full((N,), 3.0, device=DEV)
+    pshattn.linear_wgrad_bf16(dy, x, dw, db)
+    assert torch.equal(dw.double(), dy.double().t() @ x.double()) and torch.equal(db.double(), dy.double().sum(0))
 
 
 def test_linear_wgrad_rows_far_apart():
