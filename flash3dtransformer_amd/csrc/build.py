@@ -1,6 +1,7 @@
 """Builds flash3dtransformer_amd/lib/libf3d_hip.so from the HIP sources in this directory.
 
     python -m flash3dtransformer_amd.csrc.build        # or: python flash3dtransformer_amd/csrc/build.py
+    python flash3dtransformer_amd/csrc/build.py --c-abi        # the library alone, without the layers' native driver
 
 hipcc cross-compiles for gfx950 without a GPU.  Objects go to csrc/build/, the library next to the
 Python binding so that it travels with the tree.
@@ -59,14 +60,25 @@ def _compile(src, incremental=False):
 
 
 def _build_host(incremental=False):
-    """the layers' native driver: a Python module over torch's C++ API that calls the library beside it"""
+    """the layers' native driver: a Python module over torch's C++ API that calls the library beside it.  None where torch or its
+    headers are absent: the library stands without it, and the layers raise when they miss it"""
     import sysconfig
 
-    import torch
+    try:
+        import torch
+    except ImportError as e:
+        sys.stderr.write(f"the layers' native driver is not built: no torch ({e})\n")
+        return None
+    if not os.path.isdir(os.path.join(os.path.dirname(torch.__file__), "include", "torch")):
+        sys.stderr.write("the layers' native driver is not built: torch comes without its headers\n")
+        return None
+    made_for, stamp = f"{torch.__version__} {int(torch._C._GLIBCXX_USE_CXX11_ABI)}", os.path.join(OBJ_DIR, "f3d_host.torch")
     newest = max(os.path.getmtime(HOST_SRC), os.path.getmtime(os.path.join(os.path.dirname(PKG), "include", "f3d_hip.h")),
                  os.path.getmtime(__file__))
-    if incremental and os.path.exists(HOST_LIB) and os.path.getmtime(HOST_LIB) > newest:
-        return HOST_LIB
+    if incremental and os.path.exists(HOST_LIB) and os.path.getmtime(HOST_LIB) > newest and os.path.exists(stamp):
+        with open(stamp) as f:
+            if f.read() == made_for:
+                return HOST_LIB
     root = os.path.dirname(torch.__file__)
     inc, libs = os.path.join(root, "include"), os.path.join(root, "lib")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
@@ -81,12 +93,15 @@ def _build_host(incremental=False):
         raise RuntimeError(f"g++ failed on {HOST_SRC}:\n{p.stderr}")
     if p.stderr.strip():
         sys.stderr.write(p.stderr + "\n")
+    with open(stamp, "w") as f:
+        f.write(made_for)
     return HOST_LIB
 
 
-def build(verbose=True, jobs=None, incremental=False):
-    """incremental=True keeps objects that are newer than their source, every header and this file (a developer's
-    shortcut: `python -m flash3dtransformer_amd.csrc.build -i`); the default compiles everything."""
+def build(verbose=True, jobs=None, incremental=False, host=True):
+    """incremental=True keeps objects that are newer than their source, every header and this file, and were made for the
+    torch that is there (a developer's shortcut: `python -m flash3dtransformer_amd.csrc.build -i`); the default compiles
+    everything.  host=False leaves the layers' native driver out."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
     srcs = sources()
@@ -97,11 +112,12 @@ def build(verbose=True, jobs=None, incremental=False):
     p = subprocess.run(cmd, capture_output=True, text=True)
     if p.returncode != 0:
         raise RuntimeError(f"link failed:\n{p.stderr}")
-    _build_host(incremental)
+    if host:
+        _build_host(incremental)
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources")
     return LIB
 
 
 if __name__ == "__main__":
-    build(incremental="-i" in sys.argv[1:])
+    build(incremental="-i" in sys.argv[1:], host="--c-abi" not in sys.argv[1:])

@@ -114,3 +114,30 @@ def test_staged_buffer_is_not_kept_by_a_call_that_prepares_nothing(lib):
         assert lib.f3d_stage_weights(at(65536), ctypes.c_size_t(1 << 20), 0) == 0
         assert call()
         assert lib.f3d_staged_weights_kept() == 0
+
+
+def test_library_builds_without_torch(monkeypatch, capsys, tmp_path):
+    """the native driver is left out with a word, where torch is absent or on request; it is compiled anew for another torch"""
+    import subprocess
+    import sys
+
+    import torch
+    from flash3dtransformer_amd.csrc import build
+    ran = []
+    monkeypatch.setattr(subprocess, "run", lambda cmd, **kw: (ran.append(cmd[0]), subprocess.CompletedProcess(cmd, 0, "", ""))[1])
+    monkeypatch.setattr(build, "_compile", lambda src, incremental: src)
+    with monkeypatch.context() as m:
+        m.setitem(sys.modules, "torch", None)
+        build.build(verbose=False)
+    assert ran == ["hipcc"] and "native driver is not built" in capsys.readouterr().err
+    build.build(verbose=False, host=False)
+    assert ran == ["hipcc"] * 2
+    monkeypatch.setattr(build, "OBJ_DIR", str(tmp_path))
+    monkeypatch.setattr(build, "HOST_LIB", os.path.join(build.OBJ_DIR, "_f3d_host.so"))
+    open(build.HOST_LIB, "w").close()
+    os.utime(build.HOST_LIB, (2e9, 2e9))
+    ran.clear()
+    for version in ("2.0", "2.0", "2.1"):
+        monkeypatch.setattr(torch, "__version__", version)
+        build._build_host(incremental=True)
+    assert ran == ["g++", "g++"]
