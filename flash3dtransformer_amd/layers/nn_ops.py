@@ -20,6 +20,7 @@ import torch
 from torch import nn
 
 from ..lib import pshattn
+from ..psh.batching import versioned
 
 
 class _TorchBackward(torch.autograd.Function):
@@ -110,8 +111,7 @@ class _Bf16Cache:
             return p.detach().to(torch.bfloat16).contiguous()
         key = (p.data_ptr(), p._version, p.dtype, p.get_device())
         if key != self._key:
-            with torch.inference_mode(False):      # a copy with a version of its own, whatever mode it is made in
-                self._val = p.detach().to(torch.bfloat16).contiguous()
+            self._val = versioned(lambda: p.detach().to(torch.bfloat16).contiguous())
             self._key = key
         return self._val
 

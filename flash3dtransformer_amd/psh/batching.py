@@ -29,6 +29,14 @@ def max_inslen_from_seps(seps: torch.Tensor) -> int:
     return max(host_sizes(seps))
 
 
+def versioned(make):
+    """make(), whose tensors are kept between calls of any mode: made outside inference mode, so that they have a version"""
+    if not torch.is_inference_mode_enabled():
+        return make()
+    with torch.inference_mode(False):
+        return make()
+
+
 def with_last_separator(seps: torch.Tensor, total: int) -> torch.Tensor:
     """A copy of `seps` whose last entry is `total` (rows appended for alignment are counted into the last cloud).
     The copy is made once per separator tensor and length, and the host-side sizes of the copy are derived from those
@@ -36,9 +44,11 @@ def with_last_separator(seps: torch.Tensor, total: int) -> torch.Tensor:
     facts = host_facts(seps)
     key = ("with_last", int(total))
     if key not in facts:
-        with torch.inference_mode(False):      # kept between calls of any mode: a tensor with a version
+        def extended():
             out = seps.clone()
             out.view(torch.int32)[-1] = int(total)
+            return out
+        out = versioned(extended)
         if "sizes" in facts:
             sizes = list(facts["sizes"])
             sizes[-1] += int(total) - sum(sizes)
@@ -63,13 +73,13 @@ def host_facts(seps: torch.Tensor) -> dict:
     tensor OBJECT (a weak reference proves it is still the same one: a new tensor that happens to reuse
     the address is a different object) and its version counter (in-place torch ops bump it).  A tensor made in inference
     mode has no version to tell a change by: nothing is remembered for it."""
-    if seps.is_inference():
-        return {}
     key = id(seps)
     hit = _HOST_FACTS.get(key)
     if hit is not None and hit[0]() is seps and hit[1] == seps._version:
         return hit[2]
     facts = {}
+    if seps.is_inference():
+        return facts
     _HOST_FACTS[key] = (weakref.ref(seps, lambda _r, k=key, d=_HOST_FACTS: d.pop(k, None)), seps._version, facts)
     return facts
 

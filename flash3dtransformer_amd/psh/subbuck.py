@@ -24,8 +24,7 @@ def calc_red_sep_sizes(seps: torch.Tensor, subbuck_size: int):
             acc += r
             cum.append(acc)
         as_dev = lambda v: torch.tensor(v, dtype=torch.int64).to(seps.dtype).to(seps.device)
-        with torch.inference_mode(False):      # kept between calls of any mode: tensors with a version
-            red_sizes, red_cum = as_dev(red), as_dev(cum)
+        red_sizes, red_cum = f3dbatch.versioned(lambda: (as_dev(red), as_dev(cum)))
         f3dbatch.host_facts(red_cum)["sizes"] = red
         facts[key] = (acc, red_sizes, red_cum)
     return facts[key]
