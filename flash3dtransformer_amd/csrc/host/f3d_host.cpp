@@ -8,7 +8,8 @@
 // argument conversion, autograd functions), more than the kernels of a small model take.
 //
 // Nothing is kept by the address or identity of an input.  A WeightCache keeps copies of parameters between eval-mode
-// forwards under no_grad while their address, version, dtype and device stay, as layers/nn_ops.py does.
+// forwards without gradients (no_grad, inference_mode) while their address, version, dtype and device stay, as
+// layers/nn_ops.py does.
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 

@@ -800,8 +800,8 @@ static int launch_mlp(const uint16_t* x, uint32_t ldx, float eps, const uint16_t
   // Whole turns of the chip run 256-row workgroups; what is left over is spread over all CUs in panels of fewer rows
   // (fewer waves with work per workgroup), so that the last turn is shorter than a full one.  That holds for a call of less
   // than one turn too: four waves or fewer have a SIMD each.  C = 128, weights prepared with it, in us, 256-row panels and now:
-  // 5,632 rows 33.0 -> 24.4, 16,384 rows 33.8 -> 25.3, 32,000 rows 34.9 -> 28.4, 45,000 rows 35.7 -> 34.7; C = 256: 2,816
-  // rows 86.8 -> 60.6, 16,384 rows 88.6 -> 63.5.
+  // 5,632 rows 33.0 -> 24.4, 16,384 rows 33.8 -> 25.3, 32,000 rows 34.9 -> 28.4, 45,000 rows 35.7 -> 34.7; C = 256 (which the
+  // layers send here below 30,000 rows on request only): 2,816 rows 86.8 -> 60.6, 16,384 rows 88.6 -> 63.5.
   static int cus[64] = {};
   int n_cu = 256;
   if (device >= 0 && device < 64) {

@@ -231,7 +231,7 @@ int launch_ystat_linear(const uint16_t* x, uint32_t ldx, const uint16_t* w, cons
   auto cost = [](uint64_t panels, uint32_t weight) { return (panels + 255) / 256 * weight; };
   const uint64_t wide = N % 256 == 0 ? cost((uint64_t)rows2 * (N / 256), 20) : ~0ull;
   const uint64_t tall = cost((uint64_t)rows2 * (N / 128), 15), small = cost((uint64_t)rows1 * (N / 128), 11);
-  // Fewer than half as many 128 x 128 panels as CUs: 128 x 64 ones, three quarters of the bytes a chunk and twice the CUs that
+  // Up to half as many 128 x 128 panels as an MI355X has CUs (256): 128 x 64 ones, three quarters of the bytes a chunk and twice the CUs that
   // ask for them.  K = 2048, N = 512, in us: 1,536 rows 22.0 -> 19.5, 4,096 rows 23.3 -> 20.6, but 8,192 rows 29 -> 39 (two
   // rounds); K = 1024, N = 256: 5,632 rows 12.7 -> 11.4.
   if (!in_place && 2u * (uint64_t)rows1 * (N / 128) <= 256)

@@ -118,7 +118,7 @@ class _Bf16Cache:
 
 class _StagedWeights:
     """Device buffer in which a dense kernel keeps the weights it prepares per call (LayerNorm folded into the weight
-    and bias, fragment-major copies) between eval-mode forwards under no_grad.  The buffer is current while the bf16
+    and bias, fragment-major copies) between eval-mode forwards without gradients.  The buffer is current while the bf16
     tensors it was made from are the same storage at the same version (the entry holds them, so their memory cannot
     be handed out again meanwhile); dropped together with the bf16 copies (train() / eval(), load_state_dict,
     refresh_weights())."""
@@ -712,7 +712,11 @@ class LayerNormMLP(_CachedParamModule):
         # activations [rows, ffn_hidden_size] are then never allocated.  None (default): where it is the faster path on
         # MI355X (measured against LayerNorm+fc1+gate followed by fc2+residual, hidden = 4 x width: widths 32 and 64
         # at every row count, 27 % faster at 3 k rows and 2.2 to 2.9 x at 0.5 to 1 M rows; width 128 at every row
-        # count, 19 to 41 % faster; width 256 from 32 k rows up, 6 to 23 % faster, and 11 % slower at 16 k rows)
+        # count, 19 to 41 % faster; width 256 from 30 k rows up).  Width 256, weights prepared before, one kernel / two in us:
+        # 5,632 rows 47.6 / 28.9, 16,384 rows 50.8 / 42.9, 20,480 rows 52.1 / 51.5, 28,000 rows 54.2 / 63.9, 32,768 rows
+        # 58.1 / 69.9, 81,920 rows 145 / 189; with the out-projection in front 16,384 rows 57.8 / 54.6, 20,480 rows 57.6 / 63.8,
+        # 28,000 rows 60.9 / 79.9.  The line of 30 k rows is older than the one kernel's panels of fewer rows, with which
+        # it is ahead from about 20,000 rows (18,000 with the projection): between the two, `fused=True` is the faster choice
         self.fused = fused
         assert activation in ("swiglu", "gelu")
         self.hidden_size, self.ffn_hidden_size, self.activation, self.eps = hidden_size, ffn_hidden_size, activation, eps
