@@ -50,6 +50,13 @@ Tensor bf16_rows(const Tensor& t) {      // bf16 with unit column stride
   Tensor r = t.scalar_type() == at::kBFloat16 ? t : t.to(at::kBFloat16);
   return r.stride(-1) == 1 ? r : r.contiguous();
 }
+// an output's gradient for the kernels, as autograd hands it over (a column slice of a wider one, one row expanded to all):
+// copied where its rows are not at multiples of 16 bytes, each with a place of its own
+Tensor grad_rows(const Tensor& t) {
+  const Tensor r = bf16_rows(t);
+  const bool readable = r.stride(0) >= r.size(1) && r.stride(0) % 8 == 0 && ((uintptr_t)r.data_ptr() & 15u) == 0;
+  return readable ? r : r.clone(at::MemoryFormat::Contiguous);
+}
 bool master(const Tensor& p, const Tensor& x, at::IntArrayRef shape) {      // an fp32 parameter this module takes
   return !p.defined() || (p.scalar_type() == at::kFloat && p.device() == x.device() && p.is_contiguous() && p.sizes() == shape);
 }
@@ -207,7 +214,7 @@ struct LinearNode : torch::autograd::Function<LinearNode> {
     const Tensor &x = s[0], &weight = s[1], &bias = s[2], &residual = s[3], &ln_w = s[4], &ln_b = s[5], &g16 = s[6], &b16 = s[7], &wt = s[8];
     const Wanted want(ctx, "edges");
     const double eps = ctx->saved_data["eps"].toDouble();
-    const Tensor dy = bf16_rows(grads[0]), x2 = bf16_rows(x);
+    const Tensor dy = grad_rows(grads[0]), x2 = bf16_rows(x);
     const int64_t m = x2.size(0), k = x2.size(1), n = dy.size(1);
     Tensor h = x2;
     if (ln_w.defined()) {
@@ -256,7 +263,7 @@ struct ForkNode : torch::autograd::Function<ForkNode> {
     const Tensor &x = s[0], &weight = s[1], &bias = s[2], &ln_w = s[3], &ln_b = s[4], &g16 = s[5], &b16 = s[6], &wt = s[7];
     const Wanted want(ctx, "edges");
     const double eps = ctx->saved_data["eps"].toDouble();
-    const Tensor dy = bf16_rows(grads[0]), dres = bf16_rows(grads[1]), x2 = bf16_rows(x);
+    const Tensor dy = grad_rows(grads[0]), dres = grad_rows(grads[1]), x2 = bf16_rows(x);
     const int64_t m = x2.size(0), k = x2.size(1), n = dy.size(1);
     const Tensor h = empty_like_device({m, k}, at::kBFloat16, x2);
     layernorm(x2.contiguous(), g16, b16, h, eps);
@@ -330,7 +337,7 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
                  &be16 = s[9], &w1_16 = s[10], &b1_16 = s[11], &w1t = s[12], &w2t = s[13];
     const Wanted want(ctx, "edges");
     const double eps = ctx->saved_data["eps"].toDouble();
-    const Tensor dy = bf16_rows(grads[0]), x2 = bf16_rows(x).contiguous();
+    const Tensor dy = grad_rows(grads[0]), x2 = bf16_rows(x).contiguous();
     const int64_t m = x2.size(0), c = x2.size(1), hid = w2.size(1);
     const Tensor h = empty_like_device({m, c}, at::kBFloat16, x2);
     layernorm(x2, g16, be16, h, eps);

@@ -255,6 +255,15 @@ def as_bf16_2d(x: torch.Tensor) -> torch.Tensor:
     return x
 
 
+def _grad_rows(g: torch.Tensor) -> torch.Tensor:
+    """an output's gradient for the kernels, as autograd hands it over (a column slice of a wider one, one row expanded to all):
+    copied where its rows are not at multiples of 16 bytes, each with a place of its own"""
+    g = as_bf16_2d(g)
+    if g.stride(0) >= g.shape[1] and g.stride(0) % 8 == 0 and g.data_ptr() % 16 == 0:
+        return g
+    return g.clone(memory_format=torch.contiguous_format)
+
+
 def _fresh_copies(caches, params, transposed=(), apart=()):
     """bf16 copies of a layer's parameters for a forward that records gradients (they are made anew on every such forward,
     as _Bf16Cache does), in one launch, with the transposed copies that the backward multiplies with; a forward whose backward
@@ -300,7 +309,7 @@ class _LayerNormGrad(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, weight, bias, g16 = ctx.saved_tensors
-        dx, dg, db = _ln_backward(as_bf16_2d(x), as_bf16_2d(dy.reshape(x.shape)), g16, None, ctx.eps)
+        dx, dg, db = _ln_backward(as_bf16_2d(x), _grad_rows(dy.reshape(x.shape)), g16, None, ctx.eps)
         return (None, _grad_out(dx, x) if ctx.needs_input_grad[1] else None,
                 _grad_out(dg, weight) if ctx.needs_input_grad[2] else None,
                 _grad_out(db, bias) if bias is not None and ctx.needs_input_grad[3] else None, None, None)
@@ -321,7 +330,7 @@ class _LinearGrad(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight, bias, residual, ln_w, ln_b, w16, g16, b16, w16t = ctx.saved_tensors
         need = ctx.needs_input_grad
-        dy2 = as_bf16_2d(dy)
+        dy2 = _grad_rows(dy)
         x2 = as_bf16_2d(x)
         m, k = x2.shape
         n = dy2.shape[1]
@@ -369,7 +378,7 @@ class _GatedMLPGrad(torch.autograd.Function):
     def backward(ctx, dy):
         x, residual, ln_w, ln_b, w1, b1, w2, b2, g16, be16, w1_16, b1_16, w2_16, w1t, w2t = ctx.saved_tensors
         need = ctx.needs_input_grad
-        dy2 = as_bf16_2d(dy)
+        dy2 = _grad_rows(dy)
         x2 = as_bf16_2d(x).contiguous()
         m, c = x2.shape
         hid = w2.shape[1]

@@ -281,6 +281,34 @@ def test_linear_inference_copies_its_parameters_once(training, monkeypatch):
     assert len(asked) == 2
 
 
+@pytest.mark.parametrize("layout", ["one row for all", "columns of 67", "columns at 3"])
+@pytest.mark.parametrize("kind", ["linear", "norm_linear", "residual_linear", "mlp", "norm", "block", "no dx"])
+def test_gradients_in_any_layout(kind, layout, python_path):
+    """what autograd hands to a layer's backward behind a sum over the rows or a concatenation of columns: an expanded row, rows at
+    an odd stride, rows off 16 bytes.  The gradients of the same values in a tensor of their own, by either path"""
+    from flash3dtransformer_amd import layers as L
+    from flash3dtransformer_amd.psh.bucket_scope import SwinPlan
+    torch.manual_seed(7)
+    C, rows = 64, 512
+    lin, norm, mlp = L.Linear(C, C).to(DEV), L.LayerNorm(C).to(DEV), L.LayerNormMLP(C, 2 * C).to(DEV)
+    blk = L.XFMR(C, 4 * C, 2, 512, True, SwinPlan("swin", 512, 1, 0), lambda ch: L.LayerNorm(ch)).to(DEV)
+    module, call = {"linear": (lin, lin), "norm_linear": (nn.ModuleList([lin, norm]), lambda t: lin(t, pre_norm=norm)),
+                    "residual_linear": (lin, lambda t: lin(t, residual=t)), "mlp": (mlp, lambda t: mlp(t, residual=t)), "norm": (norm, norm),
+                    "block": (blk, lambda t: blk(None, t, None)), "no dx": (lin, lambda t: lin(t.detach()))}[kind]
+    x = torch.randn(rows, C, device=DEV).to(torch.bfloat16)
+    wide = torch.randn(rows, C + 3, device=DEV).to(torch.bfloat16)
+    g = {"one row for all": wide[0, :C].expand(rows, C), "columns of 67": wide[:, :C], "columns at 3": wide[:, 3:]}[layout]
+
+    def step(grad):
+        t = x.clone().requires_grad_()
+        module.zero_grad(set_to_none=True)
+        call(t).backward(grad)
+        return ([] if kind == "no dx" else [t.grad]) + [p.grad for p in module.parameters()]
+    want = step(g.contiguous())
+    _same(step(g), want)
+    _same(python_path(lambda: step(g)), python_path(lambda: step(g.contiguous())))
+
+
 def test_layers_without_columns_raise():
     """no output columns, or no input columns, beside a residual: an error, in training and in inference"""
     from flash3dtransformer_amd import layers as L
