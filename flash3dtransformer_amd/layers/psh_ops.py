@@ -7,7 +7,7 @@ from torch import nn
 from ..lib import pshattn
 from ..psh import arithmatic as f3darith
 from ..psh import psh_main as pm
-from .nn_ops import CoordEmbedding, Linear, torch_backward
+from .nn_ops import CoordEmbedding, Linear, _grad_rows, torch_backward
 
 
 class _PermuteRows(torch.autograd.Function):
@@ -64,9 +64,7 @@ class _CoordEmbedGrad(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         weight, bias, coord = ctx.saved_tensors
-        dy2 = dy if dy.dtype == torch.bfloat16 else dy.to(torch.bfloat16)
-        if dy2.stride(-1) != 1:
-            dy2 = dy2.contiguous()
+        dy2 = _grad_rows(dy)
         c8 = torch.zeros(coord.shape[0], 8, dtype=torch.bfloat16, device=coord.device)
         c8[:, :3] = coord
         dw8 = torch.empty(weight.shape[0], 8, dtype=torch.float32, device=coord.device)

@@ -282,7 +282,7 @@ def test_linear_inference_copies_its_parameters_once(training, monkeypatch):
 
 
 @pytest.mark.parametrize("layout", ["one row for all", "columns of 67", "columns at 3"])
-@pytest.mark.parametrize("kind", ["linear", "norm_linear", "residual_linear", "mlp", "norm", "block", "no dx"])
+@pytest.mark.parametrize("kind", ["linear", "norm_linear", "residual_linear", "mlp", "norm", "block", "no dx", "embedding"])
 def test_gradients_in_any_layout(kind, layout, python_path):
     """what autograd hands to a layer's backward behind a sum over the rows or a concatenation of columns: an expanded row, rows at
     an odd stride, rows off 16 bytes.  The gradients of the same values in a tensor of their own, by either path"""
@@ -292,7 +292,9 @@ def test_gradients_in_any_layout(kind, layout, python_path):
     C, rows = 64, 512
     lin, norm, mlp = L.Linear(C, C).to(DEV), L.LayerNorm(C).to(DEV), L.LayerNormMLP(C, 2 * C).to(DEV)
     blk = L.XFMR(C, 4 * C, 2, 512, True, SwinPlan("swin", 512, 1, 0), lambda ch: L.LayerNorm(ch)).to(DEV)
-    module, call = {"linear": (lin, lin), "norm_linear": (nn.ModuleList([lin, norm]), lambda t: lin(t, pre_norm=norm)),
+    emb, seps = L.PSH3DCoordEmbedding(C, 16, rows).to(DEV), torch.tensor([rows], dtype=torch.int32, device=DEV).view(torch.uint32)
+    coords = torch.rand(rows, 3, device=DEV).half()
+    module, call = {"embedding": (emb, lambda t: emb(coords, seps, 1)), "linear": (lin, lin), "norm_linear": (nn.ModuleList([lin, norm]), lambda t: lin(t, pre_norm=norm)),
                     "residual_linear": (lin, lambda t: lin(t, residual=t)), "mlp": (mlp, lambda t: mlp(t, residual=t)), "norm": (norm, norm),
                     "block": (blk, lambda t: blk(None, t, None)), "no dx": (lin, lambda t: lin(t.detach()))}[kind]
     x = torch.randn(rows, C, device=DEV).to(torch.bfloat16)
@@ -303,7 +305,7 @@ def test_gradients_in_any_layout(kind, layout, python_path):
         t = x.clone().requires_grad_()
         module.zero_grad(set_to_none=True)
         call(t).backward(grad)
-        return ([] if kind == "no dx" else [t.grad]) + [p.grad for p in module.parameters()]
+        return ([] if kind in ("no dx", "embedding") else [t.grad]) + [p.grad for p in module.parameters()]
     want = step(g.contiguous())
     _same(step(g), want)
     _same(python_path(lambda: step(g)), python_path(lambda: step(g.contiguous())))
