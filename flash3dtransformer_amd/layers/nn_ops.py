@@ -220,8 +220,9 @@ class _CachedParamModule(nn.Module):
 
     def _load_from_state_dict(self, state_dict, prefix, *args, **kwargs):
         # TransformerEngine modules of the reference store one `_extra_state` entry each (fp8 recipe state, of no use
-        # to a bf16 kernel): dropped, so that such a checkpoint loads with strict=True
-        state_dict.pop(prefix + "_extra_state", None)
+        # to a bf16 kernel): dropped, so that such a checkpoint loads with strict=True; a subclass that takes one keeps it
+        if type(self).set_extra_state is nn.Module.set_extra_state:
+            state_dict.pop(prefix + "_extra_state", None)
         self.refresh_weights()
         return super()._load_from_state_dict(state_dict, prefix, *args, **kwargs)
 

@@ -207,3 +207,22 @@ def test_block_pickled_without_the_drivers_cache(monkeypatch):
     x = torch.zeros(512, 64, dtype=torch.bfloat16)
     for _ in range(2):
         assert old._whole_block(x, plan.gen_scopes_from_plan(512, "cpu"))[0] == "WeightCache"
+
+
+def test_extra_state_of_a_subclass_is_loaded():
+    """layers drop the entry TransformerEngine's modules store, but not that of a subclass that has one of its own"""
+    from flash3dtransformer_amd.psh.bucket_scope import SwinPlan
+
+    class Counting(L.XFMR):
+        steps = 0
+
+        def get_extra_state(self):
+            return {"steps": self.steps}
+
+        def set_extra_state(self, state):
+            self.steps = state["steps"]
+    make = lambda: Counting(32, 64, 1, 512, True, SwinPlan("swin", 512, 1, 0), L.LayerNorm)
+    a, b = make(), make()
+    a.steps = 5
+    b.load_state_dict(a.state_dict())
+    assert b.steps == 5
