@@ -1,6 +1,7 @@
 """The native driver of the layers against the layers' own Python code: the same kernels in the same order on the same
 operands, so every output and gradient is compared bit for bit."""
 import copy
+import gc
 
 import pytest
 import torch
@@ -204,10 +205,11 @@ def test_block_after_a_call_that_ran_out_of_memory(python_path):
     with torch.no_grad():
         big = torch.zeros(rows, 512, dtype=torch.bfloat16, device=DEV)
         torch.cuda.synchronize()
+        gc.collect()
         torch.cuda.empty_cache()
         room = rows * (3 * 512 * 2 + 3 * 512 * 2 + 16 * 4) + (64 << 20)      # qkv; o, mid, y; lse; weight copies
         total = torch.cuda.get_device_properties(0).total_memory
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / total)
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_allocated() + room) / total)      # the call needs 200 MB more
         try:
             with pytest.raises(torch.cuda.OutOfMemoryError):
                 blk(None, big, None)
